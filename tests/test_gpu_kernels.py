@@ -983,6 +983,32 @@ def test_seeded_sampling_matches_the_plain_sampler(vocab):
             assert edge <= 1e-4 * total, f"row {r}: kernel {got[r]}, plain {tok}, u {u}"
 
 
+@pytest.mark.parametrize("vocab", [1, 3, 1023, 1025, 16384, 16385, 32769, 50257, 53249, 65536, 65537])
+def test_sampling_from_held_rows(vocab):
+    """Rows of up to 65,536 logits are held in registers, 1 to 64 a thread; longer ones are read again.  The lists of the
+    two searches, their ends, ties, infinities and a temperature that makes different logits equal."""
+    g = torch.Generator().manual_seed(vocab)
+    opts = [(0.8, 0, 1.0), (0.7, 50, 0.95), (1.0, 1, 1.0), (1.3, 0, 0.9), (0.5, 0, 0.05), (3.9, 512, 0.99), (1.0, 513, 1.0),
+            (5.0, 20, 1.0), (1e9, 3, 1.0), (0.9, vocab, 0.5), (0.9, max(vocab - 1, 1), 0.5), (1.0, 40, 1.0)]
+    m = 3 * len(opts)
+    logits = rnd(g, m, vocab, scale=2.0)
+    logits[len(opts):2 * len(opts)] = (logits[len(opts):2 * len(opts)] * 4).round() / 4          # ties, lists too long
+    low = logits[2 * len(opts):]
+    low[torch.rand(low.shape, generator=g) < 0.5] = float("-inf")                                # masked rows
+    low[:, -1] = 1.5
+    temps, top_k, top_p = (list(x) * 3 for x in zip(*opts))
+    seeds, idx = list(range(7, 7 + m)), [5 * i for i in range(m)]
+    got = _sample(logits, temps, top_k, top_p, seeds, idx, engine_seed=11)
+    assert got == _sample(logits, temps, top_k, top_p, seeds, idx, engine_seed=11)
+    for r in range(m):
+        u = P.plain_uniform(11, seeds[r], idx[r])
+        tok, lo, hi, total = P.plain_sample(logits[r].numpy(), temps[r], top_k[r] or None,
+                                            top_p[r] if top_p[r] < 1 else None, u)
+        if got[r] != tok:      # sums of float32: u must sit on a boundary, as above
+            edge = min(abs(u * total - lo), abs(u * total - hi))
+            assert edge <= 1e-4 * total, f"row {r}: kernel {got[r]}, plain {tok}, u {u}, options {opts[r % len(opts)]}"
+
+
 def test_reference_vectors_top_k_top_p():
     # reference tests/test_sampling.py:25-38
     logits = torch.tensor([[1.0, 5.0, 3.0, 2.0, 4.0]] * 64)

@@ -1,0 +1,302 @@
+// out[n, o] = sum_k A[n, k] W[o, k] (+ bias[o]) with an optional GELU-tanh, squared-relu or residual-add epilogue, all in
+// 32 bits on the matrix cores (v_mfma_f32_16x16x4_f32: float32 products and sums): the product of the true 32-bit path
+// (reference: src/minigpt_infer/model.py:43-44,96-101).
+//
+// The order of an element's sum depends on nothing but k, so that a token's logits are the same bits however the tokens
+// were cut into steps: k is cut into blocks of 256; a block's sum runs over groups of 16 k from zero, a group as four
+// matrix instructions of which the i-th takes k = i, 4 + i, 8 + i, 12 + i (what a lane loads as one 16-byte piece serves
+// all four); the blocks' sums are added up in order, then the bias.  What is missing to a group counts as zeros.  All
+// kernels below keep to that, whatever their tiles, and whether one wave has all blocks of an element or each wave some.
+#include "common.h"
+#include "linear_exact.h"
+
+#define EPI_NONE 0
+#define EPI_GELU 1
+#define EPI_RESIDUAL 2  // out += result
+#define EPI_RELU2 5     // max(result, 0)^2
+
+#define EX_BLOCK 256    // k of a block
+#define EX_GROUP 16     // k of a group
+
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float ex_f4;
+
+template <int EPI>
+__device__ __forceinline__ float ex_epilogue(float v, float old) {
+  if (EPI == EPI_GELU) return gelu_tanh(v);
+  if (EPI == EPI_RELU2) return relu_squared(v);
+  if (EPI == EPI_RESIDUAL) return old + v;
+  return v;
+}
+
+// Four k of a row from k on; those at or beyond k_dim count as zero.  VEC: rows are 16-byte aligned and k_dim is a multiple
+// of 4.
+template <bool VEC>
+__device__ __forceinline__ ex_f4 ex_load(const float* __restrict__ row, int k, int k_dim) {
+  ex_f4 v = {0.f, 0.f, 0.f, 0.f};
+  if (VEC) {
+    if (k < k_dim) v = *reinterpret_cast<const ex_f4*>(row + k);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (k + i < k_dim) v[i] = row[k + i];
+  }
+  return v;
+}
+
+// Many rows: a workgroup of four waves per tile of 32 T rows x 32 T columns, a wave 16 T x 16 T of them; steps of 32 k
+// through two buffers of LDS, rows of 128 bytes whose 16-byte pieces are XORed with the row's low bits.  The matrix
+// cores' float32 rate (a sixteenth of bfloat16's) is what bounds it, with T = 4 from about 256 tiles on.
+#define EX_BK 32
+template <int T, int EPI, bool VEC>
+__global__ __launch_bounds__(256) void linear_exact_tile_kernel(
+    const float* __restrict__ A, long lda, const float* __restrict__ W, const float* __restrict__ bias,
+    float* __restrict__ out, long ldo, int n_rows, int n_out, int k_dim, int row_tiles, int vec_out) {
+  constexpr int B = 32 * T;                          // rows and columns of the tile
+  constexpr int PIECES = B * EX_BK / 4 / 256;        // 16-byte pieces of one operand's slice that a thread stages
+  extern __shared__ __align__(16) float ex_lds[];    // [2][2 B][EX_BK]: rows of activations, then of W
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int row0 = (int)(blockIdx.x % row_tiles) * B, col0 = (int)(blockIdx.x / row_tiles) * B;
+  const int wr = (wave & 1) * 16 * T, wc = (wave >> 1) * 16 * T;
+  const int l16 = lane & 15, lk = lane >> 4;
+
+  // rows past the end are read from the last one: their results are never stored
+  constexpr int ROW = EX_BK / 4, STEP = 256 / ROW;   // pieces of a row, rows that 256 threads stage at a time
+  const int srow = tid / ROW, sc = tid % ROW;        // this thread's piece of a slice: row srow + STEP p
+  const float* ap[PIECES];
+  const float* wp[PIECES];
+#pragma unroll
+  for (int p = 0; p < PIECES; ++p) {
+    const int r = row0 + srow + STEP * p, c = col0 + srow + STEP * p;
+    ap[p] = A + (long)(r < n_rows ? r : n_rows - 1) * lda;
+    wp[p] = W + (long)(c < n_out ? c : n_out - 1) * k_dim;
+  }
+  const int s_lds = srow * EX_BK + ((sc ^ (srow & 7)) << 2);
+  ex_f4 ga[PIECES], gw[PIECES];
+  auto load = [&](int k0) {
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p) {
+      ga[p] = ex_load<VEC>(ap[p], k0 + 4 * sc, k_dim);
+      gw[p] = ex_load<VEC>(wp[p], k0 + 4 * sc, k_dim);
+    }
+  };
+  auto store = [&](int buf) {
+    float* dst = ex_lds + buf * (2 * B * EX_BK) + s_lds;
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p) {
+      *reinterpret_cast<ex_f4*>(dst + STEP * p * EX_BK) = ga[p];
+      *reinterpret_cast<ex_f4*>(dst + (B + STEP * p) * EX_BK) = gw[p];
+    }
+  };
+
+  ex_f4 acc[T][T], sum[T][T];                        // [column tile][row tile]: the block's sum, the blocks' sum
+#pragma unroll
+  for (int i = 0; i < T; ++i)
+#pragma unroll
+    for (int j = 0; j < T; ++j) acc[i][j] = sum[i][j] = (ex_f4){0.f, 0.f, 0.f, 0.f};
+
+  load(0);
+  store(0);
+  __syncthreads();
+  for (int k0 = 0, buf = 0; k0 < k_dim; k0 += EX_BK, buf ^= 1) {
+    const bool more = k0 + EX_BK < k_dim;
+    if (more) load(k0 + EX_BK);
+    const float* as = ex_lds + buf * (2 * B * EX_BK) + (wr + l16) * EX_BK;
+    const float* ws = ex_lds + buf * (2 * B * EX_BK) + (B + wc + l16) * EX_BK;
+#pragma unroll
+    for (int g = 0; g < EX_BK / EX_GROUP; ++g) {
+      const int piece = ((4 * g + lk) ^ (l16 & 7)) << 2;
+      ex_f4 af[T], wf[T];
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        af[t] = *reinterpret_cast<const ex_f4*>(as + t * 16 * EX_BK + piece);
+        wf[t] = *reinterpret_cast<const ex_f4*>(ws + t * 16 * EX_BK + piece);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < T; ++i)
+#pragma unroll
+          for (int j = 0; j < T; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[i][e], af[j][e], acc[i][j], 0, 0, 0);
+    }
+    if (((k0 + EX_BK) & (EX_BLOCK - 1)) == 0 || !more) {
+#pragma unroll
+      for (int i = 0; i < T; ++i)
+#pragma unroll
+        for (int j = 0; j < T; ++j) {
+          sum[i][j] += acc[i][j];
+          acc[i][j] = (ex_f4){0.f, 0.f, 0.f, 0.f};
+        }
+    }
+    if (more) store(buf ^ 1);
+    __syncthreads();
+  }
+
+  // a lane has four consecutive columns of a row
+#pragma unroll
+  for (int j = 0; j < T; ++j) {
+    const int r = row0 + wr + 16 * j + l16;
+    if (r >= n_rows) continue;
+#pragma unroll
+    for (int i = 0; i < T; ++i) {
+      const int c = col0 + wc + 16 * i + 4 * lk;
+      float* dst = out + (long)r * ldo + c;
+      if (vec_out && c + 4 <= n_out) {
+        ex_f4 v = sum[i][j];
+        if (bias) v += *reinterpret_cast<const ex_f4*>(bias + c);
+        ex_f4 old = {0.f, 0.f, 0.f, 0.f};
+        if (EPI == EPI_RESIDUAL) old = *reinterpret_cast<const ex_f4*>(dst);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = ex_epilogue<EPI>(v[e], old[e]);
+        *reinterpret_cast<ex_f4*>(dst) = v;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (c + e < n_out) {
+            float v = sum[i][j][e];
+            if (bias) v += bias[c + e];
+            dst[e] = ex_epilogue<EPI>(v, EPI == EPI_RESIDUAL ? dst[e] : 0.f);
+          }
+      }
+    }
+  }
+}
+
+// Few rows, or a product whose tiles would leave compute units idle: a workgroup per 16 rows x 16 columns, each of its
+// waves on blocks of its own (wave w: blocks w, w + waves, ...), operands straight from memory; the blocks' sums meet in
+// LDS and are added up in order.  Four groups of a block are loaded while the four before are multiplied.  Nothing is
+// shared between waves, so beyond a few dozen rows its loads bound it, at 33 TFLOP/s.
+template <int EPI, bool VEC>
+__global__ __launch_bounds__(1024) void linear_exact_rows_kernel(
+    const float* __restrict__ A, long lda, const float* __restrict__ W, const float* __restrict__ bias,
+    float* __restrict__ out, long ldo, int n_rows, int n_out, int k_dim, int row_tiles) {
+  constexpr int N = 256;                             // elements of the tile
+  constexpr int U = 4;                               // groups on their way
+  extern __shared__ __align__(16) float ex_lds[];    // [waves][N]
+  const int tid = threadIdx.x, lane = tid & 63, waves = blockDim.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int row0 = (int)(blockIdx.x % row_tiles) * 16, col0 = (int)(blockIdx.x / row_tiles) * 16;
+  const int l16 = lane & 15, lk = lane >> 4;
+  const int blocks = (k_dim + EX_BLOCK - 1) / EX_BLOCK;
+  const int lr = row0 + l16, lc = col0 + l16;
+  const float* ap = A + (long)(lr < n_rows ? lr : n_rows - 1) * lda;
+  const float* wp = W + (long)(lc < n_out ? lc : n_out - 1) * k_dim;
+
+  // element e of the tile: row e / 16, column e % 16; a thread adds up e = tid, tid + threads, ...
+  float total[N / 64] = {0.f, 0.f, 0.f, 0.f};
+  for (int b0 = 0; b0 < blocks; b0 += waves) {
+    const int b = b0 + wave;
+    ex_f4 acc = {0.f, 0.f, 0.f, 0.f};
+    if (b < blocks) {
+      const int kb = b * EX_BLOCK + 4 * lk;
+      ex_f4 af[2][U], wf[2][U];
+      auto load = [&](int set, int k) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          wf[set][u] = ex_load<VEC>(wp, k + u * EX_GROUP, k_dim);
+          af[set][u] = ex_load<VEC>(ap, k + u * EX_GROUP, k_dim);
+        }
+      };
+      load(0, kb);
+#pragma unroll
+      for (int q = 0; q < EX_BLOCK / EX_GROUP / U; ++q) {
+        if (q + 1 < EX_BLOCK / EX_GROUP / U) load((q + 1) & 1, kb + (q + 1) * U * EX_GROUP);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[q & 1][u][e], af[q & 1][u][e], acc, 0, 0, 0);
+      }
+    }
+    if (b0) __syncthreads();                         // the round before has been added up
+    *reinterpret_cast<ex_f4*>(ex_lds + wave * N + l16 * 16 + 4 * lk) = acc;
+    __syncthreads();
+    const int here = blocks - b0 < waves ? blocks - b0 : waves;
+#pragma unroll
+    for (int m = 0; m < N / 64; ++m) {
+      const int e = tid + m * (waves << 6);
+      if (e < N)
+        for (int w = 0; w < here; ++w) total[m] += ex_lds[w * N + e];
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < N / 64; ++m) {
+    const int e = tid + m * (waves << 6);
+    const int r = row0 + (e >> 4), c = col0 + (e & 15);
+    if (e < N && r < n_rows && c < n_out) {
+      float* dst = out + (long)r * ldo + c;
+      float v = total[m];
+      if (bias) v += bias[c];
+      *dst = ex_epilogue<EPI>(v, EPI == EPI_RESIDUAL ? *dst : 0.f);
+    }
+  }
+}
+
+struct ExactArgs {
+  const float* A; long lda; const float* W; const float* bias; float* out; long ldo;
+  int n_rows, n_out, k_dim;
+};
+
+template <int T, int EPI, bool VEC>
+static int launch_tile(const ExactArgs& a, hipStream_t stream) {
+  constexpr int B = 32 * T, bytes = 2 * 2 * B * EX_BK * (int)sizeof(float);
+  static_assert(bytes <= 64 * 1024, "what a kernel gets without asking");
+  const int row_tiles = (a.n_rows + B - 1) / B, col_tiles = (a.n_out + B - 1) / B;
+  if ((long)row_tiles * col_tiles > 0x7fffffffL) return MGPT_ERR_TOO_LARGE;
+  const int vec_out = a.ldo % 4 == 0 && ((reinterpret_cast<uintptr_t>(a.out) | reinterpret_cast<uintptr_t>(a.bias)) & 15) == 0;
+  hipLaunchKernelGGL((linear_exact_tile_kernel<T, EPI, VEC>), dim3(row_tiles * col_tiles), dim3(256), bytes, stream, a.A, a.lda,
+                     a.W, a.bias, a.out, a.ldo, a.n_rows, a.n_out, a.k_dim, row_tiles, vec_out);
+  return mgpt_last_error();
+}
+
+template <int EPI, bool VEC>
+static int launch_rows(const ExactArgs& a, hipStream_t stream) {
+  const int row_tiles = (a.n_rows + 15) / 16, col_tiles = (a.n_out + 15) / 16;
+  if ((long)row_tiles * col_tiles > 0x7fffffffL) return MGPT_ERR_TOO_LARGE;
+  const int blocks = (a.k_dim + EX_BLOCK - 1) / EX_BLOCK;
+  const int rounds = (blocks + 15) / 16, waves = (blocks + rounds - 1) / rounds;
+  hipLaunchKernelGGL((linear_exact_rows_kernel<EPI, VEC>), dim3(row_tiles * col_tiles), dim3(64 * waves),
+                     waves * 256 * (int)sizeof(float), stream, a.A, a.lda, a.W, a.bias, a.out, a.ldo, a.n_rows, a.n_out,
+                     a.k_dim, row_tiles);
+  return mgpt_last_error();
+}
+
+enum { EX_ROWS, EX_TILE64, EX_TILE128 };
+
+// The kernel that takes least by what was measured (us; a call's fixed part is the same for all): the rows kernel by its
+// rate; a tile kernel by the rounds of 256 workgroups that it needs, a round of 64 x 64 tiles 0.019 us a k (0.0225 alone on
+// a compute unit), of 128 x 128 tiles 0.068.  Rows kernel / 64 / 128, us: 64 rows 768 -> 2304 12.1 / 22 / 60; 256 rows
+// 32.9 / 23.3 / 61; 1,100 rows 116 / 48.7 / 63; 256 rows 3072 -> 768 41 / 78 / 223; 1,100 rows 512 -> 50304 1525 / 536 / 512.
+// The 64 x 64 FMA tiles that these kernels replace reached 10 to 15 TFLOP/s (1,100 rows 2048 -> 512: 163 us, here 54), the
+// FMA kernel for few rows took 57 us for 16 rows 3072 -> 768 (here 14).
+static int choose_kernel(const ExactArgs& a) {
+  const double k = a.k_dim, rows = 2.0 * a.n_rows * a.n_out * k / 34e6;
+  auto rounds = [&](int b) {
+    const long tiles = (long)((a.n_rows + b - 1) / b) * ((a.n_out + b - 1) / b);
+    return (double)((tiles + 255) / 256);
+  };
+  const double r64 = rounds(64), t64 = r64 > 1 ? r64 * 0.019 * k : 0.0225 * k, t128 = rounds(128) * 0.068 * k;
+  if (rows <= t64 && rows <= t128) return EX_ROWS;
+  return t64 <= t128 ? EX_TILE64 : EX_TILE128;
+}
+
+template <int EPI, bool VEC>
+static int launch_kernel(const ExactArgs& a, int kernel, hipStream_t stream) {
+  if (kernel == EX_ROWS) return launch_rows<EPI, VEC>(a, stream);
+  return kernel == EX_TILE64 ? launch_tile<2, EPI, VEC>(a, stream) : launch_tile<4, EPI, VEC>(a, stream);
+}
+
+int mgpt_linear_exact_launch(const float* A, long lda, const float* W, const float* bias, float* out, long ldo, int n_rows,
+                             int n_out, int k_dim, int epi, hipStream_t stream) {
+  const ExactArgs a = {A, lda, W, bias, out, ldo, n_rows, n_out, k_dim};
+  const bool vec = k_dim % 4 == 0 && lda % 4 == 0 && ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(W)) & 15) == 0;
+  const int kernel = choose_kernel(a);
+#define EX_LAUNCH(E) return vec ? launch_kernel<E, true>(a, kernel, stream) : launch_kernel<E, false>(a, kernel, stream)
+  if (epi == EPI_NONE) EX_LAUNCH(EPI_NONE);
+  if (epi == EPI_GELU) EX_LAUNCH(EPI_GELU);
+  if (epi == EPI_RELU2) EX_LAUNCH(EPI_RELU2);
+  if (epi == EPI_RESIDUAL) EX_LAUNCH(EPI_RESIDUAL);
+#undef EX_LAUNCH
+  return MGPT_ERR_BAD_SHAPE;
+}

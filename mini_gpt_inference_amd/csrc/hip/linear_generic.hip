@@ -3,12 +3,13 @@
 // GELU-tanh, squared-relu or residual-add epilogue: y = x W^T + b as nn.Linear
 // (reference: src/minigpt_infer/model.py:43-44,96-101).
 //
-// This is the kernel of the true 32-bit path: k runs 0..K-1 in order for every
-// output element, so a row's result does not depend on which other rows share
-// the launch.  The bfloat16 serving path uses it only for shapes the MFMA
-// kernels refuse.
+// k runs 0..K-1 in order for every output element, so a row's result does not
+// depend on which other rows share the launch.  The bfloat16 path uses it for
+// shapes the MFMA kernels refuse and for matrices stored in 32-bit; a product
+// that is float32 throughout goes to the matrix cores (linear_exact.hip).
 #include "common.h"
 #include "launchers.h"
+#include "linear_exact.h"
 
 #define EPI_NONE 0
 #define EPI_GELU 1
@@ -87,7 +88,7 @@ __global__ __launch_bounds__(256) void linear_generic_kernel(
   }
 }
 
-// The same product for few rows (a decode step on the 32-bit path): with 64 x 64 tiles a product of
+// The same product for few rows (a decode step): with 64 x 64 tiles a product of
 // one row by 512 columns is eight workgroups that each walk the whole inner size.  Here a workgroup
 // owns 16 rows x 16 columns, one output element a thread, so there are as many workgroups as the
 // matrix has groups of 16 columns.  Every element is the same chain as above (acc = fma(a[k], w[k],
@@ -187,8 +188,11 @@ extern "C" int mgpt_linear_generic(const void* A, int a_dtype, long lda, const v
   if (n_rows < 0 || n_out < 0 || k_dim <= 0 || lda < k_dim || ldo < n_out)
     return MGPT_ERR_BAD_SHAPE;
   if ((n_rows + TILE - 1) / TILE > 65535) return MGPT_ERR_TOO_LARGE;
-  if (a_dtype == MGPT_F32 && w_dtype == MGPT_F32)
-    return launch_out<float, float>(A, lda, W, bias, out, ldo, n_rows, n_out, k_dim, epilogue, out_dtype, stream);
+  if (a_dtype == MGPT_F32 && w_dtype == MGPT_F32 && out_dtype == MGPT_F32)
+    return mgpt_linear_exact_launch((const float*)A, lda, (const float*)W, bias, (float*)out, ldo, n_rows, n_out, k_dim,
+                                    epilogue, stream);
+  if (a_dtype == MGPT_F32 && w_dtype == MGPT_F32 && out_dtype == MGPT_BF16 && epilogue != EPI_RESIDUAL)
+    return launch_epi<float, float, bf16_t>(A, lda, W, bias, out, ldo, n_rows, n_out, k_dim, epilogue, stream);
   if (a_dtype == MGPT_BF16 && w_dtype == MGPT_BF16)
     return launch_out<bf16_t, bf16_t>(A, lda, W, bias, out, ldo, n_rows, n_out, k_dim, epilogue, out_dtype, stream);
   if (a_dtype == MGPT_BF16 && w_dtype == MGPT_F32)

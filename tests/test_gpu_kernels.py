@@ -91,8 +91,8 @@ def test_linear_generic(a_dt, w_dt, o_dt, epi):
                                                 ("bfloat16", "float32", "bfloat16", kernels.EPI_GELU),
                                                 ("bfloat16", "bfloat16", "float32", kernels.EPI_NONE)])
 def test_linear_generic_few_rows_and_many_agree_bit_for_bit(a_dt, w_dt, o_dt, epi, n_few):
-    """Up to 32 rows go to a kernel with a workgroup per 16 x 16 outputs, more to 64 x 64 tiles: every
-    element is the same chain of fused multiply-adds along k in both, so a row's result is the same
+    """Few rows go to a kernel with a workgroup per 16 x 16 outputs, more to tiles: every element's sum
+    runs in the same order along k in both, so a row's result is the same
     bits whichever kernel its step's size chooses (a decode step against a prompt's step)."""
     g = torch.Generator().manual_seed(23)
     n, k, o = 50, 208, 137      # an inner size that is no multiple of the few-rows kernel's stage of 64
@@ -123,6 +123,27 @@ def test_linear_generic_takes_any_inner_size(a_dt, w_dt, o_dt, n, k):
     helpers.assert_close(out[:n], _linear_want(a[:n], w, bias, kernels.EPI_GELU, None), o_dt if o_dt == "bfloat16" else "float32",
                          f"inner size {k}")
     assert (out[n] == 7.0).all()
+
+
+@pytest.mark.parametrize("k", [1, 15, 17, 256, 258, 300, 512, 4100, 4352])
+def test_float32_product_keeps_its_sums_whatever_the_tiles(k):
+    """A product that is float32 throughout goes to one of three kernels by its size: a workgroup per 16 x 16 outputs with
+    a wave per 256 of k (several rounds of them beyond 16 waves), tiles of 64 x 64 and of 128 x 128.  An element's bits
+    are the same in all, also where rows of the operands are not 16-byte aligned; the error against 64 bits is that of
+    float32 sums (a chain of at most 64 groups of four products in a block of 256, then the blocks: below 1e-6 of the
+    result's norm)."""
+    g = torch.Generator().manual_seed(k)
+    o, n = 8192 if k <= 300 else 1100, 1030            # enough tiles for the largest one where that is cheap
+    a, w, bias = rnd(g, n, k + 3).to(DEV), rnd(g, o, k).to(DEV), rnd(g, o).to(DEV)
+    whole = torch.empty(n, o, device=DEV)
+    kernels.linear_generic(a[:, :k], w, bias, whole, n)          # a row stride that is not the inner size
+    want = a[:, :k].double() @ w.double().T + bias.double()
+    assert ((whole.double() - want).norm() / want.norm()).item() < 1e-6
+    for rows, cols in ((1, o), (16, o), (17, 37), (70, 200), (130, o), (300, 515), (n, 130)):
+        part = torch.full((rows + 1, cols), 7.0, device=DEV)
+        kernels.linear_generic(a[:rows, :k].contiguous(), w[:cols].contiguous(), bias[:cols].contiguous(), part, rows)
+        assert torch.equal(part[:rows], whole[:rows, :cols]), f"{rows} rows, {cols} columns"
+        assert (part[rows] == 7.0).all()
 
 
 def test_linear_generic_refuses_tensors_off_the_gpu():

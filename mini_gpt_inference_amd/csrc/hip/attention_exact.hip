@@ -1,0 +1,240 @@
+// Attention of the 32-bit path on the float32 matrix cores (v_mfma_f32_16x16x4_f32), paged, causal, softmax in float32:
+// what the general kernel (attention_generic.hip, which says what the arguments mean) computes, for head sizes 16, 32,
+// 64 and 128 and softmax weights (reference: src/minigpt_infer/model.py:61-87).
+//
+// A workgroup has 16 queries of one request, a head and eight waves.  Keys are taken in chunks of 64 that start at
+// multiples of 64; chunk c belongs to wave c % 8, which walks its chunks with a running maximum and sum; the waves'
+// results are put together in the order of the waves.  All of that depends on a key's position only, and what a query
+// does not see adds zeros, so a query's output is the same bits in a prompt, in a portion of one and in a decode step.
+// Keys that no query of the tile sees are never loaded.
+//
+// The scores of a chunk are made transposed, S^T = K Q^T: a lane then has, of query lane % 16, the keys
+// 16 t + 4 (lane / 16) + i, which is just how O^T = V^T P^T takes them as its second operand.  Weights, maxima and sums
+// stay in the lanes; nothing goes through LDS before the end.  Keys and values come straight from the pages, 16 bytes a
+// lane; of the values a lane takes the head size / 16 consecutive channels that are its row in as many tiles of O^T.
+//
+// The general kernel walks a query's keys with one wave and 4-byte loads: 352 us for the prompts of 4 requests (1,098
+// tokens, 8 heads of 64) and 134 us for decode steps of 16 requests x 12 heads behind 16 to 280 keys.
+#include "attention_exact.h"
+#include "attention_mask.h"
+#include "common.h"
+
+#define AX_WAVES 8
+#define AX_QUERIES 16
+#define AX_CHUNK 64
+#define AX_NONE 0xffffffffu     // not a row of the pool
+
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float ax_f4;
+
+// over the four lanes that share a query
+__device__ __forceinline__ float ax_max4(float v) {
+  v = fmaxf(v, __shfl_xor(v, 16, MGPT_WAVE));
+  return fmaxf(v, __shfl_xor(v, 32, MGPT_WAVE));
+}
+__device__ __forceinline__ float ax_sum4(float v) {
+  v += __shfl_xor(v, 16, MGPT_WAVE);
+  return v + __shfl_xor(v, 32, MGPT_WAVE);
+}
+
+template <int D>
+__global__ __launch_bounds__(64 * AX_WAVES) void attention_exact_kernel(AttentionExactArgs a) {
+  constexpr int G = D / 16;            // groups of 16 channels; also the channels of a lane's row of V^T
+  constexpr int LD = D + 4;
+  extern __shared__ __align__(16) float ax_lds[];      // [waves][queries][LD]
+  __shared__ float m_s[AX_WAVES][AX_QUERIES], l_s[AX_WAVES][AX_QUERIES];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, lk = lane >> 4;
+  const int h = blockIdx.y, hk = h / (a.n_head / a.n_kv_head);
+
+  // the request and the tile of it that this workgroup has: requests' tiles are numbered one behind the other
+  int r = -1, tile = blockIdx.x;
+  for (int r0 = 0; r0 < a.n_req; r0 += MGPT_WAVE) {
+    const int rr = r0 + lane;
+    int tiles = rr < a.n_req ? (a.cu_q[rr + 1] - a.cu_q[rr] + AX_QUERIES - 1) / AX_QUERIES : 0;
+    int upto = tiles;                                   // tiles of the requests up to this lane's
+    for (int off = 1; off < MGPT_WAVE; off <<= 1) {
+      const int o = __shfl_up(upto, off, MGPT_WAVE);
+      if (lane >= off) upto += o;
+    }
+    const uint64_t past = __ballot(upto > tile);
+    if (past) {
+      const int at = __ffsll((unsigned long long)past) - 1;
+      r = r0 + at;
+      tile -= __shfl(upto - tiles, at, MGPT_WAVE);
+      break;
+    }
+    tile -= __shfl(upto, MGPT_WAVE - 1, MGPT_WAVE);
+  }
+  if (r < 0) return;                                    // beyond the step's tiles: the whole workgroup
+  r = __builtin_amdgcn_readfirstlane(r);
+  const int q_start = a.cu_q[r], q_len = a.cu_q[r + 1] - q_start;
+  const int q0 = __builtin_amdgcn_readfirstlane(tile) * AX_QUERIES;
+  const int ctx = a.seq_lens[r] - q_len;
+  const int n_here = q_len - q0 < AX_QUERIES ? q_len - q0 : AX_QUERIES;
+  const int pos_lo = ctx + q0, pos_hi = pos_lo + n_here - 1;
+  const int tile_begin = first_seen(pos_lo, a.window, a.chunked);
+  const bool q_ok = l16 < n_here;
+  const int my_pos = pos_lo + l16, my_begin = first_seen(my_pos, a.window, a.chunked);
+  const int* bt = a.block_tables + (long)r * a.max_blocks;
+
+  ax_f4 qf[G];
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    qf[g] = (ax_f4){0.f, 0.f, 0.f, 0.f};
+    if (q_ok) qf[g] = *reinterpret_cast<const ax_f4*>(a.q + (long)(q_start + q0 + l16) * a.ldq + (long)h * D + 16 * g + 4 * lk);
+  }
+  const float slope = a.slopes ? a.slopes[h] : 0.f;
+  const float* dist = a.dist_bias ? a.dist_bias + (long)h * a.bias_len : nullptr;
+
+  float m = -INFINITY, l = 0.f;
+  ax_f4 acc[G];                                         // O^T tile dt, rows 4 lk + i: channel G (4 lk + i) + dt
+#pragma unroll
+  for (int g = 0; g < G; ++g) acc[g] = (ax_f4){0.f, 0.f, 0.f, 0.f};
+
+  for (int c = wave; c * AX_CHUNK <= pos_hi; c += AX_WAVES) {
+    const int c0 = c * AX_CHUNK;
+    if (c0 + AX_CHUNK <= tile_begin && c0 >= a.keep_first) continue;
+    // the pool rows of this lane's four keys, c0 + 16 t + l16
+    unsigned int row[4];                                // 2^32 rows of 16 channels are 275 GB
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int j = c0 + 16 * t + l16;
+      row[t] = AX_NONE;
+      if (j <= pos_hi && (j >= tile_begin || j < a.keep_first)) {
+        const int idx = j / a.page_size;
+        row[t] = ((unsigned int)bt[idx] * a.n_kv_head + hk) * a.page_size + (j - idx * a.page_size);
+      }
+    }
+    ax_f4 s[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      s[t] = (ax_f4){0.f, 0.f, 0.f, 0.f};
+      ax_f4 kf[G];
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        kf[g] = (ax_f4){0.f, 0.f, 0.f, 0.f};
+        if (row[t] != AX_NONE) kf[g] = *reinterpret_cast<const ax_f4*>(a.kpool + (long)row[t] * D + 16 * g + 4 * lk);
+      }
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[g][e], qf[g][e], s[t], 0, 0, 0);
+    }
+    float top = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int j = c0 + 16 * t + 4 * lk + i;
+        float v = s[t][i] * a.scale;
+        if (dist) v += dist[distance_entry(my_pos - j, a.bias_len)];
+        if (a.softcap > 0.f) v = a.softcap * tanhf(v / a.softcap);
+        if (a.slopes) v -= slope * (float)(my_pos - j);
+        if (!(q_ok && j <= my_pos && (j >= my_begin || j < a.keep_first))) v = -INFINITY;
+        s[t][i] = v;
+        top = fmaxf(top, v);
+      }
+    const float m_new = fmaxf(m, ax_max4(top));
+    const float m_sub = m_new == -INFINITY ? 0.f : m_new;   // nothing seen so far: every weight is exp(-inf)
+    const float alpha = expf(m - m_sub);
+    float sum = 0.f;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        s[t][i] = expf(s[t][i] - m_sub);
+        sum += s[t][i];
+      }
+    l = l * alpha + ax_sum4(sum);
+    m = m_new;
+#pragma unroll
+    for (int g = 0; g < G; ++g) acc[g] *= alpha;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      float vf[4][G];                                   // of key 16 t + 4 lk + i the channels G l16 .. G l16 + G - 1
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const unsigned int vr = __shfl(row[t], 4 * lk + i, MGPT_WAVE);
+        const float* src = a.vpool + (long)vr * D + G * l16;
+        if constexpr (G >= 4) {
+#pragma unroll
+          for (int g = 0; g < G; g += 4) {
+            ax_f4 v = {0.f, 0.f, 0.f, 0.f};
+            if (vr != AX_NONE) v = *reinterpret_cast<const ax_f4*>(src + g);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) vf[i][g + e] = v[e];
+          }
+        } else {
+#pragma unroll
+          for (int g = 0; g < G; ++g) vf[i][g] = vr != AX_NONE ? src[g] : 0.f;
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int g = 0; g < G; ++g) acc[g] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[i][g], s[t][i], acc[g], 0, 0, 0);
+    }
+  }
+
+  if (lk == 0) {
+    m_s[wave][l16] = m;
+    l_s[wave][l16] = l;
+  }
+  float* mine = ax_lds + (wave * AX_QUERIES + l16) * LD + 4 * G * lk;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int g = 0; g < G; ++g) mine[i * G + g] = acc[g][i];
+  __syncthreads();
+
+  for (int e = tid; e < n_here * D; e += 64 * AX_WAVES) {
+    const int qi = e / D, d = e % D;
+    float top = a.sinks ? a.sinks[h] : -INFINITY;       // one more term of the denominator, with no value
+#pragma unroll
+    for (int w = 0; w < AX_WAVES; ++w) top = fmaxf(top, m_s[w][qi]);
+    float num = 0.f, den = 0.f;
+#pragma unroll
+    for (int w = 0; w < AX_WAVES; ++w) {
+      const float f = expf(m_s[w][qi] - top);
+      den += l_s[w][qi] * f;
+      num += ax_lds[(w * AX_QUERIES + qi) * LD + d] * f;
+    }
+    if (a.sinks) den += expf(a.sinks[h] - top);
+    const long n = q_start + q0 + qi;
+    float inv = 1.0f / den;
+    if (a.gate) inv *= 1.0f / (1.0f + expf(-a.gate[n * a.ldg + h]));
+    a.out[n * a.ldo + (long)h * D + d] = num * inv;
+  }
+}
+
+template <int D>
+static int launch(const AttentionExactArgs& a, int n_tokens, hipStream_t stream) {
+  constexpr int bytes = AX_WAVES * AX_QUERIES * (D + 4) * (int)sizeof(float);
+  static bool allowed = bytes <= 48 * 1024;            // more LDS than a kernel gets without asking
+  if (!allowed) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(attention_exact_kernel<D>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (e != hipSuccess) return (int)e;
+    allowed = true;
+  }
+  // at most so many tiles: a request's last one may be short
+  const long tiles = ((long)n_tokens + (long)(AX_QUERIES - 1) * (a.n_req < n_tokens ? a.n_req : n_tokens)) / AX_QUERIES;
+  if (tiles > 0x7fffffffL) return MGPT_ERR_TOO_LARGE;
+  hipLaunchKernelGGL(attention_exact_kernel<D>, dim3((unsigned int)tiles, a.n_head), dim3(64 * AX_WAVES), bytes, stream, a);
+  return mgpt_last_error();
+}
+
+bool mgpt_attention_exact_takes(const AttentionExactArgs& a, int head_dim) {
+  const uintptr_t together = reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.kpool) |
+                             reinterpret_cast<uintptr_t>(a.vpool);
+  return (head_dim == 16 || head_dim == 32 || head_dim == 64 || head_dim == 128) && (together & 15) == 0 && a.ldq % 4 == 0;
+}
+
+int mgpt_attention_exact_launch(const AttentionExactArgs& a, int n_tokens, int head_dim, hipStream_t stream) {
+  if (head_dim == 16) return launch<16>(a, n_tokens, stream);
+  if (head_dim == 32) return launch<32>(a, n_tokens, stream);
+  if (head_dim == 64) return launch<64>(a, n_tokens, stream);
+  return launch<128>(a, n_tokens, stream);
+}

@@ -20,11 +20,13 @@
 // y = P v (reference: src/minigpt_infer/model.py:61-87,
 // the rule col <= cache_len + row of src/minigpt_infer/batch.py:202-227).
 //
-// The general kernel runs one wave per (token, head).  Keys are reduced in
+// On the 32-bit path softmax attention with head sizes 16, 32, 64 and 128 goes to the matrix cores
+// (attention_exact.hip).  The general kernel runs one wave per (token, head).  Keys are reduced in
 // chunks of 64 that start at absolute positions that are multiples of 64, so the
 // order of the sums for a query depends only on its position, never on how the
 // tokens were cut into steps or what else is in the batch.  Slots outside
 // [begin, end) are never loaded.
+#include "attention_exact.h"
 #include "attention_mask.h"
 #include "common.h"
 #include "launchers.h"
@@ -183,22 +185,29 @@ __global__ __launch_bounds__(64) void paged_attention_generic_kernel(
 
 // q: [n_tokens, n_head*head_dim] with row stride ldq; out likewise with ldo.
 // q_req[t] = index of token t's request in this step (or -1 for a padded token),
-// cu_q[r]..cu_q[r+1] = the tokens of request r, seq_lens[r] = its length after this step.
+// cu_q[r]..cu_q[r+1] = the tokens of request r (r < n_req), seq_lens[r] = its length after this step.
 extern "C" int mgpt_paged_attention_generic(
     const void* q, long ldq, void* out, long ldo, const void* kpool, const void* vpool,
     const int* block_tables, int max_blocks, const int* cu_q, const int* seq_lens, const int* q_req,
-    int n_tokens, int n_head, int n_kv_head, int head_dim, int page_size, float scale, int window,
+    int n_tokens, int n_req, int n_head, int n_kv_head, int head_dim, int page_size, float scale, int window,
     int dtype, int fast_exp, const float* sinks, float softcap, const void* gate, long ldg, int keep_first,
     const float* score_bias, int chunked, const float* dist_bias, int bias_len, const float* slopes,
     hipStream_t stream) {
   if (n_tokens == 0) return MGPT_OK;
   if (!q || !out || !kpool || !vpool || !block_tables || !cu_q || !seq_lens || !q_req) return MGPT_ERR_NULL;
-  if (n_tokens < 0 || n_head <= 0 || n_kv_head <= 0 || (n_head % n_kv_head) != 0 || head_dim <= 0 ||
+  if (n_tokens < 0 || n_req < 0 || n_head <= 0 || n_kv_head <= 0 || (n_head % n_kv_head) != 0 || head_dim <= 0 ||
       head_dim > MAX_DPL * MGPT_WAVE || page_size <= 0 || max_blocks <= 0 || window < 0 || keep_first < 0 || (score_bias && (sinks || softcap > 0.f)) ||
       (dist_bias && (bias_len <= 0 || score_bias || softcap > 0.f)) || (slopes && (dist_bias || score_bias)))
     return MGPT_ERR_BAD_SHAPE;
   if (n_head > 65535) return MGPT_ERR_TOO_LARGE;
   if (window == 0) keep_first = 0;   // every key is seen anyway
+  if (dtype == MGPT_F32 && !fast_exp && !score_bias) {
+    const AttentionExactArgs args = {(const float*)q, ldq, (float*)out, ldo, (const float*)kpool, (const float*)vpool,
+                                     block_tables, max_blocks, cu_q, seq_lens, n_req, n_head, n_kv_head, page_size, scale,
+                                     window, sinks, softcap, (const float*)gate, ldg, keep_first, chunked, dist_bias,
+                                     bias_len, slopes};
+    if (mgpt_attention_exact_takes(args, head_dim)) return mgpt_attention_exact_launch(args, n_tokens, head_dim, stream);
+  }
   dim3 grid(n_tokens, n_head), block(MGPT_WAVE);
 #define LAUNCH(T, F)                                                                              \
   hipLaunchKernelGGL((paged_attention_generic_kernel<T, F>), grid, block, 0, stream, (const T*)q, ldq, \

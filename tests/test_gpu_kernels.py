@@ -638,6 +638,46 @@ ATTENTION_CASES = [
 ]
 
 
+@pytest.mark.parametrize("window,mask", [(0, {}), (100, {}), (100, {"keep_first": 70}), (96, {"chunked": True})])
+@pytest.mark.parametrize("d", [16, 32, 64, 128])
+def test_float32_attention_keeps_its_sums_whatever_the_portion(d, window, mask):
+    """The matrix-core kernel of the 32-bit path has tiles of 16 queries and chunks of 64 keys dealt out over 8 waves (512
+    keys a round): a query's output is the same bits as part of a whole prompt, of a portion and alone, around the ends of
+    all of these, and with more requests than the 64 that a wave numbers the tiles of at a time."""
+    lens = [1, 15, 16, 17, 63, 64, 65, 511, 512, 513, 600]
+    c = PagedCase(lens, lens, h=4, hk=2, d=d, page=12, dtype="float32", seed=d)
+    g = torch.Generator().manual_seed(d + 1)
+    extra = {"sinks": torch.randn(4, generator=g).to(DEV), "softcap": 0.0 if mask else 20.0,
+             "gate": torch.randn(c.n, 4, generator=g).to(DEV)}
+
+    def attend(req, first, q_lens, rows):
+        out = torch.full((len(rows), 4 * d), float("nan"), device=DEV)
+        cu = i32(np.concatenate([[0], np.cumsum(q_lens)]))
+        kernels.paged_attention_generic(
+            c.q_flat[rows].contiguous(), out, c.kp, c.vp, c.bt[req].contiguous(), cu,
+            i32([f + q for f, q in zip(first, q_lens)]), i32([i for i, q in enumerate(q_lens) for _ in range(q)]), len(rows),
+            len(req), 4, d ** -0.5, window, **{**extra, "gate": extra["gate"][rows].contiguous()}, **mask)
+        return out
+
+    starts = np.concatenate([[0], np.cumsum(lens)])
+    whole = attend(list(range(len(lens))), [0] * len(lens), lens, list(range(c.n)))
+    if not mask:
+        want = c.want(d ** -0.5, window)               # without sink, cap and gate
+        plain = torch.empty_like(whole)
+        kernels.paged_attention_generic(c.q_flat, plain, c.kp, c.vp, c.bt, c.cu, c.sl, c.q_req, c.n, len(lens), 4, d ** -0.5,
+                                        window)
+        helpers.assert_close(plain, want, "float32", "matrix-core attention")
+    # every request's tokens from a third of it on, in one portion, with others before and behind it
+    cut = [n // 3 for n in lens]
+    rows = [starts[r] + t for r, n in enumerate(lens) for t in range(cut[r], n)]
+    assert torch.equal(attend(list(range(len(lens))), cut, [n - x for n, x in zip(lens, cut)], rows), whole[rows])
+    # single tokens, eighty requests' worth of them
+    pick = [(r, t) for r, n in enumerate(lens) for t in sorted({0, n // 2, max(n - 2, 0), n - 1, min(64, n - 1)})]
+    pick = (pick * 3)[:80]
+    rows = [starts[r] + t for r, t in pick]
+    assert torch.equal(attend([r for r, _ in pick], [t for _, t in pick], [1] * len(pick), rows), whole[rows])
+
+
 @pytest.mark.parametrize("window", [0, 5, 70])
 @pytest.mark.parametrize("case", range(len(ATTENTION_CASES)))
 @pytest.mark.parametrize("kernel", ["generic-float32", "generic-bfloat16", "split-bfloat16", "splitfast-bfloat16",

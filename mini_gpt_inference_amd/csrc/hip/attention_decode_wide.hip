@@ -12,7 +12,7 @@
 //    lie beyond the sequence are never followed (their keys are masked before the load), and
 //    an entry's page number is clamped to the pool so that a stale entry cannot send a load
 //    outside it;
-//  * eight waves, each with one 64-key chunk in flight (sixteen 16-byte loads per lane), so a
+//  * eight waves (four with many tokens and heads), each with one 64-key chunk in flight (sixteen 16-byte loads per lane), so a
 //    context of up to 512 keys is one pass;
 //  * D/8 lanes share a key: scores with v_dot2_f32_bf16 on the packed rows as loaded, summed
 //    over the D/8 lanes with DPP moves; one wave-wide maximum per chunk (DPP within rows of 16,
@@ -30,8 +30,6 @@
 #include "attention_mask.h"
 #include "common.h"
 #include "launchers.h"
-
-#define AW_WAVES 8
 
 typedef __attribute__((ext_vector_type(2))) __bf16 aw_bf16x2_t;
 
@@ -70,8 +68,13 @@ __device__ __forceinline__ float aw_dot2(unsigned int a, unsigned int b, float c
 }
 
 // IDENT: token n is request n (or padded), so its block table row is known before anything is loaded
-template <int D, bool IDENT, int BIAS>
-__global__ __launch_bounds__(AW_WAVES * 64) void paged_attention_decode_kernel(
+// W: waves of the workgroup.  A context of up to 512 keys is one pass of eight waves; with more (token, head) pairs than
+// the chip holds such workgroups at a time (two a compute unit, one with a head size of 128 and its 166 registers), four
+// waves: more workgroups at a time, and fewer waves without a chunk under short contexts.  Eight / four waves, us: 32
+// tokens x 25 heads of 64 behind 40, 150, 400 and 1,000 keys 8.0 / 5.3, 9.0 / 6.8, 16.7 / 16.6, 34.4 / 34.4; 256 x 25 behind 40
+// and 400 40 / 20, 116 / 116 (5.6 TB/s); 40 x 16 of 128 behind 150 and 1,000 19.4 / 12.7, 64 / 59.
+template <int D, bool IDENT, int BIAS, int W>
+__global__ __launch_bounds__(W * 64) void paged_attention_decode_kernel(
     const bf16_t* __restrict__ q, long ldq, bf16_t* __restrict__ out, long ldo,
     const bf16_t* __restrict__ kpool, const bf16_t* __restrict__ vpool,
     const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ positions,
@@ -81,9 +84,10 @@ __global__ __launch_bounds__(AW_WAVES * 64) void paged_attention_decode_kernel(
     int chunked, const float* __restrict__ dist_bias, int bias_len, const float* __restrict__ slopes) {
   constexpr int LPK = D / 8;     // lanes per key
   constexpr int KPI = 64 / LPK;  // keys per load instruction
-  constexpr int ROWS = AW_WAVES * KPI;      // partial results: one per (key subgroup, wave)
-  constexpr int SUBSETS = AW_WAVES * 64 / D;  // groups of AW_WAVES partial rows, one thread per channel each
-  __shared__ float m_s[AW_WAVES];
+  constexpr int ROWS = W * KPI;      // partial results: one per (key subgroup, wave)
+  constexpr int SUBSETS = W * 64 / D;  // groups of 8 partial rows, one thread per channel each
+  static_assert(ROWS == SUBSETS * 8 && 8 % W == 0, "a thread adds up 8 partial rows of its channel");
+  __shared__ float m_s[W];
   __shared__ float l_s[ROWS];        // [sub][wave]
   __shared__ float acc_s[ROWS * D];  // [sub][wave][channel]
   __shared__ float part_s[SUBSETS * D];
@@ -133,7 +137,7 @@ __global__ __launch_bounds__(AW_WAVES * 64) void paged_attention_decode_kernel(
     }
     kv_end = qr < 0 ? 0 : qpos + 1;
     kv_begin = first_key;
-    c_base += 64 * AW_WAVES;
+    c_base += 64 * W;
     // a chunk without a visible key costs its wave nothing more (the same decision in all lanes)
     if (__builtin_amdgcn_readfirstlane((c0 >= kv_end) | ((c0 + 64 <= kv_begin) & (c0 >= keep_first)))) continue;
     // ---- second round trip: keys and values of this wave's chunk.  Every lane loads (a masked
@@ -205,9 +209,9 @@ __global__ __launch_bounds__(AW_WAVES * 64) void paged_attention_decode_kernel(
   // ---- merge: partial rows [sub][wave] of D channels; every key's weight sits on LPK lanes, so
   // lane dg == 0 speaks for the group's sum
   if (lane == 0) m_s[wave] = m;
-  if (dg == 0) l_s[sub * AW_WAVES + wave] = l;
+  if (dg == 0) l_s[sub * W + wave] = l;
   {
-    float4* dst = reinterpret_cast<float4*>(acc_s + (sub * AW_WAVES + wave) * D + dg * 8);
+    float4* dst = reinterpret_cast<float4*>(acc_s + (sub * W + wave) * D + dg * 8);
     dst[0] = make_float4(acc[0], acc[1], acc[2], acc[3]);
     dst[1] = make_float4(acc[4], acc[5], acc[6], acc[7]);
   }
@@ -215,15 +219,15 @@ __global__ __launch_bounds__(AW_WAVES * 64) void paged_attention_decode_kernel(
   {
     float mx = m_s[0];
 #pragma unroll
-    for (int w = 1; w < AW_WAVES; ++w) mx = fmaxf(mx, m_s[w]);
+    for (int w = 1; w < W; ++w) mx = fmaxf(mx, m_s[w]);
     if (sinks) mx = fmaxf(mx, sinks[h] * 1.4426950408889634f);   // the sink, in the scores' units of log2 e
-    const int c = tid % D, sset = tid / D;  // this thread: channel c of the partial rows sset*AW_WAVES ..
+    const int c = tid % D, sset = tid / D;  // this thread: channel c of the partial rows 8 * sset ..
     float a = 0.f, lt = 0.f;
 #pragma unroll
-    for (int w = 0; w < AW_WAVES; ++w) {
-      const float f = __builtin_amdgcn_exp2f(m_s[w] - mx);  // a wave without keys: exp2(-inf) = 0, and its sums are 0
-      a = fmaf(acc_s[(sset * AW_WAVES + w) * D + c], f, a);
-      lt = fmaf(l_s[sset * AW_WAVES + w], f, lt);
+    for (int i = 0; i < 8; ++i) {
+      const float f = __builtin_amdgcn_exp2f(m_s[i % W] - mx);  // a wave without keys: exp2(-inf) = 0, and its sums are 0
+      a = fmaf(acc_s[(sset * 8 + i) * D + c], f, a);
+      lt = fmaf(l_s[sset * 8 + i], f, lt);
     }
     part_s[sset * D + c] = a;
     if (c == 0) lpart_s[sset] = lt;
@@ -241,7 +245,7 @@ __global__ __launch_bounds__(AW_WAVES * 64) void paged_attention_decode_kernel(
       const float sink = sinks[h] * 1.4426950408889634f;
       float mx = sink;
 #pragma unroll
-      for (int w = 0; w < AW_WAVES; ++w) mx = fmaxf(mx, m_s[w]);
+      for (int w = 0; w < W; ++w) mx = fmaxf(mx, m_s[w]);
       lt += __builtin_amdgcn_exp2f(sink - mx);
     }
     float res = score_bias ? a : a / lt;
@@ -279,13 +283,19 @@ extern "C" int mgpt_paged_attention_decode_bf16(
   if (pool_bytes >= (1L << 32)) return MGPT_ERR_BAD_SHAPE;
   const unsigned int page_bytes = (unsigned int)(n_kv_head * page_size * head_dim * 2);
   const float scale_log2e = scale * 1.4426950408889634f;
-  dim3 grid(n_tokens, n_head), block(AW_WAVES * 64);
-#define AW_LAUNCH3(DD, ID, BI)                                                                                 \
-  hipLaunchKernelGGL((paged_attention_decode_kernel<DD, ID, BI>), grid, block, 0, stream, (const bf16_t*)q, ldq, \
+  const bool many = (long)n_tokens * n_head > (head_dim == 128 ? 256 : 512);
+  dim3 grid(n_tokens, n_head);
+#define AW_LAUNCH4(DD, ID, BI, W)                                                                              \
+  hipLaunchKernelGGL((paged_attention_decode_kernel<DD, ID, BI, W>), grid, dim3(W * 64), 0, stream, (const bf16_t*)q, ldq, \
                      (bf16_t*)out, ldo, (const bf16_t*)kpool, (const bf16_t*)vpool, block_tables,          \
                      max_blocks, positions, q_req, cu_q, n_head, n_kv_head, page_shift, num_pages, page_bytes, \
                      scale_log2e, window, sinks, softcap > 0.f ? softcap * 1.4426950408889634f : 0.f, \
                      (const bf16_t*)gate, ldg, keep_first, score_bias, chunked, dist_bias, bias_len, slopes)
+#define AW_LAUNCH3(DD, ID, BI)                 \
+  do {                                         \
+    if (many) AW_LAUNCH4(DD, ID, BI, 4);       \
+    else AW_LAUNCH4(DD, ID, BI, 8);            \
+  } while (0)
 #define AW_LAUNCH2(DD, ID)                     \
   do {                                         \
     if (slopes) AW_LAUNCH3(DD, ID, 2);         \
@@ -307,5 +317,6 @@ extern "C" int mgpt_paged_attention_decode_bf16(
 #undef AW_LAUNCH
 #undef AW_LAUNCH2
 #undef AW_LAUNCH3
+#undef AW_LAUNCH4
   return mgpt_last_error();
 }

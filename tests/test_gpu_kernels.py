@@ -638,6 +638,19 @@ ATTENTION_CASES = [
 ]
 
 
+@pytest.mark.parametrize("window", [0, 100])
+@pytest.mark.parametrize("d,n", [(16, 129), (32, 129), (64, 128), (64, 129), (128, 64), (128, 65)])
+def test_decode_attention_of_many_tokens(d, n, window):
+    """More (token, head) pairs than the chip holds workgroups of eight waves go to workgroups of four, whose pass is 256
+    keys: around the line between the two, contexts around a chunk and around one and two passes."""
+    lens = ([1, 63, 64, 65, 255, 256, 257, 511, 512, 513, 40] * 12)[:n]
+    c = PagedCase(lens, [1] * n, h=4, hk=2, d=d, page=16, dtype="bfloat16", seed=d + n)
+    out = torch.full((n, 4 * d), float("nan"), dtype=torch.bfloat16, device=DEV)
+    assert kernels.paged_attention_decode_bf16(c.q_flat, out, c.kp, c.vp, c.bt, i32([x - 1 for x in lens]), c.q_req, n, 4,
+                                               d ** -0.5, window, identity=True)
+    helpers.assert_close(out, c.want(d ** -0.5, window), "bfloat16", "decode attention")
+
+
 @pytest.mark.parametrize("window,mask", [(0, {}), (100, {}), (100, {"keep_first": 70}), (96, {"chunked": True})])
 @pytest.mark.parametrize("d", [16, 32, 64, 128])
 def test_float32_attention_keeps_its_sums_whatever_the_portion(d, window, mask):

@@ -8,11 +8,13 @@
 // all four); the blocks' sums are added up in order, then the bias.  What is missing to a group counts as zeros.  All
 // kernels below keep to that, whatever their tiles, and whether one wave has all blocks of an element or each wave some.
 #include "common.h"
+#include "launchers.h"
 #include "linear_exact.h"
 
 #define EPI_NONE 0
 #define EPI_GELU 1
 #define EPI_RESIDUAL 2  // out += result
+#define EPI_QKV 3       // out = result; key and value columns also into their pages
 #define EPI_RELU2 5     // max(result, 0)^2
 
 #define EX_BLOCK 256    // k of a block
@@ -26,6 +28,18 @@ __device__ __forceinline__ float ex_epilogue(float v, float old) {
   if (EPI == EPI_RELU2) return relu_squared(v);
   if (EPI == EPI_RESIDUAL) return old + v;
   return v;
+}
+
+// Where a key or value column c >= q_width of token row r goes, or null (a padded row).
+__device__ __forceinline__ float* ex_page_row(const ExactScatter& sc, int r, int c) {
+  const int slot = sc.slot_mapping[r];
+  if (slot < 0) return nullptr;
+  c -= sc.q_width;
+  float* pool = c < sc.kv_width ? sc.kpool : sc.vpool;
+  if (c >= sc.kv_width) c -= sc.kv_width;
+  const int page = slot / sc.page_size, h = c / sc.head_dim;
+  return pool + ((long)(page * (sc.kv_width / sc.head_dim) + h) * sc.page_size + (slot - page * sc.page_size)) * sc.head_dim +
+         (c - h * sc.head_dim);
 }
 
 // Four k of a row from k on; those at or beyond k_dim count as zero.  VEC: rows are 16-byte aligned and k_dim is a multiple
@@ -50,7 +64,7 @@ __device__ __forceinline__ ex_f4 ex_load(const float* __restrict__ row, int k, i
 template <int T, int EPI, bool VEC>
 __global__ __launch_bounds__(256) void linear_exact_tile_kernel(
     const float* __restrict__ A, long lda, const float* __restrict__ W, const float* __restrict__ bias,
-    float* __restrict__ out, long ldo, int n_rows, int n_out, int k_dim, int row_tiles, int vec_out) {
+    float* __restrict__ out, long ldo, int n_rows, int n_out, int k_dim, int row_tiles, int vec_out, ExactScatter sc) {
   constexpr int B = 32 * T;                          // rows and columns of the tile
   constexpr int PIECES = B * EX_BK / 4 / 256;        // 16-byte pieces of one operand's slice that a thread stages
   extern __shared__ __align__(16) float ex_lds[];    // [2][2 B][EX_BK]: rows of activations, then of W
@@ -62,7 +76,7 @@ __global__ __launch_bounds__(256) void linear_exact_tile_kernel(
 
   // rows past the end are read from the last one: their results are never stored
   constexpr int ROW = EX_BK / 4, STEP = 256 / ROW;   // pieces of a row, rows that 256 threads stage at a time
-  const int srow = tid / ROW, sc = tid % ROW;        // this thread's piece of a slice: row srow + STEP p
+  const int srow = tid / ROW, sp = tid % ROW;        // this thread's piece of a slice: row srow + STEP p
   const float* ap[PIECES];
   const float* wp[PIECES];
 #pragma unroll
@@ -71,13 +85,13 @@ __global__ __launch_bounds__(256) void linear_exact_tile_kernel(
     ap[p] = A + (long)(r < n_rows ? r : n_rows - 1) * lda;
     wp[p] = W + (long)(c < n_out ? c : n_out - 1) * k_dim;
   }
-  const int s_lds = srow * EX_BK + ((sc ^ (srow & 7)) << 2);
+  const int s_lds = srow * EX_BK + ((sp ^ (srow & 7)) << 2);
   ex_f4 ga[PIECES], gw[PIECES];
   auto load = [&](int k0) {
 #pragma unroll
     for (int p = 0; p < PIECES; ++p) {
-      ga[p] = ex_load<VEC>(ap[p], k0 + 4 * sc, k_dim);
-      gw[p] = ex_load<VEC>(wp[p], k0 + 4 * sc, k_dim);
+      ga[p] = ex_load<VEC>(ap[p], k0 + 4 * sp, k_dim);
+      gw[p] = ex_load<VEC>(wp[p], k0 + 4 * sp, k_dim);
     }
   };
   auto store = [&](int buf) {
@@ -150,13 +164,19 @@ __global__ __launch_bounds__(256) void linear_exact_tile_kernel(
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] = ex_epilogue<EPI>(v[e], old[e]);
         *reinterpret_cast<ex_f4*>(dst) = v;
+        if (EPI == EPI_QKV && c >= sc.q_width) {       // four columns of one head: all sizes are multiples of 4
+          if (float* at = ex_page_row(sc, r, c)) *reinterpret_cast<ex_f4*>(at) = v;
+        }
       } else {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
           if (c + e < n_out) {
             float v = sum[i][j][e];
             if (bias) v += bias[c + e];
-            dst[e] = ex_epilogue<EPI>(v, EPI == EPI_RESIDUAL ? dst[e] : 0.f);
+            dst[e] = v = ex_epilogue<EPI>(v, EPI == EPI_RESIDUAL ? dst[e] : 0.f);
+            if (EPI == EPI_QKV && c + e >= sc.q_width) {
+              if (float* at = ex_page_row(sc, r, c + e)) *at = v;
+            }
           }
       }
     }
@@ -170,7 +190,7 @@ __global__ __launch_bounds__(256) void linear_exact_tile_kernel(
 template <int EPI, bool VEC>
 __global__ __launch_bounds__(1024) void linear_exact_rows_kernel(
     const float* __restrict__ A, long lda, const float* __restrict__ W, const float* __restrict__ bias,
-    float* __restrict__ out, long ldo, int n_rows, int n_out, int k_dim, int row_tiles) {
+    float* __restrict__ out, long ldo, int n_rows, int n_out, int k_dim, int row_tiles, ExactScatter sc) {
   constexpr int N = 256;                             // elements of the tile
   constexpr int U = 4;                               // groups on their way
   extern __shared__ __align__(16) float ex_lds[];    // [waves][N]
@@ -228,7 +248,10 @@ __global__ __launch_bounds__(1024) void linear_exact_rows_kernel(
       float* dst = out + (long)r * ldo + c;
       float v = total[m];
       if (bias) v += bias[c];
-      *dst = ex_epilogue<EPI>(v, EPI == EPI_RESIDUAL ? *dst : 0.f);
+      *dst = v = ex_epilogue<EPI>(v, EPI == EPI_RESIDUAL ? *dst : 0.f);
+      if (EPI == EPI_QKV && c >= sc.q_width) {
+        if (float* at = ex_page_row(sc, r, c)) *at = v;
+      }
     }
   }
 }
@@ -236,6 +259,7 @@ __global__ __launch_bounds__(1024) void linear_exact_rows_kernel(
 struct ExactArgs {
   const float* A; long lda; const float* W; const float* bias; float* out; long ldo;
   int n_rows, n_out, k_dim;
+  ExactScatter sc;
 };
 
 template <int T, int EPI, bool VEC>
@@ -244,9 +268,13 @@ static int launch_tile(const ExactArgs& a, hipStream_t stream) {
   static_assert(bytes <= 64 * 1024, "what a kernel gets without asking");
   const int row_tiles = (a.n_rows + B - 1) / B, col_tiles = (a.n_out + B - 1) / B;
   if ((long)row_tiles * col_tiles > 0x7fffffffL) return MGPT_ERR_TOO_LARGE;
-  const int vec_out = a.ldo % 4 == 0 && ((reinterpret_cast<uintptr_t>(a.out) | reinterpret_cast<uintptr_t>(a.bias)) & 15) == 0;
+  uintptr_t stored = reinterpret_cast<uintptr_t>(a.out) | reinterpret_cast<uintptr_t>(a.bias);
+  if (EPI == EPI_QKV) stored |= reinterpret_cast<uintptr_t>(a.sc.kpool) | reinterpret_cast<uintptr_t>(a.sc.vpool);
+  const int vec_out = a.ldo % 4 == 0 && (stored & 15) == 0 &&
+                      (EPI != EPI_QKV || (a.sc.q_width % 4 == 0 && a.sc.head_dim % 4 == 0));
   hipLaunchKernelGGL((linear_exact_tile_kernel<T, EPI, VEC>), dim3(row_tiles * col_tiles), dim3(256), bytes, stream, a.A, a.lda,
-                     a.W, a.bias, a.out, a.ldo, a.n_rows, a.n_out, a.k_dim, row_tiles, vec_out);
+                     a.W, a.bias, a.out, a.ldo, a.n_rows, a.n_out, a.k_dim, row_tiles, vec_out,
+                     a.sc);
   return mgpt_last_error();
 }
 
@@ -258,7 +286,7 @@ static int launch_rows(const ExactArgs& a, hipStream_t stream) {
   const int rounds = (blocks + 15) / 16, waves = (blocks + rounds - 1) / rounds;
   hipLaunchKernelGGL((linear_exact_rows_kernel<EPI, VEC>), dim3(row_tiles * col_tiles), dim3(64 * waves),
                      waves * 256 * (int)sizeof(float), stream, a.A, a.lda, a.W, a.bias, a.out, a.ldo, a.n_rows, a.n_out,
-                     a.k_dim, row_tiles);
+                     a.k_dim, row_tiles, a.sc);
   return mgpt_last_error();
 }
 
@@ -288,8 +316,8 @@ static int launch_kernel(const ExactArgs& a, int kernel, hipStream_t stream) {
 }
 
 int mgpt_linear_exact_launch(const float* A, long lda, const float* W, const float* bias, float* out, long ldo, int n_rows,
-                             int n_out, int k_dim, int epi, hipStream_t stream) {
-  const ExactArgs a = {A, lda, W, bias, out, ldo, n_rows, n_out, k_dim};
+                             int n_out, int k_dim, int epi, const ExactScatter& sc, hipStream_t stream) {
+  const ExactArgs a = {A, lda, W, bias, out, ldo, n_rows, n_out, k_dim, sc};
   const bool vec = k_dim % 4 == 0 && lda % 4 == 0 && ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(W)) & 15) == 0;
   const int kernel = choose_kernel(a);
 #define EX_LAUNCH(E) return vec ? launch_kernel<E, true>(a, kernel, stream) : launch_kernel<E, false>(a, kernel, stream)
@@ -297,6 +325,22 @@ int mgpt_linear_exact_launch(const float* A, long lda, const float* W, const flo
   if (epi == EPI_GELU) EX_LAUNCH(EPI_GELU);
   if (epi == EPI_RELU2) EX_LAUNCH(EPI_RELU2);
   if (epi == EPI_RESIDUAL) EX_LAUNCH(EPI_RESIDUAL);
+  if (epi == EPI_QKV) EX_LAUNCH(EPI_QKV);
 #undef EX_LAUNCH
   return MGPT_ERR_BAD_SHAPE;
+}
+
+// The product whose key and value columns (kv_width each, behind q_width columns of queries) also go to the pools at
+// slot_mapping[row] (a negative one: nowhere), [num_pages][kv_width / head_dim][page_size][head_dim].  The separate kernel
+// that copied them took 4.6 us a layer of a decode step, which is what a kernel costs there.
+extern "C" int mgpt_linear_exact_qkv(const float* A, long lda, const float* W, const float* bias, float* out, long ldo,
+                                     int n_rows, int n_out, int k_dim, float* kpool, float* vpool, const int* slot_mapping,
+                                     int q_width, int kv_width, int head_dim, int page_size, hipStream_t stream) {
+  if (n_rows == 0 || n_out == 0) return MGPT_OK;
+  if (!A || !W || !out || !kpool || !vpool || !slot_mapping) return MGPT_ERR_NULL;
+  if (n_rows < 0 || n_out < 0 || k_dim <= 0 || lda < k_dim || ldo < n_out || q_width < 0 || head_dim <= 0 || page_size <= 0 ||
+      kv_width <= 0 || kv_width % head_dim != 0 || q_width + 2 * kv_width != n_out)
+    return MGPT_ERR_BAD_SHAPE;
+  const ExactScatter sc = {kpool, vpool, slot_mapping, q_width, kv_width, head_dim, page_size};
+  return mgpt_linear_exact_launch(A, lda, W, bias, out, ldo, n_rows, n_out, k_dim, EPI_QKV, sc, stream);
 }

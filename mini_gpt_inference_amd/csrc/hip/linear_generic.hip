@@ -190,7 +190,7 @@ extern "C" int mgpt_linear_generic(const void* A, int a_dtype, long lda, const v
   if ((n_rows + TILE - 1) / TILE > 65535) return MGPT_ERR_TOO_LARGE;
   if (a_dtype == MGPT_F32 && w_dtype == MGPT_F32 && out_dtype == MGPT_F32)
     return mgpt_linear_exact_launch((const float*)A, lda, (const float*)W, bias, (float*)out, ldo, n_rows, n_out, k_dim,
-                                    epilogue, stream);
+                                    epilogue, ExactScatter{}, stream);
   if (a_dtype == MGPT_F32 && w_dtype == MGPT_F32 && out_dtype == MGPT_BF16 && epilogue != EPI_RESIDUAL)
     return launch_epi<float, float, bf16_t>(A, lda, W, bias, out, ldo, n_rows, n_out, k_dim, epilogue, stream);
   if (a_dtype == MGPT_BF16 && w_dtype == MGPT_BF16)

@@ -159,6 +159,34 @@ def linear_generic(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor
     _check(rc, "linear_generic")
 
 
+def linear_exact_qkv(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor, n_rows: int,
+                     scatter) -> bool:
+    """out[:n_rows] = a[:n_rows] @ w.T (+ bias), float32 throughout, and the key and value columns also into their pages:
+    scatter = (k_pool, v_pool, slot_mapping, q_width, kv_width).  False if a tensor is not float32."""
+    k_pool, v_pool, slot_mapping, q_width, kv_width = scatter
+    _need_cuda(a, w, bias, out, k_pool, v_pool, slot_mapping)
+    if any(t.dtype != torch.float32 for t in (a, w, out, k_pool, v_pool)):
+        return False
+    n_out, k_dim = w.shape
+    _need(w.is_contiguous(), "weight must be dense [out, in]")
+    _need(a.dim() == 2 and a.stride(1) == 1 and a.shape[1] == k_dim and a.shape[0] >= n_rows,
+          f"activation must be [>=n_rows, {k_dim}] with unit inner stride")
+    _need(out.dim() == 2 and out.stride(1) == 1 and out.shape[1] == n_out and out.shape[0] >= n_rows,
+          f"output must be [>=n_rows, {n_out}] with unit inner stride")
+    _need(bias is None or (bias.dtype == torch.float32 and bias.numel() == n_out), "bias must be float32 [out]")
+    _need(k_pool.shape == v_pool.shape and k_pool.dim() == 4 and k_pool.is_contiguous() and v_pool.is_contiguous(),
+          "key and value pools must be dense [pages, kv_heads, page_size, head_dim]")
+    _, n_kv_head, page_size, head_dim = k_pool.shape
+    _need(kv_width == n_kv_head * head_dim and q_width + 2 * kv_width == n_out,
+          "the output's columns must be the queries, then the keys and values of the pools' heads")
+    _need_i32("slot_mapping", slot_mapping, n_rows)
+    rc = library.kernels().mgpt_linear_exact_qkv(
+        _ptr(a), a.stride(0), _ptr(w), _ptr(bias), _ptr(out), out.stride(0), n_rows, n_out, k_dim, _ptr(k_pool), _ptr(v_pool),
+        _ptr(slot_mapping), q_width, kv_width, head_dim, page_size, _stream())
+    _check(rc, "linear_exact_qkv")
+    return True
+
+
 def kv_write(qkv: torch.Tensor, k_off: int, v_off: int, k_pool: torch.Tensor, v_pool: torch.Tensor,
              slot_mapping: torch.Tensor, n_tokens: int) -> None:
     """Stores the new keys and values of n_tokens rows of qkv into their pages.

@@ -279,7 +279,8 @@ def linear(ctx, a: Union[torch.Tensor, LazyNorm], w: torch.Tensor, bias: Optiona
     On the bfloat16 path up to 64 rows (fewer for a very wide output) go to the decode step's MFMA kernels (reading the residual
     stream through the folded LayerNorm when `a` is a LazyNorm of a fusable norm and the rows are
     few; splitting a long inner size over workgroups when the rows are many) and more rows to the
-    tiled MFMA kernel (which also splits a long inner size when its tiles are few); the 32-bit path, and every shape those refuse, go to the 32-bit FMA kernel.  `scatter` = (k_pool, v_pool,
+    tiled MFMA kernel (which also splits a long inner size when its tiles are few); the 32-bit path, and every shape those refuse, go to the general product
+    (on the matrix cores in 32 bits where everything is float32).  `scatter` = (k_pool, v_pool,
     slot_mapping, q_width, kv_width) asks for the new keys and values to be stored into their
     pages by the same kernel; the return value says whether that was done."""
     if n_rows == 0:
@@ -327,5 +328,7 @@ def linear(ctx, a: Union[torch.Tensor, LazyNorm], w: torch.Tensor, bias: Optiona
         partials = ctx.workspace.get("linear_partials", need, 1, torch.float32) if need else None
         if kernels.linear_mfma(a, w, bias, out, n_rows, epilogue, partials=partials):
             return False
+    if scatter is not None and epilogue == kernels.EPI_NONE and kernels.linear_exact_qkv(a, w, bias, out, n_rows, scatter):
+        return True
     kernels.linear_generic(a, w, bias, out, n_rows, epilogue)
     return False

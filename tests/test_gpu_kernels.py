@@ -146,6 +146,30 @@ def test_float32_product_keeps_its_sums_whatever_the_tiles(k):
         assert (part[rows] == 7.0).all()
 
 
+@pytest.mark.parametrize("n,k,h,hk,d", [(1, 64, 4, 4, 16), (16, 300, 3, 1, 10), (40, 36, 3, 3, 12), (300, 512, 8, 8, 64),
+                                        (1030, 256, 24, 20, 128), (70, 33, 1, 1, 33)])
+def test_float32_product_stores_keys_and_values(n, k, h, hk, d):
+    """The projection that also stores its key and value columns into their pages: the same bits as the plain product
+    followed by the kernel that copies them, in each of the product's kernels and also where no four columns of a head
+    lie together; a padded row (slot -1) is stored nowhere."""
+    g = torch.Generator().manual_seed(n)
+    q_width, kv_width, page = h * d, hk * d, 5
+    o = q_width + 2 * kv_width
+    a, w, bias = rnd(g, n, k).to(DEV), rnd(g, o, k).to(DEV), rnd(g, o).to(DEV)
+    pages = -(-n // page) + 1
+    slots = torch.randperm(pages * page, generator=g)[:n].to(torch.int32)
+    slots[n // 2] = -1 if n > 1 else slots[n // 2]
+    slots = slots.to(DEV)
+    got, want = torch.full((n, o), 7.0, device=DEV), torch.full((n, o), 7.0, device=DEV)
+    pools = [torch.full((pages, hk, page, d), float("nan"), device=DEV) for _ in range(4)]
+    assert kernels.linear_exact_qkv(a, w, bias, got, n, (pools[0], pools[1], slots, q_width, kv_width))
+    kernels.linear_generic(a, w, bias, want, n)
+    kernels.kv_write(want, q_width, q_width + kv_width, pools[2], pools[3], slots, n)
+    assert torch.equal(got, want)
+    assert torch.equal(pools[0].nan_to_num(9.0), pools[2].nan_to_num(9.0))
+    assert torch.equal(pools[1].nan_to_num(9.0), pools[3].nan_to_num(9.0))
+
+
 def test_linear_generic_refuses_tensors_off_the_gpu():
     a, w = torch.zeros(4, 40, device=DEV), torch.zeros(8, 40, device=DEV)
     with pytest.raises(kernels.KernelError, match="GPU"):

@@ -232,6 +232,130 @@ __global__ __launch_bounds__(T) void streams_step_kernel(
   }
 }
 
+// The same for up to four streams and rows that 16-byte pieces cover (up to 8,192 columns): T threads a token, just as many as
+// the row has pieces (up to 1,024, then V pieces a thread), so that every load of the token is on its way at once and none
+// is made for columns that are not there.  The kernel above walks 16 columns a thread whatever the width, 4 bytes a load:
+// in a decode step of 8 tokens x 2 streams x 2,048 columns 9.8 us against 4.1 here, with 3,000 tokens 51 against 36.
+// The threads depend on the width alone, so a token's sums run in one order in every step.
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float ss_f4;
+
+template <typename OT, int T, int V, int S>
+__global__ __launch_bounds__(T) void streams_step_vec_kernel(
+    float* __restrict__ x, const float* __restrict__ mix, const float* __restrict__ out, float* __restrict__ y,
+    int fold, int clear, const float* __restrict__ coef, float* __restrict__ u, const float* __restrict__ gain,
+    const float* __restrict__ beta, float eps, OT* __restrict__ h, int width) {
+  __shared__ float red[T / 64][2];
+  const int tid = threadIdx.x;
+  const long n = blockIdx.x;
+  float* xr = x + n * (long)S * width;
+  float* yr = y + n * (long)width;
+  const ss_f4 zero = {0.f, 0.f, 0.f, 0.f};
+  ss_f4 old[V][S], yv[V], gk[V], bk[V], keep[V];
+#pragma unroll
+  for (int i = 0; i < V; ++i) {
+    const int c = 4 * (tid + i * T), at = c < width ? c : 0;
+#pragma unroll
+    for (int s = 0; s < S; ++s) old[i][s] = *reinterpret_cast<const ss_f4*>(xr + (long)s * width + at);
+    yv[i] = zero;
+    if (fold) yv[i] = *reinterpret_cast<const ss_f4*>(yr + at);
+    gk[i] = *reinterpret_cast<const ss_f4*>(gain + at);
+    bk[i] = zero;
+    if (beta) bk[i] = *reinterpret_cast<const ss_f4*>(beta + at);
+  }
+  float sum = 0.f;
+#pragma unroll
+  for (int i = 0; i < V; ++i) {
+    const int c = 4 * (tid + i * T);
+    keep[i] = zero;
+    if (c >= width) continue;
+#pragma unroll
+    for (int t = 0; t < S; ++t) {
+      ss_f4 acc = old[i][t];
+      if (fold) {
+        acc = zero;
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[e] = fmaf(mix[s * S + t], old[i][s][e], acc[e]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] = fmaf(out[t], yv[i][e], acc[e]);
+        *reinterpret_cast<ss_f4*>(xr + (long)t * width + c) = acc;
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) keep[i][e] = fmaf(coef[t], acc[e], keep[i][e]);
+    }
+    if (clear) *reinterpret_cast<ss_f4*>(yr + c) = zero;
+    *reinterpret_cast<ss_f4*>(u + n * (long)width + c) = keep[i];
+    sum += (keep[i][0] + keep[i][1]) + (keep[i][2] + keep[i][3]);
+  }
+  // the sum over the token, then those of the distances from the mean and of their squares in one go
+  const int wave = tid >> 6, lane = tid & 63;
+  sum = wave_sum(sum);
+  if (lane == 0) red[wave][0] = sum;
+  __syncthreads();
+  float mean = 0.f;
+#pragma unroll
+  for (int w = 0; w < T / 64; ++w) mean += red[w][0];
+  mean /= (float)width;
+  float e1 = 0.f, e2 = 0.f;
+#pragma unroll
+  for (int i = 0; i < V; ++i) {
+    if (4 * (tid + i * T) >= width) continue;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      keep[i][e] -= mean;
+      e1 += keep[i][e];
+      e2 = fmaf(keep[i][e], keep[i][e], e2);
+    }
+  }
+  e1 = wave_sum(e1);
+  e2 = wave_sum(e2);
+  __syncthreads();   // the last use of red is over
+  if (lane == 0) {
+    red[wave][0] = e1;
+    red[wave][1] = e2;
+  }
+  __syncthreads();
+  float corr = 0.f, var = 0.f;
+#pragma unroll
+  for (int w = 0; w < T / 64; ++w) {
+    corr += red[w][0];
+    var += red[w][1];
+  }
+  corr /= (float)width;
+  var = fmaxf(var / (float)width - corr * corr, 0.f);
+  const float rstd = 1.0f / sqrtf(var + eps);
+#pragma unroll
+  for (int i = 0; i < V; ++i) {
+    const int c = 4 * (tid + i * T);
+    if (c >= width) continue;
+    float r[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) r[e] = (keep[i][e] - corr) * rstd * gk[i][e] + bk[i][e];
+    OT* dst = h + n * (long)width + c;
+    if (sizeof(OT) == 4) {
+      *reinterpret_cast<ss_f4*>(dst) = (ss_f4){r[0], r[1], r[2], r[3]};
+    } else {
+      *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf16x2(r[0], r[1]), pack_bf16x2(r[2], r[3]));
+    }
+  }
+}
+
+template <typename OT, int T, int V>
+static int launch_step_vec(float* x, const float* mix, const float* out, float* y, int fold, int clear, const float* coef,
+                           float* u, const float* gain, const float* beta, float eps, void* h, int n_rows, int width,
+                           int streams, hipStream_t stream) {
+#define SV_LAUNCH(S)                                                                                                  \
+  hipLaunchKernelGGL((streams_step_vec_kernel<OT, T, V, S>), dim3(n_rows), dim3(T), 0, stream, x, mix, out, y, fold,  \
+                     clear, coef, u, gain, beta, eps, (OT*)h, width)
+  if (streams == 1) SV_LAUNCH(1);
+  else if (streams == 2) SV_LAUNCH(2);
+  else if (streams == 3) SV_LAUNCH(3);
+  else SV_LAUNCH(4);
+#undef SV_LAUNCH
+  return mgpt_last_error();
+}
+
 // y [n_rows, width]: with fold, the output of the sublayer whose write is still to be made (without, the
 // streams are read as they are); with clear, it is zero afterwards.  u: float32 [n_rows, width]; h:
 // [n_rows, width] in h_dtype.  x, y, u and h are four different buffers.
@@ -241,6 +365,22 @@ extern "C" int mgpt_streams_step(float* x, const float* mix, const float* out, f
   if (n_rows == 0) return MGPT_OK;
   if (!x || !coef || !u || !gain || !h || (fold && (!mix || !out)) || ((fold || clear) && !y)) return MGPT_ERR_NULL;
   if (n_rows < 0 || width <= 0 || streams <= 0 || streams > MGPT_MAX_STREAMS) return MGPT_ERR_BAD_SHAPE;
+  const uintptr_t together = (uintptr_t)x | (uintptr_t)y | (uintptr_t)u | (uintptr_t)gain | (uintptr_t)beta | (uintptr_t)h;
+  if (streams <= 4 && width % 4 == 0 && width <= 8192 && (together & 15) == 0 && (h_dtype == MGPT_F32 || h_dtype == MGPT_BF16)) {
+    const int pieces = width / 4;
+#define SV_WIDTH(T, V)                                                                                                \
+  return h_dtype == MGPT_F32 ? launch_step_vec<float, T, V>(x, mix, out, y, fold, clear, coef, u, gain, beta, eps, h, \
+                                                            n_rows, width, streams, stream)                           \
+                             : launch_step_vec<bf16_t, T, V>(x, mix, out, y, fold, clear, coef, u, gain, beta, eps,   \
+                                                             h, n_rows, width, streams, stream)
+    if (pieces <= 64) SV_WIDTH(64, 1);
+    if (pieces <= 128) SV_WIDTH(128, 1);
+    if (pieces <= 256) SV_WIDTH(256, 1);
+    if (pieces <= 512) SV_WIDTH(512, 1);
+    if (pieces <= 1024) SV_WIDTH(1024, 1);
+    SV_WIDTH(1024, 2);
+#undef SV_WIDTH
+  }
   const bool few = n_rows <= 128 && width > 1024;   // more than four columns a thread otherwise
 #define SS_LAUNCH(OT, T)                                                                                          \
   hipLaunchKernelGGL((streams_step_kernel<OT, T>), dim3(n_rows), dim3(T), 0, stream, x, mix, out, y, fold, clear, \

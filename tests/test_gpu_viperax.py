@@ -78,6 +78,15 @@ def test_streams_write_read_and_norm_in_one_pass(dtype, streams, width, n):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("streams,width,n", [(1, 4, 1), (2, 256, 3), (3, 260, 2), (4, 516, 2), (5, 516, 2), (2, 1028, 5),
+                                             (2, 2048, 140), (4, 2052, 2), (2, 8192, 2), (2, 8196, 2), (3, 2046, 2)])
+def test_streams_write_read_and_norm_around_the_ends_of_its_kernels(dtype, streams, width, n):
+    """A thread per 16-byte piece of a row up to 4,096 columns, two pieces up to 8,192; more streams than four, wider rows
+    and rows that pieces do not cover go to the general kernel."""
+    test_streams_write_read_and_norm_in_one_pass(dtype, streams, width, n)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_embed_scaled_fills_every_stream(dtype):
     g = torch.Generator().manual_seed(1)
     table = _rnd(g, 50, 36, dtype=dtype)

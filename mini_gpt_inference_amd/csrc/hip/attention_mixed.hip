@@ -1,0 +1,124 @@
+// Attention of a step that has both, single tokens of decoding requests and prompt portions (bfloat16, head sizes 64 and 128),
+// in one launch.
+//
+// The two kind of tokens have kernels of their own (attention_decode_wide.hip, attention_prefill.hip), neither of which fills
+// the chip in such a step: a portion of 512 tokens x 12 heads is 96 tiles, eleven decoding requests are 132 workgroups, on 256
+// compute units, one behind the other 11.4 + 8.9 us a layer.  Here the first workgroups of the launch are tiles and the ones
+// behind them (token, head) pairs, both with the bodies of those kernels, so that they run side by side.  A pair's workgroup
+// holds a tile's LDS and registers, which is a compute unit, so it is done for up to 256 pairs; more go to their own kernel.
+//
+// Tiles are numbered over the requests on the device, 64 queries each: the launch is sized by how many tiles so many tokens of
+// so many requests can make at most, not by the longest portion times the requests.
+#include "attention_decode_wide.h"
+#include "attention_prefill.h"
+#include "launchers.h"
+
+struct MixedArgs {
+  const bf16_t* q; long ldq; bf16_t* out; long ldo;
+  const bf16_t* kpool; const bf16_t* vpool;
+  const int* block_tables; int max_blocks;
+  const int* positions; const int* q_req; const int* cu_q; const int* seq_lens;
+  int n_decode, first_req, n_req, tiles, single_below, n_head, n_kv_head, page_size, page_shift, num_pages;
+  unsigned int page_bytes;
+  float scale; int window;
+  const float* sinks; float softcap;
+  const bf16_t* gate; long ldg;
+  int keep_first; const float* score_bias; int chunked;
+};
+
+// IDENT: the single tokens are those of requests 0 .. n_decode - 1; else q_req names a token's request, and requests with more
+// than one token are passed over
+template <int D, int G, bool IDENT>
+__global__ __launch_bounds__(256 * G) void mixed_attention_kernel(MixedArgs a) {
+  constexpr int W = 4 * G;
+  static_assert(aw_lds_floats<D, W>() * (int)sizeof(float) <= pf_lds_bytes<D, G, 0>(), "one kind's LDS serves the other");
+  extern __shared__ __align__(16) bf16_t mx_lds[];
+  int b = blockIdx.x;
+  const int n_tiles = a.tiles * a.n_head;
+  if (b >= n_tiles) {
+    b -= n_tiles;
+    const float log2e = 1.4426950408889634f;
+    aw_decode<D, IDENT, 0, W>(a.q, a.ldq, a.out, a.ldo, a.kpool, a.vpool, a.block_tables, a.max_blocks, a.positions, a.q_req,
+                              IDENT ? nullptr : a.cu_q, a.n_head, a.n_kv_head, a.page_shift, a.num_pages, a.page_bytes,
+                              a.scale * log2e, a.window, a.sinks, a.softcap > 0.f ? a.softcap * log2e : 0.f, a.gate, a.ldg,
+                              a.keep_first, a.score_bias, a.chunked, nullptr, 0, nullptr, b % a.n_decode, b / a.n_decode,
+                              reinterpret_cast<float*>(mx_lds));
+    return;
+  }
+  const int h = b / a.tiles;
+  int tile = b - h * a.tiles, r = -1;
+  const int lane = threadIdx.x & 63;
+  for (int r0 = 0; r0 < a.n_req; r0 += MGPT_WAVE) {
+    const int rr = a.first_req + r0 + lane;
+    int tiles = 0;
+    if (r0 + lane < a.n_req) {
+      const int start = a.cu_q[rr], len = a.cu_q[rr + 1] - start;
+      if (!(len == 1 && start < a.single_below)) tiles = (len + PF_QT - 1) / PF_QT;
+    }
+    int upto = tiles;                                   // tiles of the requests up to this lane's
+    for (int off = 1; off < MGPT_WAVE; off <<= 1) {
+      const int o = __shfl_up(upto, off, MGPT_WAVE);
+      if (lane >= off) upto += o;
+    }
+    const uint64_t past = __ballot(upto > tile);
+    if (past) {
+      const int at = __ffsll((unsigned long long)past) - 1;
+      r = a.first_req + r0 + at;
+      tile -= __shfl(upto - tiles, at, MGPT_WAVE);
+      break;
+    }
+    tile -= __shfl(upto, MGPT_WAVE - 1, MGPT_WAVE);
+  }
+  if (r < 0) return;                                    // beyond the step's tiles: the whole workgroup
+  pf_tile<D, G, 0>(a.q, a.ldq, a.out, a.ldo, a.kpool, a.vpool, a.block_tables, a.max_blocks, a.cu_q, a.seq_lens, a.n_head,
+                   a.n_kv_head, a.page_size, a.scale, a.window, a.single_below, a.sinks, a.softcap, a.gate, a.ldg, a.keep_first,
+                   a.score_bias, a.chunked, nullptr, 0, nullptr, __builtin_amdgcn_readfirstlane(tile),
+                   __builtin_amdgcn_readfirstlane(r), h, mx_lds);
+}
+
+template <int D, int G, bool IDENT>
+static int launch(const MixedArgs& a, hipStream_t stream) {
+  constexpr int bytes = pf_lds_bytes<D, G, 0>();
+  static bool allowed = false;  // more LDS than a kernel gets without asking
+  if (!allowed) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(mixed_attention_kernel<D, G, IDENT>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (e != hipSuccess) return (int)e;
+    allowed = true;
+  }
+  hipLaunchKernelGGL((mixed_attention_kernel<D, G, IDENT>), dim3((a.tiles + a.n_decode) * a.n_head), dim3(256 * G), bytes, stream,
+                     a);
+  return mgpt_last_error();
+}
+
+// The step's first n_decode tokens: identity != 0: one each of requests 0 .. n_decode - 1; else those of them whose request
+// brings no other token.  And the tokens of requests first_req .. first_req + n_req - 1, n_tokens at most, without requests that
+// bring a single token as one of the step's first single_below.  positions, q_req: per token; cu_q, seq_lens, block_tables: per
+// request, from request 0 on.  The rest as mgpt_prefill_attention_bf16.  Refused (MGPT_ERR_BAD_SHAPE, nothing launched): other
+// head sizes than 64 and 128, page sizes that are no power of two, pools of 4 GiB and more, more than 256 (token, head) pairs.
+extern "C" int mgpt_mixed_attention_bf16(
+    const void* q, long ldq, void* out, long ldo, const void* kpool, const void* vpool, const int* block_tables, int max_blocks,
+    const int* positions, const int* q_req, const int* cu_q, const int* seq_lens, int n_decode, int identity, int first_req,
+    int n_req, int n_tokens, int single_below, int n_head, int n_kv_head, int head_dim, int page_size, int num_pages, float scale,
+    int window, const float* sinks, float softcap, const void* gate, long ldg, int keep_first, const float* score_bias,
+    int chunked, hipStream_t stream) {
+  if (!q || !out || !kpool || !vpool || !block_tables || !positions || !q_req || !cu_q || !seq_lens) return MGPT_ERR_NULL;
+  if (n_decode <= 0 || first_req < 0 || n_req <= 0 || n_tokens <= 0 || n_head <= 0 || n_kv_head <= 0 || n_head % n_kv_head != 0 ||
+      page_size <= 0 || (page_size & (page_size - 1)) != 0 || num_pages <= 0 || max_blocks <= 0 || window < 0 || ldq % 8 != 0 ||
+      ldo % 4 != 0 || (((size_t)out) & 7) != 0 || !(scale > 0.f) || keep_first < 0 || (score_bias && (sinks || softcap > 0.f)) ||
+      (head_dim != 64 && head_dim != 128) || (long)n_decode * n_head > 256 ||
+      (long)num_pages * n_kv_head * page_size * head_dim * 2 >= (1L << 32))
+    return MGPT_ERR_BAD_SHAPE;
+  const long tiles = ((long)n_tokens + (long)(PF_QT - 1) * (n_req < n_tokens ? n_req : n_tokens)) / PF_QT;
+  if ((tiles + n_decode) * n_head > 0x7fffffffL) return MGPT_ERR_TOO_LARGE;
+  int page_shift = 0;
+  while ((1 << page_shift) < page_size) ++page_shift;
+  const MixedArgs a = {(const bf16_t*)q, ldq, (bf16_t*)out, ldo, (const bf16_t*)kpool, (const bf16_t*)vpool, block_tables,
+                       max_blocks, positions, q_req, cu_q, seq_lens, n_decode, first_req, n_req, (int)tiles, single_below, n_head,
+                       n_kv_head, page_size, page_shift, num_pages, (unsigned int)(n_kv_head * page_size * head_dim * 2), scale,
+                       window, sinks, softcap, (const bf16_t*)gate, ldg, window == 0 ? 0 : keep_first, score_bias, chunked};
+  // two wave groups a tile while the tiles are few, as for prompt portions alone
+  if (head_dim == 128) return identity ? launch<128, 1, true>(a, stream) : launch<128, 1, false>(a, stream);
+  if (tiles * n_head <= 320) return identity ? launch<64, 2, true>(a, stream) : launch<64, 2, false>(a, stream);
+  return identity ? launch<64, 1, true>(a, stream) : launch<64, 1, false>(a, stream);
+}

@@ -35,6 +35,12 @@ int mgpt_paged_attention_generic(const void* q, long ldq, void* out, long ldo, c
     int fast_exp, const float* sinks, float softcap, const void* gate, long ldg, int keep_first, const float*
     score_bias, int chunked,
     const float* dist_bias, int bias_len, const float* slopes, hipStream_t stream);
+// attention_mixed.hip
+int mgpt_mixed_attention_bf16(const void* q, long ldq, void* out, long ldo, const void* kpool, const void* vpool, const int*
+    block_tables, int max_blocks, const int* positions, const int* q_req, const int* cu_q, const int* seq_lens, int n_decode,
+    int identity, int first_req, int n_req, int n_tokens, int single_below, int n_head, int n_kv_head, int head_dim, int
+    page_size, int num_pages, float scale, int window, const float* sinks, float softcap, const void* gate, long ldg, int
+    keep_first, const float* score_bias, int chunked, hipStream_t stream);
 // attention_prefill.hip
 int mgpt_prefill_attention_bf16(const void* q, long ldq, void* out, long ldo, const void* kpool, const void*
     vpool, const int* block_tables, int max_blocks, const int* cu_q, const int* seq_lens, int n_req, int
@@ -261,6 +267,7 @@ int mgpt_linear_mfma_grouped(const void* act, long lda, const void* w, long w_st
   X(mgpt_paged_attention_decode_bf16) \
   X(mgpt_kv_write) \
   X(mgpt_paged_attention_generic) \
+  X(mgpt_mixed_attention_bf16) \
   X(mgpt_prefill_attention_bf16) \
   X(mgpt_embed) \
   X(mgpt_layernorm) \

@@ -12,7 +12,7 @@ def _mixed_step(ctx, q, out, k_pool, v_pool, group, n_head: int, scale: float, w
     """A step with prompt portions.  The requests that lead the step with one token each (a scheduler
     puts the decoding requests first) go to the decode kernel, token n being request n; the rest,
     prompt portions mostly, to the MFMA tile kernel, which would spend a 64-query tile on a single
-    token.  False, having launched nothing, if the tile kernel does not take the case."""
+    token; both in one launch where the single tokens are few.  False, having launched nothing, if the tile kernel does not take the case."""
     mask = mask or {}
     q_lens = ctx.host_q_lens
     lead = 0
@@ -20,6 +20,10 @@ def _mixed_step(ctx, q, out, k_pool, v_pool, group, n_head: int, scale: float, w
         while lead < len(q_lens) and q_lens[lead] == 1:
             lead += 1
     rest = ctx.n_req - lead
+    if lead and rest and kernels.mixed_attention_bf16(
+            q, out, k_pool, v_pool, group.block_tables, ctx.positions, ctx.q_req, ctx.cu_q, ctx.seq_lens, lead, True, lead, rest,
+            ctx.n_tokens - lead, 0, n_head, scale, window, sinks=sinks, softcap=softcap, gate=gate, **mask):
+        return True
     if lead and rest and kernels.prefill_attention_bf16(
             q, out, k_pool, v_pool, group.block_tables[lead:], ctx.cu_q[lead:], ctx.seq_lens[lead:], rest,
             ctx.max_q_len, n_head, scale, window, sinks=sinks, softcap=softcap, gate=gate, **mask):
@@ -47,6 +51,10 @@ def _padded_mixed_step(ctx, q, out, k_pool, v_pool, group, n_head: int, scale: f
     mask = mask or {}
     r = ctx.cu_q.numel() - 1
     lead = min(ctx.lead_cap, ctx.n_rows)
+    if lead > 0 and kernels.mixed_attention_bf16(
+            q, out, k_pool, v_pool, group.block_tables, ctx.positions, ctx.q_req, ctx.cu_q, ctx.seq_lens, lead, False, 0, r,
+            ctx.n_rows, lead, n_head, scale, window, sinks=sinks, softcap=softcap, gate=gate, **mask):
+        return True
     singles = lead > 0 and kernels.paged_attention_decode_bf16(
         q, out, k_pool, v_pool, group.block_tables, ctx.positions, ctx.q_req, lead, n_head, scale, window,
         cu_q=ctx.cu_q, sinks=sinks, softcap=softcap, gate=gate, **mask)

@@ -808,6 +808,51 @@ def prefill_attention_bf16(q: torch.Tensor, out: torch.Tensor, k_pool: torch.Ten
     return True
 
 
+def mixed_attention_bf16(q: torch.Tensor, out: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor,
+                         block_tables: torch.Tensor, positions: torch.Tensor, q_req: torch.Tensor, cu_q: torch.Tensor,
+                         seq_lens: torch.Tensor, n_decode: int, identity: bool, first_req: int, n_req: int, n_tokens: int,
+                         single_below: int, n_head: int, scale: float, window: int = 0,
+                         sinks: Optional[torch.Tensor] = None, softcap: float = 0.0, gate: Optional[torch.Tensor] = None,
+                         keep_first: int = 0, score_bias: Optional[torch.Tensor] = None, chunked: bool = False,
+                         dist_bias: Optional[torch.Tensor] = None, slopes: Optional[torch.Tensor] = None) -> bool:
+    """What paged_attention_decode_bf16 does for a step's first n_decode tokens (identity: token n is request n's; else
+    those of requests that bring one token) and prefill_attention_bf16 for its requests first_req .. first_req + n_req - 1
+    (n_tokens tokens at most), in one launch.  False, having launched nothing, if it does not take the case."""
+    if q.dtype != torch.bfloat16 or dist_bias is not None or slopes is not None or n_decode <= 0 or n_req <= 0:
+        return False
+    _need_cuda(q, out, k_pool, v_pool, block_tables, positions, q_req, cu_q, seq_lens)
+    _need(k_pool.shape == v_pool.shape and k_pool.dim() == 4 and k_pool.is_contiguous() and v_pool.is_contiguous(),
+          "key and value pools must be dense [pages, kv_heads, page_size, head_dim]")
+    num_pages, n_kv_head, page_size, head_dim = k_pool.shape
+    if head_dim not in (64, 128) or q.stride(0) % 8 != 0 or q.data_ptr() % 16 != 0 \
+            or k_pool.data_ptr() % 16 != 0 or v_pool.data_ptr() % 16 != 0:
+        return False
+    _need(q.dtype == out.dtype == k_pool.dtype == v_pool.dtype, "queries, output and pools must share a dtype")
+    _need(q.dim() == 2 and q.stride(1) == 1 and out.dim() == 2 and out.stride(1) == 1,
+          "query and output rows must have unit inner stride")
+    _need(q.shape[0] >= max(n_decode, n_tokens) and out.shape[0] >= max(n_decode, n_tokens)
+          and q.shape[1] >= n_head * head_dim and out.shape[1] >= n_head * head_dim, "query/output buffers are too small")
+    _need(n_head % n_kv_head == 0, "n_head must be a multiple of the number of key/value heads")
+    r = max(first_req + n_req, n_decode if identity else 0)
+    _need(block_tables.dim() == 2 and block_tables.dtype == torch.int32 and block_tables.is_contiguous()
+          and block_tables.shape[0] >= r, "block_tables must be dense int32 [>=requests, max_blocks]")
+    _need_i32("positions", positions, n_decode)
+    _need_i32("q_req", q_req, n_decode)
+    _need_i32("cu_q", cu_q, r + 1)
+    _need_i32("seq_lens", seq_lens, r)
+    _need_sinks(sinks, n_head)
+    rc = library.kernels().mgpt_mixed_attention_bf16(
+        _ptr(q), q.stride(0), _ptr(out), out.stride(0), _ptr(k_pool), _ptr(v_pool), _ptr(block_tables), block_tables.shape[1],
+        _ptr(positions), _ptr(q_req), _ptr(cu_q), _ptr(seq_lens), n_decode, int(identity), first_req, n_req, n_tokens,
+        int(single_below), n_head, n_kv_head, head_dim, page_size, num_pages, float(scale), int(window), _ptr(sinks),
+        float(softcap), *_gate_args(gate, q, q.shape[0], n_head),
+        *_mask_args(keep_first, score_bias, n_head, sinks, softcap, chunked)[:3], _stream())
+    if rc == -2:
+        return False
+    _check(rc, "mixed_attention_bf16")
+    return True
+
+
 # ---------------------------------------------------------------- decode steps of few rows, fused
 FUSED_MAX_WIDTH = 512
 FUSED_MLP_SLICE = 64

@@ -137,6 +137,7 @@ def _declare_optional(lib: ctypes.CDLL) -> None:
         "mgpt_linear_mfma_partials": [I, I, I, I],
         "mgpt_linear_mfma_parts": [P, L, P, P, P, L, I, I, I, P],
         "mgpt_linear_mfma_qkv": [P, L, P, P, P, L, I, I, I, P, P, P, I, I, I, I, I, I, P],
+        "mgpt_mixed_attention_bf16": [P, L, P, L, P, P, P, I, P, P, P, P, I, I, I, I, I, I, I, I, I, I, I, F, I, P, F, P, L, I, P, I, P],
         "mgpt_prefill_attention_bf16": [P, L, P, L, P, P, P, I, P, P, I, I, I, I, I, I, F, I, I, P, F, P, L, I, P, I, P, I, P, P],
         # a residual that is still a sum: base, partials, n_parts, part_stride, token table, position table, ids, positions
         "mgpt_fused_attention_decode": [P, P, I, L, P, P, P, P, P, P, P, P, F, P, P, P, P, P, L, P, P, P, P, I, P, P,

@@ -662,6 +662,38 @@ ATTENTION_CASES = [
 ]
 
 
+@pytest.mark.parametrize("window", [0, 90])
+@pytest.mark.parametrize("d,h,hk", [(64, 12, 12), (64, 4, 1), (128, 8, 2)])
+@pytest.mark.parametrize("seq_lens,q_lens", [([40, 513, 700], [1, 1, 130]), ([1, 64], [1, 63]), ([300] * 20 + [65, 1, 900], [1] * 20 + [65, 1, 640]),
+                                             ([9] * 3 + [70] * 70, [1] * 3 + [66] * 70), ([500, 1000], [1, 1000])])
+def test_single_tokens_and_portions_in_one_launch(seq_lens, q_lens, d, h, hk, window):
+    """The launch that has a step's single tokens beside its prompt portions: both kinds against the plain attention, as the
+    step's own requests (the leading ones are the single tokens) and as a padded step (which requests bring one token is
+    read from cu_q, the last single token of the portions' part among them; requests and tokens of the padding are left
+    alone), around a tile, few tiles and many, and with more requests than a wave numbers at a time."""
+    c = PagedCase(seq_lens, q_lens, h=h, hk=hk, d=d, page=16, dtype="bfloat16", seed=d + len(q_lens))
+    n, r = c.n, len(q_lens)
+    lead = next(i for i, q in enumerate(q_lens) if q != 1)
+    scale, want = d ** -0.5, c.want(d ** -0.5, window)
+    positions = i32([s - q + t for s, q in zip(seq_lens, q_lens) for t in range(q)])
+    out = torch.full((n, h * d), float("nan"), dtype=torch.bfloat16, device=DEV)
+    args = (c.q_flat, out, c.kp, c.vp, c.bt, positions, c.q_req, c.cu, c.sl)
+    took = lead * h <= 256
+    assert kernels.mixed_attention_bf16(*args, lead, True, lead, r - lead, n - lead, 0, h, scale, window) == took
+    if took:
+        helpers.assert_close(out, want, "bfloat16", "the step's own requests")
+    cap, rows = 16, n + 5
+    pad = lambda t, size, fill: torch.cat([t, torch.full((size - t.shape[0], *t.shape[1:]), fill, dtype=t.dtype, device=DEV)])
+    padded = torch.full((rows, h * d), 7.0, dtype=torch.bfloat16, device=DEV)
+    took = kernels.mixed_attention_bf16(
+        pad(c.q_flat, rows, 0.0), padded, c.kp, c.vp, pad(c.bt, r + 4, -1), pad(positions, rows, 0), pad(c.q_req, rows, -1),
+        pad(c.cu, r + 5, n), pad(c.sl, r + 4, 0), min(cap, rows), False, 0, r + 4, rows, min(cap, rows), h, scale, window)
+    assert took == (min(cap, rows) * h <= 256)
+    if took:
+        helpers.assert_close(padded[:n], want, "bfloat16", "a padded step")
+        assert (padded[n:] == 7.0).all()
+
+
 @pytest.mark.parametrize("window", [0, 100])
 @pytest.mark.parametrize("d,n", [(16, 129), (32, 129), (64, 128), (64, 129), (128, 64), (128, 65)])
 def test_decode_attention_of_many_tokens(d, n, window):

@@ -180,6 +180,56 @@ __global__ void layernorm_vec_kernel(const float* __restrict__ x, const float* _
   }
 }
 
+// The same for rows of 513 to 4,096 values (multiples of 4, 16-byte aligned): a workgroup a row with a vector of four a lane, W
+// waves, whose sums meet in LDS.  One wave a row has three to eight vectors a lane there, and their loads, sums and stores
+// one behind the other (us in a graph of such calls, a wave a row / here: 32 rows of 768 2.87 / 2.49, of 1,600 3.70 / 2.71; of
+// 4,096, which had 4-byte loads, 29.5 / 3.3; 512 rows of 1,600 3.97 / 3.47).  With many rows there are waves enough and the
+// meeting only costs (1,024 rows of 1,600 4.23 / 4.50): bfloat16 outputs of more than 640 rows of up to 2,048 stay with the
+// kernel above.  Float32 outputs, the 32-bit path's, always come here where it takes the row (4,096 rows of 768 5.6 / 6.6, beside
+// products of hundreds): their sums run in one order whatever the number of rows.
+template <typename OT, int W>
+__global__ __launch_bounds__(64 * W) void layernorm_row_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                               const float* __restrict__ b, OT* __restrict__ out,
+                                                               const int* __restrict__ rows, int width, float eps) {
+  __shared__ float red[W][2], red_sum[W];
+  const int tid = threadIdx.x, wave = tid >> 6;
+  const long src = rows ? rows[blockIdx.x] : (long)blockIdx.x;
+  const bool in = 4 * tid < width;
+  const int c = in ? tid : 0;
+  float4 v = reinterpret_cast<const float4*>(x + src * (long)width)[c];
+  const float4 g = reinterpret_cast<const float4*>(w)[c];
+  const float4 o = b ? reinterpret_cast<const float4*>(b)[c] : make_float4(0.f, 0.f, 0.f, 0.f);
+  const float s = wave_sum(in ? (v.x + v.y) + (v.z + v.w) : 0.f);
+  if ((tid & 63) == 0) red_sum[wave] = s;
+  __syncthreads();
+  float mean = 0.f;
+#pragma unroll
+  for (int i = 0; i < W; ++i) mean += red_sum[i];
+  mean /= (float)width;
+  v.x -= mean; v.y -= mean; v.z -= mean; v.w -= mean;
+  const float e = wave_sum(in ? (v.x + v.y) + (v.z + v.w) : 0.f);
+  const float q = wave_sum(in ? fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, v.w * v.w))) : 0.f);
+  if ((tid & 63) == 0) {
+    red[wave][0] = e;
+    red[wave][1] = q;
+  }
+  __syncthreads();
+  float corr = 0.f, var = 0.f;
+#pragma unroll
+  for (int i = 0; i < W; ++i) {
+    corr += red[i][0];
+    var += red[i][1];
+  }
+  corr /= (float)width;
+  const float rstd = 1.0f / sqrtf(fmaxf(var / (float)width - corr * corr, 0.f) + eps);
+  if (!in) return;
+  const float y0 = (v.x - corr) * rstd * g.x + o.x, y1 = (v.y - corr) * rstd * g.y + o.y;
+  const float y2 = (v.z - corr) * rstd * g.z + o.z, y3 = (v.w - corr) * rstd * g.w + o.w;
+  OT* orow = out + (long)blockIdx.x * width;
+  if (sizeof(OT) == 4) reinterpret_cast<float4*>(orow)[tid] = make_float4(y0, y1, y2, y3);
+  else reinterpret_cast<uint2*>(orow)[tid] = make_uint2(pack_bf16x2(y0, y1), pack_bf16x2(y2, y3));
+}
+
 // rows: optional gather list (n_rows entries) of source rows of x; out row i <- x row rows[i].
 extern "C" int mgpt_layernorm(const float* x, const float* w, const float* b, void* out,
                               const int* rows, int n_rows, int width, float eps, int out_dtype,
@@ -189,23 +239,38 @@ extern "C" int mgpt_layernorm(const float* x, const float* w, const float* b, vo
   if (n_rows < 0 || width <= 0) return MGPT_ERR_BAD_SHAPE;
   const int rows_per_block = 4;
   dim3 grid((n_rows + rows_per_block - 1) / rows_per_block), block(rows_per_block * MGPT_WAVE);
-  const bool vec = (width % 4) == 0 && width <= MGPT_WAVE * 4 * 8 &&
+  const bool vec = (width % 4) == 0 && width <= 4096 &&
                    ((((size_t)x) | ((size_t)w) | ((size_t)b) | ((size_t)out)) & 15) == 0;
-  const int need = (width / 4 + MGPT_WAVE - 1) / MGPT_WAVE;   // vectors of four per lane
+  const int need = (width / 4 + MGPT_WAVE - 1) / MGPT_WAVE;   // vectors of four per lane of one wave
 #define LN_LAUNCH(OT, V) \
   hipLaunchKernelGGL((layernorm_vec_kernel<OT, V>), grid, block, 0, stream, x, w, b, (OT*)out, rows, n_rows, width, eps)
-#define LN_PICK(OT)                    \
-  if (need <= 1) LN_LAUNCH(OT, 1);     \
-  else if (need <= 2) LN_LAUNCH(OT, 2); \
-  else if (need <= 3) LN_LAUNCH(OT, 3); \
+#define LN_ROW(OT, W) \
+  hipLaunchKernelGGL((layernorm_row_kernel<OT, W>), dim3(n_rows), dim3(64 * W), 0, stream, x, w, b, (OT*)out, rows, width, eps)
+#define LN_PICK_WAVE(OT)                \
+  if (need <= 3) LN_LAUNCH(OT, 3);      \
   else if (need <= 4) LN_LAUNCH(OT, 4); \
   else if (need <= 6) LN_LAUNCH(OT, 6); \
   else LN_LAUNCH(OT, 8)
+#define LN_PICK_ROW(OT)               \
+  if (need <= 3) LN_ROW(OT, 3);       \
+  else if (need <= 4) LN_ROW(OT, 4);  \
+  else if (need <= 5) LN_ROW(OT, 5);  \
+  else if (need <= 6) LN_ROW(OT, 6);  \
+  else if (need <= 7) LN_ROW(OT, 7);  \
+  else if (need <= 8) LN_ROW(OT, 8);  \
+  else LN_ROW(OT, 16)
   if (vec && out_dtype == MGPT_F32) {
-    LN_PICK(float);
+    if (need <= 1) LN_LAUNCH(float, 1);
+    else if (need <= 2) LN_LAUNCH(float, 2);
+    else { LN_PICK_ROW(float); }
   } else if (vec && out_dtype == MGPT_BF16) {
-    LN_PICK(bf16_t);
-#undef LN_PICK
+    if (need <= 1) LN_LAUNCH(bf16_t, 1);
+    else if (need <= 2) LN_LAUNCH(bf16_t, 2);
+    else if (n_rows <= 640 || need > 8) { LN_PICK_ROW(bf16_t); }
+    else { LN_PICK_WAVE(bf16_t); }
+#undef LN_PICK_ROW
+#undef LN_PICK_WAVE
+#undef LN_ROW
 #undef LN_LAUNCH
   } else if (out_dtype == MGPT_F32) {
     hipLaunchKernelGGL(layernorm_kernel<float>, grid, block, 0, stream, x, w, b, (float*)out, rows,

@@ -109,6 +109,14 @@ def test_the_step_between_two_sublayers(h_dtype, branches, n, width):
             assert (h[n] == 5.0).all()
 
 
+@pytest.mark.parametrize("h_dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("branches,n,width", [(1, 2, 4), (2, 2, 256), (1, 3, 260), (2, 2, 512), (2, 2, 516), (1, 2, 1028),
+                                              (2, 2, 4096), (1, 2, 4096), (1, 2, 4100), (2, 2, 2050)])
+def test_the_step_between_two_sublayers_around_the_ends_of_its_kernels(h_dtype, branches, n, width):
+    """A 16-byte piece a lane in 1, 2, 4, 8 or 16 waves; longer rows and rows that pieces do not cover go to the general kernel."""
+    test_the_step_between_two_sublayers(h_dtype, branches, n, width)
+
+
 def _freq(dims, base, factor=1.0):
     return torch.tensor([base ** (-2.0 * i / dims) / factor for i in range(dims // 2)], dtype=torch.float64).float()
 

@@ -58,6 +58,13 @@ def test_layer_norm(out_dtype, width, bias, eps):
     helpers.assert_close(out2, want[rows], out_dtype, "layer_norm gather")
 
 
+@pytest.mark.parametrize("out_dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("width", [516, 772, 1028, 1540, 2044, 4096, 4100])
+def test_layer_norm_of_rows_in_several_waves(out_dtype, width):
+    """A 16-byte piece a lane in 3, 4, 6, 8 or 16 waves; longer rows go to the kernel with a wave a row."""
+    test_layer_norm(out_dtype, width, True, 1e-5)
+
+
 # ----------------------------------------------------------------------------- linear
 def _linear_want(a, w, bias, epi, prev):
     y = P.plain_linear(a.double(), w.double(), None if bias is None else bias.double())

@@ -217,11 +217,26 @@ __global__ __launch_bounds__(256) void state_inputs_kernel(const void* __restric
   }
 }
 
-template <int EB>     // value channels a workgroup: 32, or 16 where that is what fills the machine
+// A request's chunks are a chain, 5 to 7 us each, and a step of few long prompts has few chains: 8 requests x 8 heads with the
+// longest of 1,024 tokens took 224 us, 32 chunks one behind the other.  With scratch for them the requests are cut into segments
+// of 256 tokens instead (numbered over the requests one behind the other): a first launch makes, for all segments but a request's
+// last, what the segment adds to the state (sum_t L^(n-1-t) k_t v_t^T, a third of a chunk's work; the first segment starts from
+// the request's state and so leaves the state behind it, and copies that state to the last segment's place, where nobody adds);
+// a second launch puts a segment's starting state together from those before it, S <- L^256 S + added, and runs its chunks.
+// 49 + 115 us there; segments of 128 tokens take 47 + 127.  The caller decides where that is less (a chunk's work is then done
+// 1.4 times, so not where the chains fill the chip).  Error against 64 bits over 1,024 tokens: 3.8e-7, whole 4.5e-7.
+#define DC_SEGMENT 256
+#define DC_WHOLE 0      // a request's chunks one behind the other
+#define DC_ADDED 1      // what the segments add
+#define DC_OUTPUTS 2    // the segments' outputs, and the last one's state
+
+// EB: value channels a workgroup: 32, or 16 where that is what fills the machine.  added: [segments][n_head][E][Dp].
+template <int EB, int MODE>
 __global__ __launch_bounds__(256) void decay_state_chunk_kernel(
     const float* __restrict__ qk, const void* __restrict__ z, int dtype, long ldz, int v_off, int n_head, int D, int E,
     int act, const int* __restrict__ positions, const float* __restrict__ decay, float* __restrict__ state,
-    const int* __restrict__ state_slots, const int* __restrict__ cu_q, float* __restrict__ out, long ldo) {
+    const int* __restrict__ state_slots, const int* __restrict__ cu_q, float* __restrict__ out, long ldo, int n_req,
+    float* __restrict__ added) {
   constexpr int NJ = EB / 16;     // column tiles of the workgroup's value channels
   // queries and keys [token][d]; the state and the values transposed, [value channel][d] and [value channel][token];
   // P [token][token].  Every product's index of summation runs along a row, so that a lane's operands of four
@@ -230,21 +245,69 @@ __global__ __launch_bounds__(256) void decay_state_chunk_kernel(
   __shared__ __attribute__((aligned(16))) float Qs[DC_C][DC_LDQ], Ks[DC_C][DC_LDQ], St[EB][DC_LDQ], Vt[EB][DC_LDP],
       Ps[DC_C][DC_LDP];
   __shared__ float pw[DC_C + 1];
-  const int r = blockIdx.x, h = blockIdx.y, e0 = blockIdx.z * EB, tid = threadIdx.x;
-  const int slot = state_slots[r];
-  const int t_begin = cu_q[r], t_end = cu_q[r + 1];
-  if (slot < 0 || t_end <= t_begin) return;     // a request of the padding
+  const int h = blockIdx.y, e0 = blockIdx.z * EB, tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63, r16 = lane & 15, g = lane >> 4;
+  int r = blockIdx.x, seg = 0, first = 0;       // the request, its segment, the number of its first segment
+  if (MODE != DC_WHOLE) {
+    int left = blockIdx.x;
+    r = -1;
+    for (int r0 = 0; r0 < n_req; r0 += 64) {
+      const int rr = r0 + lane;
+      const int mine = rr < n_req ? (cu_q[rr + 1] - cu_q[rr] + DC_SEGMENT - 1) / DC_SEGMENT : 0;
+      int upto = mine;                          // segments of the requests up to this lane's
+      for (int off = 1; off < 64; off <<= 1) {
+        const int o = __shfl_up(upto, off, 64);
+        if (lane >= off) upto += o;
+      }
+      const unsigned long long past = __ballot(upto > left);
+      if (past) {
+        const int at = __ffsll(past) - 1;
+        r = r0 + at;
+        seg = left - __shfl(upto - mine, at, 64);
+        break;
+      }
+      left -= __shfl(upto, 63, 64);
+    }
+    if (r < 0) return;                          // beyond the step's segments: the whole workgroup
+    first = (int)blockIdx.x - seg;
+  }
+  const int slot = state_slots[r];
+  int t_begin = cu_q[r], t_end = cu_q[r + 1];
+  if (slot < 0 || t_end <= t_begin) return;     // a request of the padding
+  const int n_seg = (t_end - t_begin + DC_SEGMENT - 1) / DC_SEGMENT;
+  if (MODE == DC_ADDED && seg == n_seg - 1) return;
+  const bool fresh = positions[t_begin] == 0;
+  if (MODE != DC_WHOLE) {
+    t_begin += seg * DC_SEGMENT;
+    if (seg != n_seg - 1) t_end = t_begin + DC_SEGMENT;
+  }
   const int Dp = (D + 15) & ~15;                // rows of S and steps along d, padded with zeros
   const int HD = n_head * D;
   const float lambda = decay[h];
   const float log_l = logf(lambda);
   if (tid <= DC_C) pw[tid] = tid == 0 ? 1.0f : expf((float)tid * log_l);
   float* st = state + ((long)slot * n_head + h) * (long)D * E;
-  const bool fresh = positions[t_begin] == 0;
-  for (int i = tid; i < Dp * EB; i += 256) {
-    const int d = i / EB, c = i - d * EB;
-    St[c][d] = (!fresh && d < D && e0 + c < E) ? st[(long)d * E + e0 + c] : 0.f;
+  // a segment's place in `added`, and its row of value channel e0 + c
+  auto place = [&](int number, int c) { return added + (((long)number * n_head + h) * E + e0 + c) * Dp; };
+  if (MODE == DC_OUTPUTS && n_seg > 1) {
+    const float across = expf((float)DC_SEGMENT * log_l);
+    for (int i = tid; i < Dp * EB; i += 256) {
+      const int c = i / Dp, d = i - c * Dp;
+      float v = 0.f;
+      if (e0 + c < E) {
+        v = place(seg == 0 ? first + n_seg - 1 : first, c)[d];
+        for (int j = 1; j < seg; ++j) v = fmaf(across, v, place(first + j, c)[d]);
+      }
+      St[c][d] = v;
+    }
+  } else {
+    const bool empty = fresh || (MODE == DC_ADDED && seg > 0);
+    for (int i = tid; i < Dp * EB; i += 256) {
+      const int d = i / EB, c = i - d * EB;
+      const float v = (!empty && d < D && e0 + c < E) ? st[(long)d * E + e0 + c] : 0.f;
+      St[c][d] = v;
+      if (MODE == DC_ADDED && seg == 0 && e0 + c < E) place(first + n_seg - 1, c)[d] = v;
+    }
   }
   const int ti = wave >> 1, tj = wave & 1;      // this wave's 16 x 16 tile of P and of the chunk's outputs
 
@@ -259,7 +322,7 @@ __global__ __launch_bounds__(256) void decay_state_chunk_kernel(
       const int i = tid + u * 256, tt = i / Dp, d = i - tt * Dp;
       const bool ok = i < DC_C * Dp && tt < nt && d < D;
       const long at = (long)(t0 + tt) * 2 * HD + (long)h * D + d;
-      q_r[u] = ok ? qk[at] : 0.f;
+      if (MODE != DC_ADDED) q_r[u] = ok ? qk[at] : 0.f;
       k_r[u] = ok ? qk[at + HD] : 0.f;
     }
 #pragma unroll
@@ -278,7 +341,7 @@ __global__ __launch_bounds__(256) void decay_state_chunk_kernel(
     for (int u = 0; u < QK_PT; ++u) {
       const int i = tid + u * 256, tt = i / Dp, d = i - tt * Dp;
       if (i < DC_C * Dp) {
-        Qs[tt][d] = q_r[u];
+        if (MODE != DC_ADDED) Qs[tt][d] = q_r[u];
         Ks[tt][d] = k_r[u];
       }
     }
@@ -289,49 +352,51 @@ __global__ __launch_bounds__(256) void decay_state_chunk_kernel(
     }
     __syncthreads();
     fetch(t0 + DC_C);     // (behind the last chunk: no token is left, nothing is loaded)
-    // ---- P = Q K^T with the decay of the distance, lower triangle
-    {
-      f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-      if (tj <= ti) {
+    if (MODE != DC_ADDED) {
+      // ---- P = Q K^T with the decay of the distance, lower triangle
+      {
+        f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+        if (tj <= ti) {
 #pragma unroll 2
-        for (int k0 = 0; k0 < Dp; k0 += 16) {
-          const f32x4_t a = *reinterpret_cast<const f32x4_t*>(&Qs[ti * 16 + r16][k0 + 4 * g]);
-          const f32x4_t b = *reinterpret_cast<const f32x4_t*>(&Ks[tj * 16 + r16][k0 + 4 * g]);
+          for (int k0 = 0; k0 < Dp; k0 += 16) {
+            const f32x4_t a = *reinterpret_cast<const f32x4_t*>(&Qs[ti * 16 + r16][k0 + 4 * g]);
+            const f32x4_t b = *reinterpret_cast<const f32x4_t*>(&Ks[tj * 16 + r16][k0 + 4 * g]);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], acc, 0, 0, 0);
+            for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], acc, 0, 0, 0);
+          }
+        }
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int i = ti * 16 + 4 * g + v, j = tj * 16 + r16;
+          Ps[i][j] = j <= i ? acc[v] * pw[i - j] : 0.f;
         }
       }
+      __syncthreads();
+      // ---- o = P V + L^(i+1) Q S: the tiles (oi, oj) of the chunk's [32, EB] outputs
+      for (int t = wave; t < 2 * NJ; t += 4) {
+        const int oi = t / NJ, oj = t - oi * NJ;
+        f32x4_t a1 = {0.f, 0.f, 0.f, 0.f}, a2 = {0.f, 0.f, 0.f, 0.f};
+        for (int k0 = 0; k0 < (oi + 1) * 16; k0 += 16) {
+          const f32x4_t a = *reinterpret_cast<const f32x4_t*>(&Ps[oi * 16 + r16][k0 + 4 * g]);
+          const f32x4_t b = *reinterpret_cast<const f32x4_t*>(&Vt[oj * 16 + r16][k0 + 4 * g]);
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int i = ti * 16 + 4 * g + v, j = tj * 16 + r16;
-        Ps[i][j] = j <= i ? acc[v] * pw[i - j] : 0.f;
-      }
-    }
-    __syncthreads();
-    // ---- o = P V + L^(i+1) Q S: the tiles (oi, oj) of the chunk's [32, EB] outputs
-    for (int t = wave; t < 2 * NJ; t += 4) {
-      const int oi = t / NJ, oj = t - oi * NJ;
-      f32x4_t a1 = {0.f, 0.f, 0.f, 0.f}, a2 = {0.f, 0.f, 0.f, 0.f};
-      for (int k0 = 0; k0 < (oi + 1) * 16; k0 += 16) {
-        const f32x4_t a = *reinterpret_cast<const f32x4_t*>(&Ps[oi * 16 + r16][k0 + 4 * g]);
-        const f32x4_t b = *reinterpret_cast<const f32x4_t*>(&Vt[oj * 16 + r16][k0 + 4 * g]);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) a1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], a1, 0, 0, 0);
-      }
+          for (int e = 0; e < 4; ++e) a1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], a1, 0, 0, 0);
+        }
 #pragma unroll 2
-      for (int k0 = 0; k0 < Dp; k0 += 16) {
-        const f32x4_t a = *reinterpret_cast<const f32x4_t*>(&Qs[oi * 16 + r16][k0 + 4 * g]);
-        const f32x4_t b = *reinterpret_cast<const f32x4_t*>(&St[oj * 16 + r16][k0 + 4 * g]);
+        for (int k0 = 0; k0 < Dp; k0 += 16) {
+          const f32x4_t a = *reinterpret_cast<const f32x4_t*>(&Qs[oi * 16 + r16][k0 + 4 * g]);
+          const f32x4_t b = *reinterpret_cast<const f32x4_t*>(&St[oj * 16 + r16][k0 + 4 * g]);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) a2 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], a2, 0, 0, 0);
-      }
+          for (int e = 0; e < 4; ++e) a2 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], a2, 0, 0, 0);
+        }
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int i = oi * 16 + 4 * g + v, c = e0 + oj * 16 + r16;
-        if (i < nt && c < E) out[(long)(t0 + i) * ldo + (long)h * E + c] = a1[v] + pw[i + 1] * a2[v];
+        for (int v = 0; v < 4; ++v) {
+          const int i = oi * 16 + 4 * g + v, c = e0 + oj * 16 + r16;
+          if (i < nt && c < E) out[(long)(t0 + i) * ldo + (long)h * E + c] = a1[v] + pw[i + 1] * a2[v];
+        }
       }
+      __syncthreads();     // every wave has read the old S
     }
-    __syncthreads();     // every wave has read the old S
     // ---- S <- L^n S + sum_t L^(n-1-t) k_t v_t^T: the tiles (di, sj) of the [Dp, EB] state, dealt out over the waves
     for (int t = wave; t < (Dp >> 4) * NJ; t += 4) {
       const int di = t / NJ, sj = t - di * NJ;
@@ -353,6 +418,14 @@ __global__ __launch_bounds__(256) void decay_state_chunk_kernel(
     }
   }
   __syncthreads();
+  if (MODE == DC_ADDED) {
+    for (int i = tid; i < Dp * EB; i += 256) {
+      const int c = i / Dp, d = i - c * Dp;
+      if (e0 + c < E) place(first + seg, c)[d] = St[c][d];
+    }
+    return;
+  }
+  if (MODE == DC_OUTPUTS && seg != n_seg - 1) return;
   for (int i = tid; i < D * EB; i += 256) {
     const int d = i / EB, c = i - d * EB;
     if (e0 + c < E) st[(long)d * E + e0 + c] = St[c][d];
@@ -361,12 +434,15 @@ __global__ __launch_bounds__(256) void decay_state_chunk_kernel(
 
 // The chunked form for steps with prompt portions: qk is scratch, float32 [n_tokens, 2 * n_head * head_dim]; out is
 // float32 [n_tokens, >= n_head * value_dim]: the heads' raw outputs (norm and gate are the caller's next kernel).
-// Head sizes up to 128 (value sizes up to 256); others are refused with MGPT_ERR_BAD_SHAPE and nothing launched.
+// Head sizes up to 128 (value sizes up to 256); others are refused with MGPT_ERR_BAD_SHAPE and nothing launched.  added
+// (optional): scratch of added_floats floats; with it the requests are cut into segments, for which it must hold
+// n_head * value_dim * (head_dim rounded up to 16) floats each, (n_tokens + 255 * min(n_req, n_tokens)) / 256 of them.
 extern "C" int mgpt_decay_state_chunked(const void* z, int dtype, long ldz, int q_off, int k_off, int v_off, int n_head,
                                         int head_dim, int value_dim, int act, const int* positions, const float* freq,
                                         int rot_dims, float k_scale, const float* decay, float* state,
                                         const int* state_slots, const int* cu_q, int n_req, int n_tokens, float* qk,
-                                        float* out, long ldo, hipStream_t stream) {
+                                        float* out, long ldo, float* added, long added_floats,
+                                        hipStream_t stream) {
   if (n_req == 0 || n_tokens == 0) return MGPT_OK;
   if (!z || !positions || !decay || !state || !state_slots || !cu_q || !out || !qk) return MGPT_ERR_NULL;
   if (!dtype_ok(dtype)) return MGPT_ERR_BAD_DTYPE;
@@ -375,14 +451,28 @@ extern "C" int mgpt_decay_state_chunked(const void* z, int dtype, long ldz, int 
       (rot_dims & 1) || rot_dims > D || (act != 0 && act != 1))
     return MGPT_ERR_BAD_SHAPE;
   if (n_head > 65535) return MGPT_ERR_TOO_LARGE;
+  const long segments = ((long)n_tokens + (DC_SEGMENT - 1L) * (n_req < n_tokens ? n_req : n_tokens)) / DC_SEGMENT;
+  if (added && (segments > 0x7fffffffL || added_floats < segments * n_head * E * ((D + 15) & ~15))) return MGPT_ERR_BAD_SHAPE;
   hipLaunchKernelGGL(state_inputs_kernel, dim3(n_tokens), dim3(256), 0, stream, z, dtype, ldz, q_off, k_off, n_head, D, act,
                      positions, rot_dims ? freq : nullptr, rot_dims, k_scale, qk, n_tokens);
   // 32 value channels a workgroup; 16 where that many workgroups would leave compute units idle
-  if ((long)n_req * n_head * ((E + 31) / 32) >= 256)
-    hipLaunchKernelGGL(decay_state_chunk_kernel<32>, dim3(n_req, n_head, (E + 31) / 32), dim3(256), 0, stream, qk, z, dtype,
-                       ldz, v_off, n_head, D, E, act, positions, decay, state, state_slots, cu_q, out, ldo);
-  else
-    hipLaunchKernelGGL(decay_state_chunk_kernel<16>, dim3(n_req, n_head, (E + 15) / 16), dim3(256), 0, stream, qk, z, dtype,
-                       ldz, v_off, n_head, D, E, act, positions, decay, state, state_slots, cu_q, out, ldo);
+#define DC_LAUNCH(EB, MODE, X)                                                                                             \
+  hipLaunchKernelGGL((decay_state_chunk_kernel<EB, MODE>), dim3((unsigned int)(X), n_head, (E + EB - 1) / EB), dim3(256), 0, \
+                     stream, qk, z, dtype, ldz, v_off, n_head, D, E, act, positions, decay, state, state_slots, cu_q, out, \
+                     ldo, n_req, added)
+  if (added) {
+    if (segments * n_head * ((E + 31) / 32) >= 256) {
+      DC_LAUNCH(32, DC_ADDED, segments);
+      DC_LAUNCH(32, DC_OUTPUTS, segments);
+    } else {
+      DC_LAUNCH(16, DC_ADDED, segments);
+      DC_LAUNCH(16, DC_OUTPUTS, segments);
+    }
+  } else if ((long)n_req * n_head * ((E + 31) / 32) >= 256) {
+    DC_LAUNCH(32, DC_WHOLE, n_req);
+  } else {
+    DC_LAUNCH(16, DC_WHOLE, n_req);
+  }
+#undef DC_LAUNCH
   return mgpt_last_error();
 }

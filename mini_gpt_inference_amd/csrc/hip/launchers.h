@@ -253,7 +253,7 @@ int mgpt_decay_state(const void* z, int dtype, long ldz, int q_off, int k_off, i
 int mgpt_decay_state_chunked(const void* z, int dtype, long ldz, int q_off, int k_off, int v_off, int n_head,
     int head_dim, int value_dim, int act, const int* positions, const float* freq, int rot_dims, float k_scale,
     const float* decay, float* state, const int* state_slots, const int* cu_q, int n_req, int n_tokens, float* qk,
-    float* out, long ldo, hipStream_t stream);
+    float* out, long ldo, float* added, long added_floats, hipStream_t stream);
 // linear_mfma.hip
 int mgpt_linear_mfma_grouped(const void* act, long lda, const void* w, long w_stride, const int* row_expert, const
     int* row_valid, int group_rows, void* out, int out_dtype, long ldo, int n_rows, int n_out, int k_dim,

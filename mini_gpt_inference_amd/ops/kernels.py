@@ -1885,9 +1885,12 @@ CHUNKED_STATE_MAX_DIM = 128     # largest head size that the chunked form of the
 def decay_state_chunked(z: torch.Tensor, q_off: int, k_off: int, v_off: int, n_head: int, head_dim: int, value_dim: int,
                         decay: torch.Tensor, state: torch.Tensor, state_slots: torch.Tensor, cu_q: torch.Tensor,
                         n_req: int, n_tokens: int, positions: torch.Tensor, qk: torch.Tensor, out: torch.Tensor,
-                        silu_inputs: bool = False, freq: Optional[torch.Tensor] = None, k_scale: float = 1.0) -> bool:
+                        silu_inputs: bool = False, freq: Optional[torch.Tensor] = None, k_scale: float = 1.0,
+                        added: Optional[torch.Tensor] = None) -> bool:
     """decay_state for steps with prompt portions: the recurrence 32 tokens at a time as float32 matrix products.
     out: float32 rows, the heads' raw outputs (no norm, no gate); qk: float32 scratch [>= n_tokens, 2 * heads * dim].
+    added: float32 scratch of decay_state_segments(...) floats at least: the requests' tokens are then cut into segments that
+    run side by side.
     False, with nothing launched, for head sizes beyond CHUNKED_STATE_MAX_DIM."""
     if head_dim > CHUNKED_STATE_MAX_DIM:
         return False
@@ -1897,6 +1900,8 @@ def decay_state_chunked(z: torch.Tensor, q_off: int, k_off: int, v_off: int, n_h
           and out.shape[1] >= n_head * value_dim, "decay_state_chunked: out must be float32 rows of all heads' values")
     _need(qk.dtype == torch.float32 and qk.is_contiguous() and qk.shape[0] >= n_tokens
           and qk.shape[1] == 2 * n_head * head_dim, "decay_state_chunked: qk must be float32 [tokens, 2 * heads * dim]")
+    _need(added is None or (added.is_cuda and added.dtype == torch.float32 and added.is_contiguous()),
+          "decay_state_chunked: added must be dense float32")
     _need(z.shape[1] >= max(q_off, k_off) + n_head * head_dim and z.shape[1] >= v_off + n_head * value_dim,
           "decay_state_chunked: z is too narrow")
     _need(decay.dtype == torch.float32 and decay.numel() == n_head, "decay_state: one float32 decay per head")
@@ -1913,9 +1918,26 @@ def decay_state_chunked(z: torch.Tensor, q_off: int, k_off: int, v_off: int, n_h
     rc = library.kernels().mgpt_decay_state_chunked(
         _ptr(z), _dtype_code(z), z.stride(0), q_off, k_off, v_off, n_head, head_dim, value_dim, int(silu_inputs),
         _ptr(positions), _ptr(freq), rot_dims, float(k_scale), _ptr(decay), _ptr(state), _ptr(state_slots), _ptr(cu_q),
-        n_req, n_tokens, _ptr(qk), _ptr(out), out.stride(0), _stream())
-    _check(rc, "decay_state_chunked", 2)
+        n_req, n_tokens, _ptr(qk), _ptr(out), out.stride(0), _ptr(added), 0 if added is None else added.numel(), _stream())
+    _check(rc, "decay_state_chunked", 2 if added is None else 3)
     return True
+
+
+DECAY_SEGMENT = 256     # tokens of a segment
+
+
+def decay_state_segments(n_tokens: int, n_req: int, max_q_len: int, n_head: int, head_dim: int, value_dim: int) -> int:
+    """Floats of scratch with which decay_state_chunked should cut requests into segments; 0 where the requests' chunks one
+    behind the other take no longer.  In us, for heads of 128 x 128: a chunk of the longest request 6.75 (5.1 while the chain's
+    workgroups have 16 value channels); cut, 40 and 8.3 for every chunk that each of 256 compute units has of all requests'
+    chunks, heads and 32 value channels.  Whole / cut: 2 requests of 1,024 tokens x 8 heads 175 / 129, x 16 heads 184 / 193;
+    one of 2,048 x 16 337 / 160; 8 of 100 to 1,024 x 8 236 / 205; 4 of 600 x 16 153 / 204; 16 of 1,024 x 8 332 / 482."""
+    blocks = -(-value_dim // 32) * n_head
+    whole = max_q_len / 32 * (6.75 if n_req * blocks >= 256 else 5.1)
+    if max_q_len <= DECAY_SEGMENT or whole <= 40 + 8.3 * n_tokens / 32 * blocks / 256:
+        return 0
+    segments = (n_tokens + (DECAY_SEGMENT - 1) * min(n_req, n_tokens)) // DECAY_SEGMENT
+    return segments * n_head * value_dim * (-(-head_dim // 16) * 16)
 
 
 GATED_STATE_MODES = {"channel_sigmoid": 0, "head_softplus": 1}

@@ -174,7 +174,7 @@ def _declare_optional(lib: ctypes.CDLL) -> None:
         "mgpt_cast_rows": [P, L, P, I, L, I, I, P],
         "mgpt_qk_prepare": [P, I, L, I, I, I, I, I, I, I, I, P, P, I, F, P, P, L, I, P, P, P, I, I, I, P, P, I, F, I, F, I, P],
         "mgpt_decay_state": [P, I, L, I, I, I, I, I, I, I, I, P, P, I, F, P, P, P, P, I, F, P, I, L, P],
-        "mgpt_decay_state_chunked": [P, I, L, I, I, I, I, I, I, I, P, P, I, F, P, P, P, P, I, I, P, P, L, P],
+        "mgpt_decay_state_chunked": [P, I, L, I, I, I, I, I, I, I, P, P, I, F, P, P, P, P, I, I, P, P, L, P, L, P],
         "mgpt_expert_route": [P, P, P, I, I, I, P, P, P, P, I, I, I, P],
         "mgpt_gather_rows": [P, L, P, P, L, I, I, P],
         "mgpt_linear_mfma_grouped": [P, L, P, L, P, P, I, P, I, L, I, I, I, I, P],

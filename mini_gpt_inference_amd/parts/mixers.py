@@ -679,10 +679,14 @@ class DecayStateMixer(Mixer):
         if not ctx.decode_only and self.head_dim <= kernels.CHUNKED_STATE_MAX_DIM:
             sums = ws.get("decay_state_sums", n, self.v_width, torch.float32)
             qk = ws.get("decay_state_qk", n, 2 * self.qk_width, torch.float32)
+            # (a padded step's longest portion is not known, only a bound of it: chunks one behind the other)
+            need = 0 if ctx.host_q_lens is None else kernels.decay_state_segments(n, n_req, ctx.max_q_len, self.n_head,
+                                                                                  self.head_dim, self.value_dim)
+            added = ws.get("decay_state_added", need, 1, torch.float32) if need else None
             chunked = kernels.decay_state_chunked(z, 0, self.k_off, self.v_off, self.n_head, self.head_dim, self.value_dim,
                                                   self._decays(z.device), state, ctx.state_slots, ctx.cu_q, n_req, n,
                                                   ctx.positions, qk, sums, silu_inputs=self.silu_inputs, freq=freq,
-                                                  k_scale=self.k_scale)
+                                                  k_scale=self.k_scale, added=added)
         gated_inside = self.head_norm_eps is not None and not chunked
         if not chunked:
             sums = y if gated_inside else ws.get("decay_state_sums", n, self.v_width, torch.float32)

@@ -297,6 +297,37 @@ def test_decaying_state_whole_in_portions_and_slots_used_again(dtype, H, D, E):
         helpers.assert_close(state[1:4], whole_state[1:4], "float32", f"{variant} state")
 
 
+@pytest.mark.parametrize("H,D,E", [(2, 128, 128), (3, 40, 24), (1, 16, 130)])
+@pytest.mark.parametrize("lens", [[1, 255, 256, 257], [511, 512, 513, 0, 700], [1300], [300] * 70, [4] * 66 + [600]])
+def test_decaying_state_in_segments(lens, H, D, E):
+    """Requests cut into segments of 256 tokens that run side by side against their chunks one behind the other (which is
+    what the plain recurrence is compared with): outputs and states after two steps in a row, so that the second starts
+    from the first one's states, with requests of the padding behind, around a segment's end and beyond the 64 requests
+    that a wave numbers at a time."""
+    g = torch.Generator().manual_seed(D + len(lens))
+    n, r = sum(lens), len(lens) + 2
+    k_off, v_off = H * D, 2 * H * D
+    decay = torch.tensor(([0.9995, 0.6, 0.97] * 3)[:H]).to(DEV)
+    cu = torch.tensor([0] + list(np.cumsum(lens)) + [n] * 2, dtype=torch.int32, device=DEV)
+    slots = torch.tensor(list(range(len(lens), 0, -1)) + [-1, 0], dtype=torch.int32, device=DEV)
+    need = (n + 255 * min(r, n)) // 256 * H * E * (-(-D // 16) * 16)
+    states = [torch.full((r, H * D * E), float("nan"), device=DEV) for _ in range(2)]
+    outs = [torch.zeros(n, H * E, device=DEV) for _ in range(2)]
+    first = [0] * len(lens)
+    for _ in range(2):
+        z = _rnd(g, n, v_off + H * E, scale=0.5).to(DEV)
+        pos = torch.tensor([f + t for f, T in zip(first, lens) for t in range(T)], dtype=torch.int32, device=DEV)
+        for state, out, added in zip(states, outs, (None, torch.full((need + 3,), float("nan"), device=DEV))):
+            assert kernels.decay_state_chunked(z, 0, k_off, v_off, H, D, E, decay, state, slots, cu, r, n, pos,
+                                               torch.zeros(n, 2 * H * D, device=DEV), out, added=added)
+        live = [len(lens) - i for i, T in enumerate(lens) if T]
+        for what, (whole, cut) in (("outputs", outs), ("states", [s[live] for s in states])):
+            assert (whole - cut).norm() <= 2e-6 * whole.norm(), what    # the same sums of float32 put together otherwise
+        first = list(lens)
+    dead = [i for i in range(r) if i not in live]
+    assert torch.isnan(states[1][dead]).all()
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("H,D,E", [(2, 16, 24), (1, 64, 64), (2, 128, 128), (3, 20, 12), (1, 128, 200), (2, 8, 256),
                                    (1, 1, 1), (1, 30, 33), (8, 16, 200), (9, 64, 160)])     # (the last two: 32 channels a workgroup)

@@ -325,7 +325,7 @@ int mgpt_linear_exact_launch(const float* A, long lda, const float* W, const flo
   if (epi == EPI_GELU) EX_LAUNCH(EPI_GELU);
   if (epi == EPI_RELU2) EX_LAUNCH(EPI_RELU2);
   if (epi == EPI_RESIDUAL) EX_LAUNCH(EPI_RESIDUAL);
-  if (epi == EPI_QKV) EX_LAUNCH(EPI_QKV);
+  if (epi == EPI_QKV && sc.kpool && sc.vpool && sc.slot_mapping) EX_LAUNCH(EPI_QKV);   // a plain product has no pages
 #undef EX_LAUNCH
   return MGPT_ERR_BAD_SHAPE;
 }

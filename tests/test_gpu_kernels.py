@@ -177,6 +177,17 @@ def test_float32_product_stores_keys_and_values(n, k, h, hk, d):
     assert torch.equal(pools[1].nan_to_num(9.0), pools[3].nan_to_num(9.0))
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_linear_generic_refuses_epilogues_that_it_does_not_have(dtype):
+    """The code that sends key and value columns to their pages among them: the plain product has no pages to send them to."""
+    a, w = torch.zeros(4, 40, dtype=getattr(torch, dtype), device=DEV), torch.zeros(8, 40, dtype=getattr(torch, dtype), device=DEV)
+    out = torch.full((4, 8), 7.0, dtype=a.dtype, device=DEV)
+    for epilogue in (kernels.SK_EPI_QKV, 4, 6, -1):
+        with pytest.raises(kernels.KernelError):
+            kernels.linear_generic(a, w, None, out, 4, epilogue)
+    assert (out == 7.0).all()
+
+
 def test_linear_generic_refuses_tensors_off_the_gpu():
     a, w = torch.zeros(4, 40, device=DEV), torch.zeros(8, 40, device=DEV)
     with pytest.raises(kernels.KernelError, match="GPU"):

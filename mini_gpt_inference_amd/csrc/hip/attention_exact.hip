@@ -6,7 +6,11 @@
 // multiples of 64; chunk c belongs to wave c % 8, which walks its chunks with a running maximum and sum; the waves'
 // results are put together in the order of the waves.  All of that depends on a key's position only, and what a query
 // does not see adds zeros, so a query's output is the same bits in a prompt, in a portion of one and in a decode step.
-// Keys that no query of the tile sees are never loaded.
+// Keys that no query of the tile sees are never loaded.  A value that is infinite or NaN shows in the wave's sums, where a
+// weight of zero has made NaN of it for queries that do not see its key: the wave then walks its chunks again and takes such
+// values out of the products of chunks that not all queries see whole, adding them to the queries that see them.  The walk
+// is there twice for that: with the look at the values in the one loop, prompts of 15 requests x 12 heads of 64 took 48.2 us
+// for 44.6, now 45; so they did with more than 96 registers, which the launch bounds of that head size keep to.
 //
 // The scores of a chunk are made transposed, S^T = K Q^T: a lane then has, of query lane % 16, the keys
 // 16 t + 4 (lane / 16) + i, which is just how O^T = V^T P^T takes them as its second operand.  Weights, maxima and sums
@@ -18,6 +22,7 @@
 #include "attention_exact.h"
 #include "attention_mask.h"
 #include "common.h"
+#include <type_traits>
 
 #define AX_WAVES 8
 #define AX_QUERIES 16
@@ -36,8 +41,50 @@ __device__ __forceinline__ float ax_sum4(float v) {
   return v + __shfl_xor(v, 32, MGPT_WAVE);
 }
 
+__device__ __forceinline__ bool ax_unusual(float v) { return !(fabsf(v) <= 3.402823466e38f); }   // infinite or NaN
+
+// Takes the infinite and NaN values out of vf (values of keys j0 .. j0 + 15, whose rows of the pool the lanes' `row` says,
+// as the kernel holds them) and adds each, times its weight, to the outputs of the queries that see its key.
+template <int G>
+__device__ __forceinline__ void ax_take_unusual(float (&vf)[4][G], const ax_f4& p, ax_f4 (&acc)[G],
+                                                const float* __restrict__ vpool, unsigned int row, int j0, int my_pos,
+                                                int my_begin, int keep_first) {
+  const int lane = threadIdx.x & 63, l16 = lane & 15, lk = lane >> 4;
+  float zero = 0.f;                                                     // NaN if one of them is unusual
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int g = 0; g < G; ++g) zero = fmaf(vf[i][g], 0.f, zero);
+  const uint64_t all = __ballot(zero != zero);
+  if (!all) return;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int g = 0; g < G; ++g) vf[i][g] = ax_unusual(vf[i][g]) ? 0.f : vf[i][g];
+  for (uint64_t lanes = all; lanes; lanes &= lanes - 1) {               // lanes that have one, in order
+    const int from = __builtin_amdgcn_readfirstlane(__ffsll((unsigned long long)lanes) - 1);
+    const int from_k = from >> 4, from_c = from & 15;
+#pragma unroll 1
+    for (int i = 0; i < 4; ++i) {
+      const int j = j0 + 4 * from_k + i;
+      const unsigned int vr = __builtin_amdgcn_readlane(row, 4 * from_k + i);
+      const float w = __shfl(i == 0 ? p[0] : (i == 1 ? p[1] : (i == 2 ? p[2] : p[3])), 16 * from_k + l16, MGPT_WAVE);
+      const bool mine = vr != AX_NONE && j <= my_pos && (j >= my_begin || j < keep_first) && lk == from_c >> 2;
+      if (!mine) continue;
+      const float* src = vpool + (long)vr * (16 * G) + G * from_c;     // channel G from_c + g: element from_c % 4 of acc[g]
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        const float v = src[g];
+        if (!ax_unusual(v)) continue;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[g][e] = e == (from_c & 3) ? fmaf(w, v, acc[g][e]) : acc[g][e];
+      }
+    }
+  }
+}
+
 template <int D>
-__global__ __launch_bounds__(64 * AX_WAVES) void attention_exact_kernel(AttentionExactArgs a) {
+__global__ __launch_bounds__(64 * AX_WAVES, D == 64 ? 5 : 1) void attention_exact_kernel(AttentionExactArgs a) {
   constexpr int G = D / 16;            // groups of 16 channels; also the channels of a lane's row of V^T
   constexpr int LD = D + 4;
   extern __shared__ __align__(16) float ax_lds[];      // [waves][queries][LD]
@@ -74,7 +121,7 @@ __global__ __launch_bounds__(64 * AX_WAVES) void attention_exact_kernel(Attentio
   const int ctx = a.seq_lens[r] - q_len;
   const int n_here = q_len - q0 < AX_QUERIES ? q_len - q0 : AX_QUERIES;
   const int pos_lo = ctx + q0, pos_hi = pos_lo + n_here - 1;
-  const int tile_begin = first_seen(pos_lo, a.window, a.chunked);
+  const int tile_begin = first_seen(pos_lo, a.window, a.chunked), last_begin = first_seen(pos_hi, a.window, a.chunked);
   const bool q_ok = l16 < n_here;
   const int my_pos = pos_lo + l16, my_begin = first_seen(my_pos, a.window, a.chunked);
   const int* bt = a.block_tables + (long)r * a.max_blocks;
@@ -88,96 +135,111 @@ __global__ __launch_bounds__(64 * AX_WAVES) void attention_exact_kernel(Attentio
   const float slope = a.slopes ? a.slopes[h] : 0.f;
   const float* dist = a.dist_bias ? a.dist_bias + (long)h * a.bias_len : nullptr;
 
-  float m = -INFINITY, l = 0.f;
+  float m, l;
   ax_f4 acc[G];                                         // O^T tile dt, rows 4 lk + i: channel G (4 lk + i) + dt
+  // the wave's walk over its chunks; CAREFUL: for values that are infinite or NaN
+  auto walk = [&](auto careful) __attribute__((always_inline)) {
+    constexpr bool CAREFUL = decltype(careful)::value;
+    m = -INFINITY;
+    l = 0.f;
 #pragma unroll
-  for (int g = 0; g < G; ++g) acc[g] = (ax_f4){0.f, 0.f, 0.f, 0.f};
-
-  for (int c = wave; c * AX_CHUNK <= pos_hi; c += AX_WAVES) {
-    const int c0 = c * AX_CHUNK;
-    if (c0 + AX_CHUNK <= tile_begin && c0 >= a.keep_first) continue;
-    // the pool rows of this lane's four keys, c0 + 16 t + l16
-    unsigned int row[4];                                // 2^32 rows of 16 channels are 275 GB
+    for (int g = 0; g < G; ++g) acc[g] = (ax_f4){0.f, 0.f, 0.f, 0.f};
+    for (int c = wave; c * AX_CHUNK <= pos_hi; c += AX_WAVES) {
+      const int c0 = c * AX_CHUNK;
+      if (c0 + AX_CHUNK <= tile_begin && c0 >= a.keep_first) continue;
+      // whether every query of the tile sees every key that is loaded (always so for a single query)
+      const bool whole = (c0 + AX_CHUNK - 1 < pos_hi ? c0 + AX_CHUNK - 1 : pos_hi) <= pos_lo &&
+                         ((c0 > tile_begin ? c0 : tile_begin) >= last_begin || c0 + AX_CHUNK <= a.keep_first);
+      // the pool rows of this lane's four keys, c0 + 16 t + l16
+      unsigned int row[4];                                // 2^32 rows of 16 channels are 275 GB
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int j = c0 + 16 * t + l16;
-      row[t] = AX_NONE;
-      if (j <= pos_hi && (j >= tile_begin || j < a.keep_first)) {
-        const int idx = j / a.page_size;
-        row[t] = ((unsigned int)bt[idx] * a.n_kv_head + hk) * a.page_size + (j - idx * a.page_size);
-      }
-    }
-    ax_f4 s[4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      s[t] = (ax_f4){0.f, 0.f, 0.f, 0.f};
-      ax_f4 kf[G];
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        kf[g] = (ax_f4){0.f, 0.f, 0.f, 0.f};
-        if (row[t] != AX_NONE) kf[g] = *reinterpret_cast<const ax_f4*>(a.kpool + (long)row[t] * D + 16 * g + 4 * lk);
-      }
-#pragma unroll
-      for (int g = 0; g < G; ++g)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[g][e], qf[g][e], s[t], 0, 0, 0);
-    }
-    float top = -INFINITY;
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int j = c0 + 16 * t + 4 * lk + i;
-        float v = s[t][i] * a.scale;
-        if (dist) v += dist[distance_entry(my_pos - j, a.bias_len)];
-        if (a.softcap > 0.f) v = a.softcap * tanhf(v / a.softcap);
-        if (a.slopes) v -= slope * (float)(my_pos - j);
-        if (!(q_ok && j <= my_pos && (j >= my_begin || j < a.keep_first))) v = -INFINITY;
-        s[t][i] = v;
-        top = fmaxf(top, v);
-      }
-    const float m_new = fmaxf(m, ax_max4(top));
-    const float m_sub = m_new == -INFINITY ? 0.f : m_new;   // nothing seen so far: every weight is exp(-inf)
-    const float alpha = expf(m - m_sub);
-    float sum = 0.f;
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        s[t][i] = expf(s[t][i] - m_sub);
-        sum += s[t][i];
-      }
-    l = l * alpha + ax_sum4(sum);
-    m = m_new;
-#pragma unroll
-    for (int g = 0; g < G; ++g) acc[g] *= alpha;
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      float vf[4][G];                                   // of key 16 t + 4 lk + i the channels G l16 .. G l16 + G - 1
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const unsigned int vr = __shfl(row[t], 4 * lk + i, MGPT_WAVE);
-        const float* src = a.vpool + (long)vr * D + G * l16;
-        if constexpr (G >= 4) {
-#pragma unroll
-          for (int g = 0; g < G; g += 4) {
-            ax_f4 v = {0.f, 0.f, 0.f, 0.f};
-            if (vr != AX_NONE) v = *reinterpret_cast<const ax_f4*>(src + g);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) vf[i][g + e] = v[e];
-          }
-        } else {
-#pragma unroll
-          for (int g = 0; g < G; ++g) vf[i][g] = vr != AX_NONE ? src[g] : 0.f;
+      for (int t = 0; t < 4; ++t) {
+        const int j = c0 + 16 * t + l16;
+        row[t] = AX_NONE;
+        if (j <= pos_hi && (j >= tile_begin || j < a.keep_first)) {
+          const int idx = j / a.page_size;
+          row[t] = ((unsigned int)bt[idx] * a.n_kv_head + hk) * a.page_size + (j - idx * a.page_size);
         }
       }
+      ax_f4 s[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int t = 0; t < 4; ++t) {
+        s[t] = (ax_f4){0.f, 0.f, 0.f, 0.f};
+        ax_f4 kf[G];
 #pragma unroll
-        for (int g = 0; g < G; ++g) acc[g] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[i][g], s[t][i], acc[g], 0, 0, 0);
+        for (int g = 0; g < G; ++g) {
+          kf[g] = (ax_f4){0.f, 0.f, 0.f, 0.f};
+          if (row[t] != AX_NONE) kf[g] = *reinterpret_cast<const ax_f4*>(a.kpool + (long)row[t] * D + 16 * g + 4 * lk);
+        }
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[g][e], qf[g][e], s[t], 0, 0, 0);
+      }
+      float top = -INFINITY;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int j = c0 + 16 * t + 4 * lk + i;
+          float v = s[t][i] * a.scale;
+          if (dist) v += dist[distance_entry(my_pos - j, a.bias_len)];
+          if (a.softcap > 0.f) v = a.softcap * tanhf(v / a.softcap);
+          if (a.slopes) v -= slope * (float)(my_pos - j);
+          if (!(q_ok && j <= my_pos && (j >= my_begin || j < a.keep_first))) v = -INFINITY;
+          s[t][i] = v;
+          top = fmaxf(top, v);
+        }
+      const float m_new = fmaxf(m, ax_max4(top));
+      const float m_sub = m_new == -INFINITY ? 0.f : m_new;   // nothing seen so far: every weight is exp(-inf)
+      const float alpha = expf(m - m_sub);
+      float sum = 0.f;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          s[t][i] = expf(s[t][i] - m_sub);
+          sum += s[t][i];
+        }
+      l = l * alpha + ax_sum4(sum);
+      m = m_new;
+#pragma unroll
+      for (int g = 0; g < G; ++g) acc[g] *= alpha;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        float vf[4][G];                                   // of key 16 t + 4 lk + i the channels G l16 .. G l16 + G - 1
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const unsigned int vr = __shfl(row[t], 4 * lk + i, MGPT_WAVE);
+          const float* src = a.vpool + (long)vr * D + G * l16;
+          if constexpr (G >= 4) {
+#pragma unroll
+            for (int g = 0; g < G; g += 4) {
+              ax_f4 v = {0.f, 0.f, 0.f, 0.f};
+              if (vr != AX_NONE) v = *reinterpret_cast<const ax_f4*>(src + g);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) vf[i][g + e] = v[e];
+            }
+          } else {
+#pragma unroll
+            for (int g = 0; g < G; ++g) vf[i][g] = vr != AX_NONE ? src[g] : 0.f;
+          }
+        }
+        if (CAREFUL && !whole) ax_take_unusual<G>(vf, s[t], acc, a.vpool, row[t], c0 + 16 * t, my_pos, my_begin, a.keep_first);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int g = 0; g < G; ++g) acc[g] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[i][g], s[t][i], acc[g], 0, 0, 0);
+      }
     }
-  }
-
+  };
+  walk(std::false_type{});
+  float zero = 0.f;                                     // an infinity or NaN among the sums stays one to the end
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) zero = fmaf(acc[g][i], 0.f, zero);
+  if (__ballot(zero != zero)) walk(std::true_type{});
   if (lk == 0) {
     m_s[wave][l16] = m;
     l_s[wave][l16] = l;

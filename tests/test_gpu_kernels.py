@@ -765,6 +765,39 @@ def test_float32_attention_keeps_its_sums_whatever_the_portion(d, window, mask):
     assert torch.equal(attend([r for r, _ in pick], [t for _, t in pick], [1] * len(pick), rows), whole[rows])
 
 
+@pytest.mark.parametrize("window,mask", [(0, {}), (20, {}), (20, {"keep_first": 9}), (24, {"chunked": True})])
+@pytest.mark.parametrize("d", [16, 32, 48, 64, 128])
+def test_float32_attention_keeps_what_a_query_does_not_see_out_of_it(d, window, mask):
+    """A value that is infinite or NaN reaches the queries that see its key, in its channel, and nobody else: every other
+    output is the same bits as without it, also of the queries that share a tile with one that sees it.  (48: the general
+    kernel; the others: the matrix-core kernel, prompts, portions and single tokens.)"""
+    seq_lens, q_lens = [40, 65, 130, 7, 90, 150], [40, 65, 130, 7, 33, 1]
+    c = PagedCase(seq_lens, q_lens, h=4, hk=2, d=d, page=12, dtype="float32", seed=d)
+
+    def attend():
+        out = torch.full((c.n, 4 * d), 7.0, device=DEV)
+        kernels.paged_attention_generic(c.q_flat, out, c.kp, c.vp, c.bt, c.cu, c.sl, c.q_req, c.n, len(q_lens), 4, d ** -0.5,
+                                        window, **mask)
+        return out.view(c.n, 4, d)
+
+    want = attend()
+    assert torch.isfinite(want).all()
+    unusual = []                                       # request, key, head of keys, channel, value
+    for r, s in enumerate(seq_lens):
+        for i, j in enumerate(sorted({s - 1, s - 2, s // 2, s // 2 + 1, 4})):
+            unusual.append((r, j, i % 2, (5 * i + r) % d, (float("inf"), float("nan"), float("-inf"))[i % 3]))
+    for r, j, hk, ch, value in unusual:
+        c.vp[int(c.bt[r, j // 12]), hk, j % 12, ch] = value
+    starts = c.cu.tolist()
+    for r, j, hk, ch, value in unusual:
+        for t in range(q_lens[r]):
+            p = seq_lens[r] - q_lens[r] + t
+            first = 0 if not window else (p - p % window if mask.get("chunked") else p - window + 1)
+            if j <= p and (j >= first or j < mask.get("keep_first", 0)):
+                want[starts[r] + t, 2 * hk:2 * hk + 2, ch] = value
+    assert torch.equal(attend().nan_to_num(1e30, 2e30, 3e30), want.nan_to_num(1e30, 2e30, 3e30))
+
+
 @pytest.mark.parametrize("window", [0, 5, 70])
 @pytest.mark.parametrize("case", range(len(ATTENTION_CASES)))
 @pytest.mark.parametrize("kernel", ["generic-float32", "generic-bfloat16", "split-bfloat16", "splitfast-bfloat16",

@@ -8,8 +8,8 @@ struct AttentionExactArgs {
   float* out; long ldo;
   const float* kpool; const float* vpool;
   const int* block_tables; int max_blocks;
-  const int* cu_q; const int* seq_lens;
-  int n_req, n_head, n_kv_head, page_size;
+  const int* cu_q; const int* seq_lens; const int* q_req;
+  int n_tokens, n_req, n_head, n_kv_head, page_size;
   float scale; int window;
   const float* sinks; float softcap;
   const float* gate; long ldg;
@@ -18,6 +18,7 @@ struct AttentionExactArgs {
   const float* slopes;
 };
 
-// Whether the kernel takes these: nothing in it depends on a step's size, so a model's calls are all taken or none is.
+// Whether the kernel takes these: nothing in it depends on a step's size (but for a step of no requests, which has nothing to
+// do), so a model's calls are all taken or none is.
 bool mgpt_attention_exact_takes(const AttentionExactArgs& a, int head_dim);
-int mgpt_attention_exact_launch(const AttentionExactArgs& a, int n_tokens, int head_dim, hipStream_t stream);
+int mgpt_attention_exact_launch(const AttentionExactArgs& a, int head_dim, hipStream_t stream);

@@ -89,6 +89,7 @@ __global__ __launch_bounds__(64 * AX_WAVES, D == 64 ? 5 : 1) void attention_exac
   constexpr int LD = D + 4;
   extern __shared__ __align__(16) float ax_lds[];      // [waves][queries][LD]
   __shared__ float m_s[AX_WAVES][AX_QUERIES], l_s[AX_WAVES][AX_QUERIES];
+  __shared__ int req_s[AX_QUERIES];                    // negative: a token of the padding, left alone
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -119,7 +120,10 @@ __global__ __launch_bounds__(64 * AX_WAVES, D == 64 ? 5 : 1) void attention_exac
   const int q_start = a.cu_q[r], q_len = a.cu_q[r + 1] - q_start;
   const int q0 = __builtin_amdgcn_readfirstlane(tile) * AX_QUERIES;
   const int ctx = a.seq_lens[r] - q_len;
-  const int n_here = q_len - q0 < AX_QUERIES ? q_len - q0 : AX_QUERIES;
+  int n_here = q_len - q0 < AX_QUERIES ? q_len - q0 : AX_QUERIES;
+  if (a.n_tokens - q_start - q0 < n_here) n_here = a.n_tokens - q_start - q0;   // rows that the caller does not have
+  if (n_here <= 0) return;
+  const int token_req = a.q_req[q_start + q0 + (l16 < n_here ? l16 : 0)];       // for the end
   const int pos_lo = ctx + q0, pos_hi = pos_lo + n_here - 1;
   const int tile_begin = first_seen(pos_lo, a.window, a.chunked), last_begin = first_seen(pos_hi, a.window, a.chunked);
   const bool q_ok = l16 < n_here;
@@ -243,6 +247,7 @@ __global__ __launch_bounds__(64 * AX_WAVES, D == 64 ? 5 : 1) void attention_exac
   if (lk == 0) {
     m_s[wave][l16] = m;
     l_s[wave][l16] = l;
+    if (wave == 0) req_s[l16] = token_req;
   }
   float* mine = ax_lds + (wave * AX_QUERIES + l16) * LD + 4 * G * lk;
 #pragma unroll
@@ -253,6 +258,7 @@ __global__ __launch_bounds__(64 * AX_WAVES, D == 64 ? 5 : 1) void attention_exac
 
   for (int e = tid; e < n_here * D; e += 64 * AX_WAVES) {
     const int qi = e / D, d = e % D;
+    if (req_s[qi] < 0) continue;
     float top = a.sinks ? a.sinks[h] : -INFINITY;       // one more term of the denominator, with no value
 #pragma unroll
     for (int w = 0; w < AX_WAVES; ++w) top = fmaxf(top, m_s[w][qi]);
@@ -272,7 +278,7 @@ __global__ __launch_bounds__(64 * AX_WAVES, D == 64 ? 5 : 1) void attention_exac
 }
 
 template <int D>
-static int launch(const AttentionExactArgs& a, int n_tokens, hipStream_t stream) {
+static int launch(const AttentionExactArgs& a, hipStream_t stream) {
   constexpr int bytes = AX_WAVES * AX_QUERIES * (D + 4) * (int)sizeof(float);
   static bool allowed = bytes <= 48 * 1024;            // more LDS than a kernel gets without asking
   if (!allowed) {
@@ -282,7 +288,7 @@ static int launch(const AttentionExactArgs& a, int n_tokens, hipStream_t stream)
     allowed = true;
   }
   // at most so many tiles: a request's last one may be short
-  const long tiles = ((long)n_tokens + (long)(AX_QUERIES - 1) * (a.n_req < n_tokens ? a.n_req : n_tokens)) / AX_QUERIES;
+  const long tiles = ((long)a.n_tokens + (long)(AX_QUERIES - 1) * (a.n_req < a.n_tokens ? a.n_req : a.n_tokens)) / AX_QUERIES;
   if (tiles > 0x7fffffffL) return MGPT_ERR_TOO_LARGE;
   hipLaunchKernelGGL(attention_exact_kernel<D>, dim3((unsigned int)tiles, a.n_head), dim3(64 * AX_WAVES), bytes, stream, a);
   return mgpt_last_error();
@@ -291,12 +297,13 @@ static int launch(const AttentionExactArgs& a, int n_tokens, hipStream_t stream)
 bool mgpt_attention_exact_takes(const AttentionExactArgs& a, int head_dim) {
   const uintptr_t together = reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.kpool) |
                              reinterpret_cast<uintptr_t>(a.vpool);
-  return (head_dim == 16 || head_dim == 32 || head_dim == 64 || head_dim == 128) && (together & 15) == 0 && a.ldq % 4 == 0;
+  return (head_dim == 16 || head_dim == 32 || head_dim == 64 || head_dim == 128) && (together & 15) == 0 && a.ldq % 4 == 0 &&
+         a.n_req > 0;   // (without requests all tokens are padding: the general kernel leaves them alone)
 }
 
-int mgpt_attention_exact_launch(const AttentionExactArgs& a, int n_tokens, int head_dim, hipStream_t stream) {
-  if (head_dim == 16) return launch<16>(a, n_tokens, stream);
-  if (head_dim == 32) return launch<32>(a, n_tokens, stream);
-  if (head_dim == 64) return launch<64>(a, n_tokens, stream);
-  return launch<128>(a, n_tokens, stream);
+int mgpt_attention_exact_launch(const AttentionExactArgs& a, int head_dim, hipStream_t stream) {
+  if (head_dim == 16) return launch<16>(a, stream);
+  if (head_dim == 32) return launch<32>(a, stream);
+  if (head_dim == 64) return launch<64>(a, stream);
+  return launch<128>(a, stream);
 }

@@ -203,10 +203,10 @@ extern "C" int mgpt_paged_attention_generic(
   if (window == 0) keep_first = 0;   // every key is seen anyway
   if (dtype == MGPT_F32 && !fast_exp && !score_bias) {
     const AttentionExactArgs args = {(const float*)q, ldq, (float*)out, ldo, (const float*)kpool, (const float*)vpool,
-                                     block_tables, max_blocks, cu_q, seq_lens, n_req, n_head, n_kv_head, page_size, scale,
-                                     window, sinks, softcap, (const float*)gate, ldg, keep_first, chunked, dist_bias,
-                                     bias_len, slopes};
-    if (mgpt_attention_exact_takes(args, head_dim)) return mgpt_attention_exact_launch(args, n_tokens, head_dim, stream);
+                                     block_tables, max_blocks, cu_q, seq_lens, q_req, n_tokens, n_req, n_head, n_kv_head,
+                                     page_size, scale, window, sinks, softcap, (const float*)gate, ldg, keep_first, chunked,
+                                     dist_bias, bias_len, slopes};
+    if (mgpt_attention_exact_takes(args, head_dim)) return mgpt_attention_exact_launch(args, head_dim, stream);
   }
   dim3 grid(n_tokens, n_head), block(MGPT_WAVE);
 #define LAUNCH(T, F)                                                                              \

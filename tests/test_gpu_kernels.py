@@ -798,6 +798,30 @@ def test_float32_attention_keeps_what_a_query_does_not_see_out_of_it(d, window, 
     assert torch.equal(attend().nan_to_num(1e30, 2e30, 3e30), want.nan_to_num(1e30, 2e30, 3e30))
 
 
+@pytest.mark.parametrize("d", [16, 48, 64, 128])
+def test_float32_attention_leaves_other_tokens_alone(d):
+    """Rows at or beyond n_tokens, which cu_q may still count, tokens without a request and a step without requests: the
+    kernel on the matrix cores as the general one (48)."""
+    seq_lens, q_lens = [20, 40, 9, 70], [20, 3, 9, 33]
+    c = PagedCase(seq_lens, q_lens, h=4, hk=2, d=d, page=12, dtype="float32", seed=d)
+    q_req = c.q_req.clone()
+    q_req[[5, 19, 24]] = -1
+
+    def attend(n, r, q_req):
+        out = torch.full((c.n, 4 * d), 7.0, device=DEV)
+        kernels.paged_attention_generic(c.q_flat, out, c.kp, c.vp, c.bt, c.cu, c.sl, q_req, n, r, 4, d ** -0.5)
+        return out
+
+    whole = attend(c.n, len(q_lens), c.q_req)
+    assert not (whole == 7.0).all(1).any()
+    for n in (c.n, c.n - 1, 49, 48, 33, 32, 24, 21, 20, 17, 16, 3):
+        want = whole.clone()
+        want[n:] = 7.0
+        want[[5, 19, 24]] = 7.0
+        assert torch.equal(attend(n, len(q_lens), q_req), want), n
+    assert (attend(c.n, 0, torch.full_like(q_req, -1)) == 7.0).all()
+
+
 @pytest.mark.parametrize("window", [0, 5, 70])
 @pytest.mark.parametrize("case", range(len(ATTENTION_CASES)))
 @pytest.mark.parametrize("kernel", ["generic-float32", "generic-bfloat16", "split-bfloat16", "splitfast-bfloat16",

@@ -679,9 +679,11 @@ class DecayStateMixer(Mixer):
         if not ctx.decode_only and self.head_dim <= kernels.CHUNKED_STATE_MAX_DIM:
             sums = ws.get("decay_state_sums", n, self.v_width, torch.float32)
             qk = ws.get("decay_state_qk", n, 2 * self.qk_width, torch.float32)
-            # (a padded step's longest portion is not known, only a bound of it: chunks one behind the other)
-            need = 0 if ctx.host_q_lens is None else kernels.decay_state_segments(n, n_req, ctx.max_q_len, self.n_head,
-                                                                                  self.head_dim, self.value_dim)
+            # Segments put the same sums together in another order, and whether they pay hangs on the whole step.  On the
+            # 32-bit path a request's bits depend on its own tokens and cuts alone: its chunks go one behind the other.
+            # So they do in a padded step, whose longest portion is not known, only a bound of it.
+            need = 0 if ctx.exact or ctx.host_q_lens is None else kernels.decay_state_segments(
+                n, n_req, ctx.max_q_len, self.n_head, self.head_dim, self.value_dim)
             added = ws.get("decay_state_added", need, 1, torch.float32) if need else None
             chunked = kernels.decay_state_chunked(z, 0, self.k_off, self.v_off, self.n_head, self.head_dim, self.value_dim,
                                                   self._decays(z.device), state, ctx.state_slots, ctx.cu_q, n_req, n,

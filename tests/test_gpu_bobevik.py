@@ -657,6 +657,51 @@ def test_long_decoding(tmp_path_factory, dtype):
     _check(folder, "A", dtype, "long", ids, got["a"], want, "long decoding")
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("name", ["A", "B"])
+def test_a_long_prompt_alone_beside_others_and_in_a_buckets_graph(tmp_path_factory, monkeypatch, name, dtype):
+    """A prompt long enough for its decaying state to be cut into segments: on the 32-bit path it never is, and its logits
+    are the same bits alone, beside other requests and replayed from a bucket's padded graph; in bfloat16 it is cut in the
+    first two and not in the third, each within rounding of the plain implementation."""
+    folder, vocab = _folder(tmp_path_factory, name), cases.RAW[name]["vocab"]
+    rng = np.random.default_rng(21)
+    ids, n = helpers.random_ids(rng, vocab, 600), 600
+    cfg, w = P.read_model_folder(folder)
+    want = P.forward(cfg, w, ids).numpy()
+    rows = list(range(n - 100, n))
+    cut, real = [], kernels.decay_state_chunked
+
+    def chunked(*args, **kw):
+        cut.append(kw.get("added") is not None)
+        return real(*args, **kw)
+
+    monkeypatch.setattr(kernels, "decay_state_chunked", chunked)
+
+    def replayer():
+        return TraceReplayer(folder, dtype, 2048, page_size=16, max_live=4, poison=True)
+
+    entry = {"id": "long", "tokens": ids, "want": rows}
+    others = [{"id": f"o{i}", "tokens": helpers.random_ids(rng, vocab, k), "want": []} for i, k in enumerate((3, 470, 90))]
+    got = [replayer().run_step({"entries": [entry]}).cpu().numpy(),
+           replayer().run_step({"entries": others[:2] + [entry] + others[2:]}).cpu().numpy()]
+    assert set(cut) == {dtype == "bfloat16"}
+    rep = replayer()
+    for k in (590, 597, 583):      # other lengths of the same bucket: the third makes its graph
+        rep.run_step({"entries": [{"id": "x", "tokens": helpers.random_ids(rng, vocab, k), "want": rows[:70]}], "end": ["x"]})
+    before = rep.runner.num_replayed_steps
+    got.append(rep.run_step({"entries": [entry]}).cpu().numpy())
+    assert rep.runner.num_replayed_steps == before + 1
+    noise = _row_errors(_rounded_twin(cfg, w, ids)[rows], want[rows])
+    for what, logits in zip(("alone", "beside others", "a bucket's graph"), got):
+        err = _row_errors(logits, want[rows])
+        if dtype == "float32":
+            assert np.array_equal(logits, got[0]), what
+            assert err.max() <= 5e-5 * max(1.0, float(np.abs(want).max())), f"{what}: {err.max():.3e}"
+        else:     # as _assert_within_rounding has it
+            assert err.max() <= 3.0 * noise.max() and err.mean() <= 3.0 * noise.mean(), \
+                f"{what}: {err.max():.3e} / {noise.max():.3e}, mean {err.mean():.3e} / {noise.mean():.3e}"
+
+
 @pytest.mark.parametrize("name", ["A", "B"])
 def test_greedy_generation_through_the_engine(tmp_path_factory, name):
     folder = _folder(tmp_path_factory, name)

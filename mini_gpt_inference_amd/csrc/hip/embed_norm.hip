@@ -114,6 +114,38 @@ __global__ void layernorm_kernel(const float* __restrict__ x, const float* __res
   }
 }
 
+// Mean, what is left of it in the distances from it, and 1 / standard deviation of a row of n4 vectors of four, of which
+// this lane has those at lane + 64 i; they become the distances from the mean.  One order of sums for every kernel below.
+// Only the last PART of the LN_VEC may lie behind the row's end for some lanes.
+template <int LN_VEC, int PART>
+__device__ __forceinline__ void layernorm_sums(float4 (&xv)[LN_VEC], int n4, int width, float eps, float& mean, float& corr,
+                                               float& rstd) {
+  const int lane = threadIdx.x & (MGPT_WAVE - 1);
+  float s = 0.f;
+#pragma unroll
+  for (int i = 0; i < LN_VEC; ++i) {
+    if (i >= LN_VEC - PART && lane + i * MGPT_WAVE >= n4) xv[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    s += (xv[i].x + xv[i].y) + (xv[i].z + xv[i].w);
+  }
+  mean = wave_sum(s) / (float)width;
+  float e = 0.f, v2 = 0.f;
+#pragma unroll
+  for (int i = 0; i < LN_VEC; ++i) {
+    const bool in = i < LN_VEC - PART || lane + i * MGPT_WAVE < n4;
+    float* p = reinterpret_cast<float*>(&xv[i]);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const float d = in ? p[k] - mean : 0.f;
+      p[k] = d;
+      e += d;
+      v2 = fmaf(d, d, v2);
+    }
+  }
+  corr = wave_sum(e) / (float)width;
+  const float var = fmaxf(wave_sum(v2) / (float)width - corr * corr, 0.f);
+  rstd = 1.0f / sqrtf(var + eps);
+}
+
 // The same for widths that are multiples of 4 up to 64 * 4 * LN_VEC with 16-byte aligned rows: every
 // lane loads and stores vectors of four (a row of 512 is two loads per lane instead of eight).
 // LN_VEC is the number of such vectors a lane holds: the row's width / 256, rounded up to one of
@@ -139,29 +171,8 @@ __global__ void layernorm_vec_kernel(const float* __restrict__ x, const float* _
     gv[i] = w4[cc];
     bv[i] = b ? b4[cc] : make_float4(0.f, 0.f, 0.f, 0.f);
   }
-  float s = 0.f;
-#pragma unroll
-  for (int i = 0; i < LN_VEC; ++i) {
-    if (lane + i * MGPT_WAVE >= n4) xv[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-    s += (xv[i].x + xv[i].y) + (xv[i].z + xv[i].w);
-  }
-  const float mean = wave_sum(s) / (float)width;
-  float e = 0.f, v2 = 0.f;
-#pragma unroll
-  for (int i = 0; i < LN_VEC; ++i) {
-    const bool in = lane + i * MGPT_WAVE < n4;
-    float* p = reinterpret_cast<float*>(&xv[i]);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const float d = in ? p[k] - mean : 0.f;
-      p[k] = d;
-      e += d;
-      v2 = fmaf(d, d, v2);
-    }
-  }
-  const float corr = wave_sum(e) / (float)width;
-  const float var = fmaxf(wave_sum(v2) / (float)width - corr * corr, 0.f);
-  const float rstd = 1.0f / sqrtf(var + eps);
+  float mean, corr, rstd;
+  layernorm_sums<LN_VEC, LN_VEC <= 4 ? 1 : 2>(xv, n4, width, eps, mean, corr, rstd);   // (5 and 7 vectors: 6 and 8 here)
   OT* orow = out + (long)row * width;
 #pragma unroll
   for (int i = 0; i < LN_VEC; ++i) {
@@ -180,17 +191,49 @@ __global__ void layernorm_vec_kernel(const float* __restrict__ x, const float* _
   }
 }
 
-// The same for rows of 513 to 4,096 values (multiples of 4, 16-byte aligned): a workgroup a row with a vector of four a lane, W
-// waves, whose sums meet in LDS.  One wave a row has three to eight vectors a lane there, and their loads, sums and stores
-// one behind the other (us in a graph of such calls, a wave a row / here: 32 rows of 768 2.87 / 2.49, of 1,600 3.70 / 2.71; of
-// 4,096, which had 4-byte loads, 29.5 / 3.3; 512 rows of 1,600 3.97 / 3.47).  With many rows there are waves enough and the
-// meeting only costs (1,024 rows of 1,600 4.23 / 4.50): bfloat16 outputs of more than 640 rows of up to 2,048 stay with the
-// kernel above.  Float32 outputs, the 32-bit path's, always come here where it takes the row (4,096 rows of 768 5.6 / 6.6, beside
-// products of hundreds): their sums run in one order whatever the number of rows.
+// The same for rows of 513 to 2,048 values where the rows are few: a workgroup a row, a vector of four a lane, W waves.  One
+// wave a row has three to eight vectors a lane there, and their loads, sums and stores one behind the other.  The waves hand
+// each other the row through LDS and each makes all of its sums, in the order of the kernel above: a row's result is the same
+// bits in both, and so whatever the number of rows.  With many rows there are waves enough, and eight waves that make one
+// row's sums eight times only cost.  us in a graph of such calls, a wave a row / here: bfloat16 outputs, 16 rows of 768
+// 2.43 / 1.95, of 1,600 3.30 / 2.42, of 2,048 3.45 / 2.47; 200 rows of 1,600 3.41 / 2.61; 640 rows of 768 2.58 / 2.55;
+// with masks on all vectors 640 rows of 1,600 3.57 / 4.30.  The line between them, 1,920 waves (two a SIMD, nearly), lies
+// where the two meet: 640 rows of 768, 274 of 1,600, 240 of 2,048.  (Waves that each sum a part of the row and meet in LDS
+// took 2.25 us for 16 rows of 1,600, but in an order of their own, which the 32-bit path then had to keep to with many rows
+// as well: 4,096 rows of 768 took 6.2 us for 5.3.)
 template <typename OT, int W>
-__global__ __launch_bounds__(64 * W) void layernorm_row_kernel(const float* __restrict__ x, const float* __restrict__ w,
-                                                               const float* __restrict__ b, OT* __restrict__ out,
-                                                               const int* __restrict__ rows, int width, float eps) {
+__global__ __launch_bounds__(64 * W) void layernorm_shared_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                                  const float* __restrict__ b, OT* __restrict__ out,
+                                                                  const int* __restrict__ rows, int width, float eps) {
+  __shared__ float4 row_s[64 * W];
+  const int tid = threadIdx.x, lane = tid & (MGPT_WAVE - 1), n4 = width >> 2;
+  const long src = rows ? rows[blockIdx.x] : (long)blockIdx.x;
+  const int c = tid < n4 ? tid : 0;
+  const float4 v = reinterpret_cast<const float4*>(x + src * (long)width)[c];
+  const float4 g = reinterpret_cast<const float4*>(w)[c];
+  const float4 o = b ? reinterpret_cast<const float4*>(b)[c] : make_float4(0.f, 0.f, 0.f, 0.f);
+  row_s[tid] = v;
+  __syncthreads();
+  float4 xv[W];
+#pragma unroll
+  for (int i = 0; i < W; ++i) xv[i] = row_s[lane + i * MGPT_WAVE];
+  float mean, corr, rstd;
+  layernorm_sums<W, 1>(xv, n4, width, eps, mean, corr, rstd);
+  if (tid >= n4) return;
+  const float y0 = ((v.x - mean) - corr) * rstd * g.x + o.x, y1 = ((v.y - mean) - corr) * rstd * g.y + o.y;
+  const float y2 = ((v.z - mean) - corr) * rstd * g.z + o.z, y3 = ((v.w - mean) - corr) * rstd * g.w + o.w;
+  OT* orow = out + (long)blockIdx.x * width;
+  if (sizeof(OT) == 4) reinterpret_cast<float4*>(orow)[tid] = make_float4(y0, y1, y2, y3);
+  else reinterpret_cast<uint2*>(orow)[tid] = make_uint2(pack_bf16x2(y0, y1), pack_bf16x2(y2, y3));
+}
+
+// Rows of 2,049 to 4,096 values: 16 waves a row, whose sums meet in LDS (16 rows of 4,096 with the 4-byte loads of the first
+// kernel above 29 us, here 2.9; 4,096 rows 74 / 24).
+template <typename OT>
+__global__ __launch_bounds__(1024) void layernorm_row_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                             const float* __restrict__ b, OT* __restrict__ out,
+                                                             const int* __restrict__ rows, int width, float eps) {
+  constexpr int W = 16;
   __shared__ float red[W][2], red_sum[W];
   const int tid = threadIdx.x, wave = tid >> 6;
   const long src = rows ? rows[blockIdx.x] : (long)blockIdx.x;
@@ -244,33 +287,32 @@ extern "C" int mgpt_layernorm(const float* x, const float* w, const float* b, vo
   const int need = (width / 4 + MGPT_WAVE - 1) / MGPT_WAVE;   // vectors of four per lane of one wave
 #define LN_LAUNCH(OT, V) \
   hipLaunchKernelGGL((layernorm_vec_kernel<OT, V>), grid, block, 0, stream, x, w, b, (OT*)out, rows, n_rows, width, eps)
-#define LN_ROW(OT, W) \
-  hipLaunchKernelGGL((layernorm_row_kernel<OT, W>), dim3(n_rows), dim3(64 * W), 0, stream, x, w, b, (OT*)out, rows, width, eps)
-#define LN_PICK_WAVE(OT)                \
-  if (need <= 3) LN_LAUNCH(OT, 3);      \
-  else if (need <= 4) LN_LAUNCH(OT, 4); \
-  else if (need <= 6) LN_LAUNCH(OT, 6); \
+#define LN_SHARED(OT, W)                                                                                                 \
+  hipLaunchKernelGGL((layernorm_shared_kernel<OT, W>), dim3(n_rows), dim3(64 * W), 0, stream, x, w, b, (OT*)out, rows, \
+                     width, eps)
+#define LN_PICK(OT)                                                                                                  \
+  if (need <= 1) LN_LAUNCH(OT, 1);                                                                                   \
+  else if (need <= 2) LN_LAUNCH(OT, 2);                                                                              \
+  else if (need > 8)                                                                                                 \
+    hipLaunchKernelGGL((layernorm_row_kernel<OT>), dim3(n_rows), dim3(1024), 0, stream, x, w, b, (OT*)out, rows, width,     \
+                       eps);                                                                                         \
+  else if ((long)n_rows * need <= 1920) {                                                                            \
+    if (need <= 3) LN_SHARED(OT, 3);                                                                                 \
+    else if (need <= 4) LN_SHARED(OT, 4);                                                                            \
+    else if (need <= 5) LN_SHARED(OT, 5);                                                                            \
+    else if (need <= 6) LN_SHARED(OT, 6);                                                                            \
+    else if (need <= 7) LN_SHARED(OT, 7);                                                                            \
+    else LN_SHARED(OT, 8);                                                                                           \
+  } else if (need <= 3) LN_LAUNCH(OT, 3);                                                                            \
+  else if (need <= 4) LN_LAUNCH(OT, 4);                                                                              \
+  else if (need <= 6) LN_LAUNCH(OT, 6);                                                                              \
   else LN_LAUNCH(OT, 8)
-#define LN_PICK_ROW(OT)               \
-  if (need <= 3) LN_ROW(OT, 3);       \
-  else if (need <= 4) LN_ROW(OT, 4);  \
-  else if (need <= 5) LN_ROW(OT, 5);  \
-  else if (need <= 6) LN_ROW(OT, 6);  \
-  else if (need <= 7) LN_ROW(OT, 7);  \
-  else if (need <= 8) LN_ROW(OT, 8);  \
-  else LN_ROW(OT, 16)
   if (vec && out_dtype == MGPT_F32) {
-    if (need <= 1) LN_LAUNCH(float, 1);
-    else if (need <= 2) LN_LAUNCH(float, 2);
-    else { LN_PICK_ROW(float); }
+    LN_PICK(float);
   } else if (vec && out_dtype == MGPT_BF16) {
-    if (need <= 1) LN_LAUNCH(bf16_t, 1);
-    else if (need <= 2) LN_LAUNCH(bf16_t, 2);
-    else if (n_rows <= 640 || need > 8) { LN_PICK_ROW(bf16_t); }
-    else { LN_PICK_WAVE(bf16_t); }
-#undef LN_PICK_ROW
-#undef LN_PICK_WAVE
-#undef LN_ROW
+    LN_PICK(bf16_t);
+#undef LN_PICK
+#undef LN_SHARED
 #undef LN_LAUNCH
   } else if (out_dtype == MGPT_F32) {
     hipLaunchKernelGGL(layernorm_kernel<float>, grid, block, 0, stream, x, w, b, (float*)out, rows,

@@ -61,8 +61,25 @@ def test_layer_norm(out_dtype, width, bias, eps):
 @pytest.mark.parametrize("out_dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("width", [516, 772, 1028, 1540, 2044, 4096, 4100])
 def test_layer_norm_of_rows_in_several_waves(out_dtype, width):
-    """A 16-byte piece a lane in 3, 4, 6, 8 or 16 waves; longer rows go to the kernel with a wave a row."""
+    """A 16-byte piece a lane: in 3, 4, 6 or 8 waves where the rows are few, else in one; in 16 waves; longer rows go to the
+    kernel that reads them three times."""
     test_layer_norm(out_dtype, width, True, 1e-5)
+
+
+@pytest.mark.parametrize("out_dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("width", [512, 516, 768, 1000, 1280, 1284, 1600, 1796, 2044, 2048, 2052, 4096])
+def test_layer_norm_keeps_its_sums_whatever_the_number_of_rows(out_dtype, width):
+    """Few rows of 513 to 2,048 values have a workgroup of several waves each, more rows a wave each (the line lies at 1,920
+    waves): a row's result is the same bits in both."""
+    g = torch.Generator().manual_seed(width)
+    few = 1920 // (-(-width // 256))
+    x, w, b = (rnd(g, few + 1, width, scale=3.0) + 1.0).to(DEV), rnd(g, width).to(DEV), rnd(g, width).to(DEV)
+    got = [torch.empty(n, width, dtype=TDT[out_dtype], device=DEV) for n in (few + 1, few, 3)]
+    for out in got:
+        kernels.layer_norm(x, w, b, out, out.shape[0], 1e-5)
+    assert torch.equal(got[0][:few], got[1]) and torch.equal(got[0][:3], got[2])
+    helpers.assert_close(got[0][:3], torch.nn.functional.layer_norm(x[:3].double(), (width,), w.double(), b.double(), 1e-5),
+                         out_dtype, "layer_norm")
 
 
 # ----------------------------------------------------------------------------- linear

@@ -196,11 +196,15 @@ __global__ __launch_bounds__(256) void rms_post_norm_kernel(RmsBranches br, int 
     store_f(h, h_dtype, base + c, x[base + c] * rx * (offset + gain_next[c]));
 }
 
-// The same step for one or two branches and rows of W waves' 16-byte pieces, one a lane (up to 4,096 values): every value is
-// loaded once, and all of them (the row, the sublayers' outputs, the gains) are on their way before the first sum.  With 4 to 16
-// values of 4 bytes a thread and a test of the output's type for each a call took 5.4 us on average over prompts and decode
-// steps of width 1,024; here 4.1.
-template <int W, int NB>
+// The same step for one or two branches and rows of up to 4,096 values, four a lane of W waves: every value is loaded once,
+// and all of them (the row, the sublayers' outputs, the gains) are on their way before the first sum.  PIECES: rows that
+// 16-byte pieces cover; other rows have a lane's four values 64 W apart, so that a wave's 4-byte loads lie together.  A row's
+// sums then run in another order, but always in the same.  Four waves with 4 to 16 values of 4 bytes a thread and a test of the
+// output's type for each / here, us a call: 8 rows of 1,024 2.72 / 2.10, of 1,023 3.23 / 2.80, of 2,048 3.6 / 2.4, of 2,047
+// 4.2 / 3.1; 3,000 rows of 1,023 10.3 / 9.0, of 2,047 19.4 / 18.5.  The kernel above, which reads a row three to five times,
+// took 4.2 and 12.4 for 8 and 3,000 rows of 1,023, 5.7 and 22.9 for rows of 2,047.  (Five and twelve waves: 1,026 values are a
+// little over two rounds of eight waves' lanes, 3,000 such rows 11.6 us; in five waves 10.1, before 10.8.)
+template <int W, int NB, bool PIECES>
 __global__ __launch_bounds__(64 * W) void rms_post_norm_row_kernel(RmsBranches br, float coef, int join_unit,
                                                                    float* __restrict__ x, const float* __restrict__ gain_post,
                                                                    const float* __restrict__ scale_post, float offset,
@@ -208,10 +212,25 @@ __global__ __launch_bounds__(64 * W) void rms_post_norm_row_kernel(RmsBranches b
                                                                    void* __restrict__ h, int h_dtype, int width) {
   __shared__ float scratch[W];
   const int tid = threadIdx.x;
-  const bool in = 4 * tid < width;
-  const long at = (long)blockIdx.x * width + (in ? 4 * tid : 0);
-  const int c = in ? 4 * tid : 0;
-  auto load4 = [](const float* p) { return *reinterpret_cast<const float4*>(p); };
+  const bool in = (PIECES ? 4 * tid : tid) < width;
+  const int c = in ? (PIECES ? 4 * tid : tid) : 0;
+  const long base = (long)blockIdx.x * width;
+  // this thread's values of a row: four neighbouring ones, or those at tid, tid + 64 W, ... (zeros behind the row's end)
+  auto load4 = [&](const float* p) {
+    if (PIECES) return *reinterpret_cast<const float4*>(p + c);
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (in) v.x = p[c];
+    if (c + 64 * W < width) v.y = p[c + 64 * W];
+    if (c + 128 * W < width) v.z = p[c + 128 * W];
+    if (c + 192 * W < width) v.w = p[c + 192 * W];
+    return v;
+  };
+  auto each = [&](auto store) {   // !PIECES: store(place in the buffer, which value)
+    store(base + c, 0);
+    if (c + 64 * W < width) store(base + c + 64 * W, 1);
+    if (c + 128 * W < width) store(base + c + 128 * W, 2);
+    if (c + 192 * W < width) store(base + c + 192 * W, 3);
+  };
   // sum over the workgroup, the same value in every thread; waves are added in order
   auto block_sum = [&](float v) {
     v = wave_sum(in ? v : 0.f);
@@ -227,14 +246,14 @@ __global__ __launch_bounds__(64 * W) void rms_post_norm_row_kernel(RmsBranches b
   float4 yv[NB], jg[NB];
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
-    yv[b] = load4(br.y[b] + at);
-    if (NB > 1) jg[b] = load4(br.gain[b] + c);
+    yv[b] = load4(br.y[b] + base);
+    if (NB > 1) jg[b] = load4(br.gain[b]);
   }
-  float4 xv = load4(x + at);
-  const float4 gp = load4(gain_post + c);
+  float4 xv = load4(x + base);
+  const float4 gp = load4(gain_post);
   float4 sp = make_float4(1.f, 1.f, 1.f, 1.f), gn = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (scale_post) sp = load4(scale_post + c);
-  if (gain_next) gn = load4(gain_next + c);
+  if (scale_post) sp = load4(scale_post);
+  if (gain_next) gn = load4(gain_next);
   if (NB > 1) {
     // the branches' outputs, each normed with its own plain gain, averaged
     float r[NB];
@@ -255,10 +274,17 @@ __global__ __launch_bounds__(64 * W) void rms_post_norm_row_kernel(RmsBranches b
   xv.y += yv[0].y * ry * ((offset + gp.y) * sp.y);
   xv.z += yv[0].z * ry * ((offset + gp.z) * sp.z);
   xv.w += yv[0].w * ry * ((offset + gp.w) * sp.w);
-  if (in) {
-    *reinterpret_cast<float4*>(x + at) = xv;
+  if (in && PIECES) {
+    *reinterpret_cast<float4*>(x + base + c) = xv;
 #pragma unroll
-    for (int b = 0; b < NB; ++b) *reinterpret_cast<float4*>(br.y[b] + at) = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int b = 0; b < NB; ++b) *reinterpret_cast<float4*>(br.y[b] + base + c) = make_float4(0.f, 0.f, 0.f, 0.f);
+  } else if (in) {
+    const float xe[4] = {xv.x, xv.y, xv.z, xv.w};
+    each([&](long at, int e) {
+      x[at] = xe[e];
+#pragma unroll
+      for (int b = 0; b < NB; ++b) br.y[b][at] = 0.f;
+    });
   }
   if (!gain_next && !h) return;
   float4 v = xv;
@@ -268,8 +294,15 @@ __global__ __launch_bounds__(64 * W) void rms_post_norm_row_kernel(RmsBranches b
                     xv.w * rx * (offset + gn.w));
   }
   if (!in) return;
-  if (h_dtype == MGPT_F32) *reinterpret_cast<float4*>(reinterpret_cast<float*>(h) + at) = v;
-  else *reinterpret_cast<uint2*>(reinterpret_cast<bf16_t*>(h) + at) = make_uint2(pack_bf16x2(v.x, v.y), pack_bf16x2(v.z, v.w));
+  if (!PIECES) {
+    const float ve[4] = {v.x, v.y, v.z, v.w};
+    each([&](long at, int e) { store_f(h, h_dtype, at, ve[e]); });
+  } else if (h_dtype == MGPT_F32) {
+    *reinterpret_cast<float4*>(reinterpret_cast<float*>(h) + base + c) = v;
+  } else {
+    uint2* dst = reinterpret_cast<uint2*>(reinterpret_cast<bf16_t*>(h) + base + c);
+    *dst = make_uint2(pack_bf16x2(v.x, v.y), pack_bf16x2(v.z, v.w));
+  }
 }
 
 // y_ptrs / gain_ptrs: n_branches device pointers each (float32 [n_rows, width] buffers; [width] gains, unused
@@ -288,24 +321,28 @@ extern "C" int mgpt_rms_post_norm(float* y0, float* y1, float* y2, float* y3, co
     if (!br.y[b] || (n_branches > 1 && !br.gain[b])) return MGPT_ERR_NULL;
   uintptr_t together = (uintptr_t)x | (uintptr_t)gain_post | (uintptr_t)scale_post | (uintptr_t)gain_next | (uintptr_t)h;
   for (int b = 0; b < n_branches; ++b) together |= (uintptr_t)br.y[b] | (n_branches > 1 ? (uintptr_t)br.gain[b] : 0);
-  const bool pieces = width % 4 == 0 && width <= 4096 && n_branches <= 2 && (together & 15) == 0;
-#define RPN_ROW2(W, NB)                                                                                               \
-  hipLaunchKernelGGL((rms_post_norm_row_kernel<W, NB>), dim3(n_rows), dim3(64 * W), 0, stream, br, coef, join_unit, x, \
-                     gain_post, scale_post, offset, eps, mult, gain_next, h, h_dtype, width)
-#define RPN_ROW(W)                        \
-  do {                                    \
-    if (n_branches == 1) RPN_ROW2(W, 1);  \
-    else RPN_ROW2(W, 2);                  \
+  const bool row = width <= 4096 && n_branches <= 2, pieces = width % 4 == 0 && (together & 15) == 0;
+#define RPN_ROW3(W, NB, PIECES)                                                                                         \
+  hipLaunchKernelGGL((rms_post_norm_row_kernel<W, NB, PIECES>), dim3(n_rows), dim3(64 * W), 0, stream, br, coef, join_unit, \
+                     x, gain_post, scale_post, offset, eps, mult, gain_next, h, h_dtype, width)
+#define RPN_ROW(W)                                          \
+  do {                                                      \
+    if (n_branches == 1 && pieces) RPN_ROW3(W, 1, true);    \
+    else if (n_branches == 1) RPN_ROW3(W, 1, false);        \
+    else if (pieces) RPN_ROW3(W, 2, true);                  \
+    else RPN_ROW3(W, 2, false);                             \
   } while (0)
-  if (pieces && width <= 256) RPN_ROW(1);
-  else if (pieces && width <= 512) RPN_ROW(2);
-  else if (pieces && width <= 1024) RPN_ROW(4);
-  else if (pieces && width <= 2048) RPN_ROW(8);
-  else if (pieces) RPN_ROW(16);
+  if (row && width <= 256) RPN_ROW(1);
+  else if (row && width <= 512) RPN_ROW(2);
+  else if (row && width <= 1024) RPN_ROW(4);
+  else if (row && width <= 1280 && !pieces) RPN_ROW(5);
+  else if (row && width <= 2048) RPN_ROW(8);
+  else if (row && width <= 3072 && !pieces) RPN_ROW(12);
+  else if (row) RPN_ROW(16);
   else
     hipLaunchKernelGGL(rms_post_norm_kernel, dim3(n_rows), dim3(256), 0, stream, br, n_branches, coef, join_unit, x, gain_post,
                        scale_post, offset, eps, mult, gain_next, h, h_dtype, n_rows, width);
-#undef RPN_ROW2
+#undef RPN_ROW3
 #undef RPN_ROW
   return mgpt_last_error();
 }

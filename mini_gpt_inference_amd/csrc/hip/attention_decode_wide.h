@@ -146,11 +146,18 @@ __device__ __forceinline__ void aw_decode(
       dot = aw_dot2(qraw.y, kraw[i].y, dot);
       dot = aw_dot2(qraw.z, kraw[i].z, dot);
       dot = aw_dot2(qraw.w, kraw[i].w, dot);
-      dot = aw_group_sum<LPK>(dot) * scale_log2e;
-      if (cap_log2e > 0.f) dot = cap_log2e * tanh_fast(dot * __builtin_amdgcn_rcpf(cap_log2e));   // capped scores
-      if (BIAS == 1) dot = fmaf(by_dist[i], 1.4426950408889634f, dot);
-      if (BIAS == 2) dot = fmaf(-slope_log2e, (float)(qpos - (c0 + i * KPI + sub)), dot);
-      s[i] = valid[i] ? dot : -INFINITY;
+      s[i] = aw_group_sum<LPK>(dot) * scale_log2e;
+    }
+    // capped scores, in one branch around all keys: a test for every key is turned into a tanh for every key, capped or not
+    if (cap_log2e > 0.f) {
+#pragma unroll
+      for (int i = 0; i < LPK; ++i) s[i] = cap_log2e * tanh_fast(s[i] * __builtin_amdgcn_rcpf(cap_log2e));
+    }
+#pragma unroll
+    for (int i = 0; i < LPK; ++i) {
+      if (BIAS == 1) s[i] = fmaf(by_dist[i], 1.4426950408889634f, s[i]);
+      if (BIAS == 2) s[i] = fmaf(-slope_log2e, (float)(qpos - (c0 + i * KPI + sub)), s[i]);
+      s[i] = valid[i] ? s[i] : -INFINITY;
       cmax = fmaxf(cmax, s[i]);
     }
     const float m_new = weigh ? 0.f : fmaxf(m, aw_wave_max(cmax));

@@ -51,8 +51,10 @@ __device__ __forceinline__ ex_f4 ex_load(const float* __restrict__ row, int k, i
     if (k < k_dim) v = *reinterpret_cast<const ex_f4*>(row + k);
   } else {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (k + i < k_dim) v[i] = row[k + i];
+    for (int i = 0; i < 4; ++i) {
+      const float x = row[k + i < k_dim ? k + i : k_dim - 1];   // (no branch between the loads)
+      v[i] = k + i < k_dim ? x : 0.f;
+    }
   }
   return v;
 }
@@ -187,7 +189,10 @@ __global__ __launch_bounds__(256) void linear_exact_tile_kernel(
 // waves on blocks of its own (wave w: blocks w, w + waves, ...), operands straight from memory; the blocks' sums meet in
 // LDS and are added up in order.  Four groups of a block are loaded while the four before are multiplied.  Nothing is
 // shared between waves, so beyond a few dozen rows its loads bound it, at 33 TFLOP/s.
-template <int EPI, bool VEC>
+//
+// SHORT: inner sizes of up to 192, whose last groups are not there at all, not even as zeros to add (16 rows with an inner size
+// of 64 / 37: 4.2 / 6.1 us with those zeros, 3.4 / 3.5 without; the test costs longer ones 0.15 us).
+template <int EPI, bool VEC, bool SHORT>
 __global__ __launch_bounds__(1024) void linear_exact_rows_kernel(
     const float* __restrict__ A, long lda, const float* __restrict__ W, const float* __restrict__ bias,
     float* __restrict__ out, long ldo, int n_rows, int n_out, int k_dim, int row_tiles, ExactScatter sc) {
@@ -221,6 +226,7 @@ __global__ __launch_bounds__(1024) void linear_exact_rows_kernel(
       load(0, kb);
 #pragma unroll
       for (int q = 0; q < EX_BLOCK / EX_GROUP / U; ++q) {
+        if (SHORT && q && q * U * EX_GROUP >= k_dim) break;
         if (q + 1 < EX_BLOCK / EX_GROUP / U) load((q + 1) & 1, kb + (q + 1) * U * EX_GROUP);
 #pragma unroll
         for (int u = 0; u < U; ++u)
@@ -284,9 +290,13 @@ static int launch_rows(const ExactArgs& a, hipStream_t stream) {
   if ((long)row_tiles * col_tiles > 0x7fffffffL) return MGPT_ERR_TOO_LARGE;
   const int blocks = (a.k_dim + EX_BLOCK - 1) / EX_BLOCK;
   const int rounds = (blocks + 15) / 16, waves = (blocks + rounds - 1) / rounds;
-  hipLaunchKernelGGL((linear_exact_rows_kernel<EPI, VEC>), dim3(row_tiles * col_tiles), dim3(64 * waves),
-                     waves * 256 * (int)sizeof(float), stream, a.A, a.lda, a.W, a.bias, a.out, a.ldo, a.n_rows, a.n_out,
-                     a.k_dim, row_tiles, a.sc);
+#define EX_ROWS_LAUNCH(SHORT)                                                                                              \
+  hipLaunchKernelGGL((linear_exact_rows_kernel<EPI, VEC, SHORT>), dim3(row_tiles * col_tiles), dim3(64 * waves),          \
+                     waves * 256 * (int)sizeof(float), stream, a.A, a.lda, a.W, a.bias, a.out, a.ldo, a.n_rows, a.n_out, \
+                     a.k_dim, row_tiles, a.sc)
+  if (a.k_dim <= 192) EX_ROWS_LAUNCH(true);
+  else EX_ROWS_LAUNCH(false);
+#undef EX_ROWS_LAUNCH
   return mgpt_last_error();
 }
 

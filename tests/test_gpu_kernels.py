@@ -149,7 +149,7 @@ def test_linear_generic_takes_any_inner_size(a_dt, w_dt, o_dt, n, k):
     assert (out[n] == 7.0).all()
 
 
-@pytest.mark.parametrize("k", [1, 15, 17, 256, 258, 300, 512, 4100, 4352])
+@pytest.mark.parametrize("k", [1, 15, 17, 64, 65, 128, 192, 193, 256, 258, 300, 512, 4100, 4352])
 def test_float32_product_keeps_its_sums_whatever_the_tiles(k):
     """A product that is float32 throughout goes to one of three kernels by its size: a workgroup per 16 x 16 outputs with
     a wave per 256 of k (several rounds of them beyond 16 waves), tiles of 64 x 64 and of 128 x 128.  An element's bits

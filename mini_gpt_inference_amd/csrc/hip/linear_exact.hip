@@ -308,10 +308,10 @@ enum { EX_ROWS, EX_TILE64, EX_TILE128 };
 // 32.9 / 23.3 / 61; 1,100 rows 116 / 48.7 / 63; 256 rows 3072 -> 768 41 / 78 / 223; 1,100 rows 512 -> 50304 1525 / 536 / 512.
 // The 64 x 64 FMA tiles that these kernels replace reached 10 to 15 TFLOP/s (1,100 rows 2048 -> 512: 163 us, here 54), the
 // FMA kernel for few rows took 57 us for 16 rows 3072 -> 768 (here 14).
-static int choose_kernel(const ExactArgs& a) {
-  const double k = a.k_dim, rows = 2.0 * a.n_rows * a.n_out * k / 34e6;
+extern "C" int mgpt_linear_exact_kernel(int n_rows, int n_out, int k_dim) {
+  const double k = k_dim, rows = 2.0 * n_rows * n_out * k / 34e6;
   auto rounds = [&](int b) {
-    const long tiles = (long)((a.n_rows + b - 1) / b) * ((a.n_out + b - 1) / b);
+    const long tiles = (long)((n_rows + b - 1) / b) * ((n_out + b - 1) / b);
     return (double)((tiles + 255) / 256);
   };
   const double r64 = rounds(64), t64 = r64 > 1 ? r64 * 0.019 * k : 0.0225 * k, t128 = rounds(128) * 0.068 * k;
@@ -329,7 +329,7 @@ int mgpt_linear_exact_launch(const float* A, long lda, const float* W, const flo
                              int n_out, int k_dim, int epi, const ExactScatter& sc, hipStream_t stream) {
   const ExactArgs a = {A, lda, W, bias, out, ldo, n_rows, n_out, k_dim, sc};
   const bool vec = k_dim % 4 == 0 && lda % 4 == 0 && ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(W)) & 15) == 0;
-  const int kernel = choose_kernel(a);
+  const int kernel = mgpt_linear_exact_kernel(n_rows, n_out, k_dim);
 #define EX_LAUNCH(E) return vec ? launch_kernel<E, true>(a, kernel, stream) : launch_kernel<E, false>(a, kernel, stream)
   if (epi == EPI_NONE) EX_LAUNCH(EPI_NONE);
   if (epi == EPI_GELU) EX_LAUNCH(EPI_GELU);

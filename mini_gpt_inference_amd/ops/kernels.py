@@ -159,6 +159,11 @@ def linear_generic(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor
     _check(rc, "linear_generic")
 
 
+def linear_exact_kernel(n_rows: int, n_out: int, k_dim: int) -> str:
+    """Which of its kernels a float32 product of this size goes to: "rows", "tile64" or "tile128"."""
+    return ("rows", "tile64", "tile128")[library.kernels().mgpt_linear_exact_kernel(n_rows, n_out, k_dim)]
+
+
 def linear_exact_qkv(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor, n_rows: int,
                      scatter) -> bool:
     """out[:n_rows] = a[:n_rows] @ w.T (+ bias), float32 throughout, and the key and value columns also into their pages:

@@ -117,7 +117,8 @@ def test_linear_generic(a_dt, w_dt, o_dt, epi):
 def test_linear_generic_few_rows_and_many_agree_bit_for_bit(a_dt, w_dt, o_dt, epi, n_few):
     """Few rows go to a kernel with a workgroup per 16 x 16 outputs, more to tiles: every element's sum
     runs in the same order along k in both, so a row's result is the same
-    bits whichever kernel its step's size chooses (a decode step against a prompt's step)."""
+    bits whichever kernel its step's size chooses (a decode step against a prompt's step).  (What is float32
+    throughout goes to the same kernel in both here: test_float32_product_keeps_its_sums_whatever_the_tiles.)"""
     g = torch.Generator().manual_seed(23)
     n, k, o = 50, 208, 137      # an inner size that is no multiple of the few-rows kernel's stage of 64
     a, w, bias = rnd(g, n, k, dtype=a_dt), rnd(g, o, k, dtype=w_dt), rnd(g, o)
@@ -157,28 +158,60 @@ def test_float32_product_keeps_its_sums_whatever_the_tiles(k):
     float32 sums (a chain of at most 64 groups of four products in a block of 256, then the blocks: below 1e-6 of the
     result's norm)."""
     g = torch.Generator().manual_seed(k)
-    o, n = 8192 if k <= 300 else 1100, 1030            # enough tiles for the largest one where that is cheap
+    o, n = 3501, 1030                                  # 9 x 28 tiles of 128 x 128, all but the last row and column whole
     a, w, bias = rnd(g, n, k + 3).to(DEV), rnd(g, o, k).to(DEV), rnd(g, o).to(DEV)
     whole = torch.empty(n, o, device=DEV)
+    assert kernels.linear_exact_kernel(n, o, k) == "tile128"
     kernels.linear_generic(a[:, :k], w, bias, whole, n)          # a row stride that is not the inner size
     want = a[:, :k].double() @ w.double().T + bias.double()
     assert ((whole.double() - want).norm() / want.norm()).item() < 1e-6
-    for rows, cols in ((1, o), (16, o), (17, 37), (70, 200), (130, o), (300, 515), (n, 130)):
+    used = set()
+    for rows, cols in ((1, o), (16, o), (17, 37), (70, 200), (130, o), (300, 515), (n, 130), (n, 1500), (1025, 3456), (n, 3500)):
+        used.add(kernels.linear_exact_kernel(rows, cols, k))
         part = torch.full((rows + 1, cols), 7.0, device=DEV)
         kernels.linear_generic(a[:rows, :k].contiguous(), w[:cols].contiguous(), bias[:cols].contiguous(), part, rows)
         assert torch.equal(part[:rows], whole[:rows, :cols]), f"{rows} rows, {cols} columns"
         assert (part[rows] == 7.0).all()
+    assert used == {"rows", "tile64", "tile128"}
 
 
-@pytest.mark.parametrize("n,k,h,hk,d", [(1, 64, 4, 4, 16), (16, 300, 3, 1, 10), (40, 36, 3, 3, 12), (300, 512, 8, 8, 64),
-                                        (1030, 256, 24, 20, 128), (70, 33, 1, 1, 33)])
-def test_float32_product_stores_keys_and_values(n, k, h, hk, d):
+@pytest.mark.parametrize("epi", [kernels.EPI_GELU, kernels.EPI_RESIDUAL, kernels.EPI_RELU2])
+@pytest.mark.parametrize("k,o", [(64, 3500), (300, 3501), (37, 3499)])
+def test_float32_product_epilogues_whatever_the_tiles(k, o, epi):
+    """The epilogues of the three kernels, with 16-byte stores (3,500 columns) and without: the same bits in all, and those
+    of the plain product behind the plain function (a sum, a square) or within float32 rounding of it (GELU)."""
+    g, n = torch.Generator().manual_seed(o + epi), 1030
+    a, w, bias, old = rnd(g, n, k).to(DEV), rnd(g, o, k, scale=k ** -0.5).to(DEV), rnd(g, o).to(DEV), rnd(g, n, o).to(DEV)
+    plain = torch.empty(n, o, device=DEV)
+    kernels.linear_generic(a, w, bias, plain, n)
+    used, got = set(), {}
+    for rows, cols in ((n, o), (20, o), (300, 1540), (300, 1537)):
+        used.add(kernels.linear_exact_kernel(rows, cols, k))
+        out = old[:rows + 1, :cols].clone(memory_format=torch.contiguous_format)
+        kernels.linear_generic(a[:rows].contiguous(), w[:cols].contiguous(), bias[:cols].contiguous(), out, rows, epi)
+        got[rows, cols] = out[:rows]
+        assert torch.equal(got[rows, cols], got[n, o][:rows, :cols]) and (rows == n or torch.equal(out[rows], old[rows, :cols]))
+    assert used == {"rows", "tile64", "tile128"}
+    if epi == kernels.EPI_RESIDUAL:
+        assert torch.equal(got[n, o], old + plain)
+    elif epi == kernels.EPI_RELU2:
+        assert torch.equal(got[n, o], torch.relu(plain) ** 2)
+    else:
+        helpers.assert_close(got[n, o], torch.nn.functional.gelu(plain.double(), approximate="tanh"), "float32", "GELU")
+
+
+@pytest.mark.parametrize("n,k,h,hk,d,kernel", [
+    (1, 64, 4, 4, 16, "rows"), (16, 300, 3, 1, 10, "rows"), (40, 36, 3, 3, 12, "rows"), (300, 512, 8, 8, 64, "tile64"),
+    (1030, 256, 24, 20, 128, "tile64"), (70, 33, 1, 1, 33, "rows"), (1030, 256, 100, 37, 20, "tile128"),
+    (1030, 65, 60, 23, 33, "tile128"), (1025, 300, 10, 9, 124, "tile128")])
+def test_float32_product_stores_keys_and_values(n, k, h, hk, d, kernel):
     """The projection that also stores its key and value columns into their pages: the same bits as the plain product
     followed by the kernel that copies them, in each of the product's kernels and also where no four columns of a head
     lie together; a padded row (slot -1) is stored nowhere."""
     g = torch.Generator().manual_seed(n)
     q_width, kv_width, page = h * d, hk * d, 5
     o = q_width + 2 * kv_width
+    assert kernels.linear_exact_kernel(n, o, k) == kernel
     a, w, bias = rnd(g, n, k).to(DEV), rnd(g, o, k).to(DEV), rnd(g, o).to(DEV)
     pages = -(-n // page) + 1
     slots = torch.randperm(pages * page, generator=g)[:n].to(torch.int32)

@@ -1928,7 +1928,13 @@ def decay_state_chunked(z: torch.Tensor, q_off: int, k_off: int, v_off: int, n_h
     return True
 
 
-DECAY_SEGMENT = 256     # tokens of a segment
+DECAY_SEGMENT = 256     # tokens of a segment (decay_state.hip has the same; it refuses scratch that is too small)
+
+
+def decay_state_scratch(n_tokens: int, n_req: int, n_head: int, head_dim: int, value_dim: int) -> int:
+    """Floats of scratch that decay_state_chunked needs to cut the requests into segments."""
+    segments = (n_tokens + (DECAY_SEGMENT - 1) * min(n_req, n_tokens)) // DECAY_SEGMENT
+    return segments * n_head * value_dim * (-(-head_dim // 16) * 16)
 
 
 def decay_state_segments(n_tokens: int, n_req: int, max_q_len: int, n_head: int, head_dim: int, value_dim: int) -> int:
@@ -1941,8 +1947,7 @@ def decay_state_segments(n_tokens: int, n_req: int, max_q_len: int, n_head: int,
     whole = max_q_len / 32 * (6.75 if n_req * blocks >= 256 else 5.1)
     if max_q_len <= DECAY_SEGMENT or whole <= 40 + 8.3 * n_tokens / 32 * blocks / 256:
         return 0
-    segments = (n_tokens + (DECAY_SEGMENT - 1) * min(n_req, n_tokens)) // DECAY_SEGMENT
-    return segments * n_head * value_dim * (-(-head_dim // 16) * 16)
+    return decay_state_scratch(n_tokens, n_req, n_head, head_dim, value_dim)
 
 
 GATED_STATE_MODES = {"channel_sigmoid": 0, "head_softplus": 1}

@@ -314,10 +314,14 @@ def test_decaying_state_in_segments(lens, H, D, E):
     decay = torch.tensor(([0.9995, 0.6, 0.97] * 3)[:H]).to(DEV)
     cu = torch.tensor([0] + list(np.cumsum(lens)) + [n] * 2, dtype=torch.int32, device=DEV)
     slots = torch.tensor(list(range(len(lens), 0, -1)) + [-1, 0], dtype=torch.int32, device=DEV)
-    need = (n + 255 * min(r, n)) // 256 * H * E * (-(-D // 16) * 16)
+    need = kernels.decay_state_scratch(n, r, H, D, E)
     states = [torch.full((r, H * D * E), float("nan"), device=DEV) for _ in range(2)]
     outs = [torch.zeros(n, H * E, device=DEV) for _ in range(2)]
     first = [0] * len(lens)
+    with pytest.raises(kernels.KernelError):           # a float too few
+        kernels.decay_state_chunked(torch.zeros(n, v_off + H * E, device=DEV), 0, k_off, v_off, H, D, E, decay, states[1], slots, cu,
+                                    r, n, torch.zeros(n, dtype=torch.int32, device=DEV), torch.zeros(n, 2 * H * D, device=DEV),
+                                    outs[1], added=torch.zeros(need - 1, device=DEV))
     for _ in range(2):
         z = _rnd(g, n, v_off + H * E, scale=0.5).to(DEV)
         pos = torch.tensor([f + t for f, T in zip(first, lens) for t in range(T)], dtype=torch.int32, device=DEV)

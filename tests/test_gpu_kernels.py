@@ -762,6 +762,51 @@ def test_single_tokens_and_portions_in_one_launch(seq_lens, q_lens, d, h, hk, wi
         assert (padded[n:] == 7.0).all()
 
 
+MIXED_OPTIONS = {
+    "sinks": (0, ["sinks"], {}), "cap": (0, [], {"softcap": 15.0}), "gate": (0, ["gate"], {}),
+    "kept first keys": (90, [], {"keep_first": 70}), "sigmoid weights": (0, ["score_bias"], {}),
+    "chunks": (96, [], {"chunked": True}), "sinks, cap and gate in a window": (90, ["sinks", "gate"], {"softcap": 15.0}),
+    "sigmoid weights, gate and kept first keys": (90, ["score_bias", "gate"], {"keep_first": 5}),
+    "sinks in chunks": (96, ["sinks"], {"chunked": True})}
+
+
+@pytest.mark.parametrize("option", sorted(MIXED_OPTIONS))
+@pytest.mark.parametrize("d,h,hk", [(64, 12, 12), (64, 4, 1), (128, 8, 2)])
+@pytest.mark.parametrize("seq_lens,q_lens", [([40, 513, 700], [1, 1, 130]), ([300] * 20 + [65, 1, 900], [1] * 20 + [65, 1, 640])])
+def test_single_tokens_and_portions_in_one_launch_with_every_option(seq_lens, q_lens, d, h, hk, option):
+    """Each option that the launch passes on, for both kinds of tokens, as the step's own requests and as a padded step,
+    against the general kernel in 32 bits on the same numbers."""
+    window, tensors, mask = MIXED_OPTIONS[option]
+    mask = dict(mask)
+    c = PagedCase(seq_lens, q_lens, h=h, hk=hk, d=d, page=16, dtype="bfloat16", seed=d + len(q_lens))
+    n, r = c.n, len(q_lens)
+    lead = next(i for i, q in enumerate(q_lens) if q != 1)
+    g = torch.Generator().manual_seed(d + h)
+    gate = torch.randn(n, h, generator=g).to(DEV, torch.bfloat16) if "gate" in tensors else None
+    for name in ("sinks", "score_bias"):
+        if name in tensors:
+            mask[name] = (torch.randn(h, generator=g) - (3.0 if name == "score_bias" else 0.0)).to(DEV)
+    scale, positions = d ** -0.5, i32([s - q + t for s, q in zip(seq_lens, q_lens) for t in range(q)])
+    want = torch.empty(n, h * d, device=DEV)
+    kernels.paged_attention_generic(c.q_flat.float(), want, c.kp.float(), c.vp.float(), c.bt, c.cu, c.sl, c.q_req, n, r, h, scale,
+                                    window, gate=None if gate is None else gate.float(), **mask)
+    out = torch.full((n, h * d), float("nan"), dtype=torch.bfloat16, device=DEV)
+    took = kernels.mixed_attention_bf16(c.q_flat, out, c.kp, c.vp, c.bt, positions, c.q_req, c.cu, c.sl, lead, True, lead,
+                                        r - lead, n - lead, 0, h, scale, window, gate=gate, **mask)
+    assert took == (lead * h <= 256)
+    if took:
+        helpers.assert_close(out, want, "bfloat16", "the step's own requests")
+    rows, cap = n + 5, 16
+    pad = lambda t, size, fill: torch.cat([t, torch.full((size - t.shape[0], *t.shape[1:]), fill, dtype=t.dtype, device=DEV)])
+    padded = torch.full((rows, h * d), 7.0, dtype=torch.bfloat16, device=DEV)
+    assert kernels.mixed_attention_bf16(
+        pad(c.q_flat, rows, 0.0), padded, c.kp, c.vp, pad(c.bt, r + 4, -1), pad(positions, rows, 0), pad(c.q_req, rows, -1),
+        pad(c.cu, r + 5, n), pad(c.sl, r + 4, 0), cap, False, 0, r + 4, rows, cap, h, scale, window,
+        gate=None if gate is None else pad(gate, rows, 0.0), **mask)
+    helpers.assert_close(padded[:n], want, "bfloat16", "a padded step")
+    assert (padded[n:] == 7.0).all()
+
+
 @pytest.mark.parametrize("window", [0, 100])
 @pytest.mark.parametrize("d,n", [(16, 129), (32, 129), (64, 128), (64, 129), (128, 64), (128, 65)])
 def test_decode_attention_of_many_tokens(d, n, window):

@@ -48,8 +48,9 @@ constexpr int aw_lds_floats() {
   return (W * (64 / (D / 8)) + W * 64 / D) * (D + 1) + W;
 }
 
-// Token n, head h, by a workgroup of W waves.
-template <int D, bool IDENT, int BIAS, int W>
+// Token n, head h, by a workgroup of W waves.  SIDE: 0: any token; otherwise tokens that see up to (1) or more than (-1)
+// `keys` keys; others are left alone.
+template <int D, bool IDENT, int BIAS, int W, int SIDE = 0>
 __device__ __forceinline__ void aw_decode(
     const bf16_t* __restrict__ q, long ldq, bf16_t* __restrict__ out, long ldo,
     const bf16_t* __restrict__ kpool, const bf16_t* __restrict__ vpool,
@@ -58,7 +59,7 @@ __device__ __forceinline__ void aw_decode(
     int num_pages, unsigned int page_bytes, float scale_log2e, int window, const float* __restrict__ sinks,
     float cap_log2e, const bf16_t* __restrict__ gate, long ldg, int keep_first, const float* __restrict__ score_bias,
     int chunked, const float* __restrict__ dist_bias, int bias_len, const float* __restrict__ slopes, int n,
-    int h, float* __restrict__ lds) {
+    int h, float* __restrict__ lds, int keys = 0) {
   constexpr int LPK = D / 8;     // lanes per key
   constexpr int KPI = 64 / LPK;  // keys per load instruction
   constexpr int ROWS = W * KPI;      // partial results: one per (key subgroup, wave)
@@ -87,6 +88,7 @@ __device__ __forceinline__ void aw_decode(
     if (cu_q && cu_q[r + 1] - cu_q[r] != 1) qr = -1;
   }
   const int first_key = first_seen(qpos, window, chunked);   // (with a window: waits for qpos)
+  if (SIDE != 0 && (qpos + 1 - first_key + keep_first > keys) != (SIDE < 0)) return;   // the whole workgroup
   const int first_chunk = first_key / 64;
   const int* bt = block_tables + (long)r * max_blocks;
   const bool weigh = score_bias != nullptr;   // sigmoid weights, no softmax

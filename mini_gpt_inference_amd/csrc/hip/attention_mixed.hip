@@ -7,6 +7,13 @@
 // behind them (token, head) pairs, both with the bodies of those kernels, so that they run side by side.  A pair's workgroup
 // holds a tile's LDS and registers, which is a compute unit, so it is done for up to 256 pairs; more go to their own kernel.
 //
+// Where a tile has four waves (head size 128, and 64 with many tiles) a pair has four as well, a pass of 256 keys at a time,
+// and behind long contexts that chain outlasts tiles and eight waves one behind the other: 8 requests x 8 heads of 128 beside
+// a portion of 256 tokens, behind 8,000 keys: one behind the other 84.7 us, here 110.  Lengths are known on the
+// device only (a recorded launch serves steps of any length), so tokens that see more than `keys` keys are left out here and
+// done by a second launch with eight waves each, which is made where the block table or the window allows such tokens at
+// all: 81.6 us; where no token is that long it costs 1.5 us.
+//
 // Tiles are numbered over the requests on the device, 64 queries each: the launch is sized by how many tiles so many tokens of
 // so many requests can make at most, not by the longest portion times the requests.
 #include "attention_decode_wide.h"
@@ -24,7 +31,19 @@ struct MixedArgs {
   const float* sinks; float softcap;
   const bf16_t* gate; long ldg;
   int keep_first; const float* score_bias; int chunked;
+  int keys;                  // a pair with four waves: up to so many keys
 };
+
+// Pair number b of the step's single tokens and heads.
+template <int D, bool IDENT, int W, int SIDE>
+__device__ __forceinline__ void mx_pair(const MixedArgs& a, int b, float* lds) {
+  const float log2e = 1.4426950408889634f;
+  aw_decode<D, IDENT, 0, W, SIDE>(a.q, a.ldq, a.out, a.ldo, a.kpool, a.vpool, a.block_tables, a.max_blocks, a.positions,
+                                  a.q_req, IDENT ? nullptr : a.cu_q, a.n_head, a.n_kv_head, a.page_shift, a.num_pages,
+                                  a.page_bytes, a.scale * log2e, a.window, a.sinks,
+                                  a.softcap > 0.f ? a.softcap * log2e : 0.f, a.gate, a.ldg, a.keep_first, a.score_bias,
+                                  a.chunked, nullptr, 0, nullptr, b % a.n_decode, b / a.n_decode, lds, a.keys);
+}
 
 // IDENT: the single tokens are those of requests 0 .. n_decode - 1; else q_req names a token's request, and requests with more
 // than one token are passed over
@@ -37,12 +56,7 @@ __global__ __launch_bounds__(256 * G) void mixed_attention_kernel(MixedArgs a) {
   const int n_tiles = a.tiles * a.n_head;
   if (b >= n_tiles) {
     b -= n_tiles;
-    const float log2e = 1.4426950408889634f;
-    aw_decode<D, IDENT, 0, W>(a.q, a.ldq, a.out, a.ldo, a.kpool, a.vpool, a.block_tables, a.max_blocks, a.positions, a.q_req,
-                              IDENT ? nullptr : a.cu_q, a.n_head, a.n_kv_head, a.page_shift, a.num_pages, a.page_bytes,
-                              a.scale * log2e, a.window, a.sinks, a.softcap > 0.f ? a.softcap * log2e : 0.f, a.gate, a.ldg,
-                              a.keep_first, a.score_bias, a.chunked, nullptr, 0, nullptr, b % a.n_decode, b / a.n_decode,
-                              reinterpret_cast<float*>(mx_lds));
+    mx_pair<D, IDENT, W, G == 2 ? 0 : 1>(a, b, reinterpret_cast<float*>(mx_lds));
     return;
   }
   const int h = b / a.tiles;
@@ -76,6 +90,13 @@ __global__ __launch_bounds__(256 * G) void mixed_attention_kernel(MixedArgs a) {
                    __builtin_amdgcn_readfirstlane(r), h, mx_lds);
 }
 
+// Single tokens that see more than a.keys keys.
+template <int D, bool IDENT>
+__global__ __launch_bounds__(512) void long_pairs_kernel(MixedArgs a) {
+  __shared__ __align__(16) float lds[aw_lds_floats<D, 8>()];
+  mx_pair<D, IDENT, 8, -1>(a, blockIdx.x, lds);
+}
+
 template <int D, int G, bool IDENT>
 static int launch(const MixedArgs& a, hipStream_t stream) {
   constexpr int bytes = pf_lds_bytes<D, G, 0>();
@@ -88,6 +109,11 @@ static int launch(const MixedArgs& a, hipStream_t stream) {
   }
   hipLaunchKernelGGL((mixed_attention_kernel<D, G, IDENT>), dim3((a.tiles + a.n_decode) * a.n_head), dim3(256 * G), bytes, stream,
                      a);
+  if constexpr (G == 1) {
+    const long most = a.window > 0 ? (long)a.window + a.keep_first : (long)a.max_blocks * a.page_size;   // that a token can see
+    if (most > a.keys)
+      hipLaunchKernelGGL((long_pairs_kernel<D, IDENT>), dim3(a.n_decode * a.n_head), dim3(512), 0, stream, a);
+  }
   return mgpt_last_error();
 }
 
@@ -113,10 +139,14 @@ extern "C" int mgpt_mixed_attention_bf16(
   if ((tiles + n_decode) * n_head > 0x7fffffffL) return MGPT_ERR_TOO_LARGE;
   int page_shift = 0;
   while ((1 << page_shift) < page_size) ++page_shift;
+  // what four waves lose on a token against eight, 0.005 us a key, is to be no more than what the tiles beside them take and a
+  // launch, 7 us for a portion of 64 tokens, 19 for 512; head size 64 comes here with hundreds of tiles only and loses less
+  const int keys = head_dim == 64 ? 16384 : (n_tokens < 512 ? 1024 + 6 * n_tokens : 4096);
   const MixedArgs a = {(const bf16_t*)q, ldq, (bf16_t*)out, ldo, (const bf16_t*)kpool, (const bf16_t*)vpool, block_tables,
                        max_blocks, positions, q_req, cu_q, seq_lens, n_decode, first_req, n_req, (int)tiles, single_below, n_head,
                        n_kv_head, page_size, page_shift, num_pages, (unsigned int)(n_kv_head * page_size * head_dim * 2), scale,
-                       window, sinks, softcap, (const bf16_t*)gate, ldg, window == 0 ? 0 : keep_first, score_bias, chunked};
+                       window, sinks, softcap, (const bf16_t*)gate, ldg, window == 0 ? 0 : keep_first, score_bias, chunked,
+                       keys};
   // two wave groups a tile while the tiles are few, as for prompt portions alone
   if (head_dim == 128) return identity ? launch<128, 1, true>(a, stream) : launch<128, 1, false>(a, stream);
   if (tiles * n_head <= 320) return identity ? launch<64, 2, true>(a, stream) : launch<64, 2, false>(a, stream);

@@ -807,6 +807,32 @@ def test_single_tokens_and_portions_in_one_launch_with_every_option(seq_lens, q_
     assert (padded[n:] == 7.0).all()
 
 
+@pytest.mark.parametrize("d,h,hk,portion,keys,window", [(128, 4, 1, 30, 1204, 0), (128, 4, 1, 30, 1204, 1203),
+                                                        (128, 4, 1, 30, 1204, 1204), (128, 4, 1, 30, 1204, 1250),
+                                                        (128, 4, 1, 700, 4096, 0), (64, 12, 1, 2048, 16384, 0)])
+def test_single_tokens_behind_long_contexts_beside_a_portion(d, h, hk, portion, keys, window):
+    """Where a token's workgroup has four waves, tokens that see more than so many keys have a second launch of their own:
+    every token is done by one of the two, around that number, as the step's own requests and as a padded step, also with a
+    window that keeps some of them or all below it."""
+    seq_lens = [keys - 1, keys, keys + 1, 40, keys + 300, portion + 50]
+    q_lens = [1] * 5 + [portion]
+    c = PagedCase(seq_lens, q_lens, h=h, hk=hk, d=d, page=16, dtype="bfloat16", seed=portion)
+    n, r, lead, scale = c.n, len(q_lens), 5, d ** -0.5
+    positions = i32([s - q + t for s, q in zip(seq_lens, q_lens) for t in range(q)])
+    for mask in ({}, {"keep_first": 10} if window else {"softcap": 20.0}):
+        want = torch.empty(n, h * d, device=DEV)
+        kernels.paged_attention_generic(c.q_flat.float(), want, c.kp.float(), c.vp.float(), c.bt, c.cu, c.sl, c.q_req, n, r, h,
+                                        scale, window, **mask)
+        out = torch.full((n, h * d), float("nan"), dtype=torch.bfloat16, device=DEV)
+        assert kernels.mixed_attention_bf16(c.q_flat, out, c.kp, c.vp, c.bt, positions, c.q_req, c.cu, c.sl, lead, True, lead, 1,
+                                            portion, 0, h, scale, window, **mask)
+        helpers.assert_close(out, want, "bfloat16", "the step's own requests")
+        padded = torch.full((n, h * d), float("nan"), dtype=torch.bfloat16, device=DEV)
+        assert kernels.mixed_attention_bf16(c.q_flat, padded, c.kp, c.vp, c.bt, positions, c.q_req, c.cu, c.sl, 8, False, 0, r,
+                                            n, 8, h, scale, window, **mask)
+        helpers.assert_close(padded, want, "bfloat16", "a padded step")
+
+
 @pytest.mark.parametrize("window", [0, 100])
 @pytest.mark.parametrize("d,n", [(16, 129), (32, 129), (64, 128), (64, 129), (128, 64), (128, 65)])
 def test_decode_attention_of_many_tokens(d, n, window):

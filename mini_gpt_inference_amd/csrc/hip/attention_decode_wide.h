@@ -40,15 +40,14 @@ __device__ __forceinline__ float aw_dot2(unsigned int a, unsigned int b, float c
                                          c, false);
 }
 
-// IDENT: token n is request n (or padded), so its block table row is known before anything is loaded
-
 // Floats of LDS that it takes.
 template <int D, int W>
 constexpr int aw_lds_floats() {
   return (W * (64 / (D / 8)) + W * 64 / D) * (D + 1) + W;
 }
 
-// Token n, head h, by a workgroup of W waves.  SIDE: 0: any token; otherwise tokens that see up to (1) or more than (-1)
+// Token n, head h, by a workgroup of W waves.  IDENT: token n is request n (or padded), so its block table row is known before
+// anything is loaded.  SIDE: 0: any token; otherwise tokens that see up to (1) or more than (-1)
 // `keys` keys; others are left alone.
 template <int D, bool IDENT, int BIAS, int W, int SIDE = 0>
 __device__ __forceinline__ void aw_decode(

@@ -34,7 +34,8 @@
 // the chip holds such workgroups at a time (two a compute unit, one with a head size of 128 and its 166 registers), four
 // waves: more workgroups at a time, and fewer waves without a chunk under short contexts.  Eight / four waves, us: 32
 // tokens x 25 heads of 64 behind 40, 150, 400 and 1,000 keys 8.0 / 5.3, 9.0 / 6.8, 16.7 / 16.6, 34.4 / 34.4; 256 x 25 behind 40
-// and 400 40 / 20, 116 / 116 (5.6 TB/s); 40 x 16 of 128 behind 150 and 1,000 19.4 / 12.7, 64 / 59.
+// and 400 40 / 20, 116 / 116 (5.6 TB/s); 40 x 16 of 128 behind 150 and 1,000 19.4 / 12.7, 64 / 59.  (With the cap's branch
+// around a pass both are 1 to 10 % faster: 100 x 12 of 64 behind 150 and 1,000 keys 6.0 and 31.4.)
 template <int D, bool IDENT, int BIAS, int W>
 __global__ __launch_bounds__(W * 64) void paged_attention_decode_kernel(
     const bf16_t* __restrict__ q, long ldq, bf16_t* __restrict__ out, long ldo,

@@ -536,15 +536,16 @@ __device__ __forceinline__ unsigned int wave_list_floor(const unsigned int* key,
 // its 16 waves over 50 logits a thread; a row cut over workgroups would need them to meet.
 //
 // A thread's stretch comes through LDS: a wave loads its 64 stretches, which lie one behind the other, 64 logits at a
-// time, half of the lanes' stretches after the other.  Stretches and the order of the sums are those of the kernel
-// above, so that the token is the same.
+// time, half of the lanes' stretches after the other.  Stretches and the order of the inverse CDF's sums are those of the
+// kernel above: from the same kept logits the token is the same.  What top-k keeps is the same; top-p's masses are summed
+// in another order here, so a logit whose mass ends within float32 rounding of p may be kept by one and not by the other.
 //
 // Top-k: the k-th largest of the threads' own largest logits bounds the k-th largest logit from below; the few logits
 // above that bound go to a list, in which one wave finds the k-th largest and the top-p bound, with no barrier between
 // its rounds.  The bound is on the unscaled logits, eight representable numbers lower, because logits that differ by
 // less may be equal after the division by a temperature of at most 4.  Rows with infinities or NaN, higher temperatures,
 // k over 512 and rows whose list would be too long search over all registers instead; so does top-p alone, until at
-// most 1,024 logits are left undecided.
+// most SAMPLE_LIST logits are left undecided.
 template <int K>
 __global__ __launch_bounds__(SAMPLE_THREADS) void sample_held_kernel(
     const float* __restrict__ logits, long ld, int vocab, int real_vocab,
@@ -864,8 +865,8 @@ static int launch_sample(const float* logits, long ld, int n_rows, int vocab, in
 #define SAMPLE_LAUNCH_HELD(K)                                                                                          \
   {                                                                                                                    \
     constexpr int words = SAMPLE_WAVES * (32 * K + K / 2 + 1) + 2 * MGPT_WAVE;                                         \
-    constexpr int bytes = (words > 3 * SAMPLE_LIST ? words : 3 * SAMPLE_LIST) * (int)sizeof(float);                              \
-    static_assert(bytes <= 160 * 1024 && bytes >= 3 * SAMPLE_LIST * 4, "a workgroup's LDS");                               \
+    constexpr int bytes = (words > 3 * SAMPLE_LIST ? words : 3 * SAMPLE_LIST) * (int)sizeof(float);                    \
+    static_assert(bytes <= 160 * 1024 && bytes >= 3 * SAMPLE_LIST * 4, "a workgroup's LDS");                           \
     static bool allowed = false; /* more LDS than a kernel gets without asking */                                      \
     if (!allowed) {                                                                                                    \
       const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(sample_held_kernel<K>),                   \

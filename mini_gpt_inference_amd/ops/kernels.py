@@ -835,7 +835,8 @@ def mixed_attention_bf16(q: torch.Tensor, out: torch.Tensor, k_pool: torch.Tenso
     _need(q.dtype == out.dtype == k_pool.dtype == v_pool.dtype, "queries, output and pools must share a dtype")
     _need(q.dim() == 2 and q.stride(1) == 1 and out.dim() == 2 and out.stride(1) == 1,
           "query and output rows must have unit inner stride")
-    _need(q.shape[0] >= max(n_decode, n_tokens) and out.shape[0] >= max(n_decode, n_tokens)
+    rows = n_decode + n_tokens if identity else max(n_decode, n_tokens)
+    _need(q.shape[0] >= rows and out.shape[0] >= rows
           and q.shape[1] >= n_head * head_dim and out.shape[1] >= n_head * head_dim, "query/output buffers are too small")
     _need(n_head % n_kv_head == 0, "n_head must be a multiple of the number of key/value heads")
     r = max(first_req + n_req, n_decode if identity else 0)

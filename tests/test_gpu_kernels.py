@@ -833,6 +833,18 @@ def test_single_tokens_behind_long_contexts_beside_a_portion(d, h, hk, portion, 
         helpers.assert_close(padded, want, "bfloat16", "a padded step")
 
 
+@pytest.mark.parametrize("short", ["queries", "output"])
+def test_single_tokens_and_portions_refuse_buffers_that_end_before_their_tokens(short):
+    """The portions' tokens lie behind the single ones: their numbers add up.  Nothing is launched."""
+    c = PagedCase([40, 50, 70], [1, 1, 70], h=4, hk=4, d=64, page=16, dtype="bfloat16", seed=3)
+    out = torch.full((c.n, 4 * 64), 7.0, dtype=torch.bfloat16, device=DEV)
+    q, o = (c.q_flat[:c.n - 1], out) if short == "queries" else (c.q_flat, out[:c.n - 1])
+    with pytest.raises(kernels.KernelError, match="too small"):
+        kernels.mixed_attention_bf16(q, o, c.kp, c.vp, c.bt, i32([39, 49] + list(range(70))), c.q_req, c.cu, c.sl, 2, True, 2, 1,
+                                     70, 0, 4, 0.125)
+    assert (out == 7.0).all()
+
+
 @pytest.mark.parametrize("window", [0, 100])
 @pytest.mark.parametrize("d,n", [(16, 129), (32, 129), (64, 128), (64, 129), (128, 64), (128, 65)])
 def test_decode_attention_of_many_tokens(d, n, window):

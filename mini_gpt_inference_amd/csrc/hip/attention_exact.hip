@@ -97,24 +97,8 @@ __global__ __launch_bounds__(64 * AX_WAVES, D == 64 ? 5 : 1) void attention_exac
   const int h = blockIdx.y, hk = h / (a.n_head / a.n_kv_head);
 
   // the request and the tile of it that this workgroup has: requests' tiles are numbered one behind the other
-  int r = -1, tile = blockIdx.x;
-  for (int r0 = 0; r0 < a.n_req; r0 += MGPT_WAVE) {
-    const int rr = r0 + lane;
-    int tiles = rr < a.n_req ? (a.cu_q[rr + 1] - a.cu_q[rr] + AX_QUERIES - 1) / AX_QUERIES : 0;
-    int upto = tiles;                                   // tiles of the requests up to this lane's
-    for (int off = 1; off < MGPT_WAVE; off <<= 1) {
-      const int o = __shfl_up(upto, off, MGPT_WAVE);
-      if (lane >= off) upto += o;
-    }
-    const uint64_t past = __ballot(upto > tile);
-    if (past) {
-      const int at = __ffsll((unsigned long long)past) - 1;
-      r = r0 + at;
-      tile -= __shfl(upto - tiles, at, MGPT_WAVE);
-      break;
-    }
-    tile -= __shfl(upto, MGPT_WAVE - 1, MGPT_WAVE);
-  }
+  int tile = blockIdx.x;
+  int r = piece_owner(a.n_req, tile, [&](int i) { return (a.cu_q[i + 1] - a.cu_q[i] + AX_QUERIES - 1) / AX_QUERIES; });
   if (r < 0) return;                                    // beyond the step's tiles: the whole workgroup
   r = __builtin_amdgcn_readfirstlane(r);
   const int q_start = a.cu_q[r], q_len = a.cu_q[r + 1] - q_start;

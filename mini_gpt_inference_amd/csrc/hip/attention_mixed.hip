@@ -60,34 +60,17 @@ __global__ __launch_bounds__(256 * G) void mixed_attention_kernel(MixedArgs a) {
     return;
   }
   const int h = b / a.tiles;
-  int tile = b - h * a.tiles, r = -1;
-  const int lane = threadIdx.x & 63;
-  for (int r0 = 0; r0 < a.n_req; r0 += MGPT_WAVE) {
-    const int rr = a.first_req + r0 + lane;
-    int tiles = 0;
-    if (r0 + lane < a.n_req) {
-      const int start = a.cu_q[rr], len = a.cu_q[rr + 1] - start;
-      if (!(len == 1 && start < a.single_below)) tiles = (len + PF_QT - 1) / PF_QT;
-    }
-    int upto = tiles;                                   // tiles of the requests up to this lane's
-    for (int off = 1; off < MGPT_WAVE; off <<= 1) {
-      const int o = __shfl_up(upto, off, MGPT_WAVE);
-      if (lane >= off) upto += o;
-    }
-    const uint64_t past = __ballot(upto > tile);
-    if (past) {
-      const int at = __ffsll((unsigned long long)past) - 1;
-      r = a.first_req + r0 + at;
-      tile -= __shfl(upto - tiles, at, MGPT_WAVE);
-      break;
-    }
-    tile -= __shfl(upto, MGPT_WAVE - 1, MGPT_WAVE);
-  }
+  int tile = b - h * a.tiles;
+  const int* cu_q = a.cu_q + a.first_req;
+  const int r = piece_owner(a.n_req, tile, [&](int i) {
+    const int start = cu_q[i], len = cu_q[i + 1] - start;
+    return len == 1 && start < a.single_below ? 0 : (len + PF_QT - 1) / PF_QT;
+  });
   if (r < 0) return;                                    // beyond the step's tiles: the whole workgroup
   pf_tile<D, G, 0>(a.q, a.ldq, a.out, a.ldo, a.kpool, a.vpool, a.block_tables, a.max_blocks, a.cu_q, a.seq_lens, a.n_head,
                    a.n_kv_head, a.page_size, a.scale, a.window, a.single_below, a.sinks, a.softcap, a.gate, a.ldg, a.keep_first,
                    a.score_bias, a.chunked, nullptr, 0, nullptr, __builtin_amdgcn_readfirstlane(tile),
-                   __builtin_amdgcn_readfirstlane(r), h, mx_lds);
+                   __builtin_amdgcn_readfirstlane(a.first_req + r), h, mx_lds);
 }
 
 // Single tokens that see more than a.keys keys.

@@ -89,6 +89,30 @@ __device__ __forceinline__ int wave_sum_int(int v) {
          (__builtin_amdgcn_readlane(v, 32) + __builtin_amdgcn_readlane(v, 48));
 }
 
+// Pieces of work that n owners have, numbered over the owners one behind the other, count(i) of owner i: the owner of piece
+// number `piece`, which becomes its number among that owner's; -1 behind the last piece.  For whole waves, the same in all
+// lanes.
+template <typename Count>
+__device__ __forceinline__ int piece_owner(int n, int& piece, Count count) {
+  const int lane = threadIdx.x & (MGPT_WAVE - 1);
+  for (int i0 = 0; i0 < n; i0 += MGPT_WAVE) {
+    const int mine = i0 + lane < n ? count(i0 + lane) : 0;
+    int upto = mine;                                    // pieces of the owners up to this lane's
+    for (int off = 1; off < MGPT_WAVE; off <<= 1) {
+      const int o = __shfl_up(upto, off, MGPT_WAVE);
+      if (lane >= off) upto += o;
+    }
+    const uint64_t past = __ballot(upto > piece);
+    if (past) {
+      const int at = __ffsll((unsigned long long)past) - 1;
+      piece -= __shfl(upto - mine, at, MGPT_WAVE);
+      return i0 + at;
+    }
+    piece -= __shfl(upto, MGPT_WAVE - 1, MGPT_WAVE);
+  }
+  return -1;
+}
+
 __device__ __forceinline__ float relu_squared(float v) {
   const float r = fmaxf(v, 0.f);
   return r * r;

@@ -249,25 +249,8 @@ __global__ __launch_bounds__(256) void decay_state_chunk_kernel(
   const int wave = tid >> 6, lane = tid & 63, r16 = lane & 15, g = lane >> 4;
   int r = blockIdx.x, seg = 0, first = 0;       // the request, its segment, the number of its first segment
   if (MODE != DC_WHOLE) {
-    int left = blockIdx.x;
-    r = -1;
-    for (int r0 = 0; r0 < n_req; r0 += 64) {
-      const int rr = r0 + lane;
-      const int mine = rr < n_req ? (cu_q[rr + 1] - cu_q[rr] + DC_SEGMENT - 1) / DC_SEGMENT : 0;
-      int upto = mine;                          // segments of the requests up to this lane's
-      for (int off = 1; off < 64; off <<= 1) {
-        const int o = __shfl_up(upto, off, 64);
-        if (lane >= off) upto += o;
-      }
-      const unsigned long long past = __ballot(upto > left);
-      if (past) {
-        const int at = __ffsll(past) - 1;
-        r = r0 + at;
-        seg = left - __shfl(upto - mine, at, 64);
-        break;
-      }
-      left -= __shfl(upto, 63, 64);
-    }
+    seg = blockIdx.x;
+    r = piece_owner(n_req, seg, [&](int i) { return (cu_q[i + 1] - cu_q[i] + DC_SEGMENT - 1) / DC_SEGMENT; });
     if (r < 0) return;                          // beyond the step's segments: the whole workgroup
     first = (int)blockIdx.x - seg;
   }

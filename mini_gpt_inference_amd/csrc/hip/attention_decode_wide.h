@@ -46,7 +46,7 @@ constexpr int aw_lds_floats() {
   return (W * (64 / (D / 8)) + W * 64 / D) * (D + 1) + W;
 }
 
-// Token n, head h, by a workgroup of W waves.  IDENT: token n is request n (or padded), so its block table row is known before
+// Token n, head h, by W waves: a workgroup, or each half of one with its own LDS, both for the same token.  IDENT: token n is request n (or padded), so its block table row is known before
 // anything is loaded.  SIDE: 0: any token; otherwise tokens that see up to (1) or more than (-1)
 // `keys` keys; others are left alone.
 template <int D, bool IDENT, int BIAS, int W, int SIDE = 0>
@@ -70,7 +70,7 @@ __device__ __forceinline__ void aw_decode(
   float* const lpart_s = l_s + ROWS;
   float* const m_s = lpart_s + SUBSETS;        // [wave]
 
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = threadIdx.x & (W * 64 - 1), lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int sub = lane / LPK, dg = lane % LPK;
   const int hk = h / (n_head / n_kv_head);

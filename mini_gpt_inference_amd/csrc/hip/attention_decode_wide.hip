@@ -12,7 +12,7 @@
 //    lie beyond the sequence are never followed (their keys are masked before the load), and
 //    an entry's page number is clamped to the pool so that a stale entry cannot send a load
 //    outside it;
-//  * eight waves (four with many tokens and heads), each with one 64-key chunk in flight (sixteen 16-byte loads per lane), so a
+//  * eight waves (four for short contexts with many tokens and heads), each with one 64-key chunk in flight (sixteen 16-byte loads per lane), so a
 //    context of up to 512 keys is one pass;
 //  * D/8 lanes share a key: scores with v_dot2_f32_bf16 on the packed rows as loaded, summed
 //    over the D/8 lanes with DPP moves; one wave-wide maximum per chunk (DPP within rows of 16,
@@ -30,14 +30,23 @@
 #include "attention_decode_wide.h"
 #include "launchers.h"
 
-// W: waves of the workgroup.  A context of up to 512 keys is one pass of eight waves; with more (token, head) pairs than
-// the chip holds such workgroups at a time (two a compute unit, one with a head size of 128 and its 166 registers), four
-// waves: more workgroups at a time, and fewer waves without a chunk under short contexts.  Eight / four waves, us: 32
-// tokens x 25 heads of 64 behind 40, 150, 400 and 1,000 keys 8.0 / 5.3, 9.0 / 6.8, 16.7 / 16.6, 34.4 / 34.4; 256 x 25 behind 40
-// and 400 40 / 20, 116 / 116 (5.6 TB/s); 40 x 16 of 128 behind 150 and 1,000 19.4 / 12.7, 64 / 59.  (With the cap's branch
-// around a pass both are 1 to 10 % faster: 100 x 12 of 64 behind 150 and 1,000 keys 6.0 and 31.4.)
-template <int D, bool IDENT, int BIAS, int W>
-__global__ __launch_bounds__(W * 64) void paged_attention_decode_kernel(
+// Waves of a (token, head) pair.  A context of up to 512 keys is one pass of eight waves; with more pairs than the chip holds
+// such workgroups at a time (two a compute unit, one with a head size of 128 and its 166 registers) four are better where
+// contexts are short: more pairs at a time, and fewer waves without a chunk.  Behind long contexts four waves are a chain twice
+// as long, which a few long requests among short ones then wait for.
+//  AW_EIGHT: eight waves a pair.
+//  AW_FOUR: four, a workgroup each: where no token can see more than AW_SHORT keys.
+//  AW_HALVES: each token by its own length, which only the device knows: with up to AW_SHORT keys an even head's workgroup
+//  has the odd head behind it as well, four waves each (the odd head's workgroup leaves at once), with more each head has eight.
+//  The wait for the position in front of all other loads is what it costs, too much for heads of 16 and 32.
+// us, always eight / always four / this rule: 64 tokens x 12 heads of 64 behind 1 to 256 keys 8.6 / 6.4 / 6.3 (AW_FOUR), behind
+// 512 18.3 / 18.4 / 18.5, one behind 1,024 or 2,048 and the others behind 100 12.8 / 15.0 / 11.3 and 19.4 / 25.0 / 18.1; 64 x 16
+// heads of 128 on 4 of keys behind 256 and 1,024 19.9 / 12.9 / 12.7 and 43.7 / 37.0 / 39.2; 48 x 8 of 128, one behind 2,048
+// 24.8 / 30.7 / 24.7.  Worst case found: 171 x 12 of 64, half behind 60 and half behind 1,024 45.9 / 46.4 / 49.0.
+enum { AW_EIGHT, AW_FOUR, AW_HALVES };
+#define AW_SHORT(D) ((D) == 128 ? 512 : 256)
+template <int D, bool IDENT, int BIAS, int WAVES>
+__global__ __launch_bounds__(WAVES == AW_FOUR ? 256 : 512) void paged_attention_decode_kernel(
     const bf16_t* __restrict__ q, long ldq, bf16_t* __restrict__ out, long ldo,
     const bf16_t* __restrict__ kpool, const bf16_t* __restrict__ vpool,
     const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ positions,
@@ -45,11 +54,26 @@ __global__ __launch_bounds__(W * 64) void paged_attention_decode_kernel(
     int num_pages, unsigned int page_bytes, float scale_log2e, int window, const float* __restrict__ sinks,
     float cap_log2e, const bf16_t* __restrict__ gate, long ldg, int keep_first, const float* __restrict__ score_bias,
     int chunked, const float* __restrict__ dist_bias, int bias_len, const float* __restrict__ slopes) {
-  __shared__ __align__(16) float lds[aw_lds_floats<D, W>()];
-  aw_decode<D, IDENT, BIAS, W>(q, ldq, out, ldo, kpool, vpool, block_tables, max_blocks, positions, q_req, cu_q, n_head, n_kv_head,
-                               page_shift, num_pages, page_bytes, scale_log2e, window, sinks, cap_log2e, gate,
-                               ldg, keep_first, score_bias, chunked, dist_bias, bias_len, slopes, blockIdx.x,
-                               blockIdx.y, lds);
+  constexpr int FOUR = (aw_lds_floats<D, 4>() + 3) & ~3, EIGHT = aw_lds_floats<D, 8>();
+  __shared__ __align__(16) float lds[WAVES == AW_FOUR ? FOUR : (WAVES == AW_HALVES && 2 * FOUR > EIGHT ? 2 * FOUR : EIGHT)];
+  const int n = blockIdx.x, h = blockIdx.y;
+  bool four = WAVES == AW_FOUR;
+  int half = 0;
+  if (WAVES == AW_HALVES) {
+    const int qpos = positions[n];
+    four = qpos + 1 - first_seen(qpos, window, chunked) + keep_first <= AW_SHORT(D) && (h | 1) < n_head;
+    if (four && (h & 1)) return;
+    half = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  }
+  if (WAVES != AW_EIGHT && four)
+    aw_decode<D, IDENT, BIAS, 4>(q, ldq, out, ldo, kpool, vpool, block_tables, max_blocks, positions, q_req, cu_q, n_head,
+                                 n_kv_head, page_shift, num_pages, page_bytes, scale_log2e, window, sinks, cap_log2e, gate,
+                                 ldg, keep_first, score_bias, chunked, dist_bias, bias_len, slopes, n, h + half,
+                                 lds + half * FOUR);
+  else if (WAVES != AW_FOUR)
+    aw_decode<D, IDENT, BIAS, 8>(q, ldq, out, ldo, kpool, vpool, block_tables, max_blocks, positions, q_req, cu_q, n_head,
+                                 n_kv_head, page_shift, num_pages, page_bytes, scale_log2e, window, sinks, cap_log2e, gate,
+                                 ldg, keep_first, score_bias, chunked, dist_bias, bias_len, slopes, n, h, lds);
 }
 
 // positions[n]: absolute position of token n; q_req[n]: its request (block table row), -1 for a
@@ -82,17 +106,19 @@ extern "C" int mgpt_paged_attention_decode_bf16(
   const unsigned int page_bytes = (unsigned int)(n_kv_head * page_size * head_dim * 2);
   const float scale_log2e = scale * 1.4426950408889634f;
   const bool many = (long)n_tokens * n_head > (head_dim == 128 ? 256 : 512);
+  const long most = window > 0 ? (long)window + keep_first : (long)max_blocks * page_size;   // keys that a token can see
   dim3 grid(n_tokens, n_head);
-#define AW_LAUNCH4(DD, ID, BI, W)                                                                              \
-  hipLaunchKernelGGL((paged_attention_decode_kernel<DD, ID, BI, W>), grid, dim3(W * 64), 0, stream, (const bf16_t*)q, ldq, \
-                     (bf16_t*)out, ldo, (const bf16_t*)kpool, (const bf16_t*)vpool, block_tables,          \
+#define AW_LAUNCH4(DD, ID, BI, WAVES)                                                                          \
+  hipLaunchKernelGGL((paged_attention_decode_kernel<DD, ID, BI, WAVES>), grid, dim3(WAVES == AW_FOUR ? 256 : 512), 0, stream, \
+                     (const bf16_t*)q, ldq, (bf16_t*)out, ldo, (const bf16_t*)kpool, (const bf16_t*)vpool, block_tables,          \
                      max_blocks, positions, q_req, cu_q, n_head, n_kv_head, page_shift, num_pages, page_bytes, \
                      scale_log2e, window, sinks, softcap > 0.f ? softcap * 1.4426950408889634f : 0.f, \
                      (const bf16_t*)gate, ldg, keep_first, score_bias, chunked, dist_bias, bias_len, slopes)
 #define AW_LAUNCH3(DD, ID, BI)                 \
   do {                                         \
-    if (many) AW_LAUNCH4(DD, ID, BI, 4);       \
-    else AW_LAUNCH4(DD, ID, BI, 8);            \
+    if (many && most <= AW_SHORT(DD)) AW_LAUNCH4(DD, ID, BI, AW_FOUR);                    \
+    else if (many && DD >= 64) AW_LAUNCH4(DD, ID, BI, (DD >= 64 ? AW_HALVES : AW_EIGHT)); \
+    else AW_LAUNCH4(DD, ID, BI, AW_EIGHT);                                                \
   } while (0)
 #define AW_LAUNCH2(DD, ID)                     \
   do {                                         \

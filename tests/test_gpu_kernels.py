@@ -848,14 +848,48 @@ def test_single_tokens_and_portions_refuse_buffers_that_end_before_their_tokens(
 @pytest.mark.parametrize("window", [0, 100])
 @pytest.mark.parametrize("d,n", [(16, 129), (32, 129), (64, 128), (64, 129), (128, 64), (128, 65)])
 def test_decode_attention_of_many_tokens(d, n, window):
-    """More (token, head) pairs than the chip holds workgroups of eight waves go to workgroups of four, whose pass is 256
-    keys: around the line between the two, contexts around a chunk and around one and two passes."""
+    """More (token, head) pairs than the chip holds workgroups of eight waves: four a head, whose pass is 256 keys, for
+    tokens behind few keys: around the line between the two, contexts around a chunk and around one and two passes."""
     lens = ([1, 63, 64, 65, 255, 256, 257, 511, 512, 513, 40] * 12)[:n]
     c = PagedCase(lens, [1] * n, h=4, hk=2, d=d, page=16, dtype="bfloat16", seed=d + n)
     out = torch.full((n, 4 * d), float("nan"), dtype=torch.bfloat16, device=DEV)
     assert kernels.paged_attention_decode_bf16(c.q_flat, out, c.kp, c.vp, c.bt, i32([x - 1 for x in lens]), c.q_req, n, 4,
                                                d ** -0.5, window, identity=True)
     helpers.assert_close(out, c.want(d ** -0.5, window), "bfloat16", "decode attention")
+
+
+@pytest.mark.parametrize("window,mask", [(0, {}), (0, {"softcap": 15.0}), (300, {"keep_first": 3}), (300, {"chunked": True}),
+                                         (600, {}), (256, {}), (250, {"keep_first": 7})])
+@pytest.mark.parametrize("d,h,hk,n", [(16, 5, 1, 110), (32, 5, 5, 110), (64, 5, 1, 110), (64, 4, 2, 130), (128, 7, 7, 40),
+                                      (128, 4, 1, 70)])
+def test_decode_attention_of_many_tokens_short_ones_beside_long_ones(d, h, hk, n, window, mask):
+    """Where a block table or window leaves room for long contexts, a token behind up to 256 keys (512 with heads of 128) has
+    two heads in one workgroup, four waves each, and a token behind more a workgroup a head; so has an odd number's last
+    head.  As requests' own tokens, and as a step in which some tokens are padding and some are another kernel's."""
+    lens = ([1, 255, 256, 257, 40, 511, 512, 513, 700, 64, 1100, 3] * 11)[:n]
+    c = PagedCase(lens, [1] * n, h=h, hk=hk, d=d, page=16, dtype="bfloat16", seed=d + n)
+    want = torch.empty(n, h * d, device=DEV)
+    kernels.paged_attention_generic(c.q_flat.float(), want, c.kp.float(), c.vp.float(), c.bt, c.cu, c.sl, c.q_req, n, n, h,
+                                    d ** -0.5, window, **mask)
+    out = torch.full((n, h * d), float("nan"), dtype=torch.bfloat16, device=DEV)
+    positions = i32([x - 1 for x in lens])
+    assert kernels.paged_attention_decode_bf16(c.q_flat, out, c.kp, c.vp, c.bt, positions, c.q_req, n, h, d ** -0.5, window,
+                                               identity=True, **mask)
+    helpers.assert_close(out, want, "bfloat16", "decode attention")
+    q_req, cu = c.q_req.clone(), c.cu.clone()
+    left = torch.zeros(n, dtype=torch.bool)
+    left[[2, 3, 10, 11]] = True
+    q_req[[2, 10]] = -1
+    q_req[11] = q_req[12]                              # these two are one request's, as cu_q has it
+    counts = torch.ones(n, dtype=torch.int32)
+    counts[[3, 12]] = 2
+    left[12] = True
+    cu = i32(np.concatenate([[0], np.cumsum(counts.numpy())]))
+    out = torch.full((n, h * d), 7.0, dtype=torch.bfloat16, device=DEV)
+    assert kernels.paged_attention_decode_bf16(c.q_flat, out, c.kp, c.vp, c.bt, positions, q_req, n, h, d ** -0.5, window,
+                                               cu_q=cu, **mask)
+    assert (out[left.to(DEV)] == 7.0).all()
+    helpers.assert_close(out[~left.to(DEV)], want[~left.to(DEV)], "bfloat16", "beside padding and portions")
 
 
 @pytest.mark.parametrize("window,mask", [(0, {}), (100, {}), (100, {"keep_first": 70}), (96, {"chunked": True})])

@@ -17,6 +17,11 @@
 // stay in the lanes; nothing goes through LDS before the end.  Keys and values come straight from the pages, 16 bytes a
 // lane; of the values a lane takes the head size / 16 consecutive channels that are its row in as many tiles of O^T.
 //
+// Tiles whose last query is among the first 16 have a walk of their own with the one group of 16 keys that there is: 8 heads
+// of 64 behind one key 5.5 us (with the chunk's other groups, all zeros, 8.7), behind 16 5.8 (8.9); of 128 6.3 (11.4).  The
+// same in chunks of any number of groups, a test for each, kept the loads of one group behind the products of the one
+// before: 16 requests x 8 heads of 64 behind 700 keys 23.6 -> 35.0 us.
+//
 // The general kernel walks a query's keys with one wave and 4-byte loads: 352 us for the prompts of 4 requests (1,098
 // tokens, 8 heads of 64) and 134 us for decode steps of 16 requests x 12 heads behind 16 to 280 keys.
 #include "attention_exact.h"
@@ -125,9 +130,10 @@ __global__ __launch_bounds__(64 * AX_WAVES, D == 64 ? 5 : 1) void attention_exac
 
   float m, l;
   ax_f4 acc[G];                                         // O^T tile dt, rows 4 lk + i: channel G (4 lk + i) + dt
-  // the wave's walk over its chunks; CAREFUL: for values that are infinite or NaN
-  auto walk = [&](auto careful) __attribute__((always_inline)) {
+  // the wave's walk over its chunks; CAREFUL: for values that are infinite or NaN; GROUPS: of 16 keys that a chunk can have
+  auto walk = [&](auto careful, auto groups) __attribute__((always_inline)) {
     constexpr bool CAREFUL = decltype(careful)::value;
+    constexpr int GROUPS = decltype(groups)::value;
     m = -INFINITY;
     l = 0.f;
 #pragma unroll
@@ -139,9 +145,9 @@ __global__ __launch_bounds__(64 * AX_WAVES, D == 64 ? 5 : 1) void attention_exac
       const bool whole = (c0 + AX_CHUNK - 1 < pos_hi ? c0 + AX_CHUNK - 1 : pos_hi) <= pos_lo &&
                          ((c0 > tile_begin ? c0 : tile_begin) >= last_begin || c0 + AX_CHUNK <= a.keep_first);
       // the pool rows of this lane's four keys, c0 + 16 t + l16
-      unsigned int row[4];                                // 2^32 rows of 16 channels are 275 GB
+      unsigned int row[GROUPS];                                // 2^32 rows of 16 channels are 275 GB
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
+      for (int t = 0; t < GROUPS; ++t) {
         const int j = c0 + 16 * t + l16;
         row[t] = AX_NONE;
         if (j <= pos_hi && (j >= tile_begin || j < a.keep_first)) {
@@ -149,9 +155,9 @@ __global__ __launch_bounds__(64 * AX_WAVES, D == 64 ? 5 : 1) void attention_exac
           row[t] = ((unsigned int)bt[idx] * a.n_kv_head + hk) * a.page_size + (j - idx * a.page_size);
         }
       }
-      ax_f4 s[4];
+      ax_f4 s[GROUPS];
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
+      for (int t = 0; t < GROUPS; ++t) {
         s[t] = (ax_f4){0.f, 0.f, 0.f, 0.f};
         ax_f4 kf[G];
 #pragma unroll
@@ -166,7 +172,7 @@ __global__ __launch_bounds__(64 * AX_WAVES, D == 64 ? 5 : 1) void attention_exac
       }
       float top = -INFINITY;
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
+      for (int t = 0; t < GROUPS; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int j = c0 + 16 * t + 4 * lk + i;
@@ -183,7 +189,7 @@ __global__ __launch_bounds__(64 * AX_WAVES, D == 64 ? 5 : 1) void attention_exac
       const float alpha = expf(m - m_sub);
       float sum = 0.f;
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
+      for (int t = 0; t < GROUPS; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           s[t][i] = expf(s[t][i] - m_sub);
@@ -194,7 +200,7 @@ __global__ __launch_bounds__(64 * AX_WAVES, D == 64 ? 5 : 1) void attention_exac
 #pragma unroll
       for (int g = 0; g < G; ++g) acc[g] *= alpha;
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
+      for (int t = 0; t < GROUPS; ++t) {
         float vf[4][G];                                   // of key 16 t + 4 lk + i the channels G l16 .. G l16 + G - 1
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -221,13 +227,14 @@ __global__ __launch_bounds__(64 * AX_WAVES, D == 64 ? 5 : 1) void attention_exac
       }
     }
   };
-  walk(std::false_type{});
+  if (pos_hi < 16) walk(std::false_type{}, std::integral_constant<int, 1>{});
+  else walk(std::false_type{}, std::integral_constant<int, 4>{});
   float zero = 0.f;                                     // an infinity or NaN among the sums stays one to the end
 #pragma unroll
   for (int g = 0; g < G; ++g)
 #pragma unroll
     for (int i = 0; i < 4; ++i) zero = fmaf(acc[g][i], 0.f, zero);
-  if (__ballot(zero != zero)) walk(std::true_type{});
+  if (__ballot(zero != zero)) walk(std::true_type{}, std::integral_constant<int, 4>{});
   if (lk == 0) {
     m_s[wave][l16] = m;
     l_s[wave][l16] = l;

@@ -202,8 +202,9 @@ __global__ __launch_bounds__(256) void rms_post_norm_kernel(RmsBranches br, int 
 // sums then run in another order, but always in the same.  Four waves with 4 to 16 values of 4 bytes a thread and a test of the
 // output's type for each / here, us a call: 8 rows of 1,024 2.72 / 2.10, of 1,023 3.23 / 2.80, of 2,048 3.6 / 2.4, of 2,047
 // 4.2 / 3.1; 3,000 rows of 1,023 10.3 / 9.0, of 2,047 19.4 / 18.5.  The kernel above, which reads a row three to five times,
-// took 4.2 and 12.4 for 8 and 3,000 rows of 1,023, 5.7 and 22.9 for rows of 2,047.  (Five and twelve waves: 1,026 values are a
-// little over two rounds of eight waves' lanes, 3,000 such rows 11.6 us; in five waves 10.1, before 10.8.)
+// took 4.2 and 12.4 for 8 and 3,000 rows of 1,023, 5.7 and 22.9 for rows of 2,047.  (Five and twelve waves: without them
+// 1,028 values are a little over half of eight waves' lanes, 1,900 such rows 8.9 us; in five waves 7.9, before 8.4; 1,900 of
+// 2,052 15.7 / 13.9 in twelve.)
 template <int W, int NB, bool PIECES>
 __global__ __launch_bounds__(64 * W) void rms_post_norm_row_kernel(RmsBranches br, float coef, int join_unit,
                                                                    float* __restrict__ x, const float* __restrict__ gain_post,
@@ -335,9 +336,9 @@ extern "C" int mgpt_rms_post_norm(float* y0, float* y1, float* y2, float* y3, co
   if (row && width <= 256) RPN_ROW(1);
   else if (row && width <= 512) RPN_ROW(2);
   else if (row && width <= 1024) RPN_ROW(4);
-  else if (row && width <= 1280 && !pieces) RPN_ROW(5);
+  else if (row && width <= 1280) RPN_ROW(5);
   else if (row && width <= 2048) RPN_ROW(8);
-  else if (row && width <= 3072 && !pieces) RPN_ROW(12);
+  else if (row && width <= 3072) RPN_ROW(12);
   else if (row) RPN_ROW(16);
   else
     hipLaunchKernelGGL(rms_post_norm_kernel, dim3(n_rows), dim3(256), 0, stream, br, n_branches, coef, join_unit, x, gain_post,

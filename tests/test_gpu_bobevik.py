@@ -111,13 +111,15 @@ def test_the_step_between_two_sublayers(h_dtype, branches, n, width):
 
 @pytest.mark.parametrize("h_dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("branches,n,width", [(1, 2, 4), (2, 2, 256), (1, 3, 260), (2, 2, 512), (2, 2, 516), (1, 2, 1028),
-                                              (2, 2, 4096), (1, 2, 4096), (1, 2, 4100), (2, 2, 2050), (1, 3, 1), (2, 2, 255),
+                                              (2, 2, 4096), (1, 2, 4096), (1, 2, 4100), (2, 2, 2050),
+                                              (1, 2, 1280), (2, 2, 1284), (2, 2, 2052), (1, 2, 3072), (2, 2, 3076),
+                                              (1, 3, 1), (2, 2, 255),
                                               (1, 2, 257), (2, 2, 511), (1, 2, 513), (2, 2, 1023), (1, 2, 1025), (2, 2, 1279),
                                               (1, 2, 1281), (2, 2, 2047), (1, 2, 2049), (2, 2, 3071), (1, 2, 3073),
                                               (2, 2, 4095), (1, 2, 4095), (2, 2, 4097), (3, 2, 1023)])
 def test_the_step_between_two_sublayers_around_the_ends_of_its_kernels(h_dtype, branches, n, width):
-    """Four values a lane: a 16-byte piece in 1, 2, 4, 8 or 16 waves, or, where pieces do not cover the row, four values a
-    round apart in up to 16 waves; longer rows and more branches than two go to the general kernel."""
+    """Four values a lane: a 16-byte piece in 1, 2, 4, 5, 8, 12 or 16 waves, or, where pieces do not cover the row, four values a
+    round apart in as many waves; longer rows and more branches than two go to the general kernel."""
     test_the_step_between_two_sublayers(h_dtype, branches, n, width)
 
 

@@ -22,8 +22,8 @@
 // same in chunks of any number of groups, a test for each, kept the loads of one group behind the products of the one
 // before: 16 requests x 8 heads of 64 behind 700 keys 23.6 -> 35.0 us.
 //
-// The general kernel walks a query's keys with one wave and 4-byte loads: 352 us for the prompts of 4 requests (1,098
-// tokens, 8 heads of 64) and 134 us for decode steps of 16 requests x 12 heads behind 16 to 280 keys.
+// The general kernel walks a query's keys with one wave and 4-byte loads: prompts of 640, 295, 265 and 1 tokens x 8 heads of
+// 64 326 us, here 38; decode steps of 16 requests x 12 heads behind 16 to 280 keys 68 us, here 12.4.
 #include "attention_exact.h"
 #include "attention_mask.h"
 #include "common.h"

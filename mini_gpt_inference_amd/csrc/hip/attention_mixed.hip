@@ -130,8 +130,11 @@ extern "C" int mgpt_mixed_attention_bf16(
                        n_kv_head, page_size, page_shift, num_pages, (unsigned int)(n_kv_head * page_size * head_dim * 2), scale,
                        window, sinks, softcap, (const bf16_t*)gate, ldg, window == 0 ? 0 : keep_first, score_bias, chunked,
                        keys};
-  // two wave groups a tile while the tiles are few, as for prompt portions alone
+  // Two wave groups a tile while the tiles are few, as for prompt portions alone.  Their number is taken for up to eight
+  // portions: a padded step's n_req is its capacity, of which it fills few (32 single tokens x 8 heads of 64 behind up to 4,000
+  // keys beside 38 tokens, capacity 41: 30.2 us with one group and so four waves a pair, 21.2 with two).
+  const long likely = (n_tokens + PF_QT - 1L) / PF_QT + (n_req < 8 ? n_req : 8);
   if (head_dim == 128) return identity ? launch<128, 1, true>(a, stream) : launch<128, 1, false>(a, stream);
-  if (tiles * n_head <= 320) return identity ? launch<64, 2, true>(a, stream) : launch<64, 2, false>(a, stream);
+  if (likely * n_head <= 320) return identity ? launch<64, 2, true>(a, stream) : launch<64, 2, false>(a, stream);
   return identity ? launch<64, 1, true>(a, stream) : launch<64, 1, false>(a, stream);
 }

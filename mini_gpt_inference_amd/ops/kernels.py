@@ -1943,10 +1943,13 @@ def decay_state_segments(n_tokens: int, n_req: int, max_q_len: int, n_head: int,
     behind the other take no longer.  In us, for heads of 128 x 128: a chunk of the longest request 6.75 (5.1 while the chain's
     workgroups have 16 value channels); cut, 40 and 8.3 for every chunk that each of 256 compute units has of all requests'
     chunks, heads and 32 value channels.  Whole / cut: 2 requests of 1,024 tokens x 8 heads 175 / 129, x 16 heads 184 / 193;
-    one of 2,048 x 16 337 / 160; 8 of 100 to 1,024 x 8 236 / 205; 4 of 600 x 16 153 / 204; 16 of 1,024 x 8 332 / 482."""
+    one of 2,048 x 16 337 / 160; 8 of 100 to 1,024 x 8 236 / 205; 4 of 600 x 16 153 / 204; 16 of 1,024 x 8 332 / 482.  A chunk
+    of smaller heads is less work, of 64 x 64 0.72 of that: one request of 300 x 4 40 / 50, of 1,024 x 4 111 / 54, two of 600 x 16
+    75 / 65."""
     blocks = -(-value_dim // 32) * n_head
-    whole = max_q_len / 32 * (6.75 if n_req * blocks >= 256 else 5.1)
-    if max_q_len <= DECAY_SEGMENT or whole <= 40 + 8.3 * n_tokens / 32 * blocks / 256:
+    chunk = 0.44 + 0.56 * head_dim / 128
+    whole = max_q_len / 32 * chunk * (6.75 if n_req * blocks >= 256 else 5.1)
+    if max_q_len <= DECAY_SEGMENT or whole <= 40 + 8.3 * chunk * n_tokens / 32 * blocks / 256:
         return 0
     return decay_state_scratch(n_tokens, n_req, n_head, head_dim, value_dim)
 

@@ -178,13 +178,14 @@ def test_where_a_decaying_state_is_cut_into_segments():
     prompts of a segment at most and for many requests whose chains fill the chip (measured beside the rule)."""
     from mini_gpt_inference_amd.ops import kernels
 
-    def cut(n_req, longest, heads, tokens=None):
+    def cut(n_req, longest, heads, tokens=None, dim=128):
         tokens = tokens or n_req * longest
-        need = kernels.decay_state_segments(tokens, n_req, longest, heads, 128, 128)
-        assert need in (0, kernels.decay_state_scratch(tokens, n_req, heads, 128, 128))
+        need = kernels.decay_state_segments(tokens, n_req, longest, heads, dim, dim)
+        assert need in (0, kernels.decay_state_scratch(tokens, n_req, heads, dim, dim))
         return need > 0
 
     assert cut(1, 2048, 16) and cut(2, 1024, 8) and cut(8, 1024, 8, tokens=4500)
     assert not (cut(2, 1024, 16) or cut(4, 600, 16) or cut(16, 1024, 8) or cut(1, 256, 1))
+    assert cut(1, 600, 4, dim=64) and cut(2, 600, 16, dim=64) and not cut(1, 300, 4, dim=64)    # smaller chunks
     assert kernels.decay_state_scratch(257, 1, 3, 40, 24) == 2 * 3 * 24 * 48     # heads of 40: rows of 48
     assert kernels.decay_state_scratch(4, 9, 1, 16, 16) == 4 * 16 * 16           # no more segments than tokens

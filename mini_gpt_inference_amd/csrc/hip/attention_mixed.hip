@@ -122,9 +122,11 @@ extern "C" int mgpt_mixed_attention_bf16(
   if ((tiles + n_decode) * n_head > 0x7fffffffL) return MGPT_ERR_TOO_LARGE;
   int page_shift = 0;
   while ((1 << page_shift) < page_size) ++page_shift;
-  // what four waves lose on a token against eight, 0.005 us a key, is to be no more than what the tiles beside them take and a
-  // launch, 7 us for a portion of 64 tokens, 19 for 512; head size 64 comes here with hundreds of tiles only and loses less
-  const int keys = head_dim == 64 ? 16384 : (n_tokens < 512 ? 1024 + 6 * n_tokens : 4096);
+  // What four waves lose on a token against eight, 0.005 us a key, is to be no more than what the tiles beside them take and a
+  // launch, 7 us for a portion of 64 tokens, 13 for 512 (19 are saved there, but a token beyond the line then waits for those
+  // below it: one behind 8,363 keys and others behind some 4,000 beside 630 tokens 97 us as two launches, 113 with a line at
+  // 4,096 keys, 93 here).  Head size 64 comes here with hundreds of tiles only and loses less.
+  const int keys = head_dim == 64 ? 16384 : (n_tokens < 512 ? 1024 + 3 * n_tokens : 2560);
   const MixedArgs a = {(const bf16_t*)q, ldq, (bf16_t*)out, ldo, (const bf16_t*)kpool, (const bf16_t*)vpool, block_tables,
                        max_blocks, positions, q_req, cu_q, seq_lens, n_decode, first_req, n_req, (int)tiles, single_below, n_head,
                        n_kv_head, page_size, page_shift, num_pages, (unsigned int)(n_kv_head * page_size * head_dim * 2), scale,

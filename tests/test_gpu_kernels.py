@@ -809,7 +809,10 @@ def test_single_tokens_and_portions_in_one_launch_with_every_option(seq_lens, q_
 
 @pytest.mark.parametrize("d,h,hk,portion,keys,window", [(128, 4, 1, 30, 1204, 0), (128, 4, 1, 30, 1204, 1203),
                                                         (128, 4, 1, 30, 1204, 1204), (128, 4, 1, 30, 1204, 1250),
-                                                        (128, 4, 1, 700, 4096, 0), (64, 12, 1, 2048, 16384, 0)])
+                                                        (128, 4, 1, 700, 4096, 0), (64, 12, 1, 2048, 16384, 0),
+                                                        (128, 4, 1, 30, 1114, 0), (128, 4, 1, 30, 1114, 1113),
+                                                        (128, 4, 1, 30, 1114, 1114), (128, 4, 1, 30, 1114, 1160),
+                                                        (128, 4, 1, 700, 2560, 0)])
 def test_single_tokens_behind_long_contexts_beside_a_portion(d, h, hk, portion, keys, window):
     """Where a token's workgroup has four waves, tokens that see more than so many keys have a second launch of their own:
     every token is done by one of the two, around that number, as the step's own requests and as a padded step, also with a

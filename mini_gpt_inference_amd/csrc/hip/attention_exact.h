@@ -21,4 +21,5 @@ struct AttentionExactArgs {
 // Whether the kernel takes these: nothing in it depends on a step's size (but for a step of no requests, which has nothing to
 // do), so a model's calls are all taken or none is.
 bool mgpt_attention_exact_takes(const AttentionExactArgs& a, int head_dim);
-int mgpt_attention_exact_launch(const AttentionExactArgs& a, int head_dim, hipStream_t stream);
+// single: every request has one token, token n being request n's (q_req[n] < 0: padding).
+int mgpt_attention_exact_launch(const AttentionExactArgs& a, int head_dim, int single, hipStream_t stream);

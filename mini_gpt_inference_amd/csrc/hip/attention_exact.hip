@@ -23,7 +23,8 @@
 // before: 16 requests x 8 heads of 64 behind 700 keys 23.6 -> 35.0 us.
 //
 // The general kernel walks a query's keys with one wave and 4-byte loads: prompts of 640, 295, 265 and 1 tokens x 8 heads of
-// 64 326 us, here 38; decode steps of 16 requests x 12 heads behind 16 to 280 keys 68 us, here 12.4.
+// 64 326 us, here 38; decode steps of 16 requests x 12 heads behind 16 to 280 keys 68 us, here 12.4 (7.9 with the kernel for
+// steps of single tokens, further down).
 #include "attention_exact.h"
 #include "attention_mask.h"
 #include "common.h"
@@ -268,6 +269,190 @@ __global__ __launch_bounds__(64 * AX_WAVES, D == 64 ? 5 : 1) void attention_exac
   }
 }
 
+// A step of single tokens (token n is request n's only one): a workgroup per (token, head) with the same eight waves, chunks
+// and sums, so the same bits, without what the general walk spends on finding its work, on waiting and on the 15 queries
+// that are not there.
+//  * The request is the block's number; position, query, padding mark and the first chunk's block table entries are asked
+//    for together, and all of a chunk's keys at once, its values behind them as the keys' registers come free: two trips to
+//    memory, the general walk has six.  Keys that are not seen are read from the pool's first rows and dropped, which keeps
+//    the loads free of branches.
+//  * The scores come from the same matrix products, with the query in all 16 columns; of the 16 copies of its 16 scores
+//    that a row of lanes then holds each lane takes one, so that mask and exponential are done once a key.
+//  * v_mfma_f32_16x16x4_f32 is the chain of four fused multiply-adds over its k in order (compared bit for bit over 40
+//    million sums: ordinary, denormal and overflowing ones), so the values are weighted on the vector unit in the order of
+//    the general walk's products, a lane a channel: 64 instructions of 4 cycles for 64 of 32.
+// A query sees every key that it weighs, so infinite and NaN values need no second walk.
+// us in a graph of such calls, general walk / here: 1 request x 12 heads of 64 behind 100 keys 9.9 / 5.5; 16 x 12 behind 16 to
+// 280 12.0 / 7.9, 64 x 12 30 / 19; 8 x 8 behind 700 20 / 12; 64 x 8 behind 900 to 1,000 (bound by the 250 MB) 42.8 / 39.5;
+// 16 x 8 heads of 128 behind 200 to 300 19.5 / 12.5; 3 x 4 heads of 16 behind 5 to 42 7.0 / 4.6.  Heads of 64 need the 128
+// registers that let a compute unit have two workgroups: with scores kept for all 64 keys and ten registers spilled 64 x 8
+// took 44.5.  What is left at 16 x 12: the launch (1.6), two trips to memory, 64 matrix products (0.9) and the merge.
+//
+// PAGE16: pages are multiples of 16 positions, so 16 keys lie one behind the other.
+template <int D, bool PAGE16>
+__global__ __launch_bounds__(64 * AX_WAVES, D == 128 ? 2 : 4) void attention_exact_single_kernel(AttentionExactArgs a, int page_shift) {
+  constexpr int G = D / 16;
+  constexpr int C = D > 64 ? D / 64 : 1;                // channels of a lane
+  constexpr int AHEAD = G <= 4 ? 4 : 2;                 // groups of 16 keys on their way
+  typedef __attribute__((__vector_size__(C * sizeof(float)))) float ax_fc;
+  __shared__ __align__(16) float p_s[AX_WAVES][AX_CHUNK];
+  __shared__ float o_s[AX_WAVES][D];
+  __shared__ float m_s[AX_WAVES], l_s[AX_WAVES];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, lk = lane >> 4;
+  const int n = blockIdx.x, h = blockIdx.y, hk = h / (a.n_head / a.n_kv_head);
+  const int* bt = a.block_tables + (long)n * a.max_blocks;
+  auto page_of = [&](int j) { return page_shift >= 0 ? j >> page_shift : j / a.page_size; };
+  int entry[4];                                         // block table entries of the keys c0 + 16 t + l16
+  auto look_up = [&](int c) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int idx = page_of(c * AX_CHUNK + 16 * t + l16);
+      entry[t] = bt[idx < a.max_blocks ? idx : a.max_blocks - 1];
+    }
+  };
+  look_up(wave);
+  ax_f4 qf[G];
+#pragma unroll
+  for (int g = 0; g < G; ++g) qf[g] = *reinterpret_cast<const ax_f4*>(a.q + (long)n * a.ldq + (long)h * D + 16 * g + 4 * lk);
+  const int pos = a.seq_lens[n] - 1;
+  if (a.q_req[n] < 0) return;                           // a token of the padding: the whole workgroup
+  const int begin = first_seen(pos, a.window, a.chunked);
+  const float slope = a.slopes ? a.slopes[h] : 0.f;
+  const float* dist = a.dist_bias ? a.dist_bias + (long)h * a.bias_len : nullptr;
+  const float* vlane = a.vpool + C * (D >= 64 ? lane : lane % D);
+  auto sees = [&](int j) { return j <= pos && (j >= begin || j < a.keep_first); };
+
+  float m = -INFINITY, l = 0.f;
+  ax_fc acc;                                            // channels C lane ..
+#pragma unroll
+  for (int x = 0; x < C; ++x) acc[x] = 0.f;
+  for (int c = wave; c * AX_CHUNK <= pos; c += AX_WAVES) {
+    const int c0 = c * AX_CHUNK;
+    unsigned int row[4];                                // of the keys c0 + 16 t + l16
+    uint64_t seen[4];                                   // the 16 keys' bits, four times over
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int j = c0 + 16 * t + l16, idx = page_of(j);
+      const bool ok = sees(j);
+      seen[t] = __ballot(ok);
+      row[t] = (PAGE16 ? seen[t] != 0 : ok) ? ((unsigned int)entry[t] * a.n_kv_head + hk) * a.page_size + (j - idx * a.page_size)
+                                            : (PAGE16 ? l16 : 0);
+    }
+    if ((c + AX_WAVES) * AX_CHUNK <= pos) look_up(c + AX_WAVES);
+    if (c0 + AX_CHUNK <= begin && c0 >= a.keep_first) continue;
+    ax_f4 kf[AHEAD][G];
+    auto load_keys = [&](int t) {
+      const float* src = a.kpool + (long)row[t] * D + 4 * lk;
+#pragma unroll
+      for (int g = 0; g < G; ++g) kf[t % AHEAD][g] = *reinterpret_cast<const ax_f4*>(src + 16 * g);
+    };
+    ax_fc vf[4][16];
+    auto load_values = [&](int t) {
+      if constexpr (PAGE16) {
+        const float* src = vlane + (long)(unsigned int)__builtin_amdgcn_readfirstlane((int)row[t]) * D;
+#pragma unroll
+        for (int x = 0; x < 16; ++x) vf[t][x] = *reinterpret_cast<const ax_fc*>(src + x * D);
+      } else {
+#pragma unroll
+        for (int x = 0; x < 16; ++x)
+          vf[t][x] = *reinterpret_cast<const ax_fc*>(vlane + (long)(unsigned int)__builtin_amdgcn_readlane((int)row[t], x) * D);
+      }
+    };
+#pragma unroll
+    for (int t = 0; t < AHEAD; ++t) load_keys(t);
+    float v = 0.f;                                      // this lane's key: 16 (l16 / 4) + 4 lk + l16 % 4
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      ax_f4 s = {0.f, 0.f, 0.f, 0.f};                   // keys 16 t + 4 lk + i, the same in all 16 lanes
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t % AHEAD][g][e], qf[g][e], s, 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v = l16 == 4 * t + i ? s[i] : v;
+      if (t + AHEAD < 4) load_keys(t + AHEAD);
+      load_values(t);                                   // into the registers of keys that are done with
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    const int key = 16 * (l16 >> 2) + 4 * lk + (l16 & 3), j = c0 + key;
+    v *= a.scale;
+    if (dist) v += dist[distance_entry(pos - j, a.bias_len)];
+    if (a.softcap > 0.f) v = a.softcap * tanhf(v / a.softcap);
+    if (a.slopes) v -= slope * (float)(pos - j);
+    if (!sees(j)) v = -INFINITY;
+    const float m_new = fmaxf(m, wave_max(v));
+    const float m_sub = m_new == -INFINITY ? 0.f : m_new;   // nothing seen so far: every weight is exp(-inf)
+    const float alpha = expf(m - m_sub);
+    p_s[wave][key] = expf(v - m_sub);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    float sum = 0.f;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const ax_f4 p = *reinterpret_cast<const ax_f4*>(&p_s[wave][16 * t + 4 * lk]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sum += p[i];
+    }
+    l = l * alpha + ax_sum4(sum);
+    m = m_new;
+    acc *= alpha;
+    const bool whole = (seen[0] & seen[1] & seen[2] & seen[3]) == ~0ull;
+    auto weigh = [&](auto all) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        __builtin_amdgcn_sched_barrier(0);              // (or all weights are read at once, into registers that are not there)
+        ax_f4 p[4];                                     // the keys 16 t + 4 k + i, for everybody
+#pragma unroll
+        for (int k = 0; k < 4; ++k) p[k] = *reinterpret_cast<const ax_f4*>(&p_s[wave][16 * t + 4 * k]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+#pragma unroll
+            for (int x = 0; x < C; ++x) {
+              const float val = decltype(all)::value || (seen[t] >> (4 * k + i) & 1) ? vf[t][4 * k + i][x] : 0.f;
+              acc[x] = fmaf(val, p[k][i], acc[x]);
+            }
+      }
+    };
+    if (whole) weigh(std::true_type{});
+    else weigh(std::false_type{});
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  }
+  if (lane == 0) {
+    m_s[wave] = m;
+    l_s[wave] = l;
+  }
+  if (D >= 64 || lane < D) *reinterpret_cast<ax_fc*>(&o_s[wave][C * lane]) = acc;
+  __syncthreads();
+  if (tid >= D) return;
+  float top = a.sinks ? a.sinks[h] : -INFINITY;
+#pragma unroll
+  for (int w = 0; w < AX_WAVES; ++w) top = fmaxf(top, m_s[w]);
+  float num = 0.f, den = 0.f;
+#pragma unroll
+  for (int w = 0; w < AX_WAVES; ++w) {
+    const float f = expf(m_s[w] - top);
+    den += l_s[w] * f;
+    num += o_s[w][tid] * f;
+  }
+  if (a.sinks) den += expf(a.sinks[h] - top);
+  float inv = 1.0f / den;
+  if (a.gate) inv *= 1.0f / (1.0f + expf(-a.gate[(long)n * a.ldg + h]));
+  a.out[(long)n * a.ldo + (long)h * D + tid] = num * inv;
+}
+
+template <int D>
+static int launch_single(const AttentionExactArgs& a, hipStream_t stream) {
+  const int shift = (a.page_size & (a.page_size - 1)) == 0 ? __builtin_ctz(a.page_size) : -1;
+  const dim3 grid(a.n_tokens, a.n_head), block(64 * AX_WAVES);
+  if (a.page_size % 16 == 0) hipLaunchKernelGGL((attention_exact_single_kernel<D, true>), grid, block, 0, stream, a, shift);
+  else hipLaunchKernelGGL((attention_exact_single_kernel<D, false>), grid, block, 0, stream, a, shift);
+  return mgpt_last_error();
+}
+
 template <int D>
 static int launch(const AttentionExactArgs& a, hipStream_t stream) {
   constexpr int bytes = AX_WAVES * AX_QUERIES * (D + 4) * (int)sizeof(float);
@@ -292,7 +477,13 @@ bool mgpt_attention_exact_takes(const AttentionExactArgs& a, int head_dim) {
          a.n_req > 0;   // (without requests all tokens are padding: the general kernel leaves them alone)
 }
 
-int mgpt_attention_exact_launch(const AttentionExactArgs& a, int head_dim, hipStream_t stream) {
+int mgpt_attention_exact_launch(const AttentionExactArgs& a, int head_dim, int single, hipStream_t stream) {
+  if (single && a.n_tokens <= a.n_req) {
+    if (head_dim == 16) return launch_single<16>(a, stream);
+    if (head_dim == 32) return launch_single<32>(a, stream);
+    if (head_dim == 64) return launch_single<64>(a, stream);
+    return launch_single<128>(a, stream);
+  }
   if (head_dim == 16) return launch<16>(a, stream);
   if (head_dim == 32) return launch<32>(a, stream);
   if (head_dim == 64) return launch<64>(a, stream);

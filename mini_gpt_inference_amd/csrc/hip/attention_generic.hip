@@ -186,12 +186,13 @@ __global__ __launch_bounds__(64) void paged_attention_generic_kernel(
 // q: [n_tokens, n_head*head_dim] with row stride ldq; out likewise with ldo.
 // q_req[t] = index of token t's request in this step (or -1 for a padded token),
 // cu_q[r]..cu_q[r+1] = the tokens of request r (r < n_req), seq_lens[r] = its length after this step.
+// single: token n is request n's only token (the 32-bit path then has a kernel for that).
 extern "C" int mgpt_paged_attention_generic(
     const void* q, long ldq, void* out, long ldo, const void* kpool, const void* vpool,
     const int* block_tables, int max_blocks, const int* cu_q, const int* seq_lens, const int* q_req,
     int n_tokens, int n_req, int n_head, int n_kv_head, int head_dim, int page_size, float scale, int window,
     int dtype, int fast_exp, const float* sinks, float softcap, const void* gate, long ldg, int keep_first,
-    const float* score_bias, int chunked, const float* dist_bias, int bias_len, const float* slopes,
+    const float* score_bias, int chunked, const float* dist_bias, int bias_len, const float* slopes, int single,
     hipStream_t stream) {
   if (n_tokens == 0) return MGPT_OK;
   if (!q || !out || !kpool || !vpool || !block_tables || !cu_q || !seq_lens || !q_req) return MGPT_ERR_NULL;
@@ -206,7 +207,7 @@ extern "C" int mgpt_paged_attention_generic(
                                      block_tables, max_blocks, cu_q, seq_lens, q_req, n_tokens, n_req, n_head, n_kv_head,
                                      page_size, scale, window, sinks, softcap, (const float*)gate, ldg, keep_first, chunked,
                                      dist_bias, bias_len, slopes};
-    if (mgpt_attention_exact_takes(args, head_dim)) return mgpt_attention_exact_launch(args, head_dim, stream);
+    if (mgpt_attention_exact_takes(args, head_dim)) return mgpt_attention_exact_launch(args, head_dim, single, stream);
   }
   dim3 grid(n_tokens, n_head), block(MGPT_WAVE);
 #define LAUNCH(T, F)                                                                              \

@@ -34,7 +34,8 @@ int mgpt_paged_attention_generic(const void* q, long ldq, void* out, long ldo, c
     int n_tokens, int n_req, int n_head, int n_kv_head, int head_dim, int page_size, float scale, int window, int dtype,
     int fast_exp, const float* sinks, float softcap, const void* gate, long ldg, int keep_first, const float*
     score_bias, int chunked,
-    const float* dist_bias, int bias_len, const float* slopes, hipStream_t stream);
+    const float* dist_bias, int bias_len, const float* slopes, int single,
+    hipStream_t stream);
 // attention_mixed.hip
 int mgpt_mixed_attention_bf16(const void* q, long ldq, void* out, long ldo, const void* kpool, const void* vpool, const int*
     block_tables, int max_blocks, const int* positions, const int* q_req, const int* cu_q, const int* seq_lens, int n_decode,

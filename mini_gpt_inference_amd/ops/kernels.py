@@ -274,8 +274,10 @@ def paged_attention_generic(q: torch.Tensor, out: torch.Tensor, k_pool: torch.Te
                             window: int = 0, fast_exp: bool = False, sinks: Optional[torch.Tensor] = None,
                             softcap: float = 0.0, gate: Optional[torch.Tensor] = None, keep_first: int = 0,
                             score_bias: Optional[torch.Tensor] = None, chunked: bool = False,
-                            dist_bias: Optional[torch.Tensor] = None, slopes: Optional[torch.Tensor] = None) -> None:
+                            dist_bias: Optional[torch.Tensor] = None, slopes: Optional[torch.Tensor] = None,
+                            single: bool = False) -> None:
     """Causal attention of the step's tokens over their requests' pages (any q_len, any dtype).
+    single: the caller has seen that token n is request n's only token (or padding) for all of them; the result is the same.
     sinks: float32 [n_head], one more term exp(sinks[h]) in every softmax denominator of head h.
     softcap > 0: every score becomes softcap * tanh(score / softcap) before the softmax.
     keep_first: behind a window a query also sees the keys at positions below it.  score_bias: float32 [n_head];
@@ -291,7 +293,7 @@ def paged_attention_generic(q: torch.Tensor, out: torch.Tensor, k_pool: torch.Te
         _ptr(q), q.stride(0), _ptr(out), out.stride(0), _ptr(k_pool), _ptr(v_pool), _ptr(block_tables),
         block_tables.shape[1], _ptr(cu_q), _ptr(seq_lens), _ptr(q_req), n_tokens, n_req, n_head, n_kv_head, head_dim,
         page_size, float(scale), int(window), _dtype_code(q), int(fast_exp), _ptr(sinks), float(softcap), *_gate_args(gate, q, n_tokens, n_head),
-        *_mask_args(keep_first, score_bias, n_head, sinks, softcap, chunked, dist_bias, slopes), _stream())
+        *_mask_args(keep_first, score_bias, n_head, sinks, softcap, chunked, dist_bias, slopes), int(single), _stream())
     _check(rc, "paged_attention_generic")
 
 

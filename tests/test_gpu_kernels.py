@@ -935,6 +935,45 @@ def test_float32_attention_keeps_its_sums_whatever_the_portion(d, window, mask):
     assert torch.equal(attend([r for r, _ in pick], [t for _, t in pick], [1] * len(pick), rows), whole[rows])
 
 
+@pytest.mark.parametrize("window,mask", [(0, {}), (100, {}), (100, {"keep_first": 70}), (96, {"chunked": True}), (0, {"dist_bias": 9}),
+                                         (0, {"slopes": True})])
+@pytest.mark.parametrize("page", [12, 16, 32])
+@pytest.mark.parametrize("d", [16, 32, 64, 128])
+def test_float32_attention_of_single_tokens_has_the_same_bits(d, page, window, mask):
+    """The kernel for a step of single tokens against the one for any step: around the ends of groups (16), chunks (64) and
+    rounds of eight waves (512), with padding, sinks, cap and gate, and with infinite and NaN values among the seen ones."""
+    lens = [1, 2, 15, 16, 17, 63, 64, 65, 200, 511, 512, 513, 650]
+    n = len(lens)
+    c = PagedCase(lens, [1] * n, h=4, hk=2, d=d, page=page, dtype="float32", seed=d + page)
+    g = torch.Generator().manual_seed(d)
+    mask = dict(mask)
+    if "dist_bias" in mask:
+        mask["dist_bias"] = torch.randn(4, mask["dist_bias"], generator=g).to(DEV)
+    if "slopes" in mask:
+        mask["slopes"] = torch.rand(4, generator=g).to(DEV)
+    extra = {"sinks": torch.randn(4, generator=g).to(DEV), "softcap": 20.0 if not mask else 0.0,
+             "gate": torch.randn(n, 4, generator=g).to(DEV)}
+    q_req = c.q_req.clone()
+    q_req[[3, 9]] = -1
+
+    def attend(single, **kw):
+        out = torch.full((n, 4 * d), 7.0, device=DEV)
+        kernels.paged_attention_generic(c.q_flat, out, c.kp, c.vp, c.bt, c.cu, c.sl, q_req, n, n, 4, d ** -0.5, window,
+                                        single=single, **kw, **mask)
+        return out
+
+    for kw in ({}, extra):
+        want = attend(False, **kw)
+        assert torch.isfinite(want).all() and (want[[3, 9]] == 7.0).all()
+        assert torch.equal(attend(True, **kw), want)
+    for i, (r, s) in enumerate(zip(range(n), lens)):
+        j = max(s - 1 - 5 * i, 0)
+        c.vp[int(c.bt[r, j // page]), i % 2, j % page, i % d] = (float("inf"), float("nan"), float("-inf"))[i % 3]
+    want = attend(False)
+    assert not torch.isfinite(want).all()
+    assert torch.equal(attend(True).nan_to_num(1e30, 2e30, 3e30), want.nan_to_num(1e30, 2e30, 3e30))
+
+
 @pytest.mark.parametrize("window,mask", [(0, {}), (20, {}), (20, {"keep_first": 9}), (24, {"chunked": True})])
 @pytest.mark.parametrize("d", [16, 32, 48, 64, 128])
 def test_float32_attention_keeps_what_a_query_does_not_see_out_of_it(d, window, mask):

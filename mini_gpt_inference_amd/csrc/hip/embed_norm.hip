@@ -227,6 +227,56 @@ __global__ __launch_bounds__(64 * W) void layernorm_shared_kernel(const float* _
   else reinterpret_cast<uint2*>(orow)[tid] = make_uint2(pack_bf16x2(y0, y1), pack_bf16x2(y2, y3));
 }
 
+// The kernel above for float32 rows that a product has left as sums over its blocks of k (linear_exact.hip): first
+// x += ((sums[0] + sums[1]) + ...) + bias, in the order in which that product adds them up itself, so the same bits; the row
+// goes back to `settled` if there is one (the rows' own place: nobody else reads them).  Without a gain that is all.
+template <int W>
+__global__ __launch_bounds__(64 * W) void layernorm_parts_kernel(const float* __restrict__ x, const float* __restrict__ sums,
+                                                                 int n_parts, long part_stride, const float* __restrict__ add,
+                                                                 const float* __restrict__ w, const float* __restrict__ b,
+                                                                 float* __restrict__ out, const int* __restrict__ rows,
+                                                                 int width, float eps, float* settled) {
+  constexpr int AT_ONCE = 16;                       // sums on their way
+  __shared__ float4 row_s[64 * W];
+  const int tid = threadIdx.x, lane = tid & (MGPT_WAVE - 1), n4 = width >> 2;
+  const long src = rows ? rows[blockIdx.x] : (long)blockIdx.x;
+  const int c = tid < n4 ? tid : 0;
+  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+  const float4* part = reinterpret_cast<const float4*>(sums + src * (long)width) + c;
+  float4 v = reinterpret_cast<const float4*>(x + src * (long)width)[c];
+  const float4 more = add ? reinterpret_cast<const float4*>(add)[c] : zero;
+  const float4 g = w ? reinterpret_cast<const float4*>(w)[c] : zero;
+  const float4 o = b ? reinterpret_cast<const float4*>(b)[c] : zero;
+  float4 total = zero;
+  for (int p0 = 0; p0 < n_parts; p0 += AT_ONCE) {
+    float4 t[AT_ONCE];
+#pragma unroll
+    for (int p = 0; p < AT_ONCE; ++p) t[p] = part[(p0 + p < n_parts ? p0 + p : p0) * (part_stride >> 2)];
+#pragma unroll
+    for (int p = 0; p < AT_ONCE; ++p)
+      if (p0 + p < n_parts) {
+        total.x += t[p].x; total.y += t[p].y; total.z += t[p].z; total.w += t[p].w;
+      }
+  }
+  if (add) {
+    total.x += more.x; total.y += more.y; total.z += more.z; total.w += more.w;
+  }
+  v.x += total.x; v.y += total.y; v.z += total.z; v.w += total.w;
+  if (settled && tid < n4) reinterpret_cast<float4*>(settled + src * (long)width)[tid] = v;
+  if (!w) return;
+  row_s[tid] = v;
+  __syncthreads();
+  float4 xv[W];
+#pragma unroll
+  for (int i = 0; i < W; ++i) xv[i] = row_s[lane + i * MGPT_WAVE];
+  float mean, corr, rstd;
+  layernorm_sums<W, 1>(xv, n4, width, eps, mean, corr, rstd);
+  if (tid >= n4) return;
+  const float y0 = ((v.x - mean) - corr) * rstd * g.x + o.x, y1 = ((v.y - mean) - corr) * rstd * g.y + o.y;
+  const float y2 = ((v.z - mean) - corr) * rstd * g.z + o.z, y3 = ((v.w - mean) - corr) * rstd * g.w + o.w;
+  reinterpret_cast<float4*>(out + (long)blockIdx.x * width)[tid] = make_float4(y0, y1, y2, y3);
+}
+
 // Rows of 2,049 to 4,096 values: 16 waves a row, whose sums meet in LDS (16 rows of 4,096 with the 4-byte loads of the first
 // kernel above 29 us, here 2.9; 4,096 rows 74 / 24).
 template <typename OT>
@@ -323,5 +373,29 @@ extern "C" int mgpt_layernorm(const float* x, const float* w, const float* b, vo
   } else {
     return MGPT_ERR_BAD_DTYPE;
   }
+  return mgpt_last_error();
+}
+
+// Rows left as sums over blocks by mgpt_linear_exact_parts (part_stride floats apart): out row i = LayerNorm of row rows[i] (or
+// i) of x + the sums in order + add (null: none), and with `settled` (x itself, or rows of the same kind) that sum as well;
+// w null: nothing but the sum.  Widths that are multiples of 4 up to 2,048, everything 16-byte aligned.
+extern "C" int mgpt_layernorm_parts(const float* x, const float* sums, int n_parts, long part_stride, const float* add,
+                                    const float* w, const float* b, float* out, const int* rows, int n_rows, int width,
+                                    float eps, float* settled, hipStream_t stream) {
+  if (n_rows == 0) return MGPT_OK;
+  if (!x || !sums || (w ? !out : !settled)) return MGPT_ERR_NULL;
+  const size_t together = (size_t)x | (size_t)sums | (size_t)add | (size_t)w | (size_t)b | (size_t)out | (size_t)settled;
+  if (n_rows < 0 || n_parts <= 0 || width <= 0 || width % 4 != 0 || width > 2048 || part_stride % 4 != 0 || (together & 15) != 0 ||
+      (rows && settled))
+    return MGPT_ERR_BAD_SHAPE;
+#define LP_LAUNCH(V)                                                                                                       \
+  case V:                                                                                                                  \
+    hipLaunchKernelGGL(layernorm_parts_kernel<V>, dim3(n_rows), dim3(64 * V), 0, stream, x, sums, n_parts, part_stride, add, w, \
+                       b, out, rows, width, eps, settled);                                                                 \
+    break
+  switch ((width / 4 + MGPT_WAVE - 1) / MGPT_WAVE) {
+    LP_LAUNCH(1); LP_LAUNCH(2); LP_LAUNCH(3); LP_LAUNCH(4); LP_LAUNCH(5); LP_LAUNCH(6); LP_LAUNCH(7); LP_LAUNCH(8);
+  }
+#undef LP_LAUNCH
   return mgpt_last_error();
 }

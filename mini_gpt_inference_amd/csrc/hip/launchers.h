@@ -55,6 +55,12 @@ int mgpt_embed(const int* ids, const int* pos, const void* tok, const void* post
 // embed_norm.hip
 int mgpt_layernorm(const float* x, const float* w, const float* b, void* out, const int* rows, int n_rows, int
     width, float eps, int out_dtype, hipStream_t stream);
+// embed_norm.hip
+int mgpt_layernorm_parts(const float* x, const float* sums, int n_parts, long part_stride, const float* add, const float* w,
+    const float* b, float* out, const int* rows, int n_rows, int width, float eps, float* settled, hipStream_t stream);
+// linear_exact.hip
+int mgpt_linear_exact_parts(const float* A, long lda, const float* W, float* sums, int n_rows, int n_out, int k_dim,
+    hipStream_t stream);
 // fold_norm.hip
 int mgpt_fold_layernorm(const void* w, const float* gain, const float* beta, const float* bias, void* w_out,
     float* colsum, float* bias_out, int n_out, int k_dim, hipStream_t stream);
@@ -272,6 +278,8 @@ int mgpt_linear_mfma_grouped(const void* act, long lda, const void* w, long w_st
   X(mgpt_prefill_attention_bf16) \
   X(mgpt_embed) \
   X(mgpt_layernorm) \
+  X(mgpt_layernorm_parts) \
+  X(mgpt_linear_exact_parts) \
   X(mgpt_fold_layernorm) \
   X(mgpt_pack_weight) \
   X(mgpt_fused_attention_decode) \

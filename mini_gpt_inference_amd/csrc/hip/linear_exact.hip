@@ -262,6 +262,61 @@ __global__ __launch_bounds__(1024) void linear_exact_rows_kernel(
   }
 }
 
+// Few rows with an output so narrow that workgroups of 16 x 16 outputs leave compute units idle while each brings the whole
+// inner size by itself: a workgroup has one block of k, whose sum goes to memory, sums[block][row][column]; whoever reads the
+// result next adds the blocks up in order (a LayerNorm: mgpt_layernorm_parts).  A wave has 16 columns and R tiles of 16 rows;
+// the rows' slice (R x 16 KB) is shared through LDS, all of a wave's slice of W (16 KB) is on its way at once.  What bounds
+// it is what a compute unit takes in, about 50 KB a us.  us with the LayerNorm behind it, rows kernel and LayerNorm / here:
+// 1 row 3072 -> 768 12.8 / 8.7, 16 rows 16.7 / 9.0, 64 rows 17.8 / 14.0; 6400 -> 1600 23 / 16, 30 / 17, 56 / 27; 16 rows
+// 2048 -> 512 13.0 / 8.1, 768 -> 768 8.7 / 8.1; 1 row 1024 -> 1024 7.7 / 8.2, 512 -> 512 6.5 / 7.5.
+template <int R, bool VEC>
+__global__ __launch_bounds__(256) void linear_exact_parts_kernel(const float* __restrict__ A, long lda,
+                                                                 const float* __restrict__ W, float* __restrict__ sums,
+                                                                 int n_rows, int n_out, int k_dim, int row_tiles) {
+  constexpr int PIECES = EX_BLOCK / 4, GROUPS = EX_BLOCK / EX_GROUP;
+  extern __shared__ __align__(16) float ex_lds[];    // [16 R][EX_BLOCK], 16-byte pieces XORed with the row's low bits
+  const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, lk = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int b = blockIdx.y, row0 = (int)(blockIdx.x % row_tiles) * 16 * R, col0 = ((int)(blockIdx.x / row_tiles) * 4 + wave) * 16;
+  const int lc = col0 + l16, kb = b * EX_BLOCK;
+  const float* wp = W + (long)(lc < n_out ? lc : n_out - 1) * k_dim;
+  ex_f4 ga[4 * R], wf[GROUPS];
+#pragma unroll
+  for (int p = 0; p < 4 * R; ++p) {                  // a wave a row: 64 pieces
+    const int r = row0 + 4 * p + wave;
+    ga[p] = ex_load<VEC>(A + (long)(r < n_rows ? r : n_rows - 1) * lda, kb + 4 * lane, k_dim);
+  }
+#pragma unroll
+  for (int u = 0; u < GROUPS; ++u) wf[u] = ex_load<VEC>(wp, kb + u * EX_GROUP + 4 * lk, k_dim);
+#pragma unroll
+  for (int p = 0; p < 4 * R; ++p) {
+    const int r = 4 * p + wave;
+    *reinterpret_cast<ex_f4*>(ex_lds + r * EX_BLOCK + ((lane ^ (r & 7)) << 2)) = ga[p];
+  }
+  __builtin_amdgcn_s_waitcnt(0xc07f);                // lgkmcnt(0): W may still be on its way
+  __builtin_amdgcn_s_barrier();
+  ex_f4 acc[R];
+#pragma unroll
+  for (int t = 0; t < R; ++t) acc[t] = (ex_f4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int u = 0; u < GROUPS; ++u) {
+    ex_f4 af[R];
+#pragma unroll
+    for (int t = 0; t < R; ++t)
+      af[t] = *reinterpret_cast<const ex_f4*>(ex_lds + (16 * t + l16) * EX_BLOCK + (((4 * u + lk) ^ (l16 & 7)) << 2));
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int t = 0; t < R; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[u][e], af[t][e], acc[t], 0, 0, 0);
+  }
+#pragma unroll
+  for (int t = 0; t < R; ++t) {
+    const int r = row0 + 16 * t + l16;
+    if (r < n_rows && col0 + 4 * lk < n_out)         // n_out is a multiple of 4
+      *reinterpret_cast<ex_f4*>(sums + ((long)b * n_rows + r) * n_out + col0 + 4 * lk) = acc[t];
+  }
+}
+
 struct ExactArgs {
   const float* A; long lda; const float* W; const float* bias; float* out; long ldo;
   int n_rows, n_out, k_dim;
@@ -353,4 +408,29 @@ extern "C" int mgpt_linear_exact_qkv(const float* A, long lda, const float* W, c
     return MGPT_ERR_BAD_SHAPE;
   const ExactScatter sc = {kpool, vpool, slot_mapping, q_width, kv_width, head_dim, page_size};
   return mgpt_linear_exact_launch(A, lda, W, bias, out, ldo, n_rows, n_out, k_dim, EPI_QKV, sc, stream);
+}
+
+// sums[b][n][o] = the sum over block b (256 k) of A[n] W[o], dense float32 with n_out a multiple of 4, 16-byte aligned: what
+// the product above adds up in the order of b, then the bias.
+extern "C" int mgpt_linear_exact_parts(const float* A, long lda, const float* W, float* sums, int n_rows, int n_out, int k_dim,
+                                       hipStream_t stream) {
+  if (n_rows == 0 || n_out == 0) return MGPT_OK;
+  if (!A || !W || !sums) return MGPT_ERR_NULL;
+  if (n_rows < 0 || n_out < 0 || k_dim <= 0 || lda < k_dim || n_out % 4 != 0 || (reinterpret_cast<uintptr_t>(sums) & 15) != 0)
+    return MGPT_ERR_BAD_SHAPE;
+  const bool vec = k_dim % 4 == 0 && lda % 4 == 0 && ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(W)) & 15) == 0;
+  // one tile of rows a workgroup while there is a compute unit for each (17 rows 3072 -> 768, 288 of them: 11.5 us, in
+  // workgroups of two 10.2; 64 rows 2048 -> 512, 256 of them: 10.1 / 10.7), else two (four: 10 % less to 30 % more)
+  const long ones = (((long)n_rows + 15) / 16) * (((long)n_out + 63) / 64) * (((long)k_dim + EX_BLOCK - 1) / EX_BLOCK);
+  const int r16 = n_rows <= 16 || ones <= 256 ? 1 : 2;
+  const long row_tiles = ((long)n_rows + 16 * r16 - 1) / (16 * r16), tiles = row_tiles * (((long)n_out + 63) / 64);
+  const int blocks = (int)(((long)k_dim + EX_BLOCK - 1) / EX_BLOCK);
+  if (tiles > 0x7fffffffL || blocks > 65535) return MGPT_ERR_TOO_LARGE;
+#define EX_PARTS_LAUNCH(R, V)                                                                                                  \
+  hipLaunchKernelGGL((linear_exact_parts_kernel<R, V>), dim3((unsigned int)tiles, blocks), dim3(256), R * 16 * EX_BLOCK * 4, \
+                     stream, A, lda, W, sums, n_rows, n_out, k_dim, (int)row_tiles)
+  if (r16 == 1) { if (vec) EX_PARTS_LAUNCH(1, true); else EX_PARTS_LAUNCH(1, false); }
+  else { if (vec) EX_PARTS_LAUNCH(2, true); else EX_PARTS_LAUNCH(2, false); }
+#undef EX_PARTS_LAUNCH
+  return mgpt_last_error();
 }

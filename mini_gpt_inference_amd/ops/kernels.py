@@ -164,6 +164,37 @@ def linear_exact_kernel(n_rows: int, n_out: int, k_dim: int) -> str:
     return ("rows", "tile64", "tile128")[library.kernels().mgpt_linear_exact_kernel(n_rows, n_out, k_dim)]
 
 
+EXACT_BLOCK = 256       # k whose sum is one part of a float32 product
+
+
+def linear_exact_blocks(k_dim: int) -> int:
+    return -(-k_dim // EXACT_BLOCK)
+
+
+def linear_exact_leaves_parts(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], x: torch.Tensor,
+                              n_rows: int) -> bool:
+    """Whether the sums over the blocks of k of a @ w.T may be left for the LayerNorm that reads x next: a product of few
+    rows, and rows that the kernel adding them up takes."""
+    n_out, k_dim = w.shape
+    return (a.dtype == w.dtype == x.dtype == torch.float32 and n_out % 4 == 0 and n_out <= 2048 and x.data_ptr() % 16 == 0
+            and (bias is None or bias.data_ptr() % 16 == 0)
+            and linear_exact_kernel(n_rows, n_out, k_dim) == "rows")
+
+
+def linear_exact_parts(a: torch.Tensor, w: torch.Tensor, sums: torch.Tensor, n_rows: int) -> None:
+    """sums[b] = a[:n_rows] @ w.T over block b of the inner size, float32 throughout: what linear_generic adds up in the order
+    of b, then the bias."""
+    _need_cuda(a, w, sums)
+    n_out, k_dim = w.shape
+    _need(w.is_contiguous() and a.dtype == w.dtype == torch.float32, "float32 products: weight must be dense [out, in]")
+    _need(a.dim() == 2 and a.stride(1) == 1 and a.shape[1] == k_dim and a.shape[0] >= n_rows,
+          f"activation must be [>=n_rows, {k_dim}] with unit inner stride")
+    _need(sums.dtype == torch.float32 and sums.is_contiguous() and sums.shape == (linear_exact_blocks(k_dim), n_rows, n_out),
+          "sums must be dense float32 [blocks, rows, out]")
+    _check(library.kernels().mgpt_linear_exact_parts(_ptr(a), a.stride(0), _ptr(w), _ptr(sums), n_rows, n_out, k_dim, _stream()),
+           "linear_exact_parts")
+
+
 def linear_exact_qkv(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor, n_rows: int,
                      scatter) -> bool:
     """out[:n_rows] = a[:n_rows] @ w.T (+ bias), float32 throughout, and the key and value columns also into their pages:
@@ -1058,6 +1089,8 @@ def residual_layer_norm(pending, gain: torch.Tensor, beta: Optional[torch.Tensor
     """out[i] = LayerNorm of row rows[i] (or i) of a residual that is still a sum.  With `settled`
     (float32 rows; may be the sum's base itself) the rows' sums are stored there too.  False if
     the width is not taken."""
+    if pending.exact:
+        return _layer_norm_parts(pending, gain, beta, eps, rows, out, n_rows, settled)
     width = gain.numel()
     if width % 32 or width > RESIDUAL_MAX_WIDTH or pending.base is None or pending.n_parts > residual_parts_limit(width):
         return False
@@ -1082,9 +1115,40 @@ def residual_layer_norm(pending, gain: torch.Tensor, beta: Optional[torch.Tensor
     return True
 
 
+def _layer_norm_parts(pending, gain, beta, eps, rows, out, n_rows: int, settled) -> bool:
+    """residual_layer_norm, or with gain None residual_settle, for the sums that linear_exact_parts leaves."""
+    base, parts, n_parts = pending.base, pending.partials, pending.n_parts
+    width = base.shape[1]
+    _need_cuda(base, parts, pending.bias, gain, beta, rows, out, settled)
+    for name, t in (("residual", base), ("settled rows", settled)):
+        _need(t is None or (t.dtype == torch.float32 and t.is_contiguous() and t.shape[1] == width),
+              f"the {name} must be dense float32 of the residual's width")
+    _need(parts.dtype == torch.float32 and parts.dim() == 3 and parts.is_contiguous() and parts.shape[0] >= n_parts
+          and parts.shape[2] == width, "pending sums must be dense float32 [parts, rows, width]")
+    for name, t in (("gain", gain), ("beta", beta), ("bias", pending.bias)):
+        _need(t is None or (t.dtype == torch.float32 and t.is_contiguous() and t.numel() == width), f"{name} must be float32 [width]")
+    _need(settled is None or rows is None, "settling through a row gather is not supported")
+    _need(out is None or (out.dtype == torch.float32 and out.is_contiguous() and out.shape[1] == width and out.shape[0] >= n_rows),
+          "LayerNorm output too small")
+    if rows is None:
+        _need(min(base.shape[0], parts.shape[1], n_rows if settled is None else settled.shape[0]) >= n_rows,
+              "the pending residual holds fewer rows than asked for")
+    else:
+        _need_i32("rows", rows, n_rows)
+    rc = library.kernels().mgpt_layernorm_parts(_ptr(base), _ptr(parts), n_parts, parts.stride(0), _ptr(pending.bias), _ptr(gain),
+                                                _ptr(beta), _ptr(out), _ptr(rows), n_rows, width, float(eps), _ptr(settled),
+                                                _stream())
+    if rc == -2:
+        return False
+    _check(rc, "layernorm_parts")
+    return True
+
+
 def residual_settle(pending, settled: torch.Tensor, n_rows: int) -> bool:
     """settled[:n_rows] = the rows of a residual that is still a sum (settled may be its base).
     False if the width is not taken."""
+    if pending.exact:
+        return _layer_norm_parts(pending, None, None, 0.0, None, None, n_rows, settled)
     width = settled.shape[1]
     if width % 32 or width > RESIDUAL_MAX_WIDTH or pending.base is None:
         return False

@@ -204,6 +204,15 @@ LEAVE_PARTS_MIN_ROWS = 8
 LEAVE_PARTS_MAX_ROWS = 256     # (the tiled kernel's split; the decode kernel's ends at its 64 rows)
 
 
+# The 32-bit path leaves the sums over the product's blocks of k for inner sizes from EXACT_PARTS_MIN_K on at any number of
+# rows, from EXACT_PARTS_MIN_K_ROWS on above EXACT_PARTS_FEW_ROWS rows (measured at the kernel, linear_exact.hip), and only
+# where the product would go to the kernel for few rows.
+EXACT_PARTS_MIN_K = 6 * 256 + 1
+EXACT_PARTS_MIN_K_ROWS = 2 * 256 + 1
+EXACT_PARTS_FEW_ROWS = 4
+EXACT_PARTS_MAX_ROWS = 256
+
+
 def plain_residual(ctx, h, x: torch.Tensor) -> None:
     """Makes the residual rows x plain for a part that reads or adds to them with ordinary kernels.
     If they are still a sum and h is the LayerNorm of them that the part is about to read, that
@@ -222,7 +231,18 @@ def linear_add(ctx, a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tenso
     may_leave_parts: the caller and whoever reads x next know of ctx.pending.  Then a product whose
     long inner size is split over workgroups anyway (few rows, few column tiles) leaves the
     workgroups' sums as the parts of a pending residual instead of running a second kernel that adds
-    them into x; the LayerNorm that reads x next adds them up (LazyNorm.tensor)."""
+    them into x; the LayerNorm that reads x next adds them up (LazyNorm.tensor).  The 32-bit path does so with the sums over
+    the blocks of k that its products are made of, which has the bits of adding into x at once."""
+    if (may_leave_parts and ctx.exact and getattr(ctx, "pending", None) is None and 0 < n_rows <= EXACT_PARTS_MAX_ROWS
+            and n_rows == ctx.n_rows and w.shape[1] >= (EXACT_PARTS_MIN_K if n_rows <= EXACT_PARTS_FEW_ROWS
+                                                        else EXACT_PARTS_MIN_K_ROWS)
+            and x.is_contiguous() and x.shape[1] == w.shape[0] and kernels.linear_exact_leaves_parts(a, w, bias, x, n_rows)):
+        n_parts = kernels.linear_exact_blocks(w.shape[1])
+        buf = ctx.workspace.get("residual_parts", n_parts * n_rows, w.shape[0], torch.float32)
+        parts = buf[:n_parts * n_rows].view(n_parts, n_rows, w.shape[0])
+        kernels.linear_exact_parts(a, w, parts, n_rows)
+        ctx.pending = residual.PendingSums(x, parts, n_parts, exact=True, bias=bias)
+        return
     leave = (may_leave_parts and getattr(ctx, "pending", None) is None and not ctx.exact
              and ctx.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and a.dtype == torch.bfloat16
              and 0 < n_rows <= LEAVE_PARTS_MAX_ROWS and n_rows == ctx.n_rows and x.is_contiguous()

@@ -37,6 +37,8 @@ class PendingSums:
     partials: Optional[torch.Tensor]    # float32 [parts, rows, width], or None
     n_parts: int
     tables: Optional[Tuple] = None      # (token table, position table or None, token ids, positions)
+    exact: bool = False                 # the 32-bit path's: the partials are a product's sums over its blocks of k, and
+    bias: Optional[torch.Tensor] = None # base + (their sum in order + bias) has the bits of that product's own addition
 
 
 def twin_of(ctx, x: torch.Tensor) -> torch.Tensor:

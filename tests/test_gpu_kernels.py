@@ -10,6 +10,7 @@ import torch
 import helpers
 import plain_gpt as P
 from mini_gpt_inference_amd.ops import kernels
+from mini_gpt_inference_amd.ops.residual import PendingSums
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -225,6 +226,31 @@ def test_float32_product_stores_keys_and_values(n, k, h, hk, d, kernel):
     assert torch.equal(got, want)
     assert torch.equal(pools[0].nan_to_num(9.0), pools[2].nan_to_num(9.0))
     assert torch.equal(pools[1].nan_to_num(9.0), pools[3].nan_to_num(9.0))
+
+
+@pytest.mark.parametrize("n,k,o", [(1, 1, 4), (1, 1537, 512), (3, 256, 60), (4, 3072, 768), (16, 257, 64), (17, 1026, 68),
+                                   (17, 3072, 768), (33, 5000, 260), (70, 2048, 2048), (128, 768, 1028), (130, 4097, 1600)])
+def test_float32_product_left_as_sums_over_its_blocks(n, k, o):
+    """The sums over the blocks of k, added up by the LayerNorm that reads the rows next (all rows, some of them, or with no
+    LayerNorm at all): the same bits as the product that adds to the residual and the LayerNorm of that."""
+    g = torch.Generator().manual_seed(n + k)
+    a, w, x = rnd(g, n, k + k % 4).to(DEV)[:, :k], rnd(g, o, k).to(DEV), rnd(g, n, o).to(DEV)
+    bias, gain, beta = rnd(g, o).to(DEV), rnd(g, o).to(DEV), rnd(g, o).to(DEV)
+    rows = i32([(7 * i) % n for i in range(min(n, 5))])
+    for b, shift in ((bias, beta), (None, None)):
+        want_x, want, want_rows = x.clone(), torch.empty_like(x), torch.empty(len(rows), o, device=DEV)
+        kernels.linear_generic(a, w, b, want_x, n, kernels.EPI_RESIDUAL)
+        kernels.layer_norm(want_x, gain, shift, want, n, 1e-5)
+        kernels.layer_norm(want_x, gain, shift, want_rows, len(rows), 1e-5, rows)
+        sums = torch.full((kernels.linear_exact_blocks(k), n, o), float("nan"), device=DEV)
+        kernels.linear_exact_parts(a, w, sums, n)
+        got_x, got, got_rows, settled = x.clone(), torch.empty_like(x), torch.empty_like(want_rows), torch.empty_like(x)
+        pending = PendingSums(got_x, sums, len(sums), exact=True, bias=b)
+        assert kernels.residual_layer_norm(pending, gain, shift, 1e-5, rows, got_rows, len(rows))
+        assert kernels.residual_settle(pending, settled, n)
+        assert kernels.residual_layer_norm(pending, gain, shift, 1e-5, None, got, n, settled=got_x)
+        assert torch.equal(got_x, want_x) and torch.equal(settled, want_x)
+        assert torch.equal(got, want) and torch.equal(got_rows, want_rows)
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])

@@ -161,21 +161,31 @@ WIDE_OUT_DECODE_WORK = 8192
 # 32, 18.8 / 10.0 at 64; [6400 x 1600] 9.3 / 9.1, 11.4 / 9.3, 12.7 / 9.3, 19.8 / 12.0; under smaller
 # matrices the decode kernel stays ahead up to 64 rows ([3072 x 768] 5.0 / 5.6 at 32, 6.2 / 5.6 at
 # 64; [1600 x 1600] 5.8 / 8.4 and 8.0 / 8.4).  A long inner size under a narrow output is split over
-# workgroups by either; there the tiled kernel with its joining kernel is ahead from 33 rows on
-# ([1600 x 6400]: the decode kernel's first half alone, its sums left pending, 20.0 us at 64 rows, the
-# tiled pair 15.1; at 32 rows about 11.5 against 12.7).
+# workgroups by either; there the tiled kernel, whose slices go straight into LDS, is ahead from 9 rows on (either with
+# its sums left pending and the LayerNorm that adds them up, decode kernel / tiled: [1600 x 6400] 11.2 / 10.4 us at 8 rows,
+# 12.6 / 10.4 at 16, 16.0 / 10.8 at 32, 23.6 / 12.7 at 64; [1280 x 5120] 10.5 / 10.5, 11.8 / 10.4, 15.7 / 10.7; [1152 x 4608]
+# 10.4 / 10.0, 11.7 / 10.1; [1024 x 4096] 8.0 / 9.3, 8.3 / 9.4, 9.4 / 9.5), and from 17 rows on where a second kernel has
+# to add the sums up ([1600 x 6400] 9.7 / 10.0 at 12 rows, 10.4 / 10.0 at 16, 14.3 / 10.4 at 32; [2048 x 8192] 12.5 / 13.3,
+# 13.6 / 13.7, 18.5 / 14.0).
 TILED_FROM_ROWS = 17
 TILED_MIN_OUT = 4096
 TILED_MIN_MATRIX = 6_000_000
-TILED_ANY_OUT_FROM_ROWS = 33
+TILED_ANY_SHAPE_FROM_ROWS = 33
+TILED_LONG_LEFT_FROM_ROWS = 9
+TILED_LONG_MIN_INNER = 4097
+TILED_LONG_MIN_MATRIX = 5_000_000
 
 
-def tiled_at_few_rows(n_rows: int, w: torch.Tensor) -> bool:
+def tiled_at_few_rows(n_rows: int, w: torch.Tensor, left: bool = False) -> bool:
     """Whether a product of few rows (the decode kernel takes up to 64; linear_add asks for up to
-    LEAVE_PARTS_MAX_ROWS) goes to the tiled kernel rather than the decode kernel."""
-    if w.shape[0] * w.shape[1] < TILED_MIN_MATRIX:
+    LEAVE_PARTS_MAX_ROWS) goes to the tiled kernel rather than the decode kernel.  left: the sums of a split
+    product are left pending."""
+    n_out, k_dim = w.shape
+    if n_out < TILED_MIN_OUT and k_dim >= TILED_LONG_MIN_INNER and n_out * k_dim >= TILED_LONG_MIN_MATRIX:
+        return n_rows >= (TILED_LONG_LEFT_FROM_ROWS if left else TILED_FROM_ROWS)
+    if n_out * k_dim < TILED_MIN_MATRIX:
         return False
-    return n_rows >= TILED_ANY_OUT_FROM_ROWS or (n_rows >= TILED_FROM_ROWS and w.shape[0] >= TILED_MIN_OUT)
+    return n_rows >= TILED_ANY_SHAPE_FROM_ROWS or (n_rows >= TILED_FROM_ROWS and n_out >= TILED_MIN_OUT)
 
 
 def as_tensor(ctx, a: Union[torch.Tensor, LazyNorm]) -> torch.Tensor:
@@ -247,7 +257,7 @@ def linear_add(ctx, a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tenso
              and ctx.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and a.dtype == torch.bfloat16
              and 0 < n_rows <= LEAVE_PARTS_MAX_ROWS and n_rows == ctx.n_rows and x.is_contiguous()
              and x.shape[1] == w.shape[0] and w.shape[1] % 16 == 0)
-    if leave and tiled_at_few_rows(n_rows, w):
+    if leave and tiled_at_few_rows(n_rows, w, left=True):
         # the tiled kernel's split: its stretches' sums are the parts (2 to 8 of them)
         need = kernels.linear_mfma_partials(n_rows, w.shape[0], w.shape[1], kernels.EPI_RESIDUAL)
         n_parts = need // (n_rows * w.shape[0])

@@ -401,3 +401,30 @@ def test_fused_kernels_refuse_what_they_cannot_do():
                                                   torch.zeros(1, 4, dtype=torch.int32, device=DEV), i32([0]), i32([0]),
                                                   1, h, 0.125)
         assert bool((out == 7.0).all())
+
+
+@pytest.mark.parametrize("rows", [8, 9, 16, 17, 33])
+@pytest.mark.parametrize("n_out,k_dim", [(1600, 6400), (1152, 4608), (1024, 4096)])
+def test_addition_of_few_rows_under_a_long_inner_size(rows, n_out, k_dim):
+    """ops.linear.linear_add on both sides of the lines between the decode kernel's split and the tiled one, with the sums left
+    for the LayerNorm and without: x + product within the tolerance of its bfloat16 operands."""
+    from types import SimpleNamespace
+
+    from mini_gpt_inference_amd.ops import linear as L
+    from mini_gpt_inference_amd.parts.base import Workspace
+
+    g = torch.Generator().manual_seed(rows)
+    a, w, b, x = bf(rnd(g, rows, k_dim)), bf(rnd(g, n_out, k_dim, scale=0.03)), rnd(g, n_out), rnd(g, rows, n_out)
+    want = x.double() + P.plain_linear(a.double(), w.double(), b.double())
+    wd = w.to(DEV)
+    assert L.tiled_at_few_rows(rows, wd, left=True) == (rows >= 9 and k_dim > 4096)
+    assert L.tiled_at_few_rows(rows, wd) == (rows >= 17 and k_dim > 4096)
+    for left in (True, False):
+        ctx = SimpleNamespace(exact=False, dtype=torch.bfloat16, n_rows=rows, pending=None, copy_budget=None,
+                              workspace=Workspace(torch.device(DEV)))
+        got = x.to(DEV)
+        L.linear_add(ctx, a.to(DEV), wd, b.to(DEV), got, rows, may_leave_parts=left)
+        assert left or ctx.pending is None
+        if ctx.pending is not None:
+            assert kernels.residual_settle(ctx.pending, got, rows)
+        helpers.assert_close(got, want, "bfloat16", "x + product")

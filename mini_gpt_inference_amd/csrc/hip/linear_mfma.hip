@@ -29,7 +29,8 @@
 // Five further variants (DIRECT) send the slices from memory straight into LDS
 // (global_load_lds_dwordx4) instead of through registers: three or four stages for a long inner
 // size, 128 x 192 tiles for wide outputs under many rows, and four or six stages of 32 x 32 tiles for
-// the rows of a decode step under a large matrix; see the kernel, choose_direct and launch_any.
+// the rows of a decode step under a large matrix; see the kernel, choose_direct and launch_any.  Four more, for
+// many rows, also let the workgroup's two halves read and multiply in turn (linear_mfma_halves_kernel, choose_large).
 #include "common.h"
 #include <type_traits>
 #include "launchers.h"
@@ -136,6 +137,125 @@ namespace {
 constexpr int MM_BK = 64;
 constexpr int MM_LD = MM_BK;       // LDS row stride in elements: 128 bytes, eight 16-byte chunks
 constexpr int MM_GROUP = 4;         // row tiles per block of tiles
+
+// What becomes of a workgroup's sums: bias, activation, and the stores.  acc[i][j] of a lane: four neighbouring columns of one
+// row, out[row0 + wr + j*16 + (lane & 15)][col0 + wc + i*16 + (lane >> 4)*4 + e].  lds: LDS_ELEMS elements that nobody needs any
+// more once every wave is here.
+template <int WTM, int WTN, int WVM, int WVN, int T, int LDS_ELEMS, int EPI, typename OT>
+__device__ __forceinline__ void mfma_epilogue(f32x4_t (&acc)[WTN][WTM], bf16_t* lds, const float* __restrict__ bias,
+                                              OT* __restrict__ out, long ldo, int n_rows, int n_out, int row0, int col0, int wr,
+                                              int wc, const MfmaScatter& sc) {
+  constexpr int BM = WVM * WTM * 16, BN = WVN * WTN * 16;
+  const int tid = threadIdx.x, lane = tid & 63, lrow = lane & 15;
+  // the activation's coefficients, read once (a store in between would make the compiler read them again)
+  float xa_p = 0.f, xa_n = 0.f;
+  if (EPI == MM_EPI_XIELU) {
+    xa_p = sc.epi_coef[0];
+    xa_n = sc.epi_coef[1];
+  }
+  // lane holds out[row0 + wr + j*16 + (lane & 15)][col0 + wc + i*16 + (lane >> 4)*4 + e], e = 0..3
+  const bool vec = (n_out & 3) == 0 && (ldo & 3) == 0 && (((size_t)out | (size_t)bias) & 15) == 0;
+  // bfloat16 outputs go through LDS (the staged operands are done with): a lane's four columns of
+  // sixteen different rows would be sixteen 8-byte pieces per store; from LDS a thread stores 16
+  // bytes and a row's threads a whole stretch of the row, and a key's or value's eight channels
+  // go to their cache page the same way.
+  constexpr int LDT = BN + 8;   // row stride of the tile in LDS
+  // the whole tile at once if it fits, else the rows of one row of waves at a time
+  constexpr int STAGE_ROWS = BM * LDT <= LDS_ELEMS ? BM : BM / WVM;
+  constexpr bool CAN_STAGE = sizeof(OT) == 2 && STAGE_ROWS * LDT <= LDS_ELEMS;
+  if (CAN_STAGE && EPI != MM_EPI_RESIDUAL && (n_out & 7) == 0 && (ldo & 7) == 0 && (((size_t)out) & 15) == 0 &&
+      (EPI != MM_EPI_QKV || ((sc.q_width | sc.kv_width | sc.head_dim) & 7) == 0)) {
+    bf16_t* tile = lds;
+    for (int part = 0; part < BM / STAGE_ROWS; ++part) {
+      __syncthreads();   // the staged operands, or the part before this one, are done with
+      if (wr / STAGE_ROWS == part) {
+#pragma unroll
+        for (int i = 0; i < WTN; ++i) {
+          const int tc = wc + i * 16 + (lane >> 4) * 4, oc = col0 + tc;
+          float b4[4];
+          mfma_bias4(bias, oc < n_out ? oc : 0, n_out, (((size_t)bias) & 15) == 0, b4);
+#pragma unroll
+          for (int j = 0; j < WTM; ++j) {
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              v[e] = acc[i][j][e] + b4[e];
+              if (EPI == MM_EPI_GELU) v[e] = gelu_tanh_fast(v[e]);
+              if (EPI == MM_EPI_RELU2) v[e] = relu_squared(v[e]);
+              if (EPI == MM_EPI_XIELU) v[e] = mfma_xielu(v[e], xa_p, xa_n);
+            }
+            uint2 pk;
+            pk.x = pack_bf16x2(v[0], v[1]);
+            pk.y = pack_bf16x2(v[2], v[3]);
+            *reinterpret_cast<uint2*>(&tile[(wr - part * STAGE_ROWS + j * 16 + lrow) * LDT + tc]) = pk;
+          }
+        }
+      }
+      __syncthreads();
+      constexpr int CPR = BN / 8;   // 16-byte chunks per tile row
+      for (int c = tid; c < STAGE_ROWS * CPR; c += T) {
+        const int row = c / CPR, tc = (c % CPR) * 8;
+        const int n = row0 + part * STAGE_ROWS + row, oc = col0 + tc;
+        if (n >= n_rows || oc >= n_out) continue;
+        const uint4 v8 = *reinterpret_cast<const uint4*>(&tile[row * LDT + tc]);
+        *reinterpret_cast<uint4*>(reinterpret_cast<bf16_t*>(out) + (long)n * ldo + oc) = v8;
+        if (EPI == MM_EPI_QKV && oc >= sc.q_width) {
+          // the chunk's eight columns lie in one head
+          const int slot = sc.slot_mapping[n];
+          if (slot >= 0) {
+            const int page = slot / sc.page_size, off = slot - page * sc.page_size;
+            const int cq = oc - sc.q_width;  // column among keys then values
+            const bool is_v = cq >= sc.kv_width;
+            const int cc = is_v ? cq - sc.kv_width : cq;
+            const int hh = cc / sc.head_dim, d = cc - hh * sc.head_dim;
+            const long dst = (((long)page * sc.n_kv_head + hh) * sc.page_size + off) * sc.head_dim + d;
+            *reinterpret_cast<uint4*>((is_v ? sc.vpool : sc.kpool) + dst) = v8;
+          }
+        }
+      }
+    }
+    return;
+  }
+  // A key or value at (row n, column c of head hh, channel d) goes to
+  // ((page * n_kv_head + hh) * page_size + offset) * head_dim + d of its pool, page and offset from
+  // the row's slot: the row's part and the column's part of that are worked out once each.
+  long cache_row[WTM];
+  if (EPI == MM_EPI_QKV) {
+#pragma unroll
+    for (int j = 0; j < WTM; ++j) {
+      const int n = row0 + wr + j * 16 + lrow;
+      const int slot = n < n_rows ? sc.slot_mapping[n] : -1;
+      const int page = slot / sc.page_size, off = slot - page * sc.page_size;
+      cache_row[j] = slot < 0 ? -1 : ((long)page * sc.n_kv_head * sc.page_size + off) * sc.head_dim;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < WTN; ++i) {
+    const int oc = col0 + wc + i * 16 + (lane >> 4) * 4;
+    if (oc >= n_out) continue;
+    float b4[4];
+    mfma_bias4(bias, oc, n_out, vec, b4);
+    bf16_t* cache_col = nullptr;
+    if (EPI == MM_EPI_QKV && oc >= sc.q_width) {
+      const int c = oc - sc.q_width;  // column among keys then values
+      const bool is_v = c >= sc.kv_width;
+      const int cc = is_v ? c - sc.kv_width : c;
+      const int hh = cc / sc.head_dim, d = cc - hh * sc.head_dim;
+      cache_col = (is_v ? sc.vpool : sc.kpool) + (long)hh * sc.page_size * sc.head_dim + d;
+    }
+#pragma unroll
+    for (int j = 0; j < WTM; ++j) {
+      const int n = row0 + wr + j * 16 + lrow;
+      if (n >= n_rows) continue;
+      bf16_t* cache_dst = nullptr;
+      if (EPI == MM_EPI_QKV && cache_col && cache_row[j] >= 0) cache_dst = cache_col + cache_row[j];
+      if (EPI == MM_EPI_XIELU)
+        mfma_store4<EPI, OT>(acc[i][j], b4, out, ldo, n, oc, n_out, vec, cache_dst, xa_p, xa_n);
+      else
+        mfma_store4<EPI, OT>(acc[i][j], b4, out, ldo, n, oc, n_out, vec, cache_dst);
+    }
+  }
+}
 
 // WTM x WTN: 16-wide tiles per wave along the rows of the activations and along the rows of W;
 // WVM x WVN: waves in a workgroup along the same.
@@ -432,117 +552,223 @@ __global__ __launch_bounds__(64 * WVM * WVN * KG) void linear_mfma_kernel(
       }
   }
 
-  // the activation's coefficients, read once (a store in between would make the compiler read them again)
-  float xa_p = 0.f, xa_n = 0.f;
-  if (EPI == MM_EPI_XIELU) {
-    xa_p = sc.epi_coef[0];
-    xa_n = sc.epi_coef[1];
-  }
-  // lane holds out[row0 + wr + j*16 + (lane & 15)][col0 + wc + i*16 + (lane >> 4)*4 + e], e = 0..3
-  const bool vec = (n_out & 3) == 0 && (ldo & 3) == 0 && (((size_t)out | (size_t)bias) & 15) == 0;
-  // bfloat16 outputs go through LDS (the staged operands are done with): a lane's four columns of
-  // sixteen different rows would be sixteen 8-byte pieces per store; from LDS a thread stores 16
-  // bytes and a row's threads a whole stretch of the row, and a key's or value's eight channels
-  // go to their cache page the same way.
-  constexpr int LDT = BN + 8;   // row stride of the tile in LDS
-  constexpr int LDS_ELEMS = STAGES * (BM + BN) * MM_LD;
-  // the whole tile at once if it fits, else the rows of one row of waves at a time
-  constexpr int STAGE_ROWS = BM * LDT <= LDS_ELEMS ? BM : BM / WVM;
-  constexpr bool CAN_STAGE = sizeof(OT) == 2 && STAGE_ROWS * LDT <= LDS_ELEMS;
-  if (CAN_STAGE && EPI != MM_EPI_RESIDUAL && (n_out & 7) == 0 && (ldo & 7) == 0 && (((size_t)out) & 15) == 0 &&
-      (EPI != MM_EPI_QKV || ((sc.q_width | sc.kv_width | sc.head_dim) & 7) == 0)) {
-    bf16_t* tile = lds;
-    for (int part = 0; part < BM / STAGE_ROWS; ++part) {
-      __syncthreads();   // the staged operands, or the part before this one, are done with
-      if (wr / STAGE_ROWS == part) {
-#pragma unroll
-        for (int i = 0; i < WTN; ++i) {
-          const int tc = wc + i * 16 + (lane >> 4) * 4, oc = col0 + tc;
-          float b4[4];
-          mfma_bias4(bias, oc < n_out ? oc : 0, n_out, (((size_t)bias) & 15) == 0, b4);
-#pragma unroll
-          for (int j = 0; j < WTM; ++j) {
-            float v[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              v[e] = acc[i][j][e] + b4[e];
-              if (EPI == MM_EPI_GELU) v[e] = gelu_tanh_fast(v[e]);
-              if (EPI == MM_EPI_RELU2) v[e] = relu_squared(v[e]);
-              if (EPI == MM_EPI_XIELU) v[e] = mfma_xielu(v[e], xa_p, xa_n);
-            }
-            uint2 pk;
-            pk.x = pack_bf16x2(v[0], v[1]);
-            pk.y = pack_bf16x2(v[2], v[3]);
-            *reinterpret_cast<uint2*>(&tile[(wr - part * STAGE_ROWS + j * 16 + lrow) * LDT + tc]) = pk;
-          }
-        }
-      }
-      __syncthreads();
-      constexpr int CPR = BN / 8;   // 16-byte chunks per tile row
-      for (int c = tid; c < STAGE_ROWS * CPR; c += T) {
-        const int row = c / CPR, tc = (c % CPR) * 8;
-        const int n = row0 + part * STAGE_ROWS + row, oc = col0 + tc;
-        if (n >= n_rows || oc >= n_out) continue;
-        const uint4 v8 = *reinterpret_cast<const uint4*>(&tile[row * LDT + tc]);
-        *reinterpret_cast<uint4*>(reinterpret_cast<bf16_t*>(out) + (long)n * ldo + oc) = v8;
-        if (EPI == MM_EPI_QKV && oc >= sc.q_width) {
-          // the chunk's eight columns lie in one head
-          const int slot = sc.slot_mapping[n];
-          if (slot >= 0) {
-            const int page = slot / sc.page_size, off = slot - page * sc.page_size;
-            const int cq = oc - sc.q_width;  // column among keys then values
-            const bool is_v = cq >= sc.kv_width;
-            const int cc = is_v ? cq - sc.kv_width : cq;
-            const int hh = cc / sc.head_dim, d = cc - hh * sc.head_dim;
-            const long dst = (((long)page * sc.n_kv_head + hh) * sc.page_size + off) * sc.head_dim + d;
-            *reinterpret_cast<uint4*>((is_v ? sc.vpool : sc.kpool) + dst) = v8;
-          }
-        }
-      }
-    }
-    return;
-  }
-  // A key or value at (row n, column c of head hh, channel d) goes to
-  // ((page * n_kv_head + hh) * page_size + offset) * head_dim + d of its pool, page and offset from
-  // the row's slot: the row's part and the column's part of that are worked out once each.
-  long cache_row[WTM];
-  if (EPI == MM_EPI_QKV) {
-#pragma unroll
-    for (int j = 0; j < WTM; ++j) {
-      const int n = row0 + wr + j * 16 + lrow;
-      const int slot = n < n_rows ? sc.slot_mapping[n] : -1;
-      const int page = slot / sc.page_size, off = slot - page * sc.page_size;
-      cache_row[j] = slot < 0 ? -1 : ((long)page * sc.n_kv_head * sc.page_size + off) * sc.head_dim;
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < WTN; ++i) {
-    const int oc = col0 + wc + i * 16 + (lane >> 4) * 4;
-    if (oc >= n_out) continue;
-    float b4[4];
-    mfma_bias4(bias, oc, n_out, vec, b4);
-    bf16_t* cache_col = nullptr;
-    if (EPI == MM_EPI_QKV && oc >= sc.q_width) {
-      const int c = oc - sc.q_width;  // column among keys then values
-      const bool is_v = c >= sc.kv_width;
-      const int cc = is_v ? c - sc.kv_width : c;
-      const int hh = cc / sc.head_dim, d = cc - hh * sc.head_dim;
-      cache_col = (is_v ? sc.vpool : sc.kpool) + (long)hh * sc.page_size * sc.head_dim + d;
-    }
-#pragma unroll
-    for (int j = 0; j < WTM; ++j) {
-      const int n = row0 + wr + j * 16 + lrow;
-      if (n >= n_rows) continue;
-      bf16_t* cache_dst = nullptr;
-      if (EPI == MM_EPI_QKV && cache_col && cache_row[j] >= 0) cache_dst = cache_col + cache_row[j];
-      if (EPI == MM_EPI_XIELU)
-        mfma_store4<EPI, OT>(acc[i][j], b4, out, ldo, n, oc, n_out, vec, cache_dst, xa_p, xa_n);
-      else
-        mfma_store4<EPI, OT>(acc[i][j], b4, out, ldo, n, oc, n_out, vec, cache_dst);
-    }
-  }
+  mfma_epilogue<WTM, WTN, WVM, WVN, T, STAGES * (BM + BN) * MM_LD, EPI, OT>(acc, lds, bias, out, ldo, n_rows, n_out, row0,
+                                                                            col0, wr, wc, sc);
 }
 
+// The large tiles with the two halves of the workgroup out of step: 128 or 256 rows x 256 columns, eight waves of
+// (WTM * 16) x 64, slices straight into LDS as in the DIRECT variants above.
+//
+// With all waves in step, each SIMD's two waves read their operands at the same time and then multiply at the same time, and
+// the matrix units idle while the LDS works and the other way round (a step of 256 x 256 x 64 took 2.1 us for 0.9 us of
+// MFMAs).  Here a step is cut into phases of 32 MFMAs a wave (64 of its rows), each a slot of reading and a slot of multiplying
+// with a barrier between, and waves 4 to 7 (one on every SIMD) run one slot behind waves 0 to 3: in every slot one wave of a
+// SIMD multiplies, at raised priority, while the other reads the operands of its next phase and sends for slices.
+//
+// (Four phases of 16 MFMAs took 163 us for 4,096 rows 6400 -> 1600, where two take 136; at full occupancy, 4,096 columns, both
+// 160: the clock gives way.)
+// With 256 rows a step has two phases (the upper and the lower 64 rows of a wave) and LDS two stages.  W and the upper rows
+// have been read by both halves once the second half is through its first phase's reading: those of step s + 2 are sent for in
+// the second phase of step s; the lower rows of step s + 1 in its first phase.  With 128 rows a step is one phase, LDS has
+// three stages, and step s + 2 goes where step s - 1 was.  A wave waits for its own loads at the end of the slot behind which
+// the first half begins to read what they bring; younger loads stay on their way.
+template <int WTM, int WTN, int EPI, typename OT>
+__global__ __launch_bounds__(512, 2) void linear_mfma_halves_kernel(const bf16_t* __restrict__ act, long lda,
+                                                                 const bf16_t* __restrict__ w, const float* __restrict__ bias,
+                                                                 OT* __restrict__ out, long ldo, int n_rows, int n_out, int k_dim,
+                                                                 MfmaScatter sc) {
+  static_assert((WTM == 4 || WTM == 8) && (WTN == 3 || WTN == 4), "128 or 256 rows, 192 or 256 columns");
+  constexpr int WVM = 2, WVN = 4, T = 512;
+  constexpr int BM = WVM * WTM * 16, BN = WVN * WTN * 16, STAGES = WTM == 8 ? 2 : 3;
+  constexpr int LW = BN / 64;                 // a wave's loads of W's slice: 8 rows each; 2 of 64 (WTM = 8: upper, lower) rows a half
+  extern __shared__ __align__(16) bf16_t lds[];
+  bf16_t* const as_base = lds;
+  bf16_t* const ws_base = lds + STAGES * BM * MM_LD;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int row_tiles = (n_rows + BM - 1) / BM, col_tiles = (n_out + BN - 1) / BN;
+  int row_tile, col_tile;
+  {
+    const int id = mfma_xcd_tile_id(blockIdx.x, gridDim.x);
+    const int per_group = MM_GROUP * col_tiles;
+    const int group = id / per_group, in_group = id - group * per_group;
+    const int first = group * MM_GROUP;
+    const int rows_here = row_tiles - first < MM_GROUP ? row_tiles - first : MM_GROUP;
+    row_tile = first + in_group % rows_here;
+    col_tile = in_group / rows_here;
+  }
+  const int row0 = row_tile * BM, col0 = col_tile * BN;
+  if (sc.row_expert) {
+    const int e = sc.row_expert[row0 / sc.group_rows];
+    if (e < 0 || sc.row_valid[row0] < 0) return;   // the whole workgroup, before any barrier
+    w += (long)e * sc.w_stride;
+  }
+  const int half = wave >> 2;
+  const int wr = half * (WTM * 16), wc = (wave & 3) * (WTN * 16), lrow = lane & 15;
+  const int k_steps = k_dim / MM_BK;
+
+  typedef __attribute__((address_space(1))) const void* global_ptr_t;
+  typedef __attribute__((address_space(3))) void* lds_ptr_t;
+  const int lr = lane >> 3, lc = ((lane & 7) ^ lr) * 8;
+  // eight rows of the activations' slice: those numbered 16 h + 8 p + wave are rows wave * 8 .. of half h's part p (of 64 rows)
+  constexpr int PARTS = WTM / 4;
+  const bf16_t* ap[PARTS][2];
+  const bf16_t* wp[LW];
+#pragma unroll
+  for (int p = 0; p < PARTS; ++p)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int r = row0 + (PARTS * 8 * h + 8 * p + wave) * 8 + lr;
+      ap[p][h] = act + (long)(r < n_rows ? r : n_rows - 1) * lda + lc;
+    }
+#pragma unroll
+  for (int i = 0; i < LW; ++i) {
+    const int r = col0 + (wave + 8 * i) * 8 + lr;
+    wp[i] = w + (long)(r < n_out ? r : n_out - 1) * k_dim + lc;
+  }
+  auto issue_a = [&](int step, int st, int p) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      __builtin_amdgcn_global_load_lds((global_ptr_t)(ap[p][h] + step * MM_BK),
+                                       (lds_ptr_t)(as_base + st * (BM * MM_LD) + (PARTS * 8 * h + 8 * p + wave) * (8 * MM_LD)),
+                                       16, 0, 0);
+  };
+  auto issue_w = [&](int step, int st) {
+#pragma unroll
+    for (int i = 0; i < LW; ++i)
+      __builtin_amdgcn_global_load_lds((global_ptr_t)(wp[i] + step * MM_BK),
+                                       (lds_ptr_t)(ws_base + st * (BN * MM_LD) + (wave + 8 * i) * (8 * MM_LD)), 16, 0, 0);
+  };
+
+  f32x4_t acc[WTN][WTM];
+#pragma unroll
+  for (int i = 0; i < WTN; ++i)
+#pragma unroll
+    for (int j = 0; j < WTM; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  const int c0 = ((lane >> 4) ^ (lrow & 7)) * 8;
+  bf16x8_t af[2][4], wf[2][WTN];   // [half of the step][row or column tile]
+  auto read_a = [&](int st, int j0) {
+    const bf16_t* p = as_base + st * (BM * MM_LD) + (wr + j0 * 16 + lrow) * MM_LD;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) af[h][j] = *reinterpret_cast<const bf16x8_t*>(p + j * 16 * MM_LD + (c0 ^ (h * 32)));
+  };
+  auto read_w = [&](int st) {
+    const bf16_t* p = ws_base + st * (BN * MM_LD) + (wc + lrow) * MM_LD;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < WTN; ++i) wf[h][i] = *reinterpret_cast<const bf16x8_t*>(p + i * 16 * MM_LD + (c0 ^ (h * 32)));
+  };
+  auto multiply = [&](int j0) {
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < WTN; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          acc[i][j0 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[h][i], af[h][j], acc[i][j0 + j], 0, 0, 0);
+    __builtin_amdgcn_s_setprio(0);
+  };
+  // the end of a slot; what a wave has read has arrived
+  auto slot_end = [&]() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // at most `YOUNGER` of this wave's loads are still on their way; none, towards the end, where fewer have been sent for
+  constexpr int YOUNGER = WTM == 8 ? LW + 4 : LW + 2;
+  auto arrived = [&](bool sent) {
+    if (sent) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(YOUNGER) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  };
+
+#pragma unroll
+  for (int s = 0; s < 2; ++s)
+    if (s < k_steps) {
+      issue_w(s, s);
+      issue_a(s, s, 0);
+      if (WTM == 8 && s == 0) issue_a(0, 0, PARTS - 1);
+    }
+  arrived(k_steps > 1);
+  slot_end();
+  if (half == 1) slot_end();
+  for (int s = 0, st = 0; s < k_steps; ++s) {
+    const bool next = s + 1 < k_steps, more = s + 2 < k_steps;
+    read_w(st);
+    read_a(st, 0);
+    if constexpr (WTM == 8) {
+      if (next) issue_a(s + 1, st ^ 1, 1);
+      if (half == 1) arrived(next);
+      slot_end();
+      multiply(0);
+      if (half == 0) arrived(next);
+      slot_end();
+      read_a(st, 4);
+      if (more) {
+        issue_w(s + 2, st);
+        issue_a(s + 2, st, 0);
+      }
+      if (half == 1) arrived(more);
+      slot_end();
+      multiply(4);
+      if (half == 0) arrived(more);
+      slot_end();
+    } else {
+      if (more) {
+        const int far = st == 0 ? 2 : st - 1;
+        issue_w(s + 2, far);
+        issue_a(s + 2, far, 0);
+      }
+      if (half == 1) arrived(more);
+      slot_end();
+      multiply(0);
+      if (half == 0) arrived(more);
+      slot_end();
+    }
+    st = st + 1 == STAGES ? 0 : st + 1;
+  }
+  if (half == 0) slot_end();   // as many barriers as the other half
+  mfma_epilogue<WTM, WTN, WVM, WVN, T, STAGES * (BM + BN) * MM_LD, EPI, OT>(acc, lds, bias, out, ldo, n_rows, n_out, row0,
+                                                                            col0, wr, wc, sc);
+}
+
+template <int WTM, int WTN, int EPI, typename OT>
+int launch_halves_one(const void* act, long lda, const void* w, const float* bias, void* out, long ldo, int n_rows, int n_out,
+                      int k_dim, const MfmaScatter& sc, hipStream_t stream) {
+  constexpr int BM = 32 * WTM, BN = 64 * WTN;
+  constexpr size_t lds_bytes = (WTM == 8 ? 2ul : 3ul) * (BM + BN) * MM_LD * sizeof(bf16_t);
+  auto kernel = linear_mfma_halves_kernel<WTM, WTN, EPI, OT>;
+  static bool allowed = false;
+  if (!allowed) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
+    if (e != hipSuccess) return (int)e;
+    allowed = true;
+  }
+  const long tiles = (long)((n_rows + BM - 1) / BM) * ((n_out + BN - 1) / BN);
+  if (tiles > 0x7fffffffL) return MGPT_ERR_TOO_LARGE;
+  hipLaunchKernelGGL(kernel, dim3((unsigned int)tiles), dim3(512), lds_bytes, stream, (const bf16_t*)act, lda, (const bf16_t*)w,
+                     bias, (OT*)out, ldo, n_rows, n_out, k_dim, sc);
+  return mgpt_last_error();
+}
+
+template <int WTM, int WTN>
+int launch_halves(const void* act, long lda, const void* w, const float* bias, void* out, int out_dtype, long ldo, int n_rows,
+                  int n_out, int k_dim, int epilogue, const MfmaScatter& sc, hipStream_t stream) {
+#define MM_LAUNCH(E, OT) return launch_halves_one<WTM, WTN, E, OT>(act, lda, w, bias, out, ldo, n_rows, n_out, k_dim, sc, stream)
+  if (epilogue == MM_EPI_NONE && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_NONE, bf16_t);
+  if (epilogue == MM_EPI_NONE && out_dtype == MGPT_F32) MM_LAUNCH(MM_EPI_NONE, float);
+  if (epilogue == MM_EPI_GELU && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_GELU, bf16_t);
+  if (epilogue == MM_EPI_RELU2 && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_RELU2, bf16_t);
+  if (epilogue == MM_EPI_XIELU && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_XIELU, bf16_t);
+  if (epilogue == MM_EPI_RESIDUAL && out_dtype == MGPT_F32) MM_LAUNCH(MM_EPI_RESIDUAL, float);
+  if (epilogue == MM_EPI_QKV && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_QKV, bf16_t);
+#undef MM_LAUNCH
+  return MGPT_ERR_BAD_DTYPE;
+}
 template <int WTM, int WTN, int WVM, int WVN, int EPI, typename OT, int AHEAD, int KG = 1, int DIRECT = 0>
 int launch_one(const void* act, long lda, const void* w, const float* bias, void* out, long ldo, int n_rows,
                int n_out, int k_dim, int k_parts, long part_stride, const MfmaScatter& sc, hipStream_t stream) {
@@ -606,11 +832,14 @@ constexpr int MM_MAX_PARTS = 8;
 constexpr int MM_AHEAD = 4;  // steps on their way from memory in the variant for few tiles over a large matrix
 // Shape ids from MM_DIRECT_FIRST on: the variants whose slices go from memory straight into LDS, by tile
 // (rows x columns), waves and stages: 32 x 32 (four waves of 16 x 16) and 64 x 64 (four of 32 x 32) with four
-// stages, 128 x 64 (eight of 32 x 32) with three, 128 x 192 (eight of 64 x 48) with two, 32 x 32 with six.
+// stages, 128 x 64 (eight of 32 x 32) with three, 128 x 192 (eight of 64 x 48) with two, 32 x 32 with six; then the
+// variants with the halves out of step.
 constexpr int MM_DIRECT_FIRST = MM_SHAPES + 3;
-constexpr int MM_DIRECT_VARIANTS = 5;
-constexpr int MM_DIRECT_ROWS[MM_DIRECT_VARIANTS] = {32, 64, 128, 128, 32};
-constexpr int MM_DIRECT_COLS[MM_DIRECT_VARIANTS] = {32, 64, 64, 192, 32};
+constexpr int MM_DIRECT_VARIANTS = 9;
+constexpr int MM_DIRECT_ROWS[MM_DIRECT_VARIANTS] = {32, 64, 128, 128, 32, 256, 128, 256, 128};
+constexpr int MM_DIRECT_COLS[MM_DIRECT_VARIANTS] = {32, 64, 64, 192, 32, 256, 256, 192, 192};
+constexpr int MM_DIRECT_HALVES = 5;     // the first of the four variants with the halves out of step: 256 x 256, 128 x 256,
+                                        // 256 x 192, 128 x 192
 constexpr int MM_SHAPE_IDS = MM_DIRECT_FIRST + MM_DIRECT_VARIANTS;
 
 long tiles_of(int shape, int n_rows, int n_out) {
@@ -770,8 +999,13 @@ long direct_tiles(int variant, int n_rows, int n_out) {
 //   tokens: width 512 -3 %, width 768 -1 to -10 %, width 1600 at 2,048 tokens -7 %.
 // - a wide output under many rows: tiles of 128 x 192 where a round of them costs less than a round of
 //   256 x 256 (qkv and first feed-forward product at 8,192 tokens, widths 512 to 1600: -2 to -5 % of the step).
+// - many rows (512 and more) under an inner size of 12 steps and more: the variant that takes least by a model of rounds of
+//   workgroups (choose_large below).
+int choose_large(int n_rows, int n_out, int k_dim);
 int choose_direct(int n_rows, int n_out, int k_dim) {
   if (n_rows < 128 || (k_dim % MM_BK) != 0) return -1;
+  const int large = choose_large(n_rows, n_out, k_dim);
+  if (large >= 0) return large;
   if (k_dim / MM_BK >= 32) {
     const long t128 = direct_tiles(2, n_rows, n_out), t64 = direct_tiles(1, n_rows, n_out);
     if (t128 > 520) return -1;
@@ -786,6 +1020,35 @@ int choose_direct(int n_rows, int n_out, int k_dim) {
   const double cost_largest = (double)((largest + 255) / 256) * 256 * 256 * 0.72;
   if (largest >= 160 && cost_largest <= cost_wide) return -1;
   return MM_DIRECT_FIRST + 3;
+}
+
+// Of the large variants the one that takes least: rounds of as many workgroups as the chip holds, each (steps x us a step + us
+// for filling, the epilogue and the start).  The numbers are fits, within 15 %, to 23 products of 1,500 to 12,000 rows, inner
+// sizes 768 to 6,400 and 768 to 10,880 columns (alone in a graph, four sets of operands in turn; bfloat16 out, or added to
+// float32 rows, which costs up to 15 us more whatever the tile, the rows being read and written).  Two workgroups of the
+// variants with less LDS share a compute unit, and each is faster where it has one to itself.  With them, before / now, us:
+// 4,096 rows 1600 -> 4800 72 / 68, 1600 -> 6400 90 / 83, 1600 -> 1600 40 / 35, 6400 -> 1600 110 / 98; 3,300 rows 2048 -> 10880
+// 150 / 135; 1,500 rows 1600 -> 6400 40 / 34; 12,000 rows 3072 -> 768 105 / 74.  At full occupancy (4,096 rows 6400 -> 4096) the
+// 256 x 256 tile reaches 1,340 TFLOP/s, the register path's 1,180; the clock is down to 1.95 GHz there, the matrix units are
+// busy 65 % of the cycles.
+int choose_large(int n_rows, int n_out, int k_dim) {
+  const int steps = k_dim / MM_BK;
+  if (n_rows < 512 || n_out < 512 || steps < 12) return -1;
+  struct Cost { int variant, per_unit; double step, fixed, step_alone; };
+  const Cost costs[] = {{MM_DIRECT_HALVES, 1, 1.2, 9.0, 1.2},      {MM_DIRECT_HALVES + 1, 1, 0.8, 6.0, 0.8},
+                        {MM_DIRECT_HALVES + 2, 1, 1.03, 8.0, 1.03}, {MM_DIRECT_HALVES + 3, 1, 0.67, 6.0, 0.67},
+                        {3, 2, 1.3, 4.0, 0.75},                     {2, 2, 0.6, 4.0, 0.4}};
+  int best = -1;
+  double least = 0.0;
+  for (const Cost& c : costs) {
+    const long tiles = direct_tiles(c.variant, n_rows, n_out), at_once = 256L * c.per_unit;
+    if (tiles < 140) continue;   // (smaller tiles, or a split, use more of the chip)
+    const long rest = tiles % at_once;
+    double t = (double)(tiles / at_once) * (steps * c.step + c.fixed);
+    if (rest > 0) t += steps * (rest <= 256 ? c.step_alone : c.step) + c.fixed;
+    if (best < 0 || t < least) best = c.variant, least = t;
+  }
+  return best < 0 ? -1 : MM_DIRECT_FIRST + best;
 }
 
 // shape < 0: chosen by the size.  k_parts: 0 = chosen by the size, together with the shape, if
@@ -810,6 +1073,7 @@ int launch_any(int shape, int k_parts, const void* act, long lda, const void* w,
   if (shape >= MM_DIRECT_FIRST) {
     if (shape >= MM_SHAPE_IDS || !direct_ok(act, w, k_dim)) return MGPT_ERR_BAD_SHAPE;
     direct = shape - MM_DIRECT_FIRST;
+    if (direct >= MM_DIRECT_HALVES && k_parts > 1) return MGPT_ERR_BAD_SHAPE;   // (these are not split)
     shape = 3;   // (the rules below for the other variants do not apply)
     ahead = 1;
   } else if (shape == MM_SHAPES + 2) {
@@ -891,6 +1155,12 @@ int launch_any(int shape, int k_parts, const void* act, long lda, const void* w,
       case 2: rc = launch_shape<2, 2, 4, 2, 1, 3>(MM_ARGS); break;
       case 3: rc = launch_shape<4, 3, 2, 4, 1, 2>(MM_ARGS); break;
       case 4: rc = launch_shape<1, 1, 2, 2, 1, 6>(MM_ARGS); break;
+      case 5: rc = launch_halves<8, 4>(act, lda, w, b, dst, dt, ld, n_rows, n_out, k_dim, epi, sc, stream); break;
+#define MM_HALVES_ARGS act, lda, w, b, dst, dt, ld, n_rows, n_out, k_dim, epi, sc, stream
+      case 6: rc = launch_halves<4, 4>(MM_HALVES_ARGS); break;
+      case 7: rc = launch_halves<8, 3>(MM_HALVES_ARGS); break;
+      case 8: rc = launch_halves<4, 3>(MM_HALVES_ARGS); break;
+#undef MM_HALVES_ARGS
       default: break;
     }
   } else
@@ -967,7 +1237,8 @@ extern "C" int mgpt_linear_mfma_xielu(const void* act, long lda, const void* w, 
 // 3 = 64 x 64, 4 = 32 x 32, 5 and 6 = 64 x 64 and 32 x 32 with four steps on their way from memory,
 // 7 = 64 x 64 with two wave groups a tile (float32 outputs), 8 to 12 = the slices straight into LDS: 32 x 32 and
 // 64 x 64 with four stages, 128 x 64 with three, 128 x 192 with two, 32 x 32 with six (an inner size of whole steps of 64 and operands
-// aligned to 16 bytes, else refused); negative: chosen) and the number of stretches of the inner size given
+// aligned to 16 bytes, else refused), 13 to 16 = the halves out of step, 256 x 256, 128 x 256, 256 x 192, 128 x 192 (the same
+// conditions, and never split); negative: chosen) and the number of stretches of the inner size given
 // (k_parts as for launch_any above), instead of chosen by the size: for tests and measurements.
 extern "C" int mgpt_linear_mfma_shape(int shape, int k_parts, const void* act, long lda, const void* w,
                                       const float* bias, void* out, int out_dtype, long ldo, int n_rows,

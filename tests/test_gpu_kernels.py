@@ -375,6 +375,44 @@ def test_linear_mfma_slices_straight_into_lds(n, k, o, epi, o_dt, shape):
     assert torch.equal(out[n:], prev[n:].to(DEV)), "rows beyond n_rows were written"
 
 
+@pytest.mark.parametrize("n,k,o", [(1, 64, 16), (300, 64, 257), (513, 512, 520), (256, 128, 384), (1000, 192, 130), (130, 256, 400),
+                                   (257, 320, 193)])
+@pytest.mark.parametrize("epi,o_dt", [(kernels.EPI_NONE, "bfloat16"), (kernels.EPI_NONE, "float32"),
+                                      (kernels.EPI_GELU, "bfloat16"), (kernels.EPI_RESIDUAL, "float32")])
+@pytest.mark.parametrize("shape", [13, 14, 15, 16])
+def test_linear_mfma_with_its_halves_out_of_step(n, k, o, epi, o_dt, shape):
+    """The variants whose two halves read and multiply in turn (256 x 256, 128 x 256, 256 x 192 and 128 x 192), at sizes that cut
+    their tiles and at 1, 2, 3, 4, 5 and 8 steps: the sums of an element run over k in the order of the other variants, so the
+    results are those of the 32 x 32 tiles bit by bit."""
+    g = torch.Generator().manual_seed(n)
+    a, w, bias = rnd(g, n, k, dtype="bfloat16"), rnd(g, o, k, dtype="bfloat16", scale=k ** -0.5), rnd(g, o)
+    prev = rnd(g, n + 2, o, dtype=o_dt)
+    out, small = prev.clone().to(DEV), prev.clone().to(DEV)
+    assert kernels.linear_mfma(a.to(DEV), w.to(DEV), bias.to(DEV), out, n, epi, shape=shape)
+    assert kernels.linear_mfma(a.to(DEV), w.to(DEV), bias.to(DEV), small, n, epi, shape=8)
+    helpers.assert_close(out[:n], _linear_want(a, w, bias, epi, prev[:n]), "bfloat16", f"shape {shape} {n}x{k}x{o}")
+    assert torch.equal(out, small)
+
+
+@pytest.mark.parametrize("n,k,o,shape", [(1500, 1600, 4800, 14), (1500, 1600, 6400, 15), (4096, 1600, 1600, 14),
+                                         (6000, 768, 2304, 13), (2000, 768, 2304, 11), (2000, 3072, 768, 10)])
+def test_linear_mfma_of_many_rows_keeps_its_sums_whatever_the_tile(n, k, o, shape):
+    """What the model of rounds chooses among the large variants: the result equals the forced variant's bit by bit."""
+    g = torch.Generator().manual_seed(o)
+    a, w, bias = rnd(g, n, k, dtype="bfloat16").to(DEV), rnd(g, o, k, dtype="bfloat16", scale=k ** -0.5).to(DEV), rnd(g, o).to(DEV)
+    out, forced = (torch.empty(n, o, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    assert kernels.linear_mfma(a, w, bias, out, n, kernels.EPI_NONE)
+    assert kernels.linear_mfma(a, w, bias, forced, n, kernels.EPI_NONE, shape=shape)
+    assert torch.equal(out, forced)
+    want = a.float() @ w.float().T + bias
+    assert ((out.float() - want).norm() / want.norm()).item() < 4e-3      # rounding to bfloat16: 2 ** -9 of each value at most
+
+
+@pytest.mark.parametrize("n,shape,k", [(300, 13, 64), (130, 14, 192), (520, 15, 128), (257, 16, 256)])
+def test_linear_mfma_halves_store_keys_and_values(n, shape, k):
+    test_linear_mfma_stores_keys_and_values(n, shape, k)
+
+
 def test_linear_mfma_straight_into_lds_wants_whole_steps():
     """An inner size that is no multiple of 64 is refused by those variants (nothing can be zeroed on its way
     into LDS), and the library's own choice then goes through registers."""

@@ -63,13 +63,19 @@ __device__ __forceinline__ ex_f4 ex_load(const float* __restrict__ row, int k, i
 // through two buffers of LDS, rows of 128 bytes whose 16-byte pieces are XORed with the row's low bits.  The matrix
 // cores' float32 rate (a sixteenth of bfloat16's) is what bounds it, with T = 4 from about 256 tiles on.
 #define EX_BK 32
-template <int T, int EPI, bool VEC>
+//
+// STAGES > 0: the slices go from memory straight into LDS (global_load_lds_dwordx4: a wave's load brings 8 rows of 128 bytes,
+// the lane that fills piece p of row r fetching piece p ^ (r & 7)), STAGES - 1 steps on their way, for inner sizes of whole
+// steps: through registers one step is on its way, and a workgroup that is alone on its compute unit waits for memory every step.  Before / now, us: 1,201
+// rows 2048 -> 512 54.6 / 46.4, 512 -> 50304 588 / 562; 2,000 rows 768 -> 768 34.3 / 31.8, 3072 -> 768 121.7 / 108.4; 600 rows
+// 5120 -> 1280 128.8 / 108.3; 5,000 rows 1600 -> 6400 847 / 819 (125 TFLOP/s).  Eight waves a tile instead of four: the same.
+template <int T, int EPI, bool VEC, int STAGES>
 __global__ __launch_bounds__(256) void linear_exact_tile_kernel(
     const float* __restrict__ A, long lda, const float* __restrict__ W, const float* __restrict__ bias,
     float* __restrict__ out, long ldo, int n_rows, int n_out, int k_dim, int row_tiles, int vec_out, ExactScatter sc) {
   constexpr int B = 32 * T;                          // rows and columns of the tile
   constexpr int PIECES = B * EX_BK / 4 / 256;        // 16-byte pieces of one operand's slice that a thread stages
-  extern __shared__ __align__(16) float ex_lds[];    // [2][2 B][EX_BK]: rows of activations, then of W
+  extern __shared__ __align__(16) float ex_lds[];    // [buffers][2 B][EX_BK]: rows of activations, then of W
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int row0 = (int)(blockIdx.x % row_tiles) * B, col0 = (int)(blockIdx.x / row_tiles) * B;
@@ -88,7 +94,7 @@ __global__ __launch_bounds__(256) void linear_exact_tile_kernel(
     wp[p] = W + (long)(c < n_out ? c : n_out - 1) * k_dim;
   }
   const int s_lds = srow * EX_BK + ((sp ^ (srow & 7)) << 2);
-  ex_f4 ga[PIECES], gw[PIECES];
+  [[maybe_unused]] ex_f4 ga[PIECES], gw[PIECES];
   auto load = [&](int k0) {
 #pragma unroll
     for (int p = 0; p < PIECES; ++p) {
@@ -111,12 +117,8 @@ __global__ __launch_bounds__(256) void linear_exact_tile_kernel(
 #pragma unroll
     for (int j = 0; j < T; ++j) acc[i][j] = sum[i][j] = (ex_f4){0.f, 0.f, 0.f, 0.f};
 
-  load(0);
-  store(0);
-  __syncthreads();
-  for (int k0 = 0, buf = 0; k0 < k_dim; k0 += EX_BK, buf ^= 1) {
-    const bool more = k0 + EX_BK < k_dim;
-    if (more) load(k0 + EX_BK);
+  // the step at k0, whose slices lie in buffer buf
+  auto multiply = [&](int k0, int buf) {
     const float* as = ex_lds + buf * (2 * B * EX_BK) + (wr + l16) * EX_BK;
     const float* ws = ex_lds + buf * (2 * B * EX_BK) + (B + wc + l16) * EX_BK;
 #pragma unroll
@@ -136,7 +138,7 @@ __global__ __launch_bounds__(256) void linear_exact_tile_kernel(
           for (int j = 0; j < T; ++j)
             acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[i][e], af[j][e], acc[i][j], 0, 0, 0);
     }
-    if (((k0 + EX_BK) & (EX_BLOCK - 1)) == 0 || !more) {
+    if (((k0 + EX_BK) & (EX_BLOCK - 1)) == 0 || k0 + EX_BK >= k_dim) {
 #pragma unroll
       for (int i = 0; i < T; ++i)
 #pragma unroll
@@ -145,8 +147,51 @@ __global__ __launch_bounds__(256) void linear_exact_tile_kernel(
           acc[i][j] = (ex_f4){0.f, 0.f, 0.f, 0.f};
         }
     }
-    if (more) store(buf ^ 1);
+  };
+  if constexpr (STAGES > 0) {
+    constexpr int LOADS = 2 * B / 8 / 4;             // of a wave and step: 8 rows each, the activations' first
+    constexpr int D = STAGES - 1;
+    typedef __attribute__((address_space(1))) const void* global_ptr_t;
+    typedef __attribute__((address_space(3))) void* lds_ptr_t;
+    const int lr = lane >> 3, lc = ((lane & 7) ^ lr) << 2;
+    const float* dp[LOADS];
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      const int r = (wave + 4 * i) * 8 + lr;
+      if (i < LOADS / 2) dp[i] = A + (long)(row0 + r < n_rows ? row0 + r : n_rows - 1) * lda + lc;
+      else dp[i] = W + (long)(col0 + r - B < n_out ? col0 + r - B : n_out - 1) * k_dim + lc;
+    }
+    auto issue = [&](int k0, int buf) {
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i)
+        __builtin_amdgcn_global_load_lds((global_ptr_t)(dp[i] + k0),
+                                         (lds_ptr_t)(ex_lds + buf * (2 * B * EX_BK) + (wave + 4 * i) * (8 * EX_BK)), 16, 0, 0);
+    };
+    const int steps = k_dim / EX_BK;
+#pragma unroll
+    for (int j = 0; j < D; ++j)
+      if (j < steps) issue(j * EX_BK, j);
+    for (int s = 0, buf = 0; s < steps; ++s) {
+      // this wave's loads of step s have arrived (D - 1 younger steps may be on their way), then everybody's; nobody reads
+      // the buffer of step s - 1 any more, which is where step s + D goes
+      if (s + D <= steps) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((D - 1) * LOADS) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      if (s + D < steps) issue((s + D) * EX_BK, buf == 0 ? STAGES - 1 : buf - 1);
+      multiply(s * EX_BK, buf);
+      buf = buf + 1 == STAGES ? 0 : buf + 1;
+    }
+  } else {
+    load(0);
+    store(0);
     __syncthreads();
+    for (int k0 = 0, buf = 0; k0 < k_dim; k0 += EX_BK, buf ^= 1) {
+      const bool more = k0 + EX_BK < k_dim;
+      if (more) load(k0 + EX_BK);
+      multiply(k0, buf);
+      if (more) store(buf ^ 1);
+      __syncthreads();
+    }
   }
 
   // a lane has four consecutive columns of a row
@@ -323,9 +368,9 @@ struct ExactArgs {
   ExactScatter sc;
 };
 
-template <int T, int EPI, bool VEC>
+template <int T, int EPI, bool VEC, int STAGES>
 static int launch_tile(const ExactArgs& a, hipStream_t stream) {
-  constexpr int B = 32 * T, bytes = 2 * 2 * B * EX_BK * (int)sizeof(float);
+  constexpr int B = 32 * T, bytes = (STAGES > 0 ? STAGES : 2) * 2 * B * EX_BK * (int)sizeof(float);
   static_assert(bytes <= 64 * 1024, "what a kernel gets without asking");
   const int row_tiles = (a.n_rows + B - 1) / B, col_tiles = (a.n_out + B - 1) / B;
   if ((long)row_tiles * col_tiles > 0x7fffffffL) return MGPT_ERR_TOO_LARGE;
@@ -333,7 +378,7 @@ static int launch_tile(const ExactArgs& a, hipStream_t stream) {
   if (EPI == EPI_QKV) stored |= reinterpret_cast<uintptr_t>(a.sc.kpool) | reinterpret_cast<uintptr_t>(a.sc.vpool);
   const int vec_out = a.ldo % 4 == 0 && (stored & 15) == 0 &&
                       (EPI != EPI_QKV || (a.sc.q_width % 4 == 0 && a.sc.head_dim % 4 == 0));
-  hipLaunchKernelGGL((linear_exact_tile_kernel<T, EPI, VEC>), dim3(row_tiles * col_tiles), dim3(256), bytes, stream, a.A, a.lda,
+  hipLaunchKernelGGL((linear_exact_tile_kernel<T, EPI, VEC, STAGES>), dim3(row_tiles * col_tiles), dim3(256), bytes, stream, a.A, a.lda,
                      a.W, a.bias, a.out, a.ldo, a.n_rows, a.n_out, a.k_dim, row_tiles, vec_out,
                      a.sc);
   return mgpt_last_error();
@@ -374,10 +419,34 @@ extern "C" int mgpt_linear_exact_kernel(int n_rows, int n_out, int k_dim) {
   return t64 <= t128 ? EX_TILE64 : EX_TILE128;
 }
 
+// Whether tiles of 32 x 32 take the place of the kernel above (inner sizes of whole steps, aligned operands): several of their
+// workgroups share a compute unit, so few tiles spread over the chip evenly.  us a k with one, two, three and n of them on a
+// compute unit 0.010, 0.014, 0.019, 0.0065 n; the rows kernel at 29 TFLOP/s.  Rows kernel or 64 x 64 tiles / here, us: 100 rows
+// 768 -> 2304 15.7 / 13.8; 300 rows 768 -> 768 15.7 / 10.5, 3072 -> 768 51.9 / 33.6; 600 rows 512 -> 512 13.9 / 9.9, 5120 -> 1280
+// 107 / 97; 1,201 rows 2048 -> 512 45.3 / 40.8; 400 rows 512 -> 2048 14.8 / 17.6 (not taken).
+extern "C" int mgpt_linear_exact_small_tiles(int n_rows, int n_out, int k_dim) {
+  if (k_dim % EX_BK != 0) return 0;
+  const double k = k_dim, rows = 2.0 * n_rows * n_out * k / 29e6;
+  auto per_unit = [&](int b) {
+    const long tiles = (long)((n_rows + b - 1) / b) * ((n_out + b - 1) / b);
+    return (double)((tiles + 255) / 256);
+  };
+  const double r64 = per_unit(64), t64 = r64 > 1 ? r64 * 0.019 * k : 0.0225 * k, t128 = per_unit(128) * 0.068 * k;
+  const double n32 = per_unit(32), t32 = k * (n32 <= 1 ? 0.010 : n32 <= 2 ? 0.014 : n32 <= 3 ? 0.019 : 0.0065 * n32);
+  return t32 < rows && t32 < t64 && t32 < t128;
+}
+
 template <int EPI, bool VEC>
 static int launch_kernel(const ExactArgs& a, int kernel, hipStream_t stream) {
+  if constexpr (VEC) {
+    if (a.k_dim % EX_BK == 0) {                      // slices straight into LDS
+      if (mgpt_linear_exact_small_tiles(a.n_rows, a.n_out, a.k_dim)) return launch_tile<1, EPI, true, 6>(a, stream);
+      if (kernel == EX_TILE64) return launch_tile<2, EPI, true, 4>(a, stream);
+      if (kernel == EX_TILE128) return launch_tile<4, EPI, true, 2>(a, stream);
+    }
+  }
   if (kernel == EX_ROWS) return launch_rows<EPI, VEC>(a, stream);
-  return kernel == EX_TILE64 ? launch_tile<2, EPI, VEC>(a, stream) : launch_tile<4, EPI, VEC>(a, stream);
+  return kernel == EX_TILE64 ? launch_tile<2, EPI, VEC, 0>(a, stream) : launch_tile<4, EPI, VEC, 0>(a, stream);
 }
 
 int mgpt_linear_exact_launch(const float* A, long lda, const float* W, const float* bias, float* out, long ldo, int n_rows,

@@ -160,8 +160,14 @@ def linear_generic(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor
 
 
 def linear_exact_kernel(n_rows: int, n_out: int, k_dim: int) -> str:
-    """Which of its kernels a float32 product of this size goes to: "rows", "tile64" or "tile128"."""
+    """Which of its kernels a float32 product of this size goes to: "rows", "tile64" or "tile128" (or, in the place of any,
+    32 x 32 tiles: linear_exact_small_tiles)."""
     return ("rows", "tile64", "tile128")[library.kernels().mgpt_linear_exact_kernel(n_rows, n_out, k_dim)]
+
+
+def linear_exact_small_tiles(n_rows: int, n_out: int, k_dim: int) -> bool:
+    """Whether a float32 product of this size with aligned operands goes to tiles of 32 x 32."""
+    return bool(library.kernels().mgpt_linear_exact_small_tiles(n_rows, n_out, k_dim))
 
 
 EXACT_BLOCK = 256       # k whose sum is one part of a float32 product

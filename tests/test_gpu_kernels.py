@@ -176,6 +176,22 @@ def test_float32_product_keeps_its_sums_whatever_the_tiles(k):
     assert used == {"rows", "tile64", "tile128"}
 
 
+@pytest.mark.parametrize("epi", [kernels.EPI_NONE, kernels.EPI_GELU, kernels.EPI_RESIDUAL])
+@pytest.mark.parametrize("n,k,o,small", [(300, 768, 768, True), (97, 768, 2303, True), (129, 32, 1500, True), (600, 512, 515, True),
+                                         (1201, 2048, 512, True), (255, 96, 1024, True), (1030, 64, 1500, False),
+                                         (1030, 160, 3501, False)])
+def test_float32_product_straight_into_lds(n, k, o, small, epi):
+    """Slices that go straight into LDS (inner sizes of whole steps), in tiles of 32 x 32, 64 x 64 and 128 x 128 and at fewer
+    steps than stages, as many and more: the bits of the same product over rows that are not aligned for that."""
+    g = torch.Generator().manual_seed(n + k)
+    assert kernels.linear_exact_small_tiles(n, o, k) == small
+    a, w, bias, old = rnd(g, n, k + 1).to(DEV)[:, :k], rnd(g, o, k).to(DEV), rnd(g, o).to(DEV), rnd(g, n + 1, o).to(DEV)
+    want, got = old.clone(), old.clone()
+    kernels.linear_generic(a, w, bias, want, n, epi)
+    kernels.linear_generic(a.contiguous(), w, bias, got, n, epi)
+    assert torch.equal(got, want) and torch.equal(got[n], old[n])
+
+
 @pytest.mark.parametrize("epi", [kernels.EPI_GELU, kernels.EPI_RESIDUAL, kernels.EPI_RELU2])
 @pytest.mark.parametrize("k,o", [(64, 3500), (300, 3501), (37, 3499)])
 def test_float32_product_epilogues_whatever_the_tiles(k, o, epi):

@@ -1107,9 +1107,17 @@ int launch_any(int shape, int k_parts, const void* act, long lda, const void* w,
     // registers, so there can be more of them (six stages while a compute unit has one such workgroup, four
     // with more).  Decode steps of 12 layers of width 1600, in turns with the variant above on one box: 24 rows
     // 0.774 -> 0.740 ms, 32 rows 0.795 -> 0.762, 64 rows 1.000 -> 0.949 (with six stages there 0.970).
+    // Under fewer than 20 steps four stages are enough (310 rows 768 -> 768 with the LayerNorm behind it: 8.1 us with six, 7.7).
     if (ahead == MM_AHEAD && direct_ok(act, w, k_dim)) {
-      direct = tiles_of(4, n_rows, n_out) * k_parts <= 256 ? 4 : 0;
+      direct = tiles_of(4, n_rows, n_out) * k_parts <= 256 && steps >= 20 ? 4 : 0;
       ahead = 1;
+    }
+    // Prompt portions of a few hundred rows under an inner size of 20 steps and more: 64 x 64 tiles with four stages from 160
+    // tiles on (400 rows 1600 -> 1600: 32 x 32 tiles through registers 17.2 us, here 15.3; 520 rows, 64 x 64 tiles through registers
+    // 18.0, here 15.8; 310 rows, 125 tiles: 13.3 and 15.1).
+    if (direct < 0 && n_rows >= 128 && k_parts == 1 && steps >= 20 && (shape == 3 || shape == 4) && direct_ok(act, w, k_dim)) {
+      const long t64 = tiles_of(3, n_rows, n_out);
+      if (t64 >= 160 && t64 <= 256) direct = 1, ahead = 1;
     }
   }
   if (k_parts > 1) {

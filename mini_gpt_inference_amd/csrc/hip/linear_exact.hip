@@ -409,6 +409,7 @@ enum { EX_ROWS, EX_TILE64, EX_TILE128 };
 // The 64 x 64 FMA tiles that these kernels replace reached 10 to 15 TFLOP/s (1,100 rows 2048 -> 512: 163 us, here 54), the
 // FMA kernel for few rows took 57 us for 16 rows 3072 -> 768 (here 14).
 extern "C" int mgpt_linear_exact_kernel(int n_rows, int n_out, int k_dim) {
+  if ((long)n_rows * n_out <= 380000) return EX_ROWS;   // less than one round of either tile (and no divisions on the host)
   const double k = k_dim, rows = 2.0 * n_rows * n_out * k / 34e6;
   auto rounds = [&](int b) {
     const long tiles = (long)((n_rows + b - 1) / b) * ((n_out + b - 1) / b);
@@ -425,7 +426,7 @@ extern "C" int mgpt_linear_exact_kernel(int n_rows, int n_out, int k_dim) {
 // 768 -> 2304 15.7 / 13.8; 300 rows 768 -> 768 15.7 / 10.5, 3072 -> 768 51.9 / 33.6; 600 rows 512 -> 512 13.9 / 9.9, 5120 -> 1280
 // 107 / 97; 1,201 rows 2048 -> 512 45.3 / 40.8; 400 rows 512 -> 2048 14.8 / 17.6 (not taken).
 extern "C" int mgpt_linear_exact_small_tiles(int n_rows, int n_out, int k_dim) {
-  if (k_dim % EX_BK != 0) return 0;
+  if (k_dim % EX_BK != 0 || (long)n_rows * n_out <= 145000) return 0;   // the rows kernel takes less than one round of these
   const double k = k_dim, rows = 2.0 * n_rows * n_out * k / 29e6;
   auto per_unit = [&](int b) {
     const long tiles = (long)((n_rows + b - 1) / b) * ((n_out + b - 1) / b);

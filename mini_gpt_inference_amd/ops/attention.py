@@ -101,4 +101,5 @@ def paged_attention(ctx, q: torch.Tensor, out: torch.Tensor, k_pool: torch.Tenso
             return
     kernels.paged_attention_generic(q, out, k_pool, v_pool, group.block_tables, ctx.cu_q, ctx.seq_lens,
                                     ctx.q_req, n, r, n_head, scale, window, fast_exp=not ctx.exact, sinks=sinks,
-                                    softcap=softcap, gate=gate, single=ctx.decode_only and n == r, **mask)
+                                    softcap=softcap, gate=gate, single=ctx.decode_only and ctx.n_tokens == ctx.n_req,
+                                    **mask)

@@ -257,6 +257,19 @@ __device__ __forceinline__ void mfma_epilogue(f32x4_t (&acc)[WTN][WTM], bf16_t* 
   }
 }
 
+// The second chain of sums, if there is one, onto the first.
+template <int CHAINS, int WTN, int WTM>
+__device__ __forceinline__ void mfma_join_chains(f32x4_t (&chain)[CHAINS][WTN][WTM]) {
+  if constexpr (CHAINS == 2) {
+#pragma unroll
+    for (int i = 0; i < WTN; ++i)
+#pragma unroll
+      for (int j = 0; j < WTM; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) chain[0][i][j][e] += chain[1][i][j][e];
+  }
+}
+
 // WTM x WTN: 16-wide tiles per wave along the rows of the activations and along the rows of W;
 // WVM x WVN: waves in a workgroup along the same.
 // AHEAD: steps whose chunks are on their way from memory beyond the one that is being put into LDS
@@ -271,13 +284,16 @@ __device__ __forceinline__ void mfma_epilogue(f32x4_t (&acc)[WTN][WTM], bf16_t* 
 // step (float32 outputs only: the epilogue that stores them has no barrier, so group 1 is done then).
 // For few tiles of 64 x 64 under a long inner size: a compute unit that has one such tile has four
 // waves, too few to cover each other's waits for LDS and the barrier.
-template <int WTM, int WTN, int WVM, int WVN, int EPI, typename OT, int AHEAD = 1, int KG = 1, int DIRECT = 0>
+// CHAINS: 2 = an element's sum is two chains, over the first and over the second halves of the steps, added at the end: what two
+// wave groups make (the same bits), with the accumulators of both in one wave.
+template <int WTM, int WTN, int WVM, int WVN, int EPI, typename OT, int AHEAD = 1, int KG = 1, int DIRECT = 0, int CHAINS = 1>
 __global__ __launch_bounds__(64 * WVM * WVN * KG) void linear_mfma_kernel(
     const bf16_t* __restrict__ act, long lda, const bf16_t* __restrict__ w,
     const float* __restrict__ bias, OT* __restrict__ out, long ldo, int n_rows, int n_out, int k_dim,
     int k_parts, long part_stride, MfmaScatter sc) {
   static_assert(KG == 1 || (KG == 2 && sizeof(OT) == 4 && AHEAD == 1), "two wave groups: float32 outputs");
   static_assert(DIRECT == 0 || (DIRECT >= 2 && AHEAD == 1 && KG == 1), "slices straight into LDS: two stages or more");
+  static_assert(CHAINS == 1 || (CHAINS == 2 && KG == 1), "two wave groups are two chains already");
   constexpr int T = 64 * WVM * WVN * KG;
   constexpr int STAGES = DIRECT > 0 ? DIRECT : 2;   // slices of a step that LDS holds
   constexpr int HALVES = (MM_BK / 32) / KG;   // halves of a step along k that a wave multiplies
@@ -357,11 +373,14 @@ __global__ __launch_bounds__(64 * WVM * WVN * KG) void linear_mfma_kernel(
     *reinterpret_cast<bf16x8_t*>(dst + s_lds) = step * MM_BK + sk + 8 <= k_len ? gv[set][p] : zero8;
   };
 
-  f32x4_t acc[WTN][WTM];  // [column tile of W][row tile of activations]
+  f32x4_t chain[CHAINS][WTN][WTM];  // [..][column tile of W][row tile of activations]
 #pragma unroll
-  for (int i = 0; i < WTN; ++i)
+  for (int c = 0; c < CHAINS; ++c)
 #pragma unroll
-    for (int j = 0; j < WTM; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < WTN; ++i)
+#pragma unroll
+      for (int j = 0; j < WTM; ++j) chain[c][i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  auto& acc = chain[0];
 
   const int k_steps = (k_len + MM_BK - 1) / MM_BK;
   const int c0 = ((lane >> 4) ^ (lrow & 7)) * 8;  // this lane's chunk of an operand row, first half of a step
@@ -411,8 +430,10 @@ __global__ __launch_bounds__(64 * WVM * WVN * KG) void linear_mfma_kernel(
       // the compiler's scheduler would move each read down to its use again
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int i = 0; i < WTN; ++i)
-        acc[i][g % WTM] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[g / WTM][i], af[g % 3], acc[i][g % WTM], 0, 0, 0);
+      for (int i = 0; i < WTN; ++i) {
+        f32x4_t& sum = chain[g / WTM % CHAINS][i][g % WTM];
+        sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[g / WTM][i], af[g % 3], sum, 0, 0, 0);
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
     if (decltype(store_next)::value) __syncthreads();  // the other buffer's readers finished before the last barrier
@@ -551,6 +572,7 @@ __global__ __launch_bounds__(64 * WVM * WVN * KG) void linear_mfma_kernel(
         for (int e = 0; e < 4; ++e) acc[i][j][e] += t[e];
       }
   }
+  mfma_join_chains(chain);
 
   mfma_epilogue<WTM, WTN, WVM, WVN, T, STAGES * (BM + BN) * MM_LD, EPI, OT>(acc, lds, bias, out, ldo, n_rows, n_out, row0,
                                                                             col0, wr, wc, sc);
@@ -572,12 +594,15 @@ __global__ __launch_bounds__(64 * WVM * WVN * KG) void linear_mfma_kernel(
 // the second phase of step s; the lower rows of step s + 1 in its first phase.  With 128 rows a step is one phase, LDS has
 // three stages, and step s + 2 goes where step s - 1 was.  A wave waits for its own loads at the end of the slot behind which
 // the first half begins to read what they bring; younger loads stay on their way.
-template <int WTM, int WTN, int EPI, typename OT>
+//
+// CHAINS as in the kernel above (two sets of accumulators are too many for 256 rows).
+template <int WTM, int WTN, int EPI, typename OT, int CHAINS = 1>
 __global__ __launch_bounds__(512, 2) void linear_mfma_halves_kernel(const bf16_t* __restrict__ act, long lda,
                                                                  const bf16_t* __restrict__ w, const float* __restrict__ bias,
                                                                  OT* __restrict__ out, long ldo, int n_rows, int n_out, int k_dim,
                                                                  MfmaScatter sc) {
   static_assert((WTM == 4 || WTM == 8) && (WTN == 3 || WTN == 4), "128 or 256 rows, 192 or 256 columns");
+  static_assert(CHAINS == 1 || (CHAINS == 2 && WTM == 4), "accumulators");
   constexpr int WVM = 2, WVN = 4, T = 512;
   constexpr int BM = WVM * WTM * 16, BN = WVN * WTN * 16, STAGES = WTM == 8 ? 2 : 3;
   constexpr int LW = BN / 64;                 // a wave's loads of W's slice: 8 rows each; 2 of 64 (WTM = 8: upper, lower) rows a half
@@ -640,11 +665,13 @@ __global__ __launch_bounds__(512, 2) void linear_mfma_halves_kernel(const bf16_t
                                        (lds_ptr_t)(ws_base + st * (BN * MM_LD) + (wave + 8 * i) * (8 * MM_LD)), 16, 0, 0);
   };
 
-  f32x4_t acc[WTN][WTM];
+  f32x4_t chain[CHAINS][WTN][WTM];
 #pragma unroll
-  for (int i = 0; i < WTN; ++i)
+  for (int c = 0; c < CHAINS; ++c)
 #pragma unroll
-    for (int j = 0; j < WTM; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < WTN; ++i)
+#pragma unroll
+      for (int j = 0; j < WTM; ++j) chain[c][i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
   const int c0 = ((lane >> 4) ^ (lrow & 7)) * 8;
   bf16x8_t af[2][4], wf[2][WTN];   // [half of the step][row or column tile]
   auto read_a = [&](int st, int j0) {
@@ -668,8 +695,10 @@ __global__ __launch_bounds__(512, 2) void linear_mfma_halves_kernel(const bf16_t
 #pragma unroll
       for (int i = 0; i < WTN; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          acc[i][j0 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[h][i], af[h][j], acc[i][j0 + j], 0, 0, 0);
+        for (int j = 0; j < 4; ++j) {
+          f32x4_t& sum = chain[h % CHAINS][i][j0 + j];
+          sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[h][i], af[h][j], sum, 0, 0, 0);
+        }
     __builtin_amdgcn_s_setprio(0);
   };
   // the end of a slot; what a wave has read has arrived
@@ -731,16 +760,17 @@ __global__ __launch_bounds__(512, 2) void linear_mfma_halves_kernel(const bf16_t
     st = st + 1 == STAGES ? 0 : st + 1;
   }
   if (half == 0) slot_end();   // as many barriers as the other half
-  mfma_epilogue<WTM, WTN, WVM, WVN, T, STAGES * (BM + BN) * MM_LD, EPI, OT>(acc, lds, bias, out, ldo, n_rows, n_out, row0,
+  mfma_join_chains(chain);
+  mfma_epilogue<WTM, WTN, WVM, WVN, T, STAGES * (BM + BN) * MM_LD, EPI, OT>(chain[0], lds, bias, out, ldo, n_rows, n_out, row0,
                                                                             col0, wr, wc, sc);
 }
 
-template <int WTM, int WTN, int EPI, typename OT>
+template <int WTM, int WTN, int EPI, typename OT, int CHAINS>
 int launch_halves_one(const void* act, long lda, const void* w, const float* bias, void* out, long ldo, int n_rows, int n_out,
                       int k_dim, const MfmaScatter& sc, hipStream_t stream) {
   constexpr int BM = 32 * WTM, BN = 64 * WTN;
   constexpr size_t lds_bytes = (WTM == 8 ? 2ul : 3ul) * (BM + BN) * MM_LD * sizeof(bf16_t);
-  auto kernel = linear_mfma_halves_kernel<WTM, WTN, EPI, OT>;
+  auto kernel = linear_mfma_halves_kernel<WTM, WTN, EPI, OT, CHAINS>;
   static bool allowed = false;
   if (!allowed) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
@@ -755,28 +785,30 @@ int launch_halves_one(const void* act, long lda, const void* w, const float* bia
   return mgpt_last_error();
 }
 
-template <int WTM, int WTN>
+template <int WTM, int WTN, int CHAINS = 1>
 int launch_halves(const void* act, long lda, const void* w, const float* bias, void* out, int out_dtype, long ldo, int n_rows,
                   int n_out, int k_dim, int epilogue, const MfmaScatter& sc, hipStream_t stream) {
-#define MM_LAUNCH(E, OT) return launch_halves_one<WTM, WTN, E, OT>(act, lda, w, bias, out, ldo, n_rows, n_out, k_dim, sc, stream)
-  if (epilogue == MM_EPI_NONE && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_NONE, bf16_t);
+#define MM_LAUNCH(E, OT) return launch_halves_one<WTM, WTN, E, OT, CHAINS>(act, lda, w, bias, out, ldo, n_rows, n_out, k_dim, sc, stream)
   if (epilogue == MM_EPI_NONE && out_dtype == MGPT_F32) MM_LAUNCH(MM_EPI_NONE, float);
-  if (epilogue == MM_EPI_GELU && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_GELU, bf16_t);
-  if (epilogue == MM_EPI_RELU2 && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_RELU2, bf16_t);
-  if (epilogue == MM_EPI_XIELU && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_XIELU, bf16_t);
   if (epilogue == MM_EPI_RESIDUAL && out_dtype == MGPT_F32) MM_LAUNCH(MM_EPI_RESIDUAL, float);
-  if (epilogue == MM_EPI_QKV && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_QKV, bf16_t);
+  if constexpr (CHAINS == 1) {
+    if (epilogue == MM_EPI_NONE && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_NONE, bf16_t);
+    if (epilogue == MM_EPI_GELU && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_GELU, bf16_t);
+    if (epilogue == MM_EPI_RELU2 && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_RELU2, bf16_t);
+    if (epilogue == MM_EPI_XIELU && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_XIELU, bf16_t);
+    if (epilogue == MM_EPI_QKV && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_QKV, bf16_t);
+  }
 #undef MM_LAUNCH
   return MGPT_ERR_BAD_DTYPE;
 }
-template <int WTM, int WTN, int WVM, int WVN, int EPI, typename OT, int AHEAD, int KG = 1, int DIRECT = 0>
+template <int WTM, int WTN, int WVM, int WVN, int EPI, typename OT, int AHEAD, int KG = 1, int DIRECT = 0, int CHAINS = 1>
 int launch_one(const void* act, long lda, const void* w, const float* bias, void* out, long ldo, int n_rows,
                int n_out, int k_dim, int k_parts, long part_stride, const MfmaScatter& sc, hipStream_t stream) {
   static_assert(AHEAD >= 1 && AHEAD <= 4, "sets of staging registers");
   constexpr int BM = WVM * WTM * 16, BN = WVN * WTN * 16;
   constexpr size_t lds_bytes = (DIRECT > 0 ? DIRECT : 2ul) * (BM + BN) * MM_LD * sizeof(bf16_t);
   static_assert(lds_bytes <= 160 * 1024, "a workgroup's LDS");
-  auto kernel = linear_mfma_kernel<WTM, WTN, WVM, WVN, EPI, OT, AHEAD, KG, DIRECT>;
+  auto kernel = linear_mfma_kernel<WTM, WTN, WVM, WVN, EPI, OT, AHEAD, KG, DIRECT, CHAINS>;
   static bool allowed = false;  // more LDS than a kernel gets without asking
   if (!allowed) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
@@ -792,20 +824,22 @@ int launch_one(const void* act, long lda, const void* w, const float* bias, void
   return mgpt_last_error();
 }
 
-template <int WTM, int WTN, int WVM, int WVN, int AHEAD = 1, int DIRECT = 0>
+template <int WTM, int WTN, int WVM, int WVN, int AHEAD = 1, int DIRECT = 0, int CHAINS = 1>
 int launch_shape(const void* act, long lda, const void* w, const float* bias, void* out, int out_dtype, long ldo,
                  int n_rows, int n_out, int k_dim, int epilogue, int k_parts, long part_stride,
                  const MfmaScatter& sc, hipStream_t stream) {
 #define MM_LAUNCH(E, OT)                                                                                            \
-  return launch_one<WTM, WTN, WVM, WVN, E, OT, AHEAD, 1, DIRECT>(act, lda, w, bias, out, ldo, n_rows, n_out, k_dim, \
-                                                                 k_parts, part_stride, sc, stream)
-  if (epilogue == MM_EPI_NONE && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_NONE, bf16_t);
+  return launch_one<WTM, WTN, WVM, WVN, E, OT, AHEAD, 1, DIRECT, CHAINS>(act, lda, w, bias, out, ldo, n_rows, n_out, k_dim, \
+                                                                         k_parts, part_stride, sc, stream)
   if (epilogue == MM_EPI_NONE && out_dtype == MGPT_F32) MM_LAUNCH(MM_EPI_NONE, float);
-  if (epilogue == MM_EPI_GELU && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_GELU, bf16_t);
-  if (epilogue == MM_EPI_RELU2 && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_RELU2, bf16_t);
-  if (epilogue == MM_EPI_XIELU && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_XIELU, bf16_t);
   if (epilogue == MM_EPI_RESIDUAL && out_dtype == MGPT_F32) MM_LAUNCH(MM_EPI_RESIDUAL, float);
-  if (epilogue == MM_EPI_QKV && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_QKV, bf16_t);
+  if constexpr (CHAINS == 1) {
+    if (epilogue == MM_EPI_NONE && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_NONE, bf16_t);
+    if (epilogue == MM_EPI_GELU && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_GELU, bf16_t);
+    if (epilogue == MM_EPI_RELU2 && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_RELU2, bf16_t);
+    if (epilogue == MM_EPI_XIELU && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_XIELU, bf16_t);
+    if (epilogue == MM_EPI_QKV && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_QKV, bf16_t);
+  }
 #undef MM_LAUNCH
   return MGPT_ERR_BAD_DTYPE;
 }
@@ -840,7 +874,10 @@ constexpr int MM_DIRECT_ROWS[MM_DIRECT_VARIANTS] = {32, 64, 128, 128, 32, 256, 1
 constexpr int MM_DIRECT_COLS[MM_DIRECT_VARIANTS] = {32, 64, 64, 192, 32, 256, 256, 192, 192};
 constexpr int MM_DIRECT_HALVES = 5;     // the first of the four variants with the halves out of step: 256 x 256, 128 x 256,
                                         // 256 x 192, 128 x 192
-constexpr int MM_SHAPE_IDS = MM_DIRECT_FIRST + MM_DIRECT_VARIANTS;
+// then the same variants with two chains of sums (float32 outputs; those of 32 x 32, 128 x 64 and 128 rows out of step have them)
+constexpr int MM_CHAINS_FIRST = MM_DIRECT_FIRST + MM_DIRECT_VARIANTS;
+constexpr bool MM_HAS_CHAINS[MM_DIRECT_VARIANTS] = {true, false, true, false, true, false, true, false, true};
+constexpr int MM_SHAPE_IDS = MM_CHAINS_FIRST + MM_DIRECT_VARIANTS;
 
 long tiles_of(int shape, int n_rows, int n_out) {
   return (long)((n_rows + MM_TILE_ROWS[shape] - 1) / MM_TILE_ROWS[shape]) *
@@ -988,6 +1025,13 @@ long direct_tiles(int variant, int n_rows, int n_out) {
          ((n_out + MM_DIRECT_COLS[variant] - 1) / MM_DIRECT_COLS[variant]);
 }
 
+// 64 x 64 tiles under a long inner size (16 steps and more a workgroup), float32 out: two wave groups
+// a tile.  [2048 x 2048 -> 512] 12.9 us against 14.4, [1024 x 2048 -> 512] 12.2 / 13.4, [2048 x 3072 ->
+// 768] 24.2 / 25.5, [8192 x 2048 -> 512] 33.9 / 35.3; at 8 steps ([2048 x 512 -> 512]) nothing.
+// (alone in a graph the variant is ahead at 256 tiles too, 12.9 us against 14.4; inside the 2,048-token
+// prefill step it is not, 0.599-0.607 ms against 0.596-0.602 in turns on one box: more than a tile a unit)
+bool two_groups_pay(int steps, long tiles) { return steps >= 16 && tiles > 256; }
+
 // The shape id for a product of a prompt portion (128 rows and more) whose slices can go straight into
 // LDS and that gains by it, or -1: the rules further down decide.  Which products gain was measured inside
 // the prefill step, one product of the layer changed at a time (alone in a graph of its own, with its
@@ -1001,11 +1045,7 @@ long direct_tiles(int variant, int n_rows, int n_out) {
 //   256 x 256 (qkv and first feed-forward product at 8,192 tokens, widths 512 to 1600: -2 to -5 % of the step).
 // - many rows (512 and more) under an inner size of 12 steps and more: the variant that takes least by a model of rounds of
 //   workgroups (choose_large below).
-int choose_large(int n_rows, int n_out, int k_dim);
-int choose_direct(int n_rows, int n_out, int k_dim) {
-  if (n_rows < 128 || (k_dim % MM_BK) != 0) return -1;
-  const int large = choose_large(n_rows, n_out, k_dim);
-  if (large >= 0) return large;
+int choose_medium(int n_rows, int n_out, int k_dim) {
   if (k_dim / MM_BK >= 32) {
     const long t128 = direct_tiles(2, n_rows, n_out), t64 = direct_tiles(1, n_rows, n_out);
     if (t128 > 520) return -1;
@@ -1031,7 +1071,7 @@ int choose_direct(int n_rows, int n_out, int k_dim) {
 // 150 / 135; 1,500 rows 1600 -> 6400 40 / 34; 12,000 rows 3072 -> 768 105 / 74.  At full occupancy (4,096 rows 6400 -> 4096) the
 // 256 x 256 tile reaches 1,340 TFLOP/s, the register path's 1,180; the clock is down to 1.95 GHz there, the matrix units are
 // busy 65 % of the cycles.
-int choose_large(int n_rows, int n_out, int k_dim) {
+int choose_large(int n_rows, int n_out, int k_dim, bool chains) {
   const int steps = k_dim / MM_BK;
   if (n_rows < 512 || n_out < 512 || steps < 12) return -1;
   struct Cost { int variant, per_unit; double step, fixed, step_alone; };
@@ -1042,13 +1082,27 @@ int choose_large(int n_rows, int n_out, int k_dim) {
   double least = 0.0;
   for (const Cost& c : costs) {
     const long tiles = direct_tiles(c.variant, n_rows, n_out), at_once = 256L * c.per_unit;
+    if (chains && !MM_HAS_CHAINS[c.variant]) continue;
     if (tiles < 140) continue;   // (smaller tiles, or a split, use more of the chip)
     const long rest = tiles % at_once;
     double t = (double)(tiles / at_once) * (steps * c.step + c.fixed);
     if (rest > 0) t += steps * (rest <= 256 ? c.step_alone : c.step) + c.fixed;
     if (best < 0 || t < least) best = c.variant, least = t;
   }
-  return best < 0 ? -1 : MM_DIRECT_FIRST + best;
+  return best < 0 ? -1 : (chains ? MM_CHAINS_FIRST : MM_DIRECT_FIRST) + best;
+}
+
+// Float32 outputs that would go to the 64 x 64 tiles with two wave groups have their sums as two chains there; a large variant
+// in their place makes the same two: single chains, twice as long, are further from the sums in 64 bits (2,048 rows 1600 -> 1600
+// 1.08e-7 of the sums' norm, two chains 0.80e-7; 3,000 rows 6400 -> 1600 3.42e-7 / 2.39e-7).  The second set of accumulators costs
+// under 2 % (3,500 rows 5120 -> 1280 62 us either way).
+int choose_direct(int n_rows, int n_out, int k_dim, bool f32) {
+  if (n_rows < 128 || (k_dim % MM_BK) != 0) return -1;
+  const int medium = choose_medium(n_rows, n_out, k_dim);
+  const bool chains = f32 && medium < 0 && choose_shape(n_rows, n_out) == 3 &&
+                      two_groups_pay(k_dim / MM_BK, tiles_of(3, n_rows, n_out));
+  const int large = choose_large(n_rows, n_out, k_dim, chains);
+  return large >= 0 ? large : medium;
 }
 
 // shape < 0: chosen by the size.  k_parts: 0 = chosen by the size, together with the shape, if
@@ -1066,13 +1120,16 @@ int launch_any(int shape, int k_parts, const void* act, long lda, const void* w,
   int ahead = 0;  // 0: chosen below
   bool two_groups = false;  // the 64 x 64 tile with two wave groups (shape MM_SHAPES + 2)
   int direct = -1;  // which of the variants whose slices go straight into LDS (-1: through registers)
+  bool chains = false;  // two chains of sums
   if (shape < 0 && k_parts <= 1 && !leave_parts) {
-    const int chosen = direct_ok(act, w, k_dim) ? choose_direct(n_rows, n_out, k_dim) : -1;
+    const int chosen = direct_ok(act, w, k_dim) ? choose_direct(n_rows, n_out, k_dim, out_dtype == MGPT_F32) : -1;
     if (chosen >= 0) shape = chosen, k_parts = 1;
   }
   if (shape >= MM_DIRECT_FIRST) {
     if (shape >= MM_SHAPE_IDS || !direct_ok(act, w, k_dim)) return MGPT_ERR_BAD_SHAPE;
-    direct = shape - MM_DIRECT_FIRST;
+    chains = shape >= MM_CHAINS_FIRST;
+    direct = shape - (chains ? MM_CHAINS_FIRST : MM_DIRECT_FIRST);
+    if (chains && (!MM_HAS_CHAINS[direct] || out_dtype != MGPT_F32)) return MGPT_ERR_BAD_SHAPE;
     if (direct >= MM_DIRECT_HALVES && k_parts > 1) return MGPT_ERR_BAD_SHAPE;   // (these are not split)
     shape = 3;   // (the rules below for the other variants do not apply)
     ahead = 1;
@@ -1136,15 +1193,10 @@ int launch_any(int shape, int k_parts, const void* act, long lda, const void* w,
     const int dt_here = split ? MGPT_F32 : out_dtype, epi_here = split ? MM_EPI_NONE : epilogue;
     if (dt_here != MGPT_F32 || (epi_here != MM_EPI_NONE && epi_here != MM_EPI_RESIDUAL)) return MGPT_ERR_BAD_SHAPE;
   } else if (shape == 3 && ahead == 1 && direct < 0) {
-    // 64 x 64 tiles under a long inner size (16 steps and more a workgroup), float32 out: two wave groups
-    // a tile.  [2048 x 2048 -> 512] 12.9 us against 14.4, [1024 x 2048 -> 512] 12.2 / 13.4, [2048 x 3072 ->
-    // 768] 24.2 / 25.5, [8192 x 2048 -> 512] 33.9 / 35.3; at 8 steps ([2048 x 512 -> 512]) nothing.
     const int steps_here = ((k_dim + MM_BK - 1) / MM_BK + k_parts - 1) / k_parts;
     const int dt_here = split ? MGPT_F32 : out_dtype, epi_here = split ? MM_EPI_NONE : epilogue;
-    // (alone in a graph the variant is ahead at 256 tiles too, 12.9 us against 14.4; inside the 2,048-token
-    // prefill step it is not, 0.599-0.607 ms against 0.596-0.602 in turns on one box: more than a tile a unit)
-    two_groups = steps_here >= 16 && dt_here == MGPT_F32 && (epi_here == MM_EPI_NONE || epi_here == MM_EPI_RESIDUAL) &&
-                 tiles_of(3, n_rows, n_out) * k_parts > 256;
+    two_groups = two_groups_pay(steps_here, tiles_of(3, n_rows, n_out) * k_parts) && dt_here == MGPT_F32 &&
+                 (epi_here == MM_EPI_NONE || epi_here == MM_EPI_RESIDUAL);
   }
   if (leave_parts) {
     *leave_parts = split ? k_parts : 0;
@@ -1156,19 +1208,27 @@ int launch_any(int shape, int k_parts, const void* act, long lda, const void* w,
   const long ld = split ? n_out : ldo, stride = split ? (long)n_rows * n_out : 0;
 #define MM_ARGS act, lda, w, b, dst, dt, ld, n_rows, n_out, k_dim, epi, k_parts, stride, sc, stream
   int rc = MGPT_ERR_BAD_SHAPE;
-  if (direct >= 0) {
+#define MM_HALVES_ARGS act, lda, w, b, dst, dt, ld, n_rows, n_out, k_dim, epi, sc, stream
+  if (direct >= 0 && chains) {
+    switch (direct) {
+      case 0: rc = launch_shape<1, 1, 2, 2, 1, 4, 2>(MM_ARGS); break;
+      case 2: rc = launch_shape<2, 2, 4, 2, 1, 3, 2>(MM_ARGS); break;
+      case 4: rc = launch_shape<1, 1, 2, 2, 1, 6, 2>(MM_ARGS); break;
+      case 6: rc = launch_halves<4, 4, 2>(MM_HALVES_ARGS); break;
+      case 8: rc = launch_halves<4, 3, 2>(MM_HALVES_ARGS); break;
+      default: break;
+    }
+  } else if (direct >= 0) {
     switch (direct) {
       case 0: rc = launch_shape<1, 1, 2, 2, 1, 4>(MM_ARGS); break;
       case 1: rc = launch_shape<2, 2, 2, 2, 1, 4>(MM_ARGS); break;
       case 2: rc = launch_shape<2, 2, 4, 2, 1, 3>(MM_ARGS); break;
       case 3: rc = launch_shape<4, 3, 2, 4, 1, 2>(MM_ARGS); break;
       case 4: rc = launch_shape<1, 1, 2, 2, 1, 6>(MM_ARGS); break;
-      case 5: rc = launch_halves<8, 4>(act, lda, w, b, dst, dt, ld, n_rows, n_out, k_dim, epi, sc, stream); break;
-#define MM_HALVES_ARGS act, lda, w, b, dst, dt, ld, n_rows, n_out, k_dim, epi, sc, stream
+      case 5: rc = launch_halves<8, 4>(MM_HALVES_ARGS); break;
       case 6: rc = launch_halves<4, 4>(MM_HALVES_ARGS); break;
       case 7: rc = launch_halves<8, 3>(MM_HALVES_ARGS); break;
       case 8: rc = launch_halves<4, 3>(MM_HALVES_ARGS); break;
-#undef MM_HALVES_ARGS
       default: break;
     }
   } else
@@ -1184,6 +1244,7 @@ int launch_any(int shape, int k_parts, const void* act, long lda, const void* w,
       rc = ahead > 1 ? launch_shape<1, 1, 2, 2, MM_AHEAD>(MM_ARGS) : launch_shape<1, 1, 2, 2>(MM_ARGS);
       break;
   }
+#undef MM_HALVES_ARGS
 #undef MM_ARGS
   if (rc != MGPT_OK || !split || leave_parts) return rc;
   return launch_join(partials, k_parts, bias, out, out_dtype, ldo, n_rows, n_out, epilogue, stream, sc.epi_coef);
@@ -1246,7 +1307,8 @@ extern "C" int mgpt_linear_mfma_xielu(const void* act, long lda, const void* w, 
 // 7 = 64 x 64 with two wave groups a tile (float32 outputs), 8 to 12 = the slices straight into LDS: 32 x 32 and
 // 64 x 64 with four stages, 128 x 64 with three, 128 x 192 with two, 32 x 32 with six (an inner size of whole steps of 64 and operands
 // aligned to 16 bytes, else refused), 13 to 16 = the halves out of step, 256 x 256, 128 x 256, 256 x 192, 128 x 192 (the same
-// conditions, and never split); negative: chosen) and the number of stretches of the inner size given
+// conditions, and never split), 17, 19, 21, 23 and 25 = 8, 10, 12, 14 and 16 with two chains of sums (float32 outputs);
+// negative: chosen) and the number of stretches of the inner size given
 // (k_parts as for launch_any above), instead of chosen by the size: for tests and measurements.
 extern "C" int mgpt_linear_mfma_shape(int shape, int k_parts, const void* act, long lda, const void* w,
                                       const float* bias, void* out, int out_dtype, long ldo, int n_rows,

@@ -424,6 +424,36 @@ def test_linear_mfma_of_many_rows_keeps_its_sums_whatever_the_tile(n, k, o, shap
     assert ((out.float() - want).norm() / want.norm()).item() < 4e-3      # rounding to bfloat16: 2 ** -9 of each value at most
 
 
+@pytest.mark.parametrize("n,k,o", [(1, 64, 16), (300, 64, 257), (513, 512, 520), (256, 128, 384), (1000, 192, 130), (257, 320, 193)])
+@pytest.mark.parametrize("epi", [kernels.EPI_NONE, kernels.EPI_RESIDUAL])
+@pytest.mark.parametrize("shape", [17, 19, 21, 23, 25])
+def test_linear_mfma_with_two_chains_of_sums(n, k, o, epi, shape):
+    """The variants whose float32 sums are two chains, at sizes that cut their tiles and at 1, 2, 3, 5 and 8 steps: the bits of
+    the two wave groups that share a 64 x 64 tile, each a chain over its half of every step."""
+    g = torch.Generator().manual_seed(n)
+    a, w, bias = rnd(g, n, k, dtype="bfloat16"), rnd(g, o, k, dtype="bfloat16", scale=k ** -0.5), rnd(g, o)
+    prev = rnd(g, n + 2, o)
+    out, groups = prev.clone().to(DEV), prev.clone().to(DEV)
+    assert kernels.linear_mfma(a.to(DEV), w.to(DEV), bias.to(DEV), out, n, epi, shape=shape)
+    assert kernels.linear_mfma(a.to(DEV), w.to(DEV), bias.to(DEV), groups, n, epi, shape=7)
+    helpers.assert_close(out[:n], _linear_want(a, w, bias, epi, prev[:n]), "bfloat16", f"shape {shape} {n}x{k}x{o}")
+    assert torch.equal(out, groups)
+    assert not kernels.linear_mfma(a.to(DEV), w.to(DEV), bias.to(DEV), out.to(torch.bfloat16), n, kernels.EPI_NONE, shape=shape)
+
+
+@pytest.mark.parametrize("n,k,o", [(800, 1600, 1600), (2048, 1024, 1024), (4096, 1280, 1280), (3000, 3200, 1600), (6000, 3072, 768)])
+@pytest.mark.parametrize("epi", [kernels.EPI_NONE, kernels.EPI_RESIDUAL])
+def test_linear_mfma_of_many_rows_keeps_two_chains_of_float32_sums(n, k, o, epi):
+    """Float32 outputs of the sizes whose 64 x 64 tiles have two wave groups: whatever tile is chosen, the bits are theirs."""
+    g = torch.Generator().manual_seed(o)
+    a, w, bias = rnd(g, n, k, dtype="bfloat16").to(DEV), rnd(g, o, k, dtype="bfloat16", scale=k ** -0.5).to(DEV), rnd(g, o).to(DEV)
+    out = rnd(g, n, o).to(DEV)
+    groups = out.clone()
+    assert kernels.linear_mfma(a, w, bias, out, n, epi)
+    assert kernels.linear_mfma(a, w, bias, groups, n, epi, shape=7)
+    assert torch.equal(out, groups)
+
+
 @pytest.mark.parametrize("n,shape,k", [(300, 13, 64), (130, 14, 192), (520, 15, 128), (257, 16, 256)])
 def test_linear_mfma_halves_store_keys_and_values(n, shape, k):
     test_linear_mfma_stores_keys_and_values(n, shape, k)

@@ -1062,32 +1062,49 @@ int choose_medium(int n_rows, int n_out, int k_dim) {
   return MM_DIRECT_FIRST + 3;
 }
 
-// Of the large variants the one that takes least: rounds of as many workgroups as the chip holds, each (steps x us a step + us
-// for filling, the epilogue and the start).  The numbers are fits, within 15 %, to 23 products of 1,500 to 12,000 rows, inner
-// sizes 768 to 6,400 and 768 to 10,880 columns (alone in a graph, four sets of operands in turn; bfloat16 out, or added to
-// float32 rows, which costs up to 15 us more whatever the tile, the rows being read and written).  Two workgroups of the
-// variants with less LDS share a compute unit, and each is faster where it has one to itself.  With them, before / now, us:
-// 4,096 rows 1600 -> 4800 72 / 68, 1600 -> 6400 90 / 83, 1600 -> 1600 40 / 35, 6400 -> 1600 110 / 98; 3,300 rows 2048 -> 10880
-// 150 / 135; 1,500 rows 1600 -> 6400 40 / 34; 12,000 rows 3072 -> 768 105 / 74.  At full occupancy (4,096 rows 6400 -> 4096) the
-// 256 x 256 tile reaches 1,340 TFLOP/s, the register path's 1,180; the clock is down to 1.95 GHz there, the matrix units are
-// busy 65 % of the cycles.
-int choose_large(int n_rows, int n_out, int k_dim, bool chains) {
+// Of the large variants the one that takes least: rounds of as many workgroups as the chip holds, each steps x us a step + us for
+// its fill and epilogue, and behind them 0.68 us a million outputs (float32 rows, most of them read and written: 1.28).  The numbers
+// are fits to 417 products of 512 to 12,288 rows, inner sizes 768 to 6,400 and 640 to 10,880 columns (each variant alone in a graph,
+// three sets of operands in turn): half of the predictions are within 2 %, 95 of 100 within 7.  The choice takes up to 5 % longer
+// than the best variant, up to 4 % longer than the rules above without it, and 7 % less than those in the mean.  Two workgroups of
+// the variants with less LDS share a compute unit, and each is faster where it has one to itself.
+// Those rules / now, in turn, us: 4,096 rows 1600 -> 4800 69 / 68, 1600 -> 6400 87 / 81, 1600 -> 1600 added to float32 rows 40 / 35,
+// 6400 -> 1600 107 / 100; 3,300 rows 2048 -> 10880 165 / 133; 1,500 rows 1600 -> 4800 35 / 28; 12,000 rows 3072 -> 768 102 / 75.
+// At full occupancy (4,096 rows 6400 -> 4096) the 256 x 256 tile reaches 1,340 TFLOP/s, the register path's 1,180; the clock is
+// down to 1.95 GHz there, the matrix units are busy 65 % of the cycles.
+//
+// Lines: from 512 rows, 12 steps and 140 tiles on (smaller tiles, or a split, use more of the chip below).  From 32 steps on 128 x 64
+// tiles keep to the range that they have above, and 128 x 192 lose what they gain by sharing a unit (12,288 rows 6400 -> 1600
+// 288 us, 128 x 256 271).  Beyond 16,384 columns (the head over many tokens) memory counts for more than rounds: 256 x 256 from
+// 1,000 rows on, below only where their last row of tiles is more than half full and the inner size long, else the rules above
+// (rules above / 256 x 256, us, 768 -> 50304: 600 rows 73 / 88, 720 85 / 93, 850 96 / 119, 1,024 150 / 130, 2,048 304 / 264;
+// 1600 -> 50304: 512 rows 109 / 104, 720 164 / 157, 850 198 / 202, 1,300 296 / 271, 4,096 750 / 724).
+int choose_large(int n_rows, int n_out, int k_dim, bool f32, bool chains, double* least) {
   const int steps = k_dim / MM_BK;
   if (n_rows < 512 || n_out < 512 || steps < 12) return -1;
-  struct Cost { int variant, per_unit; double step, fixed, step_alone; };
-  const Cost costs[] = {{MM_DIRECT_HALVES, 1, 1.2, 9.0, 1.2},      {MM_DIRECT_HALVES + 1, 1, 0.8, 6.0, 0.8},
-                        {MM_DIRECT_HALVES + 2, 1, 1.03, 8.0, 1.03}, {MM_DIRECT_HALVES + 3, 1, 0.67, 6.0, 0.67},
-                        {3, 2, 1.3, 4.0, 0.75},                     {2, 2, 0.6, 4.0, 0.4}};
+  if (n_out > 16384) {
+    const bool full = (n_rows + 255) / 256 * 2 == (n_rows + 127) / 128 && (steps >= 20 || n_rows == 512);
+    return n_rows >= 1000 || full ? MM_DIRECT_FIRST + MM_DIRECT_HALVES : -1;
+  }
+  struct Cost { int variant, per_unit; double step, step_alone, round, round_f32; };
+  const Cost costs[] = {{2, 2, 0.56, 0.355, 0.3, 0.3},
+                        {3, 2, steps >= 32 ? 1.2 : 1.09, 0.71, 0.2, 2.2},
+                        {MM_DIRECT_HALVES, 1, 1.37, 1.30, 0.3, 7.0},
+                        {MM_DIRECT_HALVES + 1, 1, 0.825, 0.76, 0.7, 3.9},
+                        {MM_DIRECT_HALVES + 2, 1, 1.09, 1.05, 0.55, 6.4},
+                        {MM_DIRECT_HALVES + 3, 1, 0.72, 0.645, 0.7, 2.8}};
+  const double outputs = 1e-6 * n_rows * n_out, behind = f32 ? 4.6 + 1.28 * outputs : 3.6 + 0.68 * outputs;
   int best = -1;
-  double least = 0.0;
   for (const Cost& c : costs) {
     const long tiles = direct_tiles(c.variant, n_rows, n_out), at_once = 256L * c.per_unit;
-    if (chains && !MM_HAS_CHAINS[c.variant]) continue;
-    if (tiles < 140) continue;   // (smaller tiles, or a split, use more of the chip)
+    if (tiles < 140 || (chains && !MM_HAS_CHAINS[c.variant])) continue;
+    if (steps >= 32 && c.variant == 2 && tiles > 520) continue;
+    if (steps >= 48 && c.variant == 3) continue;
     const long rest = tiles % at_once;
-    double t = (double)(tiles / at_once) * (steps * c.step + c.fixed);
-    if (rest > 0) t += steps * (rest <= 256 ? c.step_alone : c.step) + c.fixed;
-    if (best < 0 || t < least) best = c.variant, least = t;
+    const double round = f32 ? c.round_f32 : c.round;
+    double t = behind + (double)(tiles / at_once) * (steps * c.step + round);
+    if (rest > 0) t += steps * (rest <= 256 ? c.step_alone : c.step) + round;
+    if (best < 0 || t < *least) best = c.variant, *least = t;
   }
   return best < 0 ? -1 : (chains ? MM_CHAINS_FIRST : MM_DIRECT_FIRST) + best;
 }
@@ -1095,13 +1112,21 @@ int choose_large(int n_rows, int n_out, int k_dim, bool chains) {
 // Float32 outputs that would go to the 64 x 64 tiles with two wave groups have their sums as two chains there; a large variant
 // in their place makes the same two: single chains, twice as long, are further from the sums in 64 bits (2,048 rows 1600 -> 1600
 // 1.08e-7 of the sums' norm, two chains 0.80e-7; 3,000 rows 6400 -> 1600 3.42e-7 / 2.39e-7).  The second set of accumulators costs
-// under 2 % (3,500 rows 5120 -> 1280 62 us either way).
+// up to 3 % (3,500 rows 5120 -> 1280 62 us instead of 61, with two wave groups 93).
+//
+// The 64 x 64 tiles themselves take 6.7 us and 0.19 us a step and round of 256 of them, several sharing a compute unit: less than a
+// large variant with one workgroup in its second round (1,600 rows 1280 -> 1280, 500 of them 14.1 us, 260 of 128 x 64 16.7).  With
+// four stages, under 32 steps and more, two on a unit take 0.39 us a step (64 x 64 / 128 x 64, us: 600 rows 2048 -> 2048 15.6 / 16.3,
+// 1,300 rows 4096 -> 1024 28.0 / 29.0; 850 rows 5120 -> 1280 38.6 / 34.1).
 int choose_direct(int n_rows, int n_out, int k_dim, bool f32) {
   if (n_rows < 128 || (k_dim % MM_BK) != 0) return -1;
-  const int medium = choose_medium(n_rows, n_out, k_dim);
-  const bool chains = f32 && medium < 0 && choose_shape(n_rows, n_out) == 3 &&
-                      two_groups_pay(k_dim / MM_BK, tiles_of(3, n_rows, n_out));
-  const int large = choose_large(n_rows, n_out, k_dim, chains);
+  const int medium = choose_medium(n_rows, n_out, k_dim), steps = k_dim / MM_BK;
+  const bool small = medium < 0 && choose_shape(n_rows, n_out) == 3;
+  const long tiles = tiles_of(3, n_rows, n_out);
+  double least = 0.0;
+  const int large = choose_large(n_rows, n_out, k_dim, f32, f32 && small && two_groups_pay(steps, tiles), &least);
+  if (small && 6.7 + (double)((tiles + 255) / 256) * (0.19 * steps + (f32 ? 1.2 : 0.35)) < least) return medium;
+  if (medium == MM_DIRECT_FIRST + 1 && (f32 ? 4.2 : 3.2) + 0.39 * steps < least) return medium;
   return large >= 0 ? large : medium;
 }
 
@@ -1274,6 +1299,12 @@ extern "C" int mgpt_linear_mfma_parts(const void* act, long lda, const void* w, 
                             partials, partials_floats, sc, stream, &parts);
   if (rc != MGPT_OK) return rc;
   return parts > 1 ? MGPT_OK : MGPT_ERR_BAD_SHAPE;
+}
+
+// Which variant whose slices go straight into LDS an unsplit product of 128 and more rows goes to (a shape id as for
+// mgpt_linear_mfma_shape, for operands aligned to 16 bytes), or -1: one of those through registers, or one of the smallest tiles.
+extern "C" int mgpt_linear_mfma_choice(int n_rows, int n_out, int k_dim, int out_dtype) {
+  return choose_direct(n_rows, n_out, k_dim, out_dtype == MGPT_F32);
 }
 
 // act: [n_rows, k_dim] bfloat16 with row stride lda (a multiple of 8, 16-byte aligned base);

@@ -1063,7 +1063,7 @@ int choose_medium(int n_rows, int n_out, int k_dim) {
 }
 
 // Of the large variants the one that takes least: rounds of as many workgroups as the chip holds, each steps x us a step + us for
-// its fill and epilogue, and behind them 0.68 us a million outputs (float32 rows, most of them read and written: 1.28).  The numbers
+// its fill and epilogue, and behind them 0.68 us a million outputs (added to float32 rows, which are read and written: 1.28).  The numbers
 // are fits to 417 products of 512 to 12,288 rows, inner sizes 768 to 6,400 and 640 to 10,880 columns (each variant alone in a graph,
 // three sets of operands in turn): half of the predictions are within 2 %, 95 of 100 within 7.  The choice takes up to 5 % longer
 // than the best variant, up to 4 % longer than the rules above without it, and 7 % less than those in the mean.  Two workgroups of
@@ -1079,21 +1079,27 @@ int choose_medium(int n_rows, int n_out, int k_dim) {
 // 1,000 rows on, below only where their last row of tiles is more than half full and the inner size long, else the rules above
 // (rules above / 256 x 256, us, 768 -> 50304: 600 rows 73 / 88, 720 85 / 93, 850 96 / 119, 1,024 150 / 130, 2,048 304 / 264;
 // 1600 -> 50304: 512 rows 109 / 104, 720 164 / 157, 850 198 / 202, 1,300 296 / 271, 4,096 750 / 724).
-int choose_large(int n_rows, int n_out, int k_dim, bool f32, bool chains, double* least) {
+//
+// Grouped rows (experts) count with their padding, which comes last in a group and in the call: the XCDs take equal stretches of all
+// tiles, so those that got the used ones take the time (counted by used tiles the choice was 8 % slower in the mean of 224 products
+// of 512 to 24,000 pairs for 8 to 64 experts, and up to 54 %; counted as here it is 8 % faster than the rules above).  Where a group's second half is padding, the two workgroups that
+// share a unit leave it to one of them: 128 x 192 then win by up to 14 % what would be a tie (16 experts 1024 -> 2048, 512 pairs:
+// 23.9 us, 256 x 192 26.5).
+int choose_large(int n_rows, int n_out, int k_dim, bool added, bool grouped, bool chains, double* least) {
   const int steps = k_dim / MM_BK;
   if (n_rows < 512 || n_out < 512 || steps < 12) return -1;
   if (n_out > 16384) {
     const bool full = (n_rows + 255) / 256 * 2 == (n_rows + 127) / 128 && (steps >= 20 || n_rows == 512);
     return n_rows >= 1000 || full ? MM_DIRECT_FIRST + MM_DIRECT_HALVES : -1;
   }
-  struct Cost { int variant, per_unit; double step, step_alone, round, round_f32; };
+  struct Cost { int variant, per_unit; double step, step_alone, round, round_added; };
   const Cost costs[] = {{2, 2, 0.56, 0.355, 0.3, 0.3},
                         {3, 2, steps >= 32 ? 1.2 : 1.09, 0.71, 0.2, 2.2},
                         {MM_DIRECT_HALVES, 1, 1.37, 1.30, 0.3, 7.0},
                         {MM_DIRECT_HALVES + 1, 1, 0.825, 0.76, 0.7, 3.9},
                         {MM_DIRECT_HALVES + 2, 1, 1.09, 1.05, 0.55, 6.4},
                         {MM_DIRECT_HALVES + 3, 1, 0.72, 0.645, 0.7, 2.8}};
-  const double outputs = 1e-6 * n_rows * n_out, behind = f32 ? 4.6 + 1.28 * outputs : 3.6 + 0.68 * outputs;
+  const double outputs = 1e-6 * n_rows * n_out, behind = added ? 4.6 + 1.28 * outputs : 3.6 + 0.68 * outputs;
   int best = -1;
   for (const Cost& c : costs) {
     const long tiles = direct_tiles(c.variant, n_rows, n_out), at_once = 256L * c.per_unit;
@@ -1101,9 +1107,10 @@ int choose_large(int n_rows, int n_out, int k_dim, bool f32, bool chains, double
     if (steps >= 32 && c.variant == 2 && tiles > 520) continue;
     if (steps >= 48 && c.variant == 3) continue;
     const long rest = tiles % at_once;
-    const double round = f32 ? c.round_f32 : c.round;
+    const double round = added ? c.round_added : c.round;
     double t = behind + (double)(tiles / at_once) * (steps * c.step + round);
     if (rest > 0) t += steps * (rest <= 256 ? c.step_alone : c.step) + round;
+    if (grouped && c.variant == 3 && tiles <= 2 * at_once) t *= 0.95;
     if (best < 0 || t < *least) best = c.variant, *least = t;
   }
   return best < 0 ? -1 : (chains ? MM_CHAINS_FIRST : MM_DIRECT_FIRST) + best;
@@ -1118,15 +1125,15 @@ int choose_large(int n_rows, int n_out, int k_dim, bool f32, bool chains, double
 // large variant with one workgroup in its second round (1,600 rows 1280 -> 1280, 500 of them 14.1 us, 260 of 128 x 64 16.7).  With
 // four stages, under 32 steps and more, two on a unit take 0.39 us a step (64 x 64 / 128 x 64, us: 600 rows 2048 -> 2048 15.6 / 16.3,
 // 1,300 rows 4096 -> 1024 28.0 / 29.0; 850 rows 5120 -> 1280 38.6 / 34.1).
-int choose_direct(int n_rows, int n_out, int k_dim, bool f32) {
+int choose_direct(int n_rows, int n_out, int k_dim, bool f32, bool added, bool grouped) {
   if (n_rows < 128 || (k_dim % MM_BK) != 0) return -1;
   const int medium = choose_medium(n_rows, n_out, k_dim), steps = k_dim / MM_BK;
   const bool small = medium < 0 && choose_shape(n_rows, n_out) == 3;
   const long tiles = tiles_of(3, n_rows, n_out);
   double least = 0.0;
-  const int large = choose_large(n_rows, n_out, k_dim, f32, f32 && small && two_groups_pay(steps, tiles), &least);
-  if (small && 6.7 + (double)((tiles + 255) / 256) * (0.19 * steps + (f32 ? 1.2 : 0.35)) < least) return medium;
-  if (medium == MM_DIRECT_FIRST + 1 && (f32 ? 4.2 : 3.2) + 0.39 * steps < least) return medium;
+  const int large = choose_large(n_rows, n_out, k_dim, added, grouped, f32 && small && two_groups_pay(steps, tiles), &least);
+  if (small && 6.7 + (double)((tiles + 255) / 256) * (0.19 * steps + (added ? 1.2 : 0.35)) < least) return medium;
+  if (medium == MM_DIRECT_FIRST + 1 && (added ? 4.2 : 3.2) + 0.39 * steps < least) return medium;
   return large >= 0 ? large : medium;
 }
 
@@ -1147,7 +1154,9 @@ int launch_any(int shape, int k_parts, const void* act, long lda, const void* w,
   int direct = -1;  // which of the variants whose slices go straight into LDS (-1: through registers)
   bool chains = false;  // two chains of sums
   if (shape < 0 && k_parts <= 1 && !leave_parts) {
-    const int chosen = direct_ok(act, w, k_dim) ? choose_direct(n_rows, n_out, k_dim, out_dtype == MGPT_F32) : -1;
+    const int chosen = direct_ok(act, w, k_dim) ? choose_direct(n_rows, n_out, k_dim, out_dtype == MGPT_F32, epilogue == MM_EPI_RESIDUAL,
+                                                              sc.row_expert != nullptr)
+                                              : -1;
     if (chosen >= 0) shape = chosen, k_parts = 1;
   }
   if (shape >= MM_DIRECT_FIRST) {
@@ -1303,8 +1312,8 @@ extern "C" int mgpt_linear_mfma_parts(const void* act, long lda, const void* w, 
 
 // Which variant whose slices go straight into LDS an unsplit product of 128 and more rows goes to (a shape id as for
 // mgpt_linear_mfma_shape, for operands aligned to 16 bytes), or -1: one of those through registers, or one of the smallest tiles.
-extern "C" int mgpt_linear_mfma_choice(int n_rows, int n_out, int k_dim, int out_dtype) {
-  return choose_direct(n_rows, n_out, k_dim, out_dtype == MGPT_F32);
+extern "C" int mgpt_linear_mfma_choice(int n_rows, int n_out, int k_dim, int out_dtype, int epilogue, int grouped) {
+  return choose_direct(n_rows, n_out, k_dim, out_dtype == MGPT_F32, epilogue == MM_EPI_RESIDUAL, grouped != 0);
 }
 
 // act: [n_rows, k_dim] bfloat16 with row stride lda (a multiple of 8, 16-byte aligned base);

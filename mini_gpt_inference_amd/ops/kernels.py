@@ -723,10 +723,12 @@ def linear_mfma_parts(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Ten
     return True
 
 
-def linear_mfma_choice(n_rows: int, n_out: int, k_dim: int, dtype: torch.dtype) -> int:
-    """The `shape` among 8 to 25 that linear_mfma chooses for 128 and more rows with outputs of this type, or -1 (one of the
-    others)."""
-    return library.kernels().mgpt_linear_mfma_choice(n_rows, n_out, k_dim, F32 if dtype == torch.float32 else BF16)
+def linear_mfma_choice(n_rows: int, n_out: int, k_dim: int, dtype: torch.dtype, epilogue: int = EPI_NONE,
+                       grouped: bool = False) -> int:
+    """The `shape` among 8 to 25 that linear_mfma (grouped: grouped_linear_tiled) chooses for 128 and more rows with outputs of
+    this type, or -1 (one of the others)."""
+    return library.kernels().mgpt_linear_mfma_choice(n_rows, n_out, k_dim, F32 if dtype == torch.float32 else BF16, epilogue,
+                                                     int(grouped))
 
 
 def linear_mfma(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor,

@@ -136,7 +136,7 @@ def _declare_optional(lib: ctypes.CDLL) -> None:
         "mgpt_linear_mfma_xielu": [P, L, P, P, P, L, I, I, I, P, P, L, P],
         "mgpt_linear_mfma_shape": [I, I, P, L, P, P, P, I, L, I, I, I, I, P, L, P],
         "mgpt_linear_mfma_partials": [I, I, I, I],
-        "mgpt_linear_mfma_choice": [I, I, I, I],
+        "mgpt_linear_mfma_choice": [I, I, I, I, I, I],
         "mgpt_linear_exact_kernel": [I, I, I],
         "mgpt_linear_exact_small_tiles": [I, I, I],
         "mgpt_linear_exact_parts": [P, L, P, P, I, I, I, P],

@@ -410,20 +410,25 @@ def test_linear_mfma_with_its_halves_out_of_step(n, k, o, epi, o_dt, shape):
     assert torch.equal(out, small)
 
 
-@pytest.mark.parametrize("n,k,o,shape,shape_f32", [
-    (1500, 1600, 4800, 14, 14), (4096, 1600, 6400, 13, 11), (4096, 1600, 4800, 15, 11), (4096, 1600, 1600, 14, 14),
-    (2000, 768, 2304, 16, 16), (2000, 3072, 768, 10, 10),
-    (511, 1600, 4800, -1, -1), (512, 1600, 4800, 10, 19),           # rows
-    (2000, 704, 2304, 11, 11),                                      # 11 steps: the rules for fewer
-    (2176, 768, 512, -1, -1), (2240, 768, 512, 10, 10),             # 136 and 144 tiles of 128 x 64
-    (1600, 1280, 1280, -1, -1), (1664, 1280, 1280, 10, 19),         # a second round of the 64 x 64 tiles and a third
-    (1300, 4096, 1024, 10, 9), (850, 5120, 1280, 10, 10), (5000, 5120, 1280, 14, 14), (1600, 2048, 10880, 11, 11),
-    (3300, 5440, 2048, 14, 14), (12288, 3072, 768, 15, 15),         # long inner sizes
-    (600, 768, 50304, 11, 11), (1024, 768, 50304, 13, 13), (720, 1600, 50304, 13, 13), (850, 1600, 50304, 11, 11)])
-def test_linear_mfma_choice_among_the_large_variants(n, k, o, shape, shape_f32):
-    """What the model of rounds chooses for bfloat16 and float32 outputs, on both sides of its lines."""
+@pytest.mark.parametrize("n,k,o,shape,shape_f32,shape_added,shape_grouped", [
+    (1500, 1600, 4800, 14, 14, 14, 14), (4096, 1600, 6400, 13, 13, 11, 13), (4096, 1600, 4800, 15, 15, 11, 11),
+    (4096, 1600, 1600, 14, 14, 14, 14), (2000, 768, 2304, 16, 16, 16, 11), (2000, 3072, 768, 10, 10, 10, 10),
+    (511, 1600, 4800, -1, -1, -1, -1), (512, 1600, 4800, 10, 19, 19, 10),       # rows
+    (2000, 704, 2304, 11, 11, 11, 11),                                          # 11 steps: the rules for fewer
+    (2176, 768, 512, -1, -1, -1, -1), (2240, 768, 512, 10, 10, 10, 10),         # 136 and 144 tiles of 128 x 64
+    (1600, 1280, 1280, -1, -1, -1, -1), (1664, 1280, 1280, 10, 19, 19, 10),     # a second round of the 64 x 64 tiles and a third
+    (1300, 4096, 1024, 10, 10, 9, 10), (850, 5120, 1280, 10, 10, 10, 10), (5000, 5120, 1280, 14, 14, 14, 14),
+    (1600, 2048, 10880, 11, 11, 11, 11), (3300, 5440, 2048, 14, 14, 14, 14), (12288, 3072, 768, 15, 15, 15, 15),
+    (4608, 1024, 2048, 15, 15, 11, 11),                                         # groups whose second half may be padding
+    (600, 768, 50304, 11, 11, 11, 11), (1024, 768, 50304, 13, 13, 13, 13), (720, 1600, 50304, 13, 13, 13, 13),
+    (850, 1600, 50304, 11, 11, 11, 11)])
+def test_linear_mfma_choice_among_the_large_variants(n, k, o, shape, shape_f32, shape_added, shape_grouped):
+    """What the model of rounds chooses for bfloat16 and float32 outputs, for sums added to float32 rows and for rows in groups, on
+    both sides of its lines."""
     assert kernels.linear_mfma_choice(n, o, k, torch.bfloat16) == shape
     assert kernels.linear_mfma_choice(n, o, k, torch.float32) == shape_f32
+    assert kernels.linear_mfma_choice(n, o, k, torch.float32, kernels.EPI_RESIDUAL) == shape_added
+    assert kernels.linear_mfma_choice(n, o, k, torch.bfloat16, grouped=True) == shape_grouped
 
 
 @pytest.mark.parametrize("n,k,o", [(1500, 1600, 4800), (1500, 1600, 6400), (4096, 1600, 1600), (6000, 768, 2304), (2000, 768, 2304),

@@ -90,6 +90,8 @@ def _linear_want(a, w, bias, epi, prev):
         y = P.plain_gelu_tanh(y)
     if epi == kernels.EPI_RESIDUAL:
         y = prev.double() + y
+    if epi == kernels.EPI_RELU2:
+        y = torch.relu(y) ** 2
     return y
 
 
@@ -394,7 +396,8 @@ def test_linear_mfma_slices_straight_into_lds(n, k, o, epi, o_dt, shape):
 @pytest.mark.parametrize("n,k,o", [(1, 64, 16), (300, 64, 257), (513, 512, 520), (256, 128, 384), (1000, 192, 130), (130, 256, 400),
                                    (257, 320, 193)])
 @pytest.mark.parametrize("epi,o_dt", [(kernels.EPI_NONE, "bfloat16"), (kernels.EPI_NONE, "float32"),
-                                      (kernels.EPI_GELU, "bfloat16"), (kernels.EPI_RESIDUAL, "float32")])
+                                      (kernels.EPI_GELU, "bfloat16"), (kernels.EPI_RELU2, "bfloat16"),
+                                      (kernels.EPI_RESIDUAL, "float32")])
 @pytest.mark.parametrize("shape", [13, 14, 15, 16])
 def test_linear_mfma_with_its_halves_out_of_step(n, k, o, epi, o_dt, shape):
     """The variants whose two halves read and multiply in turn (256 x 256, 128 x 256, 256 x 192 and 128 x 192), at sizes that cut
@@ -475,6 +478,64 @@ def test_linear_mfma_of_many_rows_keeps_two_chains_of_float32_sums(n, k, o, epi)
     assert kernels.linear_mfma(a, w, bias, out, n, epi)
     assert kernels.linear_mfma(a, w, bias, groups, n, epi, shape=7)
     assert torch.equal(out, groups)
+
+
+@pytest.mark.parametrize("pairs,experts,k,o,epi,dt", [
+    (700, 5, 1024, 2048, kernels.EPI_RELU2, "bfloat16"), (900, 9, 2048, 2816, kernels.EPI_NONE, "bfloat16"),
+    (1900, 7, 2048, 2816, kernels.EPI_RELU2, "bfloat16"), (900, 9, 768, 2560, kernels.EPI_NONE, "bfloat16"),
+    (700, 5, 768, 2600, kernels.EPI_NONE, "float32"), (2000, 17, 768, 1040, kernels.EPI_NONE, "float32"),
+    (1500, 14, 4096, 1024, kernels.EPI_NONE, "float32")])
+def test_grouped_products_of_many_rows(pairs, experts, k, o, epi, dt):
+    """Experts' products through the large variants (inner sizes of 12 steps and more, 140 tiles and more): runs that end inside a
+    group of 256 slots, an expert without pairs, groups that nobody uses; every used row has the bits of its expert's own product
+    through the 32 x 32 tiles (two chains of sums: through the two wave groups), within the tolerance of the plain one."""
+    g = torch.Generator().manual_seed(pairs + o)
+    share = torch.rand(experts, generator=g) + 0.2
+    share[experts // 2] = 0.0
+    table = torch.multinomial(share, pairs, replacement=True, generator=g).to(torch.int32)[:, None].contiguous()
+    w = rnd(g, experts, o, k, dtype="bfloat16", scale=k ** -0.5).to(DEV)
+    h = rnd(g, pairs, k, dtype="bfloat16").to(DEV)
+    slots = kernels.expert_slots(pairs, 1, experts, 256)
+    st, sp, te = (torch.zeros(n, dtype=torch.int32, device=DEV) for n in (slots, slots, slots // 256))
+    kernels.expert_route(None, None, table.to(DEV), pairs, experts, st, sp, te, 256)
+    rows = torch.zeros(slots, k, dtype=torch.bfloat16, device=DEV)
+    assert kernels.gather_rows(h, st, rows, slots)
+    out = torch.full((slots, o), 7.0, dtype=TDT[dt], device=DEV)
+    shape = kernels.linear_mfma_choice(slots, o, k, TDT[dt], epi, grouped=True)
+    assert shape >= 10 and int((te < 0).sum()) > 0
+    assert kernels.grouped_linear_tiled(rows, w, te, st, out, slots, epi)
+    for e in range(experts):
+        mine = (table[:, 0] == e).nonzero().flatten().to(DEV)
+        if e == experts // 2:
+            assert len(mine) == 0
+            continue
+        used = ((te.repeat_interleave(256) == e) & (st >= 0)).nonzero().flatten()
+        assert sorted(st[used].tolist()) == mine.tolist()
+        own = torch.empty(len(used), o, dtype=TDT[dt], device=DEV)
+        assert kernels.linear_mfma(rows[used], w[e], None, own, len(used), epi, shape=7 if shape >= 17 else 4)
+        assert torch.equal(out[used], own), f"expert {e}, shape {shape}"
+        plain = rows[used].double() @ w[e].double().T
+        want = torch.relu(plain) ** 2 if epi == kernels.EPI_RELU2 else plain
+        helpers.assert_close(own, want, "bfloat16", f"expert {e}")
+
+
+@pytest.mark.parametrize("n,k,o,shape", [(2304, 768, 5632, 13), (1600, 1024, 4096, 14), (2500, 1024, 4096, 15), (1500, 1024, 2816, 16),
+                                         (2048, 1024, 2048, 10)])
+def test_xielu_behind_a_product_of_many_rows(n, k, o, shape):
+    """The activation as the epilogue of the large variants: the bits of the same product through few rows at a time."""
+    g = torch.Generator().manual_seed(n)
+    assert kernels.linear_mfma_choice(n, o, k, torch.bfloat16) == shape
+    a, w = rnd(g, n, k, dtype="bfloat16").to(DEV), rnd(g, o, k, dtype="bfloat16", scale=k ** -0.5).to(DEV)
+    bias, coef = rnd(g, o).to(DEV), torch.tensor([0.8, 1.3], device=DEV)
+    out, few = (torch.empty(n, o, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    assert kernels.linear_mfma_xielu(a, w, bias, out, n, coef)
+    for r in range(0, n, 256):
+        rows = min(256, n - r)                 # under 512: none of the large variants
+        assert kernels.linear_mfma_xielu(a[r:r + rows], w, bias, few[r:r + rows], rows, coef)
+    assert torch.equal(out, few)
+    v = a.double() @ w.double().T + bias.double()
+    want = torch.where(v > 0, 0.8 * v * v, 1.3 * (torch.expm1(v.clamp(max=0)) - v)) + v / 2
+    helpers.assert_close(out, want, "bfloat16", "xielu")
 
 
 @pytest.mark.parametrize("n,shape,k", [(300, 13, 64), (130, 14, 192), (520, 15, 128), (257, 16, 256)])

@@ -286,7 +286,10 @@ __device__ __forceinline__ void mfma_join_chains(f32x4_t (&chain)[CHAINS][WTN][W
 // waves, too few to cover each other's waits for LDS and the barrier.
 // CHAINS: 2 = an element's sum is two chains, over the first and over the second halves of the steps, added at the end: what two
 // wave groups make (the same bits), with the accumulators of both in one wave.
-template <int WTM, int WTN, int WVM, int WVN, int EPI, typename OT, int AHEAD = 1, int KG = 1, int DIRECT = 0, int CHAINS = 1>
+// FOLD: > 0 = chains of that many steps, each added to the chains before it (with operands on their way in registers without a
+// branch: where control flow joins the compiler waits for every load in flight).
+template <int WTM, int WTN, int WVM, int WVN, int EPI, typename OT, int AHEAD = 1, int KG = 1, int DIRECT = 0, int CHAINS = 1,
+          int FOLD = 0>
 __global__ __launch_bounds__(64 * WVM * WVN * KG) void linear_mfma_kernel(
     const bf16_t* __restrict__ act, long lda, const bf16_t* __restrict__ w,
     const float* __restrict__ bias, OT* __restrict__ out, long ldo, int n_rows, int n_out, int k_dim,
@@ -294,6 +297,7 @@ __global__ __launch_bounds__(64 * WVM * WVN * KG) void linear_mfma_kernel(
   static_assert(KG == 1 || (KG == 2 && sizeof(OT) == 4 && AHEAD == 1), "two wave groups: float32 outputs");
   static_assert(DIRECT == 0 || (DIRECT >= 2 && AHEAD == 1 && KG == 1), "slices straight into LDS: two stages or more");
   static_assert(CHAINS == 1 || (CHAINS == 2 && KG == 1), "two wave groups are two chains already");
+  static_assert(FOLD == 0 || (CHAINS == 1 && KG == 1), "one way of keeping chains short");
   constexpr int T = 64 * WVM * WVN * KG;
   constexpr int STAGES = DIRECT > 0 ? DIRECT : 2;   // slices of a step that LDS holds
   constexpr int HALVES = (MM_BK / 32) / KG;   // halves of a step along k that a wave multiplies
@@ -381,6 +385,13 @@ __global__ __launch_bounds__(64 * WVM * WVN * KG) void linear_mfma_kernel(
 #pragma unroll
       for (int j = 0; j < WTM; ++j) chain[c][i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
   auto& acc = chain[0];
+  [[maybe_unused]] f32x4_t folded[WTN][WTM];
+  if constexpr (FOLD > 0) {
+#pragma unroll
+    for (int i = 0; i < WTN; ++i)
+#pragma unroll
+      for (int j = 0; j < WTM; ++j) folded[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  }
 
   const int k_steps = (k_len + MM_BK - 1) / MM_BK;
   const int c0 = ((lane >> 4) ^ (lrow & 7)) * 8;  // this lane's chunk of an operand row, first half of a step
@@ -435,6 +446,20 @@ __global__ __launch_bounds__(64 * WVM * WVN * KG) void linear_mfma_kernel(
         sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[g / WTM][i], af[g % 3], sum, 0, 0, 0);
       }
       __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (FOLD > 0) {
+      const bool ends = s % FOLD == FOLD - 1;
+      if (DIRECT == 0 || ends) {
+#pragma unroll
+        for (int i = 0; i < WTN; ++i)
+#pragma unroll
+          for (int j = 0; j < WTM; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              folded[i][j][e] += ends ? acc[i][j][e] : 0.f;
+              acc[i][j][e] = ends ? 0.f : acc[i][j][e];
+            }
+      }
     }
     if (decltype(store_next)::value) __syncthreads();  // the other buffer's readers finished before the last barrier
   };
@@ -573,6 +598,14 @@ __global__ __launch_bounds__(64 * WVM * WVN * KG) void linear_mfma_kernel(
       }
   }
   mfma_join_chains(chain);
+  if constexpr (FOLD > 0) {
+#pragma unroll
+    for (int i = 0; i < WTN; ++i)
+#pragma unroll
+      for (int j = 0; j < WTM; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[i][j][e] = folded[i][j][e] + acc[i][j][e];
+  }
 
   mfma_epilogue<WTM, WTN, WVM, WVN, T, STAGES * (BM + BN) * MM_LD, EPI, OT>(acc, lds, bias, out, ldo, n_rows, n_out, row0,
                                                                             col0, wr, wc, sc);
@@ -801,14 +834,14 @@ int launch_halves(const void* act, long lda, const void* w, const float* bias, v
 #undef MM_LAUNCH
   return MGPT_ERR_BAD_DTYPE;
 }
-template <int WTM, int WTN, int WVM, int WVN, int EPI, typename OT, int AHEAD, int KG = 1, int DIRECT = 0, int CHAINS = 1>
+template <int WTM, int WTN, int WVM, int WVN, int EPI, typename OT, int AHEAD, int KG = 1, int DIRECT = 0, int CHAINS = 1, int FOLD = 0>
 int launch_one(const void* act, long lda, const void* w, const float* bias, void* out, long ldo, int n_rows,
                int n_out, int k_dim, int k_parts, long part_stride, const MfmaScatter& sc, hipStream_t stream) {
   static_assert(AHEAD >= 1 && AHEAD <= 4, "sets of staging registers");
   constexpr int BM = WVM * WTM * 16, BN = WVN * WTN * 16;
   constexpr size_t lds_bytes = (DIRECT > 0 ? DIRECT : 2ul) * (BM + BN) * MM_LD * sizeof(bf16_t);
   static_assert(lds_bytes <= 160 * 1024, "a workgroup's LDS");
-  auto kernel = linear_mfma_kernel<WTM, WTN, WVM, WVN, EPI, OT, AHEAD, KG, DIRECT, CHAINS>;
+  auto kernel = linear_mfma_kernel<WTM, WTN, WVM, WVN, EPI, OT, AHEAD, KG, DIRECT, CHAINS, FOLD>;
   static bool allowed = false;  // more LDS than a kernel gets without asking
   if (!allowed) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
@@ -863,6 +896,7 @@ constexpr int MM_SHAPES = 5;
 constexpr int MM_TILE_ROWS[MM_SHAPES] = {256, 128, 128, 64, 32};
 constexpr int MM_TILE_COLS[MM_SHAPES] = {256, 256, 64, 64, 32};
 constexpr int MM_MAX_PARTS = 8;
+constexpr int MM_FOLD = 2;   // steps of a chain where chains are kept short
 constexpr int MM_AHEAD = 4;  // steps on their way from memory in the variant for few tiles over a large matrix
 // Shape ids from MM_DIRECT_FIRST on: the variants whose slices go from memory straight into LDS, by tile
 // (rows x columns), waves and stages: 32 x 32 (four waves of 16 x 16) and 64 x 64 (four of 32 x 32) with four
@@ -874,9 +908,9 @@ constexpr int MM_DIRECT_ROWS[MM_DIRECT_VARIANTS] = {32, 64, 128, 128, 32, 256, 1
 constexpr int MM_DIRECT_COLS[MM_DIRECT_VARIANTS] = {32, 64, 64, 192, 32, 256, 256, 192, 192};
 constexpr int MM_DIRECT_HALVES = 5;     // the first of the four variants with the halves out of step: 256 x 256, 128 x 256,
                                         // 256 x 192, 128 x 192
-// then the same variants with two chains of sums (float32 outputs; those of 32 x 32, 128 x 64 and 128 rows out of step have them)
+// then the same variants with two chains of sums (float32 outputs; those of 128 x 64 and of 128 rows out of step have them)
 constexpr int MM_CHAINS_FIRST = MM_DIRECT_FIRST + MM_DIRECT_VARIANTS;
-constexpr bool MM_HAS_CHAINS[MM_DIRECT_VARIANTS] = {true, false, true, false, true, false, true, false, true};
+constexpr bool MM_HAS_CHAINS[MM_DIRECT_VARIANTS] = {false, false, true, false, false, false, true, false, true};
 constexpr int MM_SHAPE_IDS = MM_CHAINS_FIRST + MM_DIRECT_VARIANTS;
 
 long tiles_of(int shape, int n_rows, int n_out) {
@@ -1082,9 +1116,9 @@ int choose_medium(int n_rows, int n_out, int k_dim) {
 //
 // Grouped rows (experts) count with their padding, which comes last in a group and in the call: the XCDs take equal stretches of all
 // tiles, so those that got the used ones take the time (counted by used tiles the choice was 8 % slower in the mean of 224 products
-// of 512 to 24,000 pairs for 8 to 64 experts, and up to 54 %; counted as here it is 8 % faster than the rules above).  Where a group's second half is padding, the two workgroups that
-// share a unit leave it to one of them: 128 x 192 then win by up to 14 % what would be a tie (16 experts 1024 -> 2048, 512 pairs:
-// 23.9 us, 256 x 192 26.5).
+// of 512 to 24,000 pairs for 8 to 64 experts, and up to 54 %; counted as here it is 8 % faster than the rules above).  Where a
+// group's second half is padding, the two workgroups that share a unit leave it to one of them: 128 x 192 then win by up to 14 %
+// what would be a tie (16 experts 1024 -> 2048, 512 pairs: 23.9 us, 256 x 192 26.5).
 int choose_large(int n_rows, int n_out, int k_dim, bool added, bool grouped, bool chains, double* least) {
   const int steps = k_dim / MM_BK;
   if (n_rows < 512 || n_out < 512 || steps < 12) return -1;
@@ -1221,6 +1255,10 @@ int launch_any(int shape, int k_parts, const void* act, long lda, const void* w,
     }
   }
   const bool split = k_parts > 1;
+  // Up to 32 rows under a narrow output and a long inner size, where these tiles stand in for the decode kernel, whose sums are 16
+  // chains: chains of two steps.  Error of 16 rows 6400 -> 1600 against 64 bits, relative to the sums' norm: decode kernel
+  // 1.35e-7, eight stretches of one chain 1.84e-7, of short ones 1.02e-7; 6.5 and 6.8 us.
+  const bool fold = !forced && split && shape == 4 && n_rows <= 32 && n_out < 4096 && k_dim > 4096;
   if (two_groups) {
     // forced: what this kernel stores must be float32, plain or added into the residual stream (the sums of
     // a split product are)
@@ -1242,12 +1280,16 @@ int launch_any(int shape, int k_parts, const void* act, long lda, const void* w,
   const long ld = split ? n_out : ldo, stride = split ? (long)n_rows * n_out : 0;
 #define MM_ARGS act, lda, w, b, dst, dt, ld, n_rows, n_out, k_dim, epi, k_parts, stride, sc, stream
   int rc = MGPT_ERR_BAD_SHAPE;
+#define MM_FOLD_ARGS act, lda, w, b, dst, ld, n_rows, n_out, k_dim, k_parts, stride, sc, stream
 #define MM_HALVES_ARGS act, lda, w, b, dst, dt, ld, n_rows, n_out, k_dim, epi, sc, stream
-  if (direct >= 0 && chains) {
+  if (fold) {
+    rc = direct == 4   ? launch_one<1, 1, 2, 2, MM_EPI_NONE, float, 1, 1, 6, 1, MM_FOLD>(MM_FOLD_ARGS)
+         : direct == 0 ? launch_one<1, 1, 2, 2, MM_EPI_NONE, float, 1, 1, 4, 1, MM_FOLD>(MM_FOLD_ARGS)
+         : ahead > 1   ? launch_one<1, 1, 2, 2, MM_EPI_NONE, float, MM_AHEAD, 1, 0, 1, MM_FOLD>(MM_FOLD_ARGS)
+                       : launch_one<1, 1, 2, 2, MM_EPI_NONE, float, 1, 1, 0, 1, MM_FOLD>(MM_FOLD_ARGS);
+  } else if (direct >= 0 && chains) {
     switch (direct) {
-      case 0: rc = launch_shape<1, 1, 2, 2, 1, 4, 2>(MM_ARGS); break;
       case 2: rc = launch_shape<2, 2, 4, 2, 1, 3, 2>(MM_ARGS); break;
-      case 4: rc = launch_shape<1, 1, 2, 2, 1, 6, 2>(MM_ARGS); break;
       case 6: rc = launch_halves<4, 4, 2>(MM_HALVES_ARGS); break;
       case 8: rc = launch_halves<4, 3, 2>(MM_HALVES_ARGS); break;
       default: break;
@@ -1279,6 +1321,7 @@ int launch_any(int shape, int k_parts, const void* act, long lda, const void* w,
       break;
   }
 #undef MM_HALVES_ARGS
+#undef MM_FOLD_ARGS
 #undef MM_ARGS
   if (rc != MGPT_OK || !split || leave_parts) return rc;
   return launch_join(partials, k_parts, bias, out, out_dtype, ldo, n_rows, n_out, epilogue, stream, sc.epi_coef);
@@ -1347,8 +1390,8 @@ extern "C" int mgpt_linear_mfma_xielu(const void* act, long lda, const void* w, 
 // 7 = 64 x 64 with two wave groups a tile (float32 outputs), 8 to 12 = the slices straight into LDS: 32 x 32 and
 // 64 x 64 with four stages, 128 x 64 with three, 128 x 192 with two, 32 x 32 with six (an inner size of whole steps of 64 and operands
 // aligned to 16 bytes, else refused), 13 to 16 = the halves out of step, 256 x 256, 128 x 256, 256 x 192, 128 x 192 (the same
-// conditions, and never split), 17, 19, 21, 23 and 25 = 8, 10, 12, 14 and 16 with two chains of sums (float32 outputs);
-// negative: chosen) and the number of stretches of the inner size given
+// conditions, and never split), 19, 23 and 25 = 10, 14 and 16 with two chains of sums (float32 outputs); negative:
+// chosen) and the number of stretches of the inner size given
 // (k_parts as for launch_any above), instead of chosen by the size: for tests and measurements.
 extern "C" int mgpt_linear_mfma_shape(int shape, int k_parts, const void* act, long lda, const void* w,
                                       const float* bias, void* out, int out_dtype, long ldo, int n_rows,

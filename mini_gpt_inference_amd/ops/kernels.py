@@ -742,7 +742,7 @@ def linear_mfma(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], 
     steps on their way from memory, 7 = 64 x 64 with two wave groups that share a tile, float32 outputs, 8 to 12 = operand slices straight
     into LDS with tiles of 32 x 32, 64 x 64, 128 x 64, 128 x 192, 32 x 32 with six stages, 13 to 16 = the same with the
     workgroup's halves out of step and tiles of 256 x 256, 128 x 256, 256 x 192, 128 x 192: an inner size that is a
-    multiple of 64, 17, 19, 21, 23 and 25 = 8, 10, 12, 14 and 16 with float32 sums in two chains, as 7 makes them) and
+    multiple of 64, 19, 23 and 25 = 10, 14 and 16 with float32 sums in two chains, as 7 makes them) and
     `k_parts` fix what the library otherwise chooses by the size.  False when it does not take the shape."""
     if a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
         return False

@@ -428,3 +428,30 @@ def test_addition_of_few_rows_under_a_long_inner_size(rows, n_out, k_dim):
         if ctx.pending is not None:
             assert kernels.residual_settle(ctx.pending, got, rows)
         helpers.assert_close(got, want, "bfloat16", "x + product")
+
+
+@pytest.mark.parametrize("rows", [9, 17, 32])
+@pytest.mark.parametrize("n_out,k_dim", [(1600, 6400), (1152, 4608), (1280, 4112)])
+def test_addition_of_few_rows_is_no_less_exact_in_the_tiled_kernel(rows, n_out, k_dim):
+    """Where the tiled kernel's split stands in for the decode kernel's: its float32 sums are no further from 64 bits."""
+    from types import SimpleNamespace
+
+    from mini_gpt_inference_amd.ops import linear as L
+    from mini_gpt_inference_amd.parts.base import Workspace
+
+    g = torch.Generator().manual_seed(rows)
+    a, w, b = bf(rnd(g, rows, k_dim)).to(DEV), bf(rnd(g, n_out, k_dim, scale=0.03)).to(DEV), rnd(g, n_out).to(DEV)
+    want = a.double() @ w.double().T + b.double()
+    error = lambda t: ((t.double() - want).norm() / want.norm()).item()
+    decode = torch.zeros(rows, n_out, device=DEV)
+    need = kernels.linear_skinny_partials(rows, n_out, k_dim, False, kernels.EPI_RESIDUAL)
+    parts = torch.empty(need, device=DEV) if need else None
+    assert kernels.linear_skinny(a, w, b, decode, rows, kernels.EPI_RESIDUAL, partials=parts)
+    for left in (True, False):
+        ctx = SimpleNamespace(exact=False, dtype=torch.bfloat16, n_rows=rows, pending=None, copy_budget=None,
+                              workspace=Workspace(torch.device(DEV)))
+        got = torch.zeros_like(decode)
+        L.linear_add(ctx, a, w, b, got, rows, may_leave_parts=left)
+        if ctx.pending is not None:
+            assert kernels.residual_settle(ctx.pending, got, rows)
+        assert error(got) <= 1.01 * error(decode), (left, error(got), error(decode))

@@ -452,7 +452,7 @@ def test_linear_mfma_of_many_rows_keeps_its_sums_whatever_the_tile(n, k, o):
 
 @pytest.mark.parametrize("n,k,o", [(1, 64, 16), (300, 64, 257), (513, 512, 520), (256, 128, 384), (1000, 192, 130), (257, 320, 193)])
 @pytest.mark.parametrize("epi", [kernels.EPI_NONE, kernels.EPI_RESIDUAL])
-@pytest.mark.parametrize("shape", [17, 19, 21, 23, 25])
+@pytest.mark.parametrize("shape", [19, 23, 25])
 def test_linear_mfma_with_two_chains_of_sums(n, k, o, epi, shape):
     """The variants whose float32 sums are two chains, at sizes that cut their tiles and at 1, 2, 3, 5 and 8 steps: the bits of
     the two wave groups that share a 64 x 64 tile, each a chain over its half of every step."""

@@ -429,15 +429,15 @@ static int launch_rows(const ExactArgs& a, hipStream_t stream) {
   return mgpt_last_error();
 }
 
-enum { EX_ROWS, EX_TILE64, EX_TILE128 };
+enum { EX_ROWS, EX_TILE64, EX_TILE128, EX_LDS32, EX_LDS64, EX_LDS128 };   // the last three: slices straight into LDS
 
 // The kernel that takes least by what was measured (us; a call's fixed part is the same for all): the rows kernel by its
-// rate; a tile kernel by the rounds of 256 workgroups that it needs, a round of 64 x 64 tiles 0.019 us a k (0.0225 alone on
-// a compute unit), of 128 x 128 tiles 0.068.  Rows kernel / 64 / 128, us: 64 rows 768 -> 2304 12.1 / 22 / 60; 256 rows
-// 32.9 / 23.3 / 61; 1,100 rows 116 / 48.7 / 63; 256 rows 3072 -> 768 41 / 78 / 223; 1,100 rows 512 -> 50304 1525 / 536 / 512.
-// The 64 x 64 FMA tiles that these kernels replace reached 10 to 15 TFLOP/s (1,100 rows 2048 -> 512: 163 us, here 54), the
-// FMA kernel for few rows took 57 us for 16 rows 3072 -> 768 (here 14).
-extern "C" int mgpt_linear_exact_kernel(int n_rows, int n_out, int k_dim) {
+// rate, 34 TFLOP/s against these tiles, whose calls cost 2 us more; a tile kernel by the rounds of 256 workgroups that it needs, a
+// round of 64 x 64 tiles 0.019 us a k (0.0225 alone on a compute unit), of 128 x 128 tiles 0.068.  Rows kernel / 64 / 128, us: 64 rows
+// 768 -> 2304 12.1 / 22 / 60; 256 rows 32.9 / 23.3 / 61; 1,100 rows 116 / 48.7 / 63; 256 rows 3072 -> 768 41 / 78 / 223; 1,100 rows
+// 512 -> 50304 1525 / 536 / 512.  The 64 x 64 FMA tiles that these kernels replace reached 10 to 15 TFLOP/s (1,100 rows
+// 2048 -> 512: 163 us, here 54), the FMA kernel for few rows took 57 us for 16 rows 3072 -> 768 (here 14).
+static int rows_or_tiles(int n_rows, int n_out, int k_dim) {
   if ((long)n_rows * n_out <= 380000) return EX_ROWS;   // less than one round of either tile (and no divisions on the host)
   const double k = k_dim, rows = 2.0 * n_rows * n_out * k / 34e6;
   auto rounds = [&](int b) {
@@ -451,11 +451,11 @@ extern "C" int mgpt_linear_exact_kernel(int n_rows, int n_out, int k_dim) {
 
 // Whether tiles of 32 x 32 take the place of the kernel above (inner sizes of whole steps, aligned operands): several of their
 // workgroups share a compute unit, so few tiles spread over the chip evenly.  us a k with one, two, three and n of them on a
-// compute unit 0.010, 0.014, 0.019, 0.0065 n; the rows kernel at 29 TFLOP/s.  Rows kernel or 64 x 64 tiles / here, us: 100 rows
-// 768 -> 2304 15.7 / 13.8; 300 rows 768 -> 768 15.7 / 10.5, 3072 -> 768 51.9 / 33.6; 600 rows 512 -> 512 13.9 / 9.9, 5120 -> 1280
-// 107 / 97; 1,201 rows 2048 -> 512 45.3 / 40.8; 400 rows 512 -> 2048 14.8 / 17.6 (not taken).
-extern "C" int mgpt_linear_exact_small_tiles(int n_rows, int n_out, int k_dim) {
-  if (k_dim % EX_BK != 0 || (long)n_rows * n_out <= 145000) return 0;   // the rows kernel takes less than one round of these
+// compute unit 0.010, 0.014, 0.019, 0.0065 n; the rows kernel at 29 TFLOP/s, a call of either costing the same.  Rows kernel or
+// 64 x 64 tiles / here, us: 100 rows 768 -> 2304 15.7 / 13.8; 300 rows 768 -> 768 15.7 / 10.5, 3072 -> 768 51.9 / 33.6; 600 rows
+// 512 -> 512 13.9 / 9.9, 5120 -> 1280 107 / 97; 1,201 rows 2048 -> 512 45.3 / 40.8; 400 rows 512 -> 2048 14.8 / 17.6 (not taken).
+static bool small_tiles(int n_rows, int n_out, int k_dim) {
+  if ((long)n_rows * n_out <= 145000) return false;   // the rows kernel takes less than one round of these
   const double k = k_dim, rows = 2.0 * n_rows * n_out * k / 29e6;
   auto per_unit = [&](int b) {
     const long tiles = (long)((n_rows + b - 1) / b) * ((n_out + b - 1) / b);
@@ -466,14 +466,36 @@ extern "C" int mgpt_linear_exact_small_tiles(int n_rows, int n_out, int k_dim) {
   return t32 < rows && t32 < t64 && t32 < t128;
 }
 
+// The kernel for a product; aligned: rows of both operands start 16 bytes apart at least, as loads straight into LDS want them
+// beside an inner size of whole steps.  Tiles whose slices go straight into LDS come two to a compute unit (64 KB each), through
+// registers up to five of 64 x 64.  So 64 x 64 tiles stay with the registers for short inner sizes where the chip has more than two
+// each (7,000 rows 64 -> 3000 38.6 us, straight into LDS 46.0; 4,400 rows 128 -> 3000 41.4 / 44.2; 1,500 rows 96 -> 2000 11.5 / 12.1)
+// and where there is one part round more (700 rows 256 -> 3000, 517 tiles, 19.8 / 20.6); 128 x 128 tiles where a second round is half
+// full: its workgroups come two to a unit then, on the units that end first (4,000 rows 768 -> 3072, 768 tiles, 170 / 202; 3,800 rows
+// 640 -> 3072 142 / 168; 7,000 rows 384 -> 1500 92 / 109; from inner sizes of about 1,152 on the units end far enough apart: 3,800 rows
+// 1152 -> 3072 243 / 239, 1280 -> 3840 270 / 257).
+static int exact_kernel(int n_rows, int n_out, int k_dim, bool aligned) {
+  const int kernel = rows_or_tiles(n_rows, n_out, k_dim);
+  if (!aligned || k_dim % EX_BK != 0) return kernel;
+  if (small_tiles(n_rows, n_out, k_dim)) return EX_LDS32;
+  if (kernel == EX_ROWS) return kernel;
+  const int b = kernel == EX_TILE64 ? 64 : 128;
+  const long tiles = (long)((n_rows + b - 1) / b) * ((n_out + b - 1) / b);
+  if (kernel == EX_TILE64)
+    return tiles > 512 && (k_dim <= 96 || (k_dim <= 384 && tiles <= 768) || (k_dim < 224 && tiles > 2048)) ? EX_TILE64 : EX_LDS64;
+  return tiles > 640 && tiles <= 768 && k_dim >= 160 && k_dim < 1152 ? EX_TILE128 : EX_LDS128;
+}
+
+extern "C" int mgpt_linear_exact_kernel(int n_rows, int n_out, int k_dim, int aligned) {
+  return exact_kernel(n_rows, n_out, k_dim, aligned != 0);
+}
+
 template <int EPI, bool VEC>
 static int launch_kernel(const ExactArgs& a, int kernel, hipStream_t stream) {
   if constexpr (VEC) {
-    if (a.k_dim % EX_BK == 0) {                      // slices straight into LDS
-      if (mgpt_linear_exact_small_tiles(a.n_rows, a.n_out, a.k_dim)) return launch_tile<1, EPI, true, 6>(a, stream);
-      if (kernel == EX_TILE64) return launch_tile<2, EPI, true, 4>(a, stream);
-      if (kernel == EX_TILE128) return launch_tile<4, EPI, true, 2>(a, stream);
-    }
+    if (kernel == EX_LDS32) return launch_tile<1, EPI, true, 6>(a, stream);
+    if (kernel == EX_LDS64) return launch_tile<2, EPI, true, 4>(a, stream);
+    if (kernel == EX_LDS128) return launch_tile<4, EPI, true, 2>(a, stream);
   }
   if (kernel == EX_ROWS) return launch_rows<EPI, VEC>(a, stream);
   return kernel == EX_TILE64 ? launch_tile<2, EPI, VEC, 0>(a, stream) : launch_tile<4, EPI, VEC, 0>(a, stream);
@@ -483,7 +505,7 @@ int mgpt_linear_exact_launch(const float* A, long lda, const float* W, const flo
                              int n_out, int k_dim, int epi, const ExactScatter& sc, hipStream_t stream) {
   const ExactArgs a = {A, lda, W, bias, out, ldo, n_rows, n_out, k_dim, sc};
   const bool vec = k_dim % 4 == 0 && lda % 4 == 0 && ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(W)) & 15) == 0;
-  const int kernel = mgpt_linear_exact_kernel(n_rows, n_out, k_dim);
+  const int kernel = exact_kernel(n_rows, n_out, k_dim, vec);
 #define EX_LAUNCH(E) return vec ? launch_kernel<E, true>(a, kernel, stream) : launch_kernel<E, false>(a, kernel, stream)
   if (epi == EPI_NONE) EX_LAUNCH(EPI_NONE);
   if (epi == EPI_GELU) EX_LAUNCH(EPI_GELU);

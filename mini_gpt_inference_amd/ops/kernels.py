@@ -159,15 +159,13 @@ def linear_generic(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor
     _check(rc, "linear_generic")
 
 
-def linear_exact_kernel(n_rows: int, n_out: int, k_dim: int) -> str:
-    """Which of its kernels a float32 product of this size goes to: "rows", "tile64" or "tile128" (or, in the place of any,
-    32 x 32 tiles: linear_exact_small_tiles)."""
-    return ("rows", "tile64", "tile128")[library.kernels().mgpt_linear_exact_kernel(n_rows, n_out, k_dim)]
+EXACT_KERNELS = ("rows", "tile64", "tile128", "lds32", "lds64", "lds128")
 
 
-def linear_exact_small_tiles(n_rows: int, n_out: int, k_dim: int) -> bool:
-    """Whether a float32 product of this size with aligned operands goes to tiles of 32 x 32."""
-    return bool(library.kernels().mgpt_linear_exact_small_tiles(n_rows, n_out, k_dim))
+def linear_exact_kernel(n_rows: int, n_out: int, k_dim: int, aligned: bool = True) -> str:
+    """Which of its kernels a float32 product of this size goes to: one for few rows, tiles of 64 x 64 or 128 x 128, or tiles of
+    32 x 32, 64 x 64 or 128 x 128 whose slices go straight into LDS (operands whose rows are aligned to 16 bytes only)."""
+    return EXACT_KERNELS[library.kernels().mgpt_linear_exact_kernel(n_rows, n_out, k_dim, int(aligned))]
 
 
 EXACT_BLOCK = 256       # k whose sum is one part of a float32 product
@@ -184,7 +182,7 @@ def linear_exact_leaves_parts(a: torch.Tensor, w: torch.Tensor, bias: Optional[t
     n_out, k_dim = w.shape
     return (a.dtype == w.dtype == x.dtype == torch.float32 and n_out % 4 == 0 and n_out <= 2048 and x.data_ptr() % 16 == 0
             and (bias is None or bias.data_ptr() % 16 == 0)
-            and linear_exact_kernel(n_rows, n_out, k_dim) == "rows")
+            and linear_exact_kernel(n_rows, n_out, k_dim, False) == "rows")
 
 
 def linear_exact_parts(a: torch.Tensor, w: torch.Tensor, sums: torch.Tensor, n_rows: int) -> None:

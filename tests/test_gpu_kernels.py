@@ -155,43 +155,58 @@ def test_linear_generic_takes_any_inner_size(a_dt, w_dt, o_dt, n, k):
 
 @pytest.mark.parametrize("k", [1, 15, 17, 64, 65, 128, 192, 193, 256, 258, 300, 512, 4100, 4352])
 def test_float32_product_keeps_its_sums_whatever_the_tiles(k):
-    """A product that is float32 throughout goes to one of three kernels by its size: a workgroup per 16 x 16 outputs with
-    a wave per 256 of k (several rounds of them beyond 16 waves), tiles of 64 x 64 and of 128 x 128.  An element's bits
-    are the same in all, also where rows of the operands are not 16-byte aligned; the error against 64 bits is that of
+    """A product that is float32 throughout goes to one of several kernels by its size: a workgroup per 16 x 16 outputs with
+    a wave per 256 of k (several rounds of them beyond 16 waves), tiles of 64 x 64 and of 128 x 128, and for inner sizes of whole
+    steps of 32 these and tiles of 32 x 32 with their slices straight into LDS.  An element's bits are the same in all, also where rows of the operands are not 16-byte aligned; the error against 64 bits is that of
     float32 sums (a chain of at most 64 groups of four products in a block of 256, then the blocks: below 1e-6 of the
     result's norm)."""
     g = torch.Generator().manual_seed(k)
     o, n = 3501, 1030                                  # 9 x 28 tiles of 128 x 128, all but the last row and column whole
     a, w, bias = rnd(g, n, k + 3).to(DEV), rnd(g, o, k).to(DEV), rnd(g, o).to(DEV)
     whole = torch.empty(n, o, device=DEV)
-    assert kernels.linear_exact_kernel(n, o, k) == "tile128"
+    assert kernels.linear_exact_kernel(n, o, k, aligned=False) == "tile128"
     kernels.linear_generic(a[:, :k], w, bias, whole, n)          # a row stride that is not the inner size
     want = a[:, :k].double() @ w.double().T + bias.double()
     assert ((whole.double() - want).norm() / want.norm()).item() < 1e-6
     used = set()
     for rows, cols in ((1, o), (16, o), (17, 37), (70, 200), (130, o), (300, 515), (n, 130), (n, 1500), (1025, 3456), (n, 3500)):
-        used.add(kernels.linear_exact_kernel(rows, cols, k))
+        used.add(kernels.linear_exact_kernel(rows, cols, k, aligned=k % 4 == 0))
         part = torch.full((rows + 1, cols), 7.0, device=DEV)
         kernels.linear_generic(a[:rows, :k].contiguous(), w[:cols].contiguous(), bias[:cols].contiguous(), part, rows)
         assert torch.equal(part[:rows], whole[:rows, :cols]), f"{rows} rows, {cols} columns"
         assert (part[rows] == 7.0).all()
-    assert used == {"rows", "tile64", "tile128"}
+    assert used == ({"rows", "tile64", "tile128"} if k % 32 else {"rows", "lds32", "lds64", "lds128"})
 
 
 @pytest.mark.parametrize("epi", [kernels.EPI_NONE, kernels.EPI_GELU, kernels.EPI_RESIDUAL])
-@pytest.mark.parametrize("n,k,o,small", [(300, 768, 768, True), (97, 768, 2303, True), (129, 32, 1500, True), (600, 512, 515, True),
-                                         (1201, 2048, 512, True), (255, 96, 1024, True), (1030, 64, 1500, False),
-                                         (1030, 160, 3501, False)])
-def test_float32_product_straight_into_lds(n, k, o, small, epi):
+@pytest.mark.parametrize("n,k,o,kernel", [(300, 768, 768, "lds32"), (97, 768, 2303, "lds32"), (129, 32, 1500, "lds32"),
+                                          (600, 512, 515, "lds32"), (1201, 2048, 512, "lds32"), (255, 96, 1024, "lds32"),
+                                          (1030, 64, 1500, "lds64"), (400, 512, 2048, "lds64"), (1030, 160, 3501, "lds128"),
+                                          (1500, 96, 2000, "tile64"), (3400, 160, 3072, "tile128")])
+def test_float32_product_straight_into_lds(n, k, o, kernel, epi):
     """Slices that go straight into LDS (inner sizes of whole steps), in tiles of 32 x 32, 64 x 64 and 128 x 128 and at fewer
-    steps than stages, as many and more: the bits of the same product over rows that are not aligned for that."""
+    steps than stages, as many and more, and tiles of such sizes that stay with the registers: the bits of the same product over
+    rows that are not aligned for that."""
     g = torch.Generator().manual_seed(n + k)
-    assert kernels.linear_exact_small_tiles(n, o, k) == small
+    assert kernels.linear_exact_kernel(n, o, k) == kernel and not kernels.linear_exact_kernel(n, o, k, aligned=False).startswith("lds")
     a, w, bias, old = rnd(g, n, k + 1).to(DEV)[:, :k], rnd(g, o, k).to(DEV), rnd(g, o).to(DEV), rnd(g, n + 1, o).to(DEV)
     want, got = old.clone(), old.clone()
     kernels.linear_generic(a, w, bias, want, n, epi)
     kernels.linear_generic(a.contiguous(), w, bias, got, n, epi)
     assert torch.equal(got, want) and torch.equal(got[n], old[n])
+
+
+@pytest.mark.parametrize("n,k,o,kernel,unaligned", [
+    (16, 3072, 768, "rows", "rows"), (188, 768, 768, "rows", "rows"), (190, 768, 768, "lds32", "rows"),
+    (300, 768, 2304, "lds32", "tile64"), (400, 768, 2304, "lds64", "tile64"), (2000, 512, 2048, "lds128", "tile128"),
+    (2000, 96, 1000, "lds64", "tile64"), (2300, 96, 1000, "tile64", "tile64"),            # 512 and 576 tiles
+    (700, 384, 3000, "tile64", "tile64"), (1500, 384, 3000, "lds64", "tile64"),           # a third round hardly begun, or more
+    (2000, 192, 3000, "lds64", "tile64"), (4400, 192, 3000, "tile64", "tile64"), (4400, 256, 3000, "lds64", "tile64"),
+    (3400, 768, 3072, "tile128", "tile128"), (4096, 768, 3072, "tile128", "tile128"), (5000, 768, 3072, "lds128", "tile128"),
+    (4096, 1152, 3072, "lds128", "tile128"), (4096, 96, 3072, "lds128", "tile128")])
+def test_float32_product_kernel_by_size(n, k, o, kernel, unaligned):
+    """Both sides of the lines between the kernels."""
+    assert kernels.linear_exact_kernel(n, o, k) == kernel and kernels.linear_exact_kernel(n, o, k, aligned=False) == unaligned
 
 
 @pytest.mark.parametrize("epi", [kernels.EPI_GELU, kernels.EPI_RESIDUAL, kernels.EPI_RELU2])
@@ -204,13 +219,13 @@ def test_float32_product_epilogues_whatever_the_tiles(k, o, epi):
     plain = torch.empty(n, o, device=DEV)
     kernels.linear_generic(a, w, bias, plain, n)
     used, got = set(), {}
-    for rows, cols in ((n, o), (20, o), (300, 1540), (300, 1537)):
-        used.add(kernels.linear_exact_kernel(rows, cols, k))
+    for rows, cols in ((n, o), (20, o), (300, 1540), (300, 1537), (n, 1500)):
+        used.add(kernels.linear_exact_kernel(rows, cols, k, aligned=k % 4 == 0))
         out = old[:rows + 1, :cols].clone(memory_format=torch.contiguous_format)
         kernels.linear_generic(a[:rows].contiguous(), w[:cols].contiguous(), bias[:cols].contiguous(), out, rows, epi)
         got[rows, cols] = out[:rows]
         assert torch.equal(got[rows, cols], got[n, o][:rows, :cols]) and (rows == n or torch.equal(out[rows], old[rows, :cols]))
-    assert used == {"rows", "tile64", "tile128"}
+    assert used == ({"rows", "tile64", "tile128"} if k % 32 else {"rows", "lds32", "lds64", "lds128"})
     if epi == kernels.EPI_RESIDUAL:
         assert torch.equal(got[n, o], old + plain)
     elif epi == kernels.EPI_RELU2:
@@ -220,8 +235,8 @@ def test_float32_product_epilogues_whatever_the_tiles(k, o, epi):
 
 
 @pytest.mark.parametrize("n,k,h,hk,d,kernel", [
-    (1, 64, 4, 4, 16, "rows"), (16, 300, 3, 1, 10, "rows"), (40, 36, 3, 3, 12, "rows"), (300, 512, 8, 8, 64, "tile64"),
-    (1030, 256, 24, 20, 128, "tile64"), (70, 33, 1, 1, 33, "rows"), (1030, 256, 100, 37, 20, "tile128"),
+    (1, 64, 4, 4, 16, "rows"), (16, 300, 3, 1, 10, "rows"), (40, 36, 3, 3, 12, "rows"), (300, 512, 8, 8, 64, "lds32"),
+    (300, 36, 8, 8, 64, "tile64"), (1030, 256, 24, 20, 128, "lds64"), (70, 33, 1, 1, 33, "rows"), (1030, 256, 100, 37, 20, "lds128"),
     (1030, 65, 60, 23, 33, "tile128"), (1025, 300, 10, 9, 124, "tile128")])
 def test_float32_product_stores_keys_and_values(n, k, h, hk, d, kernel):
     """The projection that also stores its key and value columns into their pages: the same bits as the plain product
@@ -230,7 +245,7 @@ def test_float32_product_stores_keys_and_values(n, k, h, hk, d, kernel):
     g = torch.Generator().manual_seed(n)
     q_width, kv_width, page = h * d, hk * d, 5
     o = q_width + 2 * kv_width
-    assert kernels.linear_exact_kernel(n, o, k) == kernel
+    assert kernels.linear_exact_kernel(n, o, k, aligned=k % 4 == 0) == kernel
     a, w, bias = rnd(g, n, k).to(DEV), rnd(g, o, k).to(DEV), rnd(g, o).to(DEV)
     pages = -(-n // page) + 1
     slots = torch.randperm(pages * page, generator=g)[:n].to(torch.int32)

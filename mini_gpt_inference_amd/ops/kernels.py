@@ -175,14 +175,11 @@ def linear_exact_blocks(k_dim: int) -> int:
     return -(-k_dim // EXACT_BLOCK)
 
 
-def linear_exact_leaves_parts(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], x: torch.Tensor,
-                              n_rows: int) -> bool:
-    """Whether the sums over the blocks of k of a @ w.T may be left for the LayerNorm that reads x next: a product of few
-    rows, and rows that the kernel adding them up takes."""
-    n_out, k_dim = w.shape
+def linear_exact_takes_parts(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], x: torch.Tensor) -> bool:
+    """Whether linear_exact_parts takes these operands, and rows x the kernel that adds its sums up."""
+    n_out = w.shape[0]
     return (a.dtype == w.dtype == x.dtype == torch.float32 and n_out % 4 == 0 and n_out <= 2048 and x.data_ptr() % 16 == 0
-            and (bias is None or bias.data_ptr() % 16 == 0)
-            and linear_exact_kernel(n_rows, n_out, k_dim, False) == "rows")
+            and (bias is None or bias.data_ptr() % 16 == 0))
 
 
 def linear_exact_parts(a: torch.Tensor, w: torch.Tensor, sums: torch.Tensor, n_rows: int) -> None:

@@ -214,13 +214,23 @@ LEAVE_PARTS_MIN_ROWS = 8
 LEAVE_PARTS_MAX_ROWS = 256     # (the tiled kernel's split; the decode kernel's ends at its 64 rows)
 
 
-# The 32-bit path leaves the sums over the product's blocks of k for inner sizes from EXACT_PARTS_MIN_K on at any number of
-# rows, from EXACT_PARTS_MIN_K_ROWS on above EXACT_PARTS_FEW_ROWS rows (measured at the kernel, linear_exact.hip), and only
-# where the product would go to the kernel for few rows.
-EXACT_PARTS_MIN_K = 6 * 256 + 1
-EXACT_PARTS_MIN_K_ROWS = 2 * 256 + 1
-EXACT_PARTS_FEW_ROWS = 4
+# The 32-bit path leaves the sums over the product's blocks of k where that and the LayerNorm which adds them up take less than
+# the product and a plain LayerNorm: (inner size, rows) from which on, and up to how many outputs for short inner sizes and others.
+# us, product and LayerNorm / sums and LayerNorm: 768 -> 768 8.1 / 8.8 at 5 rows, 8.7 / 8.9 at 12, 9.4 / 8.9 at 16, 16.1 / 12.0 at 192,
+# 13.5 / 14.7 at 240 (through 32 x 32 tiles, as at all sizes that follow); 520 -> 520 7.5 / 8.1 at 5, 8.1 / 8.2 at 48; 1280 -> 1280
+# 9.4 / 9.7 at 1, 10.0 / 9.9 at 6, 16.9 / 12.5 at 64; 1600 -> 1600 10.4 / 10.3 at 1, 28.6 / 26.9 at 224, 28.9 / 29.7 at 240; 3072 -> 768
+# 13.6 / 9.3 at 1, 35.8 / 26.1 at 256; 6400 -> 1600 89.7 / 71.9 at 224; 2048 -> 2048 33.9 / 31.6 at 176, 35.3 / 35.7 at 208.
+EXACT_PARTS_FROM = ((6 * 256 + 1, 1), (1280, 6), (768, 16))
 EXACT_PARTS_MAX_ROWS = 256
+EXACT_PARTS_MAX_OUTPUTS = 380_000
+EXACT_PARTS_SHORT_K, EXACT_PARTS_SHORT_MAX_OUTPUTS = 1024, 172_000
+
+
+def exact_leaves_parts(n_rows: int, n_out: int, k_dim: int) -> bool:
+    """Whether the 32-bit path leaves a product of this size as sums over its blocks of k for the LayerNorm behind it."""
+    most = EXACT_PARTS_MAX_OUTPUTS if k_dim >= EXACT_PARTS_SHORT_K else EXACT_PARTS_SHORT_MAX_OUTPUTS
+    return (n_rows <= EXACT_PARTS_MAX_ROWS and n_rows * n_out <= most
+            and any(k_dim >= k and n_rows >= rows for k, rows in EXACT_PARTS_FROM))
 
 
 def plain_residual(ctx, h, x: torch.Tensor) -> None:
@@ -243,10 +253,9 @@ def linear_add(ctx, a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tenso
     workgroups' sums as the parts of a pending residual instead of running a second kernel that adds
     them into x; the LayerNorm that reads x next adds them up (LazyNorm.tensor).  The 32-bit path does so with the sums over
     the blocks of k that its products are made of, which has the bits of adding into x at once."""
-    if (may_leave_parts and ctx.exact and getattr(ctx, "pending", None) is None and 0 < n_rows <= EXACT_PARTS_MAX_ROWS
-            and n_rows == ctx.n_rows and w.shape[1] >= (EXACT_PARTS_MIN_K if n_rows <= EXACT_PARTS_FEW_ROWS
-                                                        else EXACT_PARTS_MIN_K_ROWS)
-            and x.is_contiguous() and x.shape[1] == w.shape[0] and kernels.linear_exact_leaves_parts(a, w, bias, x, n_rows)):
+    if (may_leave_parts and ctx.exact and getattr(ctx, "pending", None) is None and n_rows == ctx.n_rows
+            and exact_leaves_parts(n_rows, *w.shape) and x.is_contiguous() and x.shape[1] == w.shape[0]
+            and kernels.linear_exact_takes_parts(a, w, bias, x)):
         n_parts = kernels.linear_exact_blocks(w.shape[1])
         buf = ctx.workspace.get("residual_parts", n_parts * n_rows, w.shape[0], torch.float32)
         parts = buf[:n_parts * n_rows].view(n_parts, n_rows, w.shape[0])

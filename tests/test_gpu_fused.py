@@ -455,3 +455,26 @@ def test_addition_of_few_rows_is_no_less_exact_in_the_tiled_kernel(rows, n_out, 
         if ctx.pending is not None:
             assert kernels.residual_settle(ctx.pending, got, rows)
         assert error(got) <= 1.01 * error(decode), (left, error(got), error(decode))
+
+
+@pytest.mark.parametrize("rows,n_out,k_dim,left", [
+    (1, 768, 3072, True), (1, 400, 1536, False), (5, 1280, 1280, False), (6, 1280, 1280, True), (15, 768, 768, False),
+    (16, 768, 768, True), (64, 640, 640, False), (223, 768, 768, True), (224, 772, 768, False), (224, 772, 1024, True),
+    (256, 768, 3072, True), (257, 768, 3072, False), (185, 2048, 2048, True), (186, 2048, 2048, False)])
+def test_float32_addition_leaves_sums_where_that_pays(rows, n_out, k_dim, left):
+    """ops.linear.linear_add in 32 bits on both sides of its lines: x + product either way, with the same bits."""
+    from types import SimpleNamespace
+
+    from mini_gpt_inference_amd.ops import linear as L
+    from mini_gpt_inference_amd.parts.base import Workspace
+
+    g = torch.Generator().manual_seed(rows)
+    a, w, b, x = rnd(g, rows, k_dim).to(DEV), rnd(g, n_out, k_dim, scale=0.03).to(DEV), rnd(g, n_out).to(DEV), rnd(g, rows, n_out).to(DEV)
+    want, got = x.clone(), x.clone()
+    kernels.linear_generic(a, w, b, want, rows, kernels.EPI_RESIDUAL)
+    ctx = SimpleNamespace(exact=True, dtype=torch.float32, n_rows=rows, pending=None, workspace=Workspace(torch.device(DEV)))
+    L.linear_add(ctx, a, w, b, got, rows, may_leave_parts=True)
+    assert (ctx.pending is not None) == left
+    if left:
+        assert torch.equal(got, x) and kernels.residual_settle(ctx.pending, got, rows)
+    assert torch.equal(got, want)

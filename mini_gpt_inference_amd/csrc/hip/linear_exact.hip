@@ -60,15 +60,16 @@ __device__ __forceinline__ ex_f4 ex_load(const float* __restrict__ row, int k, i
 }
 
 // Many rows: a workgroup of four waves per tile of 32 T rows x 32 T columns, a wave 16 T x 16 T of them; steps of 32 k
-// through two buffers of LDS, rows of 128 bytes whose 16-byte pieces are XORed with the row's low bits.  The matrix
-// cores' float32 rate (a sixteenth of bfloat16's) is what bounds it, with T = 4 from about 256 tiles on.
-#define EX_BK 32
+// through two buffers of LDS (STAGES == 0; else that many), rows of 128 bytes whose 16-byte pieces are XORed with the row's low
+// bits.  The matrix cores' float32 rate (a sixteenth of bfloat16's) is what bounds it, with T = 4 from about 256 tiles on.
 //
 // STAGES > 0: the slices go from memory straight into LDS (global_load_lds_dwordx4: a wave's load brings 8 rows of 128 bytes,
 // the lane that fills piece p of row r fetching piece p ^ (r & 7)), STAGES - 1 steps on their way, for inner sizes of whole
-// steps: through registers one step is on its way, and a workgroup that is alone on its compute unit waits for memory every step.  Before / now, us: 1,201
-// rows 2048 -> 512 54.6 / 46.4, 512 -> 50304 588 / 562; 2,000 rows 768 -> 768 34.3 / 31.8, 3072 -> 768 121.7 / 108.4; 600 rows
-// 5120 -> 1280 128.8 / 108.3; 5,000 rows 1600 -> 6400 847 / 819 (125 TFLOP/s).  Eight waves a tile instead of four: the same.
+// steps: through registers one step is on its way, and a workgroup that is alone on its compute unit waits for memory every step.
+// Before / now, us: 1,201 rows 2048 -> 512 54.6 / 46.4, 512 -> 50304 588 / 562; 2,000 rows 768 -> 768 34.3 / 31.8, 3072 -> 768
+// 121.7 / 108.4; 600 rows 5120 -> 1280 128.8 / 108.3; 5,000 rows 1600 -> 6400 859 / 828 (124 TFLOP/s).  Eight waves a tile instead
+// of four: the same.
+#define EX_BK 32
 template <int T, int EPI, bool VEC, int STAGES>
 __global__ __launch_bounds__(256) void linear_exact_tile_kernel(
     const float* __restrict__ A, long lda, const float* __restrict__ W, const float* __restrict__ bias,
@@ -262,7 +263,7 @@ __global__ __launch_bounds__(256) void linear_exact_tile_kernel(
 // Few rows, or a product whose tiles would leave compute units idle: a workgroup per 16 rows x 16 columns, each of its
 // waves on blocks of its own (wave w: blocks w, w + waves, ...), operands straight from memory; the blocks' sums meet in
 // LDS and are added up in order.  Four groups of a block are loaded while the four before are multiplied.  Nothing is
-// shared between waves, so beyond a few dozen rows its loads bound it, at 33 TFLOP/s.
+// shared between waves, so beyond a few dozen rows its loads bound it, at 26 to 33 TFLOP/s.
 //
 // SHORT: inner sizes of up to 192, whose last groups are not there at all, not even as zeros to add (16 rows with an inner size
 // of 64 / 37: 4.2 / 6.1 us with those zeros, 3.4 / 3.5 without; the test costs longer ones 0.15 us).
@@ -347,7 +348,7 @@ template <int R, bool VEC>
 __global__ __launch_bounds__(256) void linear_exact_parts_kernel(const float* __restrict__ A, long lda,
                                                                  const float* __restrict__ W, float* __restrict__ sums,
                                                                  int n_rows, int n_out, int k_dim, int row_tiles) {
-  constexpr int PIECES = EX_BLOCK / 4, GROUPS = EX_BLOCK / EX_GROUP;
+  constexpr int GROUPS = EX_BLOCK / EX_GROUP;
   extern __shared__ __align__(16) float ex_lds[];    // [16 R][EX_BLOCK], 16-byte pieces XORed with the row's low bits
   const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, lk = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);

@@ -1237,9 +1237,10 @@ int launch_any(int shape, int k_parts, const void* act, long lda, const void* w,
       direct = tiles_of(4, n_rows, n_out) * k_parts <= 256 && steps >= 20 ? 4 : 0;
       ahead = 1;
     }
-    // Prompt portions of a few hundred rows under an inner size of 20 steps and more: 64 x 64 tiles with four stages from 160
-    // tiles on (400 rows 1600 -> 1600: 32 x 32 tiles through registers 17.2 us, here 15.3; 520 rows, 64 x 64 tiles through registers
-    // 18.0, here 15.8; 310 rows, 125 tiles: 13.3 and 15.1).
+    // Prompt portions of a few hundred rows under an inner size of 20 to 31 steps (longer ones have their rule above): 64 x 64 tiles
+    // with four stages from 160 tiles on, up to one a compute unit.  Over inner sizes 1,280 to 1,920, outputs 768 to 4,800 and 128 to
+    // 1,024 rows they take 9 to 22 % less than 32 or 64 wide tiles through registers, alone in a graph (400 rows 1600 -> 1600 12.9 /
+    // 10.3 us); with the LayerNorm behind them 400 rows 17.2 / 15.3, 520 rows 18.0 / 15.8, 310 rows (125 tiles) 13.3 / 15.1.
     if (direct < 0 && n_rows >= 128 && k_parts == 1 && steps >= 20 && (shape == 3 || shape == 4) && direct_ok(act, w, k_dim)) {
       const long t64 = tiles_of(3, n_rows, n_out);
       if (t64 >= 160 && t64 <= 256) direct = 1, ahead = 1;

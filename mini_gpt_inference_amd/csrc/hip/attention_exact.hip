@@ -286,7 +286,10 @@ __global__ __launch_bounds__(64 * AX_WAVES, D == 64 ? 5 : 1) void attention_exac
 // 280 12.0 / 7.9, 64 x 12 30 / 19; 8 x 8 behind 700 20 / 12; 64 x 8 behind 900 to 1,000 (bound by the 250 MB) 42.8 / 39.5;
 // 16 x 8 heads of 128 behind 200 to 300 19.5 / 12.5; 3 x 4 heads of 16 behind 5 to 42 7.0 / 4.6.  Heads of 64 need the 128
 // registers that let a compute unit have two workgroups: with scores kept for all 64 keys and ten registers spilled 64 x 8
-// took 44.5.  What is left at 16 x 12: the launch (1.6), two trips to memory, 64 matrix products (0.9) and the merge.
+// took 44.5.  A chunk of which at most one group of 16 keys is there (a short request's only one, every fourth one's last) is walked
+// without the other three: behind 1 to 5 keys 64 x 25 heads of 64 take 11 us, of 128 24, with the keys that are not there 18 and
+// 40, the general walk, which leaves them out too, 16 and 31.  What is left at 16 x 12: the launch (1.6), two trips to memory, 64
+// matrix products (0.9) and the merge.
 //
 // PAGE16: pages are multiples of 16 positions, so 16 keys lie one behind the other.
 template <int D, bool PAGE16>
@@ -329,7 +332,9 @@ __global__ __launch_bounds__(64 * AX_WAVES, D == 128 ? 2 : 4) void attention_exa
   ax_fc acc;                                            // channels C lane ..
 #pragma unroll
   for (int x = 0; x < C; ++x) acc[x] = 0.f;
-  for (int c = wave; c * AX_CHUNK <= pos; c += AX_WAVES) {
+  // chunk c, of which the first GROUPS groups of 16 keys are there
+  auto walk = [&](int c, auto groups) {
+    constexpr int GROUPS = decltype(groups)::value;
     const int c0 = c * AX_CHUNK;
     unsigned int row[4];                                // of the keys c0 + 16 t + l16
     uint64_t seen[4];                                   // the 16 keys' bits, four times over
@@ -342,7 +347,7 @@ __global__ __launch_bounds__(64 * AX_WAVES, D == 128 ? 2 : 4) void attention_exa
                                             : (PAGE16 ? l16 : 0);
     }
     if ((c + AX_WAVES) * AX_CHUNK <= pos) look_up(c + AX_WAVES);
-    if (c0 + AX_CHUNK <= begin && c0 >= a.keep_first) continue;
+    if (c0 + AX_CHUNK <= begin && c0 >= a.keep_first) return;
     ax_f4 kf[AHEAD][G];
     auto load_keys = [&](int t) {
       const float* src = a.kpool + (long)row[t] * D + 4 * lk;
@@ -362,10 +367,10 @@ __global__ __launch_bounds__(64 * AX_WAVES, D == 128 ? 2 : 4) void attention_exa
       }
     };
 #pragma unroll
-    for (int t = 0; t < AHEAD; ++t) load_keys(t);
+    for (int t = 0; t < AHEAD && t < GROUPS; ++t) load_keys(t);
     float v = 0.f;                                      // this lane's key: 16 (l16 / 4) + 4 lk + l16 % 4
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
+    for (int t = 0; t < GROUPS; ++t) {
       ax_f4 s = {0.f, 0.f, 0.f, 0.f};                   // keys 16 t + 4 lk + i, the same in all 16 lanes
 #pragma unroll
       for (int g = 0; g < G; ++g)
@@ -373,7 +378,7 @@ __global__ __launch_bounds__(64 * AX_WAVES, D == 128 ? 2 : 4) void attention_exa
         for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[t % AHEAD][g][e], qf[g][e], s, 0, 0, 0);
 #pragma unroll
       for (int i = 0; i < 4; ++i) v = l16 == 4 * t + i ? s[i] : v;
-      if (t + AHEAD < 4) load_keys(t + AHEAD);
+      if (t + AHEAD < GROUPS) load_keys(t + AHEAD);
       load_values(t);                                   // into the registers of keys that are done with
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -390,7 +395,7 @@ __global__ __launch_bounds__(64 * AX_WAVES, D == 128 ? 2 : 4) void attention_exa
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     float sum = 0.f;
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
+    for (int t = 0; t < GROUPS; ++t) {
       const ax_f4 p = *reinterpret_cast<const ax_f4*>(&p_s[wave][16 * t + 4 * lk]);
 #pragma unroll
       for (int i = 0; i < 4; ++i) sum += p[i];
@@ -398,10 +403,13 @@ __global__ __launch_bounds__(64 * AX_WAVES, D == 128 ? 2 : 4) void attention_exa
     l = l * alpha + ax_sum4(sum);
     m = m_new;
     acc *= alpha;
-    const bool whole = (seen[0] & seen[1] & seen[2] & seen[3]) == ~0ull;
+    uint64_t both = ~0ull;
+#pragma unroll
+    for (int t = 0; t < GROUPS; ++t) both &= seen[t];
+    const bool whole = both == ~0ull;
     auto weigh = [&](auto all) {
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
+      for (int t = 0; t < GROUPS; ++t) {
         __builtin_amdgcn_sched_barrier(0);              // (or all weights are read at once, into registers that are not there)
         ax_f4 p[4];                                     // the keys 16 t + 4 k + i, for everybody
 #pragma unroll
@@ -420,6 +428,10 @@ __global__ __launch_bounds__(64 * AX_WAVES, D == 128 ? 2 : 4) void attention_exa
     if (whole) weigh(std::true_type{});
     else weigh(std::false_type{});
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  };
+  for (int c = wave; c * AX_CHUNK <= pos; c += AX_WAVES) {
+    if (c * AX_CHUNK + 16 > pos) walk(c, std::integral_constant<int, 1>{});
+    else walk(c, std::integral_constant<int, 4>{});
   }
   if (lane == 0) {
     m_s[wave] = m;

@@ -1256,10 +1256,10 @@ int launch_any(int shape, int k_parts, const void* act, long lda, const void* w,
     }
   }
   const bool split = k_parts > 1;
-  // Up to 32 rows under a narrow output and a long inner size, where these tiles stand in for the decode kernel, whose sums are 16
-  // chains: chains of two steps.  Error of 16 rows 6400 -> 1600 against 64 bits, relative to the sums' norm: decode kernel
+  // Up to 32 rows under a narrow output and a long inner size (64 under matrices of less than 6 million elements), where these tiles
+  // stand in for the decode kernel, whose sums are 16 chains: chains of two steps.  Error of 16 rows 6400 -> 1600 against 64 bits, relative to the sums' norm: decode kernel
   // 1.35e-7, eight stretches of one chain 1.84e-7, of short ones 1.02e-7; 6.5 and 6.8 us.
-  const bool fold = !forced && split && shape == 4 && n_rows <= 32 && n_out < 4096 && k_dim > 4096;
+  const bool fold = !forced && split && shape == 4 && n_rows <= ((long)n_out * k_dim < 6000000 ? 64 : 32) && n_out < 4096 && k_dim > 4096;
   if (two_groups) {
     // forced: what this kernel stores must be float32, plain or added into the residual stream (the sums of
     // a split product are)

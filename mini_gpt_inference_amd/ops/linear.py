@@ -160,20 +160,36 @@ WIDE_OUT_DECODE_WORK = 8192
 # decode kernel against tiled: [4800 x 1600] 8.5 / 8.5 us at 16 rows, 10.6 / 8.5 at 24, 11.7 / 8.5 at
 # 32, 18.8 / 10.0 at 64; [6400 x 1600] 9.3 / 9.1, 11.4 / 9.3, 12.7 / 9.3, 19.8 / 12.0; under smaller
 # matrices the decode kernel stays ahead up to 64 rows ([3072 x 768] 5.0 / 5.6 at 32, 6.2 / 5.6 at
-# 64; [1600 x 1600] 5.8 / 8.4 and 8.0 / 8.4).  A long inner size under a narrow output is split over
-# workgroups by either; there the tiled kernel, whose slices go straight into LDS, is ahead from 9 rows on (either with
-# its sums left pending and the LayerNorm that adds them up, decode kernel / tiled: [1600 x 6400] 11.2 / 10.4 us at 8 rows,
-# 12.6 / 10.4 at 16, 16.0 / 10.8 at 32, 23.6 / 12.7 at 64; [1280 x 5120] 10.5 / 10.5, 11.8 / 10.4, 15.7 / 10.7; [1152 x 4608]
-# 10.4 / 10.0, 11.7 / 10.1; [1024 x 4096] 8.0 / 9.3, 8.3 / 9.4, 9.4 / 9.5), and from 17 rows on where a second kernel has
-# to add the sums up ([1600 x 6400] 9.7 / 10.0 at 12 rows, 10.4 / 10.0 at 16, 14.3 / 10.4 at 32; [2048 x 8192] 12.5 / 13.3,
-# 13.6 / 13.7, 18.5 / 14.0).
+# 64; [1600 x 1600] 5.8 / 8.4 and 8.0 / 8.4).
 TILED_FROM_ROWS = 17
 TILED_MIN_OUT = 4096
 TILED_MIN_MATRIX = 6_000_000
 TILED_ANY_SHAPE_FROM_ROWS = 33
-TILED_LONG_LEFT_FROM_ROWS = 9
+# A long inner size under a narrow output is split over workgroups by the tiled kernel, and by the decode kernel where its four
+# stretches are whole and the output has fewer than 128 column tiles.  Lines (rows) where the sums are left pending for a LayerNorm,
+# and where a second kernel adds them up.  us with the LayerNorm, decode kernel / tiled:
+# - where the decode kernel splits: pending [1600 x 6400] 11.5 / 11.0 at 9 rows, 16.3 / 11.3 at 32, [1152 x 4608] 10.6 / 10.3, 15.7 /
+#   10.6; added up [1600 x 6400] 13.9 / 14.0 at 16, 14.6 / 13.7 at 17, 17.5 / 13.8 at 32.
+# - outputs of 1,024 and less, whose tiles are few: pending [1024 x 8192] 10.1 / 10.8 at 16, 11.0 / 10.8 at 17; added up 11.7 / 12.7 at
+#   17, 12.5 / 13.1 at 32.
+# - where the decode kernel does not split and the tiled one's slices go straight into LDS: pending [2048 x 4160] 11.7 / 10.8 at 9,
+#   15.3 / 11.5 at 32; added up 13.3 / 14.1 at 17, 14.5 / 14.5 at 28, [2048 x 8192] 19.0 / 18.6 at 17, [2560 x 10240] 24.5 / 25.5 at 17,
+#   26.8 / 26.3 at 28, [2560 x 5120] 17.1 / 17.7 at 32.
+# - through registers (no whole steps of 64): pending [1216 x 4128] 9.8 / 10.5 at 9, 10.5 / 10.6 at 16; added up 12.0 / 13.1 at 32,
+#   [1344 x 4128] 14.1 / 14.5 at 40, 15.1 / 14.8 at 48.
 TILED_LONG_MIN_INNER = 4097
 TILED_LONG_MIN_MATRIX = 5_000_000
+
+
+def _long_inner_lines(n_out: int, k_dim: int):
+    """(rows from which on the sums are left pending, rows from which on they are added up) by the tiled kernel."""
+    if n_out <= 1024:
+        return 17, 33
+    if kernels.linear_skinny_partials(17, n_out, k_dim, False, kernels.EPI_RESIDUAL):
+        return 9, 17
+    if k_dim % 64:
+        return 17, 33 if n_out * k_dim >= TILED_MIN_MATRIX else 41
+    return 9, 28 if n_out <= 2048 or k_dim >= 5632 else 33
 
 
 def tiled_at_few_rows(n_rows: int, w: torch.Tensor, left: bool = False) -> bool:
@@ -181,8 +197,8 @@ def tiled_at_few_rows(n_rows: int, w: torch.Tensor, left: bool = False) -> bool:
     LEAVE_PARTS_MAX_ROWS) goes to the tiled kernel rather than the decode kernel.  left: the sums of a split
     product are left pending."""
     n_out, k_dim = w.shape
-    if n_out < TILED_MIN_OUT and k_dim >= TILED_LONG_MIN_INNER and n_out * k_dim >= TILED_LONG_MIN_MATRIX:
-        return n_rows >= (TILED_LONG_LEFT_FROM_ROWS if left else TILED_FROM_ROWS)
+    if n_rows > 8 and n_out < TILED_MIN_OUT and k_dim >= TILED_LONG_MIN_INNER and n_out * k_dim >= TILED_LONG_MIN_MATRIX:
+        return n_rows >= _long_inner_lines(n_out, k_dim)[0 if left else 1]
     if n_out * k_dim < TILED_MIN_MATRIX:
         return False
     return n_rows >= TILED_ANY_SHAPE_FROM_ROWS or (n_rows >= TILED_FROM_ROWS and n_out >= TILED_MIN_OUT)

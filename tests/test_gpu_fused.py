@@ -430,7 +430,18 @@ def test_addition_of_few_rows_under_a_long_inner_size(rows, n_out, k_dim):
         helpers.assert_close(got, want, "bfloat16", "x + product")
 
 
-@pytest.mark.parametrize("rows", [9, 17, 32])
+@pytest.mark.parametrize("n_out,k_dim,left,added", [(1600, 6400, 9, 17), (1152, 4608, 9, 17), (1040, 5120, 9, 17), (1024, 5120, 17, 33),
+                                                    (768, 8192, 17, 33), (2048, 4160, 9, 28), (1376, 4160, 9, 28), (2560, 10240, 9, 28),
+                                                    (2560, 5120, 9, 33), (1344, 4128, 17, 41), (1600, 4128, 17, 33)])
+def test_rows_from_which_a_long_inner_size_goes_to_the_tiled_kernel(n_out, k_dim, left, added):
+    from mini_gpt_inference_amd.ops import linear as L
+
+    w = torch.empty(n_out, k_dim, dtype=torch.bfloat16, device=DEV)
+    assert [m for m in range(1, 65) if L.tiled_at_few_rows(m, w, left=True)] == list(range(left, 65))
+    assert [m for m in range(1, 65) if L.tiled_at_few_rows(m, w)] == list(range(added, 65))
+
+
+@pytest.mark.parametrize("rows", [9, 17, 32, 64])
 @pytest.mark.parametrize("n_out,k_dim", [(1600, 6400), (1152, 4608), (1280, 4112)])
 def test_addition_of_few_rows_is_no_less_exact_in_the_tiled_kernel(rows, n_out, k_dim):
     """Where the tiled kernel's split stands in for the decode kernel's: its float32 sums are no further from 64 bits."""
@@ -448,6 +459,8 @@ def test_addition_of_few_rows_is_no_less_exact_in_the_tiled_kernel(rows, n_out, 
     parts = torch.empty(need, device=DEV) if need else None
     assert kernels.linear_skinny(a, w, b, decode, rows, kernels.EPI_RESIDUAL, partials=parts)
     for left in (True, False):
+        if rows > 32 and n_out * k_dim >= 6_000_000:
+            continue                       # (at more than 32 rows that was the tiled kernel's from the beginning)
         ctx = SimpleNamespace(exact=False, dtype=torch.bfloat16, n_rows=rows, pending=None, copy_budget=None,
                               workspace=Workspace(torch.device(DEV)))
         got = torch.zeros_like(decode)

@@ -231,22 +231,22 @@ LEAVE_PARTS_MAX_ROWS = 256     # (the tiled kernel's split; the decode kernel's 
 
 
 # The 32-bit path leaves the sums over the product's blocks of k where that and the LayerNorm which adds them up take less than
-# the product and a plain LayerNorm: (inner size, rows) from which on, and up to how many outputs for short inner sizes and others.
+# the product and a plain LayerNorm: by the inner size from how many rows on, and up to how many outputs.
 # us, product and LayerNorm / sums and LayerNorm: 768 -> 768 8.1 / 8.8 at 5 rows, 8.7 / 8.9 at 12, 9.4 / 8.9 at 16, 16.1 / 12.0 at 192,
 # 13.5 / 14.7 at 240 (through 32 x 32 tiles, as at all sizes that follow); 520 -> 520 7.5 / 8.1 at 5, 8.1 / 8.2 at 48; 1280 -> 1280
 # 9.4 / 9.7 at 1, 10.0 / 9.9 at 6, 16.9 / 12.5 at 64; 1600 -> 1600 10.4 / 10.3 at 1, 28.6 / 26.9 at 224, 28.9 / 29.7 at 240; 3072 -> 768
 # 13.6 / 9.3 at 1, 35.8 / 26.1 at 256; 6400 -> 1600 89.7 / 71.9 at 224; 2048 -> 2048 33.9 / 31.6 at 176, 35.3 / 35.7 at 208.
-EXACT_PARTS_FROM = ((6 * 256 + 1, 1), (1280, 6), (768, 16))
 EXACT_PARTS_MAX_ROWS = 256
 EXACT_PARTS_MAX_OUTPUTS = 380_000
-EXACT_PARTS_SHORT_K, EXACT_PARTS_SHORT_MAX_OUTPUTS = 1024, 172_000
+EXACT_PARTS_SHORT_MAX_OUTPUTS = 172_000    # under inner sizes below 1,024
 
 
 def exact_leaves_parts(n_rows: int, n_out: int, k_dim: int) -> bool:
     """Whether the 32-bit path leaves a product of this size as sums over its blocks of k for the LayerNorm behind it."""
-    most = EXACT_PARTS_MAX_OUTPUTS if k_dim >= EXACT_PARTS_SHORT_K else EXACT_PARTS_SHORT_MAX_OUTPUTS
-    return (n_rows <= EXACT_PARTS_MAX_ROWS and n_rows * n_out <= most
-            and any(k_dim >= k and n_rows >= rows for k, rows in EXACT_PARTS_FROM))
+    if k_dim < 768 or n_rows > EXACT_PARTS_MAX_ROWS:
+        return False
+    from_rows = 1 if k_dim > 1536 else 6 if k_dim >= 1280 else 16
+    return n_rows >= from_rows and n_rows * n_out <= (EXACT_PARTS_MAX_OUTPUTS if k_dim >= 1024 else EXACT_PARTS_SHORT_MAX_OUTPUTS)
 
 
 def plain_residual(ctx, h, x: torch.Tensor) -> None:

@@ -510,7 +510,7 @@ __device__ __forceinline__ unsigned int list_floor(const unsigned int* key, cons
   bool keep = t < n && above < k;
   if (p < 1.0f) {
     const float z = block_sum(keep ? mass[t] : 0.f, red_f);
-    keep = keep && before <= p * z;
+    keep = keep && (before <= p * z || above == 0);   // (the largest logit stays whatever p is)
   }
   return block_min_uint(keep ? mine : 0xffffffffu, reinterpret_cast<unsigned int*>(red_i));
 }

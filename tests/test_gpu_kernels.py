@@ -1699,6 +1699,16 @@ def test_sampling_from_held_rows(vocab):
             assert edge <= 1e-4 * total, f"row {r}: kernel {got[r]}, plain {tok}, u {u}, options {opts[r % len(opts)]}"
 
 
+@pytest.mark.parametrize("top_p", [0.0, -0.5, float("-inf")])
+@pytest.mark.parametrize("vocab,top_k", [(50, 20), (3000, 512), (3000, 0), (70000, 40)])
+def test_a_top_p_of_nothing_keeps_the_largest_logit(vocab, top_k, top_p):
+    """As the reference, which drops a token for the mass before it and never the first; over the list of candidates, all
+    registers, and a row that is read again."""
+    logits = rnd(torch.Generator().manual_seed(vocab), 4, vocab)
+    got = _sample(logits, [0.9] * 4, [top_k] * 4, [top_p] * 4, list(range(4)), [1] * 4)
+    assert got == logits.argmax(dim=1).tolist()
+
+
 def test_reference_vectors_top_k_top_p():
     # reference tests/test_sampling.py:25-38
     logits = torch.tensor([[1.0, 5.0, 3.0, 2.0, 4.0]] * 64)

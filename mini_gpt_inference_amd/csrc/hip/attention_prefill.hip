@@ -38,6 +38,21 @@
 #include "attention_prefill.h"
 #include "launchers.h"
 
+// Division of numbers below 2^31 by one that the host knows (0: never asked): a multiplication that is one short at most.
+struct Divisor {
+  unsigned int by, m;
+  explicit Divisor(long d) : by((unsigned int)d), m(d > 0 ? (unsigned int)(0xffffffffL / d) : 0u) {}
+  __device__ __forceinline__ unsigned int of(unsigned int x) const {
+    const unsigned int q = __umulhi(x, m);
+    return x - q * by >= by ? q + 1 : q;
+  }
+};
+// Which tile of which request's head a block takes: n = requests x heads, of which a die has `own` to itself and `left` are dealt out.
+struct PrefillDeal {
+  Divisor n, own, left, head;
+  unsigned int tiles;
+};
+
 template <int D, int Q, int K, int BIAS>
 __global__ __launch_bounds__(64 * Q * K, (pf_waves<D, K>())) void prefill_attention_kernel(
     const bf16_t* __restrict__ q, long ldq, bf16_t* __restrict__ out, long ldo,
@@ -46,20 +61,38 @@ __global__ __launch_bounds__(64 * Q * K, (pf_waves<D, K>())) void prefill_attent
     const int* __restrict__ seq_lens, int n_head, int n_kv_head, int page_size, float scale, int window,
     int single_below, const float* __restrict__ sinks, float softcap, const bf16_t* __restrict__ gate, long ldg,
     int keep_first, const float* __restrict__ score_bias, int chunked, const float* __restrict__ dist_bias,
-    int bias_len, const float* __restrict__ slopes, int n_req) {
-  // the tiles with the most keys first; all tiles of a request's head to one of the eight dies, whose L2 then has its keys
-  const int who = blockIdx.x, req = who / n_head;
-  const int tile = (int)(gridDim.z * gridDim.y - 1 - (blockIdx.z * gridDim.y + blockIdx.y));
-  if (who >= n_req * n_head) return;
+    int bias_len, const float* __restrict__ slopes, PrefillDeal deal) {
+  // Block b runs on die b % 8.  The tiles with the most keys come first.  All tiles of a request's head go to one die, whose L2 then has
+  // its keys, as far as eight heads at a time go; the tiles of the heads left over are dealt out, so that no die has more than the
+  // others, and (but for seven) no block is there in vain, which would wait for LDS like the others.  A die's turns are rounds of eight
+  // tiles of each of its own heads with its share of the dealt ones in front.  us, all tiles of a head on one die and blocks up to a
+  // multiple of eight heads / so: 1 request, 4,096 tokens behind 4,096, 1 head 148 / 49, 4 heads 129 / 74, 12 heads 178 / 148; 640 tokens x
+  // 12 heads 13.0 / 10.4, x 9 behind 2,000 34.6 / 21.8, behind a window of 256 17.9 / 11.0.
+  const unsigned int at = (blockIdx.y * gridDim.x + blockIdx.x) >> 3, die = blockIdx.x & 7;
+  const unsigned int round = deal.n.of(at), in = at - round * deal.n.by, own = deal.own.by, left = deal.left.by;
+  const bool dealt = in < (round < deal.tiles >> 3 ? left : ((deal.tiles & 7) * left + 7) >> 3);
+  unsigned int who, turn;
+  if (!dealt && own == 0) return;
+  if (dealt) {
+    const unsigned int i = (round * left + in) * 8 + die;
+    turn = deal.left.of(i);
+    who = own * 8 + i - turn * left;
+  } else {
+    const unsigned int i = at - (round < deal.tiles >> 3 ? (round + 1) * left : round * left + (((deal.tiles & 7) * left + 7) >> 3));
+    turn = deal.own.of(i);
+    who = (i - turn * own) * 8 + die;
+  }
+  if (turn >= deal.tiles) return;
+  const int tile = __builtin_amdgcn_readfirstlane((int)(deal.tiles - 1 - turn)), req = __builtin_amdgcn_readfirstlane((int)deal.head.of(who));
   extern __shared__ __align__(16) bf16_t pf_lds[];
   pf_tile<D, Q, K, BIAS>(q, ldq, out, ldo, kpool, vpool, block_tables, max_blocks, cu_q, seq_lens, n_head, n_kv_head, page_size, scale,
                       window, single_below, sinks, softcap, gate, ldg, keep_first, score_bias, chunked,
-                      dist_bias, bias_len, slopes, tile, req, who - req * n_head, pf_lds);
+                      dist_bias, bias_len, slopes, tile, req, __builtin_amdgcn_readfirstlane((int)who - req * n_head), pf_lds);
 }
 
 // One workgroup per (tile of 32 or 64 queries, request, head); max_q_len sizes the grid and is the host's
 // upper bound on the tokens any request brings (a request may bring none: its workgroups leave at
-// once).  single_below: requests that bring exactly one token, and that as one of the step's first
+// once);  single_below: requests that bring exactly one token, and that as one of the step's first
 // single_below tokens, are left to another kernel.  Head
 // sizes 32, 64, 96, 128 and a positive scale; others are refused.
 extern "C" int mgpt_prefill_attention_bf16(
@@ -77,8 +110,8 @@ extern "C" int mgpt_prefill_attention_bf16(
     return MGPT_ERR_BAD_SHAPE;
   if (window == 0) keep_first = 0;
   if (n_req > 65535 || n_head > 65535) return MGPT_ERR_TOO_LARGE;
-  const long whos = ((long)n_req * n_head + 7) / 8 * 8;
-  if (whos > 0xffffffffL / 512) return MGPT_ERR_TOO_LARGE;   // threads of a grid along x
+  const long whos = (long)n_req * n_head;
+  constexpr long PF_GRID_X = 0xffffffffL / 512 / 8 * 8;   // threads of a grid along x, whole turns of all dies
 #define PF_LAUNCH2(DD, QQ, KK, BI)                                                                                  \
   {                                                                                                                 \
     constexpr int lds_bytes = pf_lds_bytes<DD, QQ, KK, BI>();                                                       \
@@ -90,13 +123,16 @@ extern "C" int mgpt_prefill_attention_bf16(
       allowed = true;                                                                                               \
     }                                                                                                               \
     const long q_tiles = ((long)max_q_len + QQ * PF_W - 1) / (QQ * PF_W);                                           \
-    const dim3 grid((unsigned int)whos, (unsigned int)(q_tiles < 32768 ? q_tiles : 32768),                          \
-                    (unsigned int)((q_tiles + 32767) / 32768));                                                     \
+    const long turns = q_tiles / 8 * whos + (q_tiles % 8 * (whos % 8) + 7) / 8 + q_tiles % 8 * (whos / 8);          \
+    if (8 * turns > 0x7fffffffL) return MGPT_ERR_TOO_LARGE;                                                         \
+    const long x = 8 * turns <= PF_GRID_X ? 8 * turns : PF_GRID_X;                                                  \
+    const dim3 grid((unsigned int)x, (unsigned int)((8 * turns + x - 1) / x));                                      \
     hipLaunchKernelGGL((prefill_attention_kernel<DD, QQ, KK, BI>), grid, dim3(64 * QQ * KK), lds_bytes, stream,     \
                        (const bf16_t*)q, ldq, (bf16_t*)out, ldo, (const bf16_t*)kpool, (const bf16_t*)vpool,        \
                        block_tables, max_blocks, cu_q, seq_lens, n_head, n_kv_head, page_size, scale, window,       \
                        single_below, sinks, softcap, (const bf16_t*)gate, ldg, keep_first, score_bias, chunked,     \
-                       dist_bias, bias_len, slopes, n_req);                                                         \
+                       dist_bias, bias_len, slopes,                                                                 \
+                       PrefillDeal{Divisor(whos), Divisor(whos / 8), Divisor(whos % 8), Divisor(n_head), (unsigned int)q_tiles}); \
   }
 #define PF_LAUNCH(DD, QQ, KK)                                           \
   {                                                                     \

@@ -1331,6 +1331,33 @@ def test_prefill_attention_behind_more_pages_than_lie_in_lds(r, q_len, d, h, pag
     helpers.assert_close(out, want, "bfloat16", f"{r} requests, window {window}")
 
 
+@pytest.mark.parametrize("r,h,longest", [(1, 1, 1), (1, 1, 300), (1, 3, 700), (1, 7, 256), (1, 8, 33), (3, 3, 290), (1, 15, 520), (2, 12, 64),
+                                         (5, 5, 545)])
+def test_prefill_attention_deals_every_tile_out_once(r, h, longest):
+    """Heads that are no multiple of the eight dies, with fewer tiles than eight, whole eights of them and some over."""
+    q_lens = [max(longest - 97 * i, 0) for i in range(r)]
+    c = PagedCase([q + 5 * i for i, q in enumerate(q_lens)], q_lens, h=h, hk=1, d=64, page=16, dtype="bfloat16", seed=longest)
+    out = torch.full((c.n, h * 64), float("nan"), dtype=torch.bfloat16, device=DEV)
+    assert kernels.prefill_attention_bf16(c.q_flat, out, c.kp, c.vp, c.bt, c.cu, c.sl, r, longest, h, 0.125)
+    helpers.assert_close(out, c.want(0.125, 0), "bfloat16", f"{r} requests x {h} heads")
+
+
+def test_prefill_attention_of_more_heads_than_a_grid_is_wide():
+    """129 requests x 65,535 heads, a token each behind two others."""
+    r, h, d = 129, 65535, 32
+    g = torch.Generator(device=DEV).manual_seed(3)
+    q = torch.randn(r, h * d, generator=g, device=DEV, dtype=torch.bfloat16)
+    kp, vp = (torch.randn(r, 1, 4, d, generator=g, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+    out = torch.full((r, h * d), float("nan"), dtype=torch.bfloat16, device=DEV)
+    bt = torch.arange(r, dtype=torch.int32, device=DEV).view(r, 1)
+    cu, sl = torch.arange(r + 1, dtype=torch.int32, device=DEV), torch.full((r,), 3, dtype=torch.int32, device=DEV)
+    assert kernels.prefill_attention_bf16(q, out, kp, vp, bt, cu, sl, r, 1, h, d ** -0.5)
+    for i in (0, 1, 63, 127, 128):
+        scores = q[i].float().view(h, d) @ kp[i, 0, :3].float().T * d ** -0.5
+        helpers.assert_close(out[i].view(h, d), torch.softmax(scores, 1) @ vp[i, 0, :3].float(), "bfloat16", f"request {i}")
+    assert torch.isfinite(out).all()
+
+
 @pytest.mark.parametrize("window", [0, 33])
 @pytest.mark.parametrize("d", [32, 64])
 def test_prefill_attention_with_many_tiles(d, window):

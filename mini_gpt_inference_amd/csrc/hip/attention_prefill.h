@@ -264,12 +264,24 @@ __device__ __forceinline__ void pf_tile(
       if (BIAS == 2) {
         // scaled and capped scores in units of log2 e, then minus slope * distance (the lane's first key's, and
         // the keys' places behind it as constants)
-        const float first = slope2 * (float)(c0 + g * 4 - my_pos);
+        float first = slope2 * (float)(c0 + g * 4 - my_pos);
         const float in = scale * __builtin_amdgcn_rcpf(softcap), cap2 = softcap * 1.4426950408889634f;
+        auto off = [&](int i) { return __builtin_fmaf(slope2, (float)(8 * (i >> 2) + (i & 3)), first); };
+        if (Q == 1 || D == 32) {
+          // one branch: one an element spills 70 scalar registers here (33 tokens behind 700 x 9 heads of 64 17.1 us, so 13.8; 3 x 130
+          // tokens x 25 heads 10.2, 8.8); in the other forms this one spills up to 9 vector registers
+          if (softcap > 0.f) {
+            asm volatile("" : "+v"(first));   // or the branches share 16 offsets, made and kept in front of them
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const float off = __builtin_fmaf(slope2, (float)(8 * (i >> 2) + (i & 3)), first);
-          s[i] = softcap > 0.f ? __builtin_fmaf(cap2, tanh_fast(s[i] * in), off) : __builtin_fmaf(s[i], raw2, off);
+            for (int i = 0; i < 16; ++i) s[i] = __builtin_fmaf(cap2, tanh_fast(s[i] * in), off(i));
+          } else {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) s[i] = __builtin_fmaf(s[i], raw2, off(i));
+          }
+        } else {
+#pragma unroll
+          for (int i = 0; i < 16; ++i)
+            s[i] = softcap > 0.f ? __builtin_fmaf(cap2, tanh_fast(s[i] * in), off(i)) : __builtin_fmaf(s[i], raw2, off(i));
         }
       } else if (softcap > 0.f) {
         // capped scores: cap * tanh(s * scale / cap), kept in the raw scores' units (times cap / scale)

@@ -1331,6 +1331,24 @@ def test_prefill_attention_behind_more_pages_than_lie_in_lds(r, q_len, d, h, pag
     helpers.assert_close(out, want, "bfloat16", f"{r} requests, window {window}")
 
 
+@pytest.mark.parametrize("cap", [0.0, 12.0])
+@pytest.mark.parametrize("q_lens,before", [([140, 1, 30], 300), ([1, 31, 32, 33, 65, 100] * 4, 60), ([65, 40, 129] * 10, 150)])
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_prefill_attention_with_slopes_in_each_form(d, q_lens, before, cap):
+    """Slopes by distance, behind a cap and without one, with eight, four and two times two waves, against the general kernel in 32
+    bits on the same numbers."""
+    lens = [q + (before + 37 * i) % 450 for i, q in enumerate(q_lens)]
+    c = PagedCase(lens, q_lens, h=4, hk=2, d=d, page=16, dtype="bfloat16", seed=d, poison=False)
+    slopes = torch.tensor([0.5, 0.06, 0.004, 0.0], device=DEV)
+    want = torch.empty(c.n, 4 * d, device=DEV)
+    kernels.paged_attention_generic(c.q_flat.float(), want, c.kp.float(), c.vp.float(), c.bt, c.cu, c.sl, c.q_req, c.n, len(lens), 4,
+                                    d ** -0.5, softcap=cap, slopes=slopes)
+    out = torch.full((c.n, 4 * d), float("nan"), dtype=torch.bfloat16, device=DEV)
+    assert kernels.prefill_attention_bf16(c.q_flat, out, c.kp, c.vp, c.bt, c.cu, c.sl, len(lens), max(q_lens), 4, d ** -0.5,
+                                          softcap=cap, slopes=slopes)
+    helpers.assert_close(out, want, "bfloat16", f"head size {d}, cap {cap}")
+
+
 @pytest.mark.parametrize("r,h,longest", [(1, 1, 1), (1, 1, 300), (1, 3, 700), (1, 7, 256), (1, 8, 33), (3, 3, 290), (1, 15, 520), (2, 12, 64),
                                          (5, 5, 545)])
 def test_prefill_attention_deals_every_tile_out_once(r, h, longest):

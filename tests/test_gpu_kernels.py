@@ -209,6 +209,57 @@ def test_float32_product_of_infinities_and_in_float32_precision(n, k, o, kernel)
     assert ((part - exact).norm() / exact.norm()).item() < 2e-7
 
 
+@pytest.mark.parametrize("k", [37, 320, 1100, 2048])
+def test_float32_product_done_again_has_the_same_bits_whatever_the_tiles(k):
+    """Elements of rows with a value that bfloat16 rounds to infinity, computed once more in float32, in each kernel, beside rows that
+    are not."""
+    g = torch.Generator().manual_seed(k)
+    o, n = 1500, 1030
+    a, w = rnd(g, n, k).to(DEV), rnd(g, o, k, scale=0.05).to(DEV)
+    a[::3, k // 2] = 3.4e38
+    whole = torch.empty(n, o, device=DEV)
+    kernels.linear_generic(a, w, None, whole, n)
+    want = a.double() @ w.double().T
+    assert whole.isfinite().all() and ((whole.double() - want).norm(dim=1) / want.norm(dim=1)).max().item() < 1e-6
+    for rows, cols in ((1, o), (17, 37), (70, 200), (130, o), (300, 515), (n, 130)):
+        part = torch.empty(rows, cols, device=DEV)
+        kernels.linear_generic(a[:rows], w[:cols].contiguous(), None, part, rows)
+        assert torch.equal(part, whole[:rows, :cols]), f"{rows} rows, {cols} columns"
+        if cols % 4 == 0:
+            sums = torch.empty(kernels.linear_exact_blocks(k), rows, cols, device=DEV)
+            kernels.linear_exact_parts(a[:rows], w[:cols].contiguous(), sums, rows)
+            total = torch.zeros(rows, cols, device=DEV)
+            for block in sums:
+                total += block
+            assert torch.equal(total, whole[:rows, :cols]), f"{rows} rows, {cols} columns, sums over blocks"
+
+
+@pytest.mark.parametrize("n,k,o,parts", [(1201, 2048, 512, False), (1201, 512, 2048, False), (4, 3072, 768, False), (64, 768, 2304, False),
+                                         (500, 1001, 900, False), (16, 3072, 768, True)])
+def test_float32_product_of_nan_rows_takes_no_multiple_of_its_time(n, k, o, parts):
+    """All elements are computed once more: on the matrix cores' float32 rate, 16 / 6 of the bfloat16 parts' work, with operands
+    straight from memory (measured 2 to 5 times in all; a serial sum an element took 30 to 300 times)."""
+    def us(a):
+        call = (lambda: kernels.linear_exact_parts(a, w, out, n)) if parts else (lambda: kernels.linear_generic(a, w, None, out, n))
+        times = []
+        for _ in range(8):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(20):
+                call()
+            end.record()
+            end.synchronize()
+            times.append(start.elapsed_time(end) * 50)
+        return sorted(times)[2]
+
+    g = torch.Generator().manual_seed(n)
+    a, w = rnd(g, n, k).to(DEV), rnd(g, o, k).to(DEV)
+    out = torch.empty((kernels.linear_exact_blocks(k), n, o) if parts else (n, o), device=DEV)
+    plain, nan = us(a), us(torch.full_like(a, float("nan")))
+    assert out.isnan().all()
+    assert nan < 10 * plain, f"{nan:.0f} us with rows of NaN, {plain:.0f} without"
+
+
 @pytest.mark.parametrize("epi", [kernels.EPI_NONE, kernels.EPI_GELU, kernels.EPI_RESIDUAL])
 @pytest.mark.parametrize("n,k,o,kernel", [(300, 768, 768, "lds32"), (97, 768, 2303, "lds32"), (129, 32, 1500, "lds32"),
                                           (600, 512, 515, "lds32"), (1201, 2048, 512, "lds32"), (255, 96, 1024, "lds32"),

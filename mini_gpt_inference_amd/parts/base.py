@@ -172,7 +172,9 @@ class Workspace:
                 raise WorkspaceFrozen(f"workspace buffer {name!r} would have to grow while a graph holds it")
             if buf is not None:
                 self.moved += 1
-            buf = torch.empty((rows, cols), dtype=dtype, device=self.device)
+            # Zeros: kernels leave rows of a step's padding unwritten, and what lies there goes through the products like any other
+            # row.  Bits that happen to be NaN would cost time (a float32 product does its NaN elements a second time).
+            buf = torch.zeros((rows, cols), dtype=dtype, device=self.device)
             self._buffers[key] = buf
             self.generation += 1
         return buf

@@ -33,3 +33,13 @@ def test_layers_of_different_widths_do_not_take_each_others_buffer():
         ws.get("qkv", 5, 288, torch.float32)
     with pytest.raises(WorkspaceFrozen):
         ws.get("attn_out", 1, 96, torch.float32)
+
+
+def test_a_new_buffer_holds_zeros():
+    """What a step leaves unwritten (rows of its padding) is no bits of freed memory: those can be NaN, with which a product takes
+    longer."""
+    ws = Workspace(torch.device("cpu"))
+    for cols in (8, 16, 32, 64):
+        old = torch.full((500, cols), float("nan"))
+        del old
+        assert (ws.get("x", 500, cols, torch.float32) == 0).all()

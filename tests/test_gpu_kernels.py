@@ -209,6 +209,26 @@ def test_float32_product_of_infinities_and_in_float32_precision(n, k, o, kernel)
     assert ((part - exact).norm() / exact.norm()).item() < 2e-7
 
 
+@pytest.mark.parametrize("a_size,w_size", [(1e-33, 1), (1e-35, 1), (1, 1e-37), (1e-40, 1e6), (1e-35, 1e25), (1e-18, 1e-18), (1e30, 1e-30),
+                                           (1e30, 1e3)])
+@pytest.mark.parametrize("n,k,o", [(5, 64, 257), (40, 1100, 2300), (300, 384, 768), (1030, 192, 1500), (1030, 160, 3501), (500, 301, 900)])
+def test_float32_product_of_the_smallest_and_largest_operands(n, k, o, a_size, w_size):
+    """Operands down to denormal ones, in each kernel: as close to 64 bits as others are, where the product is a float32 number that
+    is not denormal (1e-35 times its own last bit is denormal: 2^-149 / 1e-35 is 1e-10); 1e-40 itself has 2^16 steps, which the product in
+    64 bits is of too.  The bound is that of float32 sums, which the largest ones are computed by."""
+    g = torch.Generator().manual_seed(n)
+    a, w = (rnd(g, n, k).double() * a_size).float(), (rnd(g, o, k).double() * w_size).float()
+    got = torch.empty(n, o, device=DEV)
+    kernels.linear_generic(a.to(DEV), w.to(DEV), None, got, n)
+    want = a.double() @ w.double().T
+    unit = want.abs().max()
+    assert (((got.cpu().double() - want) / unit).norm() / (want / unit).norm()).item() < 5e-7
+    if o % 4 == 0:
+        sums = torch.empty(kernels.linear_exact_blocks(k), n, o, device=DEV)
+        kernels.linear_exact_parts(a.to(DEV), w.to(DEV), sums, n)
+        assert (((sums.cpu().double().sum(dim=0) - want) / unit).norm() / (want / unit).norm()).item() < 5e-7
+
+
 @pytest.mark.parametrize("k", [37, 320, 1100, 2048])
 def test_float32_product_done_again_has_the_same_bits_whatever_the_tiles(k):
     """Elements of rows with a value that bfloat16 rounds to infinity, computed once more in float32, in each kernel, beside rows that

@@ -229,6 +229,24 @@ def test_float32_product_of_the_smallest_and_largest_operands(n, k, o, a_size, w
         assert (((sums.cpu().double().sum(dim=0) - want) / unit).norm() / (want / unit).norm()).item() < 5e-7
 
 
+@pytest.mark.parametrize("k", [769, 1001, 1028, 1280, 2300, 4100, 4609])
+def test_float32_product_of_few_rows_under_long_inner_sizes(k):
+    """A wave has a block of 256 k at a time, of which the last may end anywhere, in one round or two (beyond 16 blocks): the bits of
+    the sums over blocks, added up in order."""
+    g = torch.Generator().manual_seed(k)
+    for rows, cols in ((1, 300), (16, 52), (17, 132), (40, 900)):
+        a, w = rnd(g, rows, k).to(DEV), rnd(g, cols, k).to(DEV)
+        assert kernels.linear_exact_kernel(rows, cols, k, aligned=k % 4 == 0) == "rows"
+        got = torch.full((rows + 1, cols), 7.0, device=DEV)
+        kernels.linear_generic(a, w, None, got, rows)
+        sums = torch.empty(kernels.linear_exact_blocks(k), rows, cols, device=DEV)
+        kernels.linear_exact_parts(a, w, sums, rows)
+        total = torch.zeros(rows, cols, device=DEV)
+        for block in sums:
+            total += block
+        assert torch.equal(got[:rows], total) and (got[rows] == 7.0).all(), f"{rows} rows, {cols} columns"
+
+
 @pytest.mark.parametrize("k", [37, 320, 1100, 2048])
 def test_float32_product_done_again_has_the_same_bits_whatever_the_tiles(k):
     """Elements of rows with a value that bfloat16 rounds to infinity, computed once more in float32, in each kernel, beside rows that

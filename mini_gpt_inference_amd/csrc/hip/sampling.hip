@@ -498,19 +498,20 @@ __device__ __forceinline__ unsigned int list_floor(const unsigned int* key, cons
   const int t = threadIdx.x;
   const unsigned int mine = t < n ? key[t] : 0xffffffffu;
   int above = 0;
-  float before = 0.f;
+  double before = 0.;                              // (a chain of 128 additions in 32 bits is off by up to 1.5e-6)
   if (t < n) {
     for (int q = 0; q < n; q += 4) {
       const uint4 x = *reinterpret_cast<const uint4*>(key + q);
       const float4 e = *reinterpret_cast<const float4*>(mass + q);
       above += (x.x > mine) + (x.y > mine) + (x.z > mine) + (x.w > mine);
-      before += ((x.x > mine ? e.x : 0.f) + (x.y > mine ? e.y : 0.f)) + ((x.z > mine ? e.z : 0.f) + (x.w > mine ? e.w : 0.f));
+      const float four = ((x.x > mine ? e.x : 0.f) + (x.y > mine ? e.y : 0.f)) + ((x.z > mine ? e.z : 0.f) + (x.w > mine ? e.w : 0.f));
+      before += (double)four;
     }
   }
   bool keep = t < n && above < k;
   if (p < 1.0f) {
     const float z = block_sum(keep ? mass[t] : 0.f, red_f);
-    keep = keep && (before <= p * z || above == 0);   // (the largest logit stays whatever p is)
+    keep = keep && (before <= (double)p * z || above == 0);   // (the largest logit stays whatever p is)
   }
   return block_min_uint(keep ? mine : 0xffffffffu, reinterpret_cast<unsigned int*>(red_i));
 }

@@ -1843,6 +1843,19 @@ def test_a_top_p_of_nothing_keeps_the_largest_logit(vocab, top_k, top_p):
     assert got == logits.argmax(dim=1).tolist()
 
 
+@pytest.mark.parametrize("logit,keeps", [(-0.46050000190734863, False), (-0.41769999265670776, True)])
+def test_top_p_of_a_long_list_adds_masses_up_without_a_drift(logit, keeps):
+    """One logit, 400 equal ones below it and 100 below those, of which the mass above ends 0.75e-6 beside top-p: additions one by one
+    in float32 are off by 1.5e-6 here (expf by up to 1e-7, the mass of all that is kept and p by 1e-7)."""
+    logits = torch.full((64, 600), -30.0)
+    logits[:, 0], logits[:, 1:401], logits[:, 401:501] = 0.0, logit, logit - 0.01
+    mass = logits[0, :501].double().exp()
+    above = mass[:401].sum().item()
+    p = above * (1 + (0.75e-6 if keeps else -0.75e-6)) / mass.sum().item()
+    got = _sample(logits, [1.0] * 64, [501] * 64, [p] * 64, list(range(64)), [1] * 64)
+    assert any(token > 400 for token in got) == keeps and max(got) < 501
+
+
 def test_reference_vectors_top_k_top_p():
     # reference tests/test_sampling.py:25-38
     logits = torch.tensor([[1.0, 5.0, 3.0, 2.0, 4.0]] * 64)

@@ -229,6 +229,20 @@ def test_float32_product_of_the_smallest_and_largest_operands(n, k, o, a_size, w
         assert (((sums.cpu().double().sum(dim=0) - want) / unit).norm() / (want / unit).norm()).item() < 5e-7
 
 
+@pytest.mark.parametrize("n,o", [(5, 64), (17, 260), (300, 515), (1030, 1500), (1030, 3500)])
+def test_float32_product_of_an_inner_size_of_one(n, o):
+    """One product is rounded once, in each kernel that takes inner sizes which are no whole groups."""
+    g = torch.Generator().manual_seed(n)
+    a, w = rnd(g, n, 1).to(DEV), rnd(g, o, 1).to(DEV)
+    got = torch.empty(n, o, device=DEV)
+    kernels.linear_generic(a, w, None, got, n)
+    assert torch.equal(got, a * w.T)
+    if o % 4 == 0:
+        sums = torch.empty(1, n, o, device=DEV)
+        kernels.linear_exact_parts(a, w, sums, n)
+        assert torch.equal(sums[0], a * w.T)
+
+
 @pytest.mark.parametrize("k", [769, 1001, 1028, 1280, 2300, 4100, 4609])
 def test_float32_product_of_few_rows_under_long_inner_sizes(k):
     """A wave has a block of 256 k at a time, of which the last may end anywhere, in one round or two (beyond 16 blocks): the bits of

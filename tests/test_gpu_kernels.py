@@ -314,7 +314,7 @@ def test_float32_product_of_nan_rows_takes_no_multiple_of_its_time(n, k, o, part
 
 @pytest.mark.parametrize("epi", [kernels.EPI_NONE, kernels.EPI_GELU, kernels.EPI_RESIDUAL])
 @pytest.mark.parametrize("n,k,o,kernel", [(300, 768, 768, "lds32"), (97, 768, 2303, "lds32"), (129, 32, 1500, "lds32"),
-                                          (600, 512, 515, "lds32"), (1201, 2048, 512, "lds32"), (255, 96, 1024, "lds32"),
+                                          (600, 512, 515, "lds32"), (1201, 2048, 512, "lds64"), (255, 96, 1024, "lds32"),
                                           (1030, 64, 1500, "lds64"), (400, 512, 2048, "lds64"), (1030, 160, 3501, "lds128"),
                                           (1500, 96, 2000, "tile64"), (3400, 160, 3072, "tile128")])
 def test_float32_product_straight_into_lds(n, k, o, kernel, epi):
@@ -332,7 +332,8 @@ def test_float32_product_straight_into_lds(n, k, o, kernel, epi):
 
 @pytest.mark.parametrize("n,k,o,kernel,unaligned", [
     (16, 3072, 768, "rows", "rows"), (188, 768, 768, "rows", "rows"), (190, 768, 768, "lds32", "rows"),
-    (300, 768, 2304, "lds32", "tile64"), (400, 768, 2304, "lds64", "tile64"), (2000, 512, 2048, "lds128", "tile128"),
+    (300, 768, 1600, "lds32", "tile64"), (300, 768, 2304, "lds64", "tile64"), (300, 800, 2304, "lds32", "tile64"),
+    (40, 768, 8400, "lds32", "rows"), (400, 768, 2304, "lds64", "tile64"), (2000, 512, 2048, "lds128", "tile128"),
     (2000, 96, 1000, "lds64", "tile64"), (2300, 96, 1000, "tile64", "tile64"),            # 512 and 576 tiles
     (700, 384, 3000, "tile64", "tile64"), (1500, 384, 3000, "lds64", "tile64"),           # a third round hardly begun, or more
     (2000, 192, 3000, "lds64", "tile64"), (4400, 192, 3000, "tile64", "tile64"), (4400, 256, 3000, "lds64", "tile64"),

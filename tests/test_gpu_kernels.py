@@ -155,11 +155,11 @@ def test_linear_generic_takes_any_inner_size(a_dt, w_dt, o_dt, n, k):
 
 @pytest.mark.parametrize("k", [1, 15, 17, 64, 65, 128, 192, 193, 256, 258, 300, 512, 4100, 4352])
 def test_float32_product_keeps_its_sums_whatever_the_tiles(k):
-    """A product that is float32 throughout goes to one of several kernels by its size: a workgroup per 16 x 16 outputs with
-    a wave per 256 of k (several rounds of them beyond 16 waves), tiles of 64 x 64 and of 128 x 128, and for inner sizes of whole
-    steps of 32 these and tiles of 32 x 32 with their slices straight into LDS.  An element's bits are the same in all, also where rows of the operands are not 16-byte aligned; the error against 64 bits is that of
-    float32 sums (a chain of at most 64 groups of four products in a block of 256, then the blocks: below 1e-6 of the
-    result's norm)."""
+    """A product that is float32 throughout goes to one of several kernels by its size: a workgroup per 16 x 16 outputs, whose waves
+    have groups of 32 k or blocks of 256, tiles of 64 x 64 and of 128 x 128, and for inner sizes of whole groups these without
+    checks and tiles of 32 x 32.  An element's bits are the same in all, also where rows of the operands are not 16-byte aligned;
+    the error against 64 bits is that of float32 sums (a chain of eight groups of 32 k in a block of 256, then the blocks: below
+    1e-6 of the result's norm)."""
     g = torch.Generator().manual_seed(k)
     o, n = 3501, 1030                                  # 9 x 28 tiles of 128 x 128, all but the last row and column whole
     a, w, bias = rnd(g, n, k + 3).to(DEV), rnd(g, o, k).to(DEV), rnd(g, o).to(DEV)
@@ -316,11 +316,10 @@ def test_float32_product_of_nan_rows_takes_no_multiple_of_its_time(n, k, o, part
 @pytest.mark.parametrize("n,k,o,kernel", [(300, 768, 768, "lds32"), (97, 768, 2303, "lds32"), (129, 32, 1500, "lds32"),
                                           (600, 512, 515, "lds32"), (1201, 2048, 512, "lds64"), (255, 96, 1024, "lds32"),
                                           (1030, 64, 1500, "lds64"), (400, 512, 2048, "lds64"), (1030, 160, 3501, "lds128"),
-                                          (1500, 96, 2000, "tile64"), (3400, 160, 3072, "tile128")])
+                                          (1500, 96, 2000, "tile64"), (3400, 160, 3072, "lds128")])
 def test_float32_product_straight_into_lds(n, k, o, kernel, epi):
-    """Slices that go straight into LDS (inner sizes of whole steps), in tiles of 32 x 32, 64 x 64 and 128 x 128 and at fewer
-    steps than stages, as many and more, and tiles of such sizes that stay with the registers: the bits of the same product over
-    rows that are not aligned for that."""
+    """Aligned rows of whole groups, of which nothing is checked, in tiles of 32 x 32, 64 x 64 and 128 x 128, with one step and with
+    more, and 64 x 64 tiles that keep steps of one group: the bits of the same product over rows that are not aligned for that."""
     g = torch.Generator().manual_seed(n + k)
     assert kernels.linear_exact_kernel(n, o, k) == kernel and not kernels.linear_exact_kernel(n, o, k, aligned=False).startswith("lds")
     a, w, bias, old = rnd(g, n, k + 1).to(DEV)[:, :k], rnd(g, o, k).to(DEV), rnd(g, o).to(DEV), rnd(g, n + 1, o).to(DEV)
@@ -337,7 +336,7 @@ def test_float32_product_straight_into_lds(n, k, o, kernel, epi):
     (2000, 96, 1000, "lds64", "tile64"), (2300, 96, 1000, "tile64", "tile64"),            # 512 and 576 tiles
     (700, 384, 3000, "tile64", "tile64"), (1500, 384, 3000, "lds64", "tile64"),           # a third round hardly begun, or more
     (2000, 192, 3000, "lds64", "tile64"), (4400, 192, 3000, "tile64", "tile64"), (4400, 256, 3000, "lds64", "tile64"),
-    (3400, 768, 3072, "tile128", "tile128"), (4096, 768, 3072, "tile128", "tile128"), (5000, 768, 3072, "lds128", "tile128"),
+    (3400, 768, 3072, "lds128", "tile128"), (4096, 768, 3072, "lds128", "tile128"), (5000, 768, 3072, "lds128", "tile128"),
     (4096, 1152, 3072, "lds128", "tile128"), (4096, 96, 3072, "lds128", "tile128")])
 def test_float32_product_kernel_by_size(n, k, o, kernel, unaligned):
     """Both sides of the lines between the kernels."""

@@ -231,10 +231,14 @@ LEAVE_PARTS_MAX_ROWS = 256     # (the tiled kernel's split; the decode kernel's 
 
 
 # The 32-bit path leaves the sums over the product's blocks of k where that and the LayerNorm which adds them up take less than
-# the product and a plain LayerNorm: by the inner size from how many rows on, and up to how many outputs.
-# us, product and LayerNorm / sums and LayerNorm: 768 -> 768 7.2 / 7.9 at 4 rows, 7.9 / 8.0 at 16, 8.2 / 8.1 at 17, 8.8 / 8.9 at 64; 512 -> 512
-# 6.6 / 7.8 at 4; 1024 -> 1024 9.4 / 8.4 at 16; 1600 -> 1600 11.9 / 9.8 at 1, 18.4 / 15.0 at 64; 2048 -> 512 11.7 / 7.8 at 1; 3072 -> 768
-# 15.2 / 8.7 at 1, 18.6 / 9.0 at 16, 19.2 / 13.6 at 64; 6400 -> 1600 28.0 / 16.6 at 1, 51.8 / 26.5 at 64.
+# the product and a plain LayerNorm.
+# us, product and LayerNorm / sums and LayerNorm: 768 -> 768 7.4 / 8.2 at 4 rows, 8.1 / 8.4 at 16, 8.4 / 8.6 at 64, 8.6 / 8.8 at 80, and from
+# the row on from which the product's workgroups of 16 x 16 outputs are more than compute units 11.1 / 8.9 at 96, 14.5 / 10.3 at 176,
+# 11.4 / 10.8 at 224, 11.6 / 12.8 at 256; 768 -> 512 7.3 / 7.8 at 4, 8.4 / 8.0 at 32, 8.6 / 8.8 at 128, 11.1 / 9.2 at 160.  1024 -> 1024 8.5 / 8.6
+# at 8, 9.1 / 8.6 at 16, 14.9 / 14.8 at 224; 1280 -> 1280 9.4 / 8.7 at 1, 10.7 / 9.2 at 16, 17.3 / 15.8 at 160, 17.2 / 18.3 at 176, 22.0 / 19.0 at
+# 224; 1600 -> 1600 9.8 / 9.3 at 1, 17.8 / 14.4 at 64, 26.9 / 25.5 at 224, 27.2 / 27.6 at 256; 2048 -> 512 9.6 / 7.8 at 1, 20.1 / 14.4 at 256;
+# 2048 -> 2048 30.8 / 29.5 at 176, 30.6 / 31.4 at 192; 3072 -> 768 12.2 / 8.1 at 1, 18.0 / 12.8 at 64, 32.2 / 24.3 at 256; 6400 -> 1600 23.4 /
+# 15.8 at 1, 49.7 / 27.0 at 64, 81.2 / 67.2 at 224.
 EXACT_PARTS_MAX_ROWS = 256
 EXACT_PARTS_MAX_OUTPUTS = 380_000
 EXACT_PARTS_SHORT_MAX_OUTPUTS = 172_000    # under inner sizes below 1,024
@@ -244,8 +248,9 @@ def exact_leaves_parts(n_rows: int, n_out: int, k_dim: int) -> bool:
     """Whether the 32-bit path leaves a product of this size as sums over its blocks of k for the LayerNorm behind it."""
     if k_dim < 768 or n_rows > EXACT_PARTS_MAX_ROWS:
         return False
-    from_rows = 1 if k_dim > 1536 else 6 if k_dim >= 1280 else 16
-    return n_rows >= from_rows and n_rows * n_out <= (EXACT_PARTS_MAX_OUTPUTS if k_dim >= 1024 else EXACT_PARTS_SHORT_MAX_OUTPUTS)
+    if k_dim < 1024:
+        return n_rows * n_out <= EXACT_PARTS_SHORT_MAX_OUTPUTS and -(-n_rows // 16) * -(-n_out // 16) > 256
+    return n_rows >= (1 if k_dim >= 1280 else 16) and n_rows * n_out <= EXACT_PARTS_MAX_OUTPUTS
 
 
 def plain_residual(ctx, h, x: torch.Tensor) -> None:

@@ -262,13 +262,15 @@ def test_float32_product_of_few_rows_under_long_inner_sizes(k):
 
 
 @pytest.mark.parametrize("k", [37, 320, 1100, 2048])
-def test_float32_product_done_again_has_the_same_bits_whatever_the_tiles(k):
-    """Elements of rows with a value that bfloat16 rounds to infinity, computed once more in float32, in each kernel, beside rows that
-    are not."""
+@pytest.mark.parametrize("large,beside", [(3.4e38, 1.0), (1e33, 1e-33)])
+def test_float32_product_done_again_has_the_same_bits_whatever_the_tiles(k, large, beside):
+    """Elements of rows with a value whose parts are not finite, computed once more in float32, in each kernel, beside rows that are
+    not; also where that value's product is no larger than the others', so that the bits of the other blocks show."""
     g = torch.Generator().manual_seed(k)
     o, n = 1500, 1030
     a, w = rnd(g, n, k).to(DEV), rnd(g, o, k, scale=0.05).to(DEV)
-    a[::3, k // 2] = 3.4e38
+    a[::3, k // 2] = large
+    w[:, k // 2] *= beside
     whole = torch.empty(n, o, device=DEV)
     kernels.linear_generic(a, w, None, whole, n)
     want = a.double() @ w.double().T

@@ -238,7 +238,10 @@ LEAVE_PARTS_MAX_ROWS = 256     # (the tiled kernel's split; the decode kernel's 
 # at 8, 9.1 / 8.6 at 16, 14.9 / 14.8 at 224; 1280 -> 1280 9.4 / 8.7 at 1, 10.7 / 9.2 at 16, 17.3 / 15.8 at 160, 17.2 / 18.3 at 176, 22.0 / 19.0 at
 # 224; 1600 -> 1600 9.8 / 9.3 at 1, 17.8 / 14.4 at 64, 26.9 / 25.5 at 224, 27.2 / 27.6 at 256; 2048 -> 512 9.6 / 7.8 at 1, 20.1 / 14.4 at 256;
 # 2048 -> 2048 30.8 / 29.5 at 176, 30.6 / 31.4 at 192; 3072 -> 768 12.2 / 8.1 at 1, 18.0 / 12.8 at 64, 32.2 / 24.3 at 256; 6400 -> 1600 23.4 /
-# 15.8 at 1, 49.7 / 27.0 at 64, 81.2 / 67.2 at 224.
+# 15.8 at 1, 49.7 / 27.0 at 64, 81.2 / 67.2 at 224.  That is with the matrix in the caches; read from memory, as in a decode step of a
+# GPT-2-small shape (12 layers, 50,257 tokens), what sums gain a layer at 768 -> 768 is -1.2 us at 1 row, -0.7 at 8, 0.4 to 0.9 at 16
+# (the step of 16 sampled requests 748 -> 738 us), 0 at 24 to 32, -0.4 at 48 to 64, 0.1 at 128; at 960 -> 960 -0.3 at 4, 1.0 at 16, 0.2 at 32,
+# -0.3 at 64, 0.8 at 160.  So they are left at 13 to 16 rows too, where the product has least of the chip.
 EXACT_PARTS_MAX_ROWS = 256
 EXACT_PARTS_MAX_OUTPUTS = 380_000
 EXACT_PARTS_SHORT_MAX_OUTPUTS = 172_000    # under inner sizes below 1,024
@@ -249,7 +252,8 @@ def exact_leaves_parts(n_rows: int, n_out: int, k_dim: int) -> bool:
     if k_dim < 768 or n_rows > EXACT_PARTS_MAX_ROWS:
         return False
     if k_dim < 1024:
-        return n_rows * n_out <= EXACT_PARTS_SHORT_MAX_OUTPUTS and -(-n_rows // 16) * -(-n_out // 16) > 256
+        pays = 12 < n_rows <= 16 or -(-n_rows // 16) * -(-n_out // 16) > 256
+        return pays and n_rows * n_out <= EXACT_PARTS_SHORT_MAX_OUTPUTS
     return n_rows >= (1 if k_dim >= 1280 else 16) and n_rows * n_out <= EXACT_PARTS_MAX_OUTPUTS
 
 

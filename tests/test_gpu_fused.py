@@ -472,7 +472,8 @@ def test_addition_of_few_rows_is_no_less_exact_in_the_tiled_kernel(rows, n_out, 
 
 @pytest.mark.parametrize("rows,n_out,k_dim,left", [
     (1, 768, 3072, True), (1, 400, 1536, True), (1, 1280, 1280, True), (1, 1276, 1276, False), (6, 1280, 1280, True),
-    (15, 768, 768, False), (80, 768, 768, False), (81, 768, 768, True), (15, 512, 1024, False), (16, 512, 1024, True),
+    (12, 768, 768, False), (13, 768, 768, True), (16, 768, 768, True), (17, 768, 768, False), (80, 768, 768, False),
+    (81, 768, 768, True), (15, 512, 1024, False), (16, 512, 1024, True),
     (64, 640, 640, False), (223, 768, 768, True), (224, 772, 768, False), (224, 772, 1024, True),
     (256, 768, 3072, True), (257, 768, 3072, False), (185, 2048, 2048, True), (186, 2048, 2048, False)])
 def test_float32_addition_leaves_sums_where_that_pays(rows, n_out, k_dim, left):

@@ -1,11 +1,11 @@
 // Attention of a step that has both, single tokens of decoding requests and prompt portions (bfloat16, head sizes 64 and 128),
 // in one launch.
 //
-// The two kind of tokens have kernels of their own (attention_decode_wide.hip, attention_prefill.hip), neither of which fills
+// The two kinds of tokens have kernels of their own (attention_decode_wide.hip, attention_prefill.hip), neither of which fills
 // the chip in such a step: a portion of 512 tokens x 12 heads is 192 tiles, eleven decoding requests are 132 workgroups, on 256
 // compute units, one behind the other 11.4 + 8.9 us a layer.  Here the first workgroups of the launch are tiles and the ones
 // behind them (token, head) pairs, both with the bodies of those kernels, so that they run side by side.  A pair's workgroup
-// holds a tile's LDS and registers, which is a compute unit, so it is done for up to 256 pairs; more go to their own kernel.
+// holds a tile's LDS and registers, a compute unit or half of one, so it is done for up to 256 pairs; more go to their own kernel.
 //
 // Where a tile has four waves (head size 128, and 64 with many tiles or short contexts) a pair has four as well, a pass of 256 keys at a time,
 // and behind long contexts that chain outlasts tiles and eight waves one behind the other: 8 requests x 8 heads of 128 beside
@@ -128,7 +128,8 @@ extern "C" int mgpt_mixed_attention_bf16(
   // What four waves lose on a token against eight, 0.005 us a key, is to be no more than what the tiles beside them take and a
   // launch, 7 us for a portion of 64 tokens, 13 for 512 (19 are saved there, but a token beyond the line then waits for those
   // below it: one behind 8,363 keys and others behind some 4,000 beside 630 tokens 97 us as two launches, 113 with a line at
-  // 4,096 keys, 93 here).  Head size 64 comes here with hundreds of tiles only and loses less.
+  // 4,096 keys, 93 here).  Head size 64 comes here with
+  // hundreds of tiles, where it loses less, or with 1,024 keys at most.
   const int keys = head_dim == 64 ? 16384 : (n_tokens < 512 ? 1024 + 3 * n_tokens : 2560);
   const MixedArgs a = {(const bf16_t*)q, ldq, (bf16_t*)out, ldo, (const bf16_t*)kpool, (const bf16_t*)vpool, block_tables,
                        max_blocks, positions, q_req, cu_q, seq_lens, n_decode, first_req, n_req, 0, single_below, n_head,

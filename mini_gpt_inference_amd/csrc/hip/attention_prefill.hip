@@ -92,7 +92,7 @@ __global__ __launch_bounds__(64 * Q * K, (pf_waves<D, K>())) void prefill_attent
 
 // One workgroup per (tile of 32 or 64 queries, request, head); max_q_len sizes the grid and is the host's
 // upper bound on the tokens any request brings (a request may bring none: its workgroups leave at
-// once);  single_below: requests that bring exactly one token, and that as one of the step's first
+// once).  single_below: requests that bring exactly one token, and that as one of the step's first
 // single_below tokens, are left to another kernel.  Head
 // sizes 32, 64, 96, 128 and a positive scale; others are refused.
 extern "C" int mgpt_prefill_attention_bf16(

@@ -11,8 +11,8 @@ def _mixed_step(ctx, q, out, k_pool, v_pool, group, n_head: int, scale: float, w
                 softcap: float = 0.0, gate=None, mask=None) -> bool:
     """A step with prompt portions.  The requests that lead the step with one token each (a scheduler
     puts the decoding requests first) go to the decode kernel, token n being request n; the rest,
-    prompt portions mostly, to the MFMA tile kernel, which would spend a 64-query tile on a single
-    token; both in one launch where the single tokens are few.  False, having launched nothing, if the
+    prompt portions mostly, to the MFMA tile kernel, which would spend a tile of 32 or 64 queries
+    on a single token; both in one launch where the single tokens are few.  False, having launched nothing, if the
     tile kernel does not take the case."""
     mask = mask or {}
     q_lens = ctx.host_q_lens

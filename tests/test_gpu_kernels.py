@@ -243,10 +243,10 @@ def test_float32_product_of_an_inner_size_of_one(n, o):
         assert torch.equal(sums[0], a * w.T)
 
 
-@pytest.mark.parametrize("k", [769, 1001, 1028, 1280, 2300, 4100, 4609])
+@pytest.mark.parametrize("k", [769, 1001, 1025, 1028, 1149, 1152, 1280, 2300, 4100, 4609])
 def test_float32_product_of_few_rows_under_long_inner_sizes(k):
-    """A wave has a block of 256 k at a time, of which the last may end anywhere, in one round or two (beyond 16 blocks): the bits of
-    the sums over blocks, added up in order."""
+    """A wave has two groups of 32 k at a time, three from an inner size of 1,025 on, or a block of 256 from 1,153 on, of which the last
+    may end anywhere, in one round or two (beyond 16 blocks): the bits of the sums over blocks, added up in order."""
     g = torch.Generator().manual_seed(k)
     for rows, cols in ((1, 300), (16, 52), (17, 132), (40, 900)):
         a, w = rnd(g, rows, k).to(DEV), rnd(g, cols, k).to(DEV)

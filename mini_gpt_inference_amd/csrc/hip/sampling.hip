@@ -492,7 +492,7 @@ __device__ __forceinline__ unsigned int wave_top_p(const unsigned int (&x)[N], c
 // Top-k and top-p over a list of n <= SAMPLE_LIST entries in LDS (keys, and masses by key), zeros behind them up to a
 // multiple of four: the smallest key that both keep, the same in all threads.  A thread has an entry and goes over the whole list:
 // fewer than k keys above its own, and their mass within the budget.  64 rows of 50,304 logits, temperature, top-k 50 and top-p 26.9 us
-// with two searches by halving in one wave, some 60 rounds with sums over lanes, 23.9 so.
+// with two searches by halving in one wave, some 60 rounds with sums over lanes, 24.4 so.
 __device__ __forceinline__ unsigned int list_floor(const unsigned int* key, const float* mass, int n, int k, float p, float* red_f,
                                                    int* red_i) {
   const int t = threadIdx.x;
@@ -519,7 +519,7 @@ __device__ __forceinline__ unsigned int list_floor(const unsigned int* key, cons
 // The same choice for rows of at most 1024 x K logits, each thread keeping its stretch of `per` consecutive logits in
 // registers (K of them at most), so that the row is read from memory once.  The kernel above reads it again for each of
 // the 30 to 65 counts and sums of its two searches, about 6 us a time.  Rows of 50,304 logits, 64 of them, us a call,
-// above / here: temperature, top-k 50 and top-p 447 / 28; top-p alone 414 / 118 (flat), 373 / 81 (sharp); temperature
+// above / here: temperature, top-k 50 and top-p 447 / 24; top-p alone 414 / 118 (flat), 373 / 81 (sharp); temperature
 // alone 47 / 35; greedy rows 6.3 / 6.3.  What is left is one workgroup's load of 200 KB (4 us) and the instructions of
 // its 16 waves over 50 logits a thread; a row cut over workgroups would need them to meet.
 //

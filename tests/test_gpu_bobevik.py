@@ -303,6 +303,36 @@ def test_decaying_state_whole_in_portions_and_slots_used_again(dtype, H, D, E):
         helpers.assert_close(state[1:4], whole_state[1:4], "float32", f"{variant} state")
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("H,D,E", [(2, 128, 128), (3, 20, 12), (1, 256, 64), (2, 8, 256), (1, 37, 50), (1, 64, 65)])
+def test_single_tokens_have_the_bits_of_the_walk_over_several(dtype, H, D, E):
+    """A step of single tokens goes another way through the kernel than a request's several, and adds up in the same order:
+    five tokens of three requests at once and one after the other, with rotation, norm and gate and without."""
+    g = torch.Generator().manual_seed(D + E)
+    z, k_off, v_off, g_off = _state_case(g, dtype, [5, 5, 5], H, D, E)
+    z = z.to(DEV)
+    decay = torch.tensor(([0.999, 0.6, 0.9] * 3)[:H]).to(DEV)
+    slots = torch.tensor([2, 0, 1], dtype=torch.int32, device=DEV)
+    dims = (D - 1) // 2 * 2
+    for plain in (True, False):
+        kwargs = dict(silu_inputs=plain, freq=None if plain else _freq(dims, 1000.0).to(DEV), k_scale=1.0 if plain else 0.25,
+                      norm_eps=None if plain else 1e-5)
+        results = []
+        for steps in ([5], [1] * 5):
+            state = torch.full((3, H * D * E), float("nan"), device=DEV)
+            out, done = torch.zeros(15, H * E, dtype=TDT[dtype], device=DEV), 0
+            for count in steps:
+                rows = [5 * r + done + t for r in range(3) for t in range(count)]
+                o = torch.zeros(len(rows), H * E, dtype=TDT[dtype], device=DEV)
+                kernels.decay_state(z[rows].contiguous(), 0, k_off, v_off, -1 if plain else g_off, H, D, E, decay, state, slots,
+                                    torch.tensor([0, count, 2 * count, 3 * count], dtype=torch.int32, device=DEV), 3,
+                                    torch.tensor([r % 5 for r in rows], dtype=torch.int32, device=DEV), o, **kwargs)
+                out[rows] = o
+                done += count
+            results.append((out, state))
+        assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
+
+
 @pytest.mark.parametrize("H,D,E", [(2, 128, 128), (3, 40, 24), (1, 16, 130)])
 @pytest.mark.parametrize("lens", [[1, 255, 256, 257], [511, 512, 513, 0, 700], [1300], [300] * 70, [4] * 66 + [600]])
 def test_decaying_state_in_segments(lens, H, D, E):

@@ -90,6 +90,10 @@ int mgpt_residual_settle(const float* base, const float* partials, int n_parts, 
     tok_table, const void* pos_table, const int* ids, const int* token_positions, float* settled, int n_rows,
     int width, hipStream_t stream);
 // linear_exact.hip
+int mgpt_linear_exact_normed(const float* x, const int* rows, const float* gain, const float* norm_bias, float eps,
+                             const float* W, const float* bias, float* out, long ldo, int n_rows, int n_out, int k_dim,
+                             int epilogue, float* kpool, float* vpool, const int* slot_mapping, int q_width,
+                             int kv_width, int head_dim, int page_size, hipStream_t stream);
 int mgpt_linear_exact_qkv(const float* A, long lda, const float* W, const float* bias, float* out, long ldo, int n_rows,
     int n_out, int k_dim, float* kpool, float* vpool, const int* slot_mapping, int q_width, int kv_width, int head_dim,
     int page_size, hipStream_t stream);
@@ -286,6 +290,7 @@ int mgpt_linear_mfma_grouped(const void* act, long lda, const void* w, long w_st
   X(mgpt_fused_mlp_decode) \
   X(mgpt_residual_layernorm) \
   X(mgpt_residual_settle) \
+  X(mgpt_linear_exact_normed) \
   X(mgpt_linear_exact_qkv) \
   X(mgpt_linear_generic) \
   X(mgpt_linear_mfma) \

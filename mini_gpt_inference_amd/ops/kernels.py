@@ -225,6 +225,54 @@ def linear_exact_qkv(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tens
     return True
 
 
+def linear_exact_norms(n_rows: int, n_out: int, k_dim: int) -> bool:
+    """Whether a float32 product of this size norms its rows itself (linear_exact_normed, aligned operands)."""
+    return bool(library.kernels().mgpt_linear_exact_norms(n_rows, n_out, k_dim))
+
+
+def linear_exact_normed(x: torch.Tensor, gain: torch.Tensor, norm_bias: Optional[torch.Tensor], eps: float, w: torch.Tensor,
+                        bias: Optional[torch.Tensor], out: torch.Tensor, n_rows: int, epilogue: int = EPI_NONE,
+                        rows: Optional[torch.Tensor] = None, scatter=None) -> bool:
+    """out[:n_rows] = layer_norm(x[rows] or x)[:n_rows] @ w.T (+ bias) with the epilogue, float32 throughout, in one launch: the bits
+    of layer_norm and the product behind it.  scatter as for linear_exact_qkv.  False, with nothing launched, where the
+    product has too much to do for each of its workgroups to norm its rows, and for other types and unaligned operands."""
+    _need_cuda(x, gain, norm_bias, w, bias, out, rows)
+    n_out, k_dim = w.shape
+    if epilogue not in (EPI_NONE, EPI_GELU, EPI_RELU2) or (scatter is not None and epilogue != EPI_NONE):
+        return False
+    if any(t is not None and t.dtype != torch.float32 for t in (x, gain, norm_bias, w, bias, out)):
+        return False
+    if not linear_exact_norms(n_rows, n_out, k_dim) or any(t is not None and t.data_ptr() % 16 for t in (x, gain, norm_bias, w)):
+        return False
+    _need(w.is_contiguous(), "weight must be dense [out, in]")
+    _need(x.dim() == 2 and x.is_contiguous() and x.shape[1] == k_dim and (rows is not None or x.shape[0] >= n_rows),
+          f"rows to be normed must be dense [>=n_rows, {k_dim}]")
+    _need(gain.numel() == k_dim and (norm_bias is None or norm_bias.numel() == k_dim), "LayerNorm gain and bias must be [width]")
+    _need(out.dim() == 2 and out.stride(1) == 1 and out.shape[1] == n_out and out.shape[0] >= n_rows,
+          f"output must be [>=n_rows, {n_out}] with unit inner stride")
+    _need(bias is None or bias.numel() == n_out, "bias must be float32 [out]")
+    if rows is not None:
+        _need_i32("rows", rows, n_rows)
+    pools = (None, None, None, 0, 0, 0, 0)
+    if scatter is not None:
+        k_pool, v_pool, slot_mapping, q_width, kv_width = scatter
+        if k_pool.dtype != torch.float32 or v_pool.dtype != torch.float32:
+            return False
+        _need_cuda(k_pool, v_pool, slot_mapping)
+        _need(k_pool.shape == v_pool.shape and k_pool.dim() == 4 and k_pool.is_contiguous() and v_pool.is_contiguous(),
+              "key and value pools must be dense [pages, kv_heads, page_size, head_dim]")
+        _, n_kv_head, page_size, head_dim = k_pool.shape
+        _need(kv_width == n_kv_head * head_dim and q_width + 2 * kv_width == n_out,
+              "the output's columns must be the queries, then the keys and values of the pools' heads")
+        _need_i32("slot_mapping", slot_mapping, n_rows)
+        pools = (_ptr(k_pool), _ptr(v_pool), _ptr(slot_mapping), q_width, kv_width, head_dim, page_size)
+    rc = library.kernels().mgpt_linear_exact_normed(
+        _ptr(x), _ptr(rows), _ptr(gain), _ptr(norm_bias), float(eps), _ptr(w), _ptr(bias), _ptr(out), out.stride(0), n_rows, n_out,
+        k_dim, SK_EPI_QKV if scatter is not None else epilogue, *pools, _stream())
+    _check(rc, "linear_exact_normed")
+    return True
+
+
 def kv_write(qkv: torch.Tensor, k_off: int, v_off: int, k_pool: torch.Tensor, v_pool: torch.Tensor,
              slot_mapping: torch.Tensor, n_tokens: int) -> None:
     """Stores the new keys and values of n_tokens rows of qkv into their pages.

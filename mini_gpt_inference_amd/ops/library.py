@@ -138,6 +138,8 @@ def _declare_optional(lib: ctypes.CDLL) -> None:
         "mgpt_linear_mfma_partials": [I, I, I, I],
         "mgpt_linear_mfma_choice": [I, I, I, I, I, I],
         "mgpt_linear_exact_kernel": [I, I, I, I],
+        "mgpt_linear_exact_norms": [I, I, I],
+        "mgpt_linear_exact_normed": [P, P, P, P, F, P, P, P, L, I, I, I, I, P, P, P, I, I, I, I, P],
         "mgpt_linear_exact_parts": [P, L, P, P, I, I, I, P],
         "mgpt_layernorm_parts": [P, P, I, L, P, P, P, P, P, I, I, F, P, P],
         "mgpt_linear_mfma_parts": [P, L, P, P, P, L, I, I, I, P],

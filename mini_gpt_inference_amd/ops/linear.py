@@ -343,7 +343,7 @@ def linear(ctx, a: Union[torch.Tensor, LazyNorm], w: torch.Tensor, bias: Optiona
     stream through the folded LayerNorm when `a` is a LazyNorm of a fusable norm and the rows are
     few; splitting a long inner size over workgroups when the rows are many) and more rows to the
     tiled MFMA kernel (which also splits a long inner size when its tiles are few); the 32-bit path, and every shape those refuse, go to the general product
-    (on the matrix cores in 32 bits where everything is float32).  `scatter` = (k_pool, v_pool,
+    (on the matrix cores in 32 bits where everything is float32; at few rows with the LayerNorm of a LazyNorm inside).  `scatter` = (k_pool, v_pool,
     slot_mapping, q_width, kv_width) asks for the new keys and values to be stored into their
     pages by the same kernel; the return value says whether that was done."""
     if n_rows == 0:
@@ -383,6 +383,11 @@ def linear(ctx, a: Union[torch.Tensor, LazyNorm], w: torch.Tensor, bias: Optiona
         if kernels.linear_skinny(as_tensor(ctx, a), w, bias, out, n_rows, epi, scatter=scatter, partials=partials,
                                  w_packed=packed_weight(w, ctx)):
             return scatter is not None
+    if (isinstance(a, LazyNorm) and ctx.exact and a._tensor is None and getattr(a.norm, "fusable_layer_norm", False)
+            and a.x.is_contiguous()
+            and kernels.linear_exact_normed(a.x, a.norm.weight, a.norm.bias, a.norm.eps, w, bias, out, n_rows, epilogue, a.rows,
+                                            scatter)):
+        return scatter is not None
     a = as_tensor(ctx, a)
     if fast and scatter is not None and kernels.linear_mfma(a, w, bias, out, n_rows, epilogue, scatter=scatter):
         return True

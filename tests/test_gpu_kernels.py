@@ -397,6 +397,53 @@ def test_float32_product_stores_keys_and_values(n, k, h, hk, d, kernel):
     assert torch.equal(pools[1].nan_to_num(9.0), pools[3].nan_to_num(9.0))
 
 
+@pytest.mark.parametrize("n,k,h,d", [(1, 4, 1, 4), (3, 64, 4, 16), (16, 128, 2, 64), (17, 132, 3, 20), (16, 256, 4, 64), (5, 260, 5, 32),
+                                     (16, 512, 8, 64), (33, 512, 2, 64), (2, 516, 2, 36), (16, 768, 12, 64), (1, 640, 10, 64)])
+@pytest.mark.parametrize("gather,with_bias", [(False, True), (True, False)])
+def test_float32_product_that_norms_its_rows_has_the_bits_of_both_kernels(n, k, h, d, gather, with_bias):
+    """The product with the LayerNorm inside, plain, with an activation and with keys and values into their pages, against the
+    LayerNorm kernel and the product behind it: the same bits, in rows with an infinity and a NaN too."""
+    gen = torch.Generator().manual_seed(n * 1000 + k)
+    x = rnd(gen, n + 5, k, scale=2.0)
+    x[0, 1], x[n // 2, k - 1] = float("inf"), float("nan")
+    x[n - 1] = 3.0 + 1e-3 * rnd(gen, k)                     # far from zero, nearly equal
+    x = x.to(DEV)
+    rows = torch.randperm(n + 5, generator=gen)[:n].to(torch.int32).to(DEV) if gather else None
+    gain, shift = rnd(gen, k).to(DEV), rnd(gen, k).to(DEV) if with_bias else None
+    o = 3 * h * d
+    w, bias = rnd(gen, o, k, scale=k ** -0.5).to(DEV), rnd(gen, o).to(DEV) if with_bias else None
+    assert kernels.linear_exact_norms(n, o, k)
+    normed = torch.empty(n, k, device=DEV)
+    kernels.layer_norm(x, gain, shift, normed, n, 1e-5, rows)
+    for epi in (kernels.EPI_NONE, kernels.EPI_GELU, kernels.EPI_RELU2):
+        want, got = torch.empty(n, o, device=DEV), torch.full((n + 1, o), 7.0, device=DEV)
+        kernels.linear_generic(normed, w, bias, want, n, epi)
+        assert kernels.linear_exact_normed(x, gain, shift, 1e-5, w, bias, got, n, epi, rows)
+        assert torch.equal(got[:n].nan_to_num(nan=1e30), want.nan_to_num(nan=1e30)) and (got[n] == 7.0).all()
+    slots = torch.randperm(48, generator=gen)[:n].to(torch.int32)
+    slots[n - 1] = -1
+    results = []
+    for inside in (False, True):
+        pools = torch.full((2, 3, h, 16, d), 7.0, device=DEV)
+        out = torch.full((n, o), 7.0, device=DEV)
+        scatter = (pools[0], pools[1], slots.to(DEV), h * d, h * d)
+        if inside:
+            assert kernels.linear_exact_normed(x, gain, shift, 1e-5, w, bias, out, n, rows=rows, scatter=scatter)
+        else:
+            assert kernels.linear_exact_qkv(normed, w, bias, out, n, scatter)
+        results.append((out.nan_to_num(nan=1e30), pools.nan_to_num(nan=1e30)))
+    assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
+
+
+@pytest.mark.parametrize("n,o,k,norms", [(16, 4096, 512, True), (16, 4097, 512, False), (32, 2048, 512, True), (33, 2048, 512, False),
+                                         (3, 300, 768, True), (3, 300, 772, False), (3, 300, 66, False)])
+def test_which_float32_products_norm_their_rows(n, o, k, norms):
+    assert kernels.linear_exact_norms(n, o, k) == norms
+    if not norms:
+        x, gain, w = torch.zeros(n, k, device=DEV), torch.ones(k, device=DEV), torch.zeros(o, k, device=DEV)
+        assert not kernels.linear_exact_normed(x, gain, None, 1e-5, w, None, torch.zeros(n, o, device=DEV), n)
+
+
 @pytest.mark.parametrize("n,k,o", [(1, 1, 4), (1, 1537, 512), (3, 256, 60), (4, 3072, 768), (16, 257, 64), (17, 1026, 68),
                                    (17, 3072, 768), (33, 5000, 260), (70, 2048, 2048), (128, 768, 1028), (130, 4097, 1600)])
 def test_float32_product_left_as_sums_over_its_blocks(n, k, o):

@@ -79,6 +79,27 @@ def test_rms_norm_segments_gate_and_accumulate(dtype, groups, width, stride):
     helpers.assert_close(out, _d(acc) + 0.5 * base.reshape(n, -1), "float32", "accumulate")
 
 
+@pytest.mark.parametrize("x_dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("gate_dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("out_dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("width", [1, 63, 128, 129, 257, 512, 1025, 4096, 4097])
+def test_rms_norm_of_every_combination_of_types(x_dtype, gate_dtype, out_dtype, width):
+    """The values a thread holds (1, 2, 4, 16 of them, or none) and the types of input, gate and output, the gate behind the norm
+    and in front of it, with rows gathered."""
+    g = torch.Generator().manual_seed(width)
+    n = 3
+    x, gate = _rnd(g, n + 2, width, dtype=x_dtype, scale=2.0), _rnd(g, n, width, dtype=gate_dtype, scale=2.0)
+    gain, rows = _rnd(g, width) + 1.0, [4, 0, 3]
+    for act in ("sigmoid", "silu_first"):
+        out = torch.full((n + 1, width), 3.0, dtype=TDT[out_dtype], device=DEV)
+        kernels.rms_norm(x.to(DEV), gain.to(DEV), out, n, 1e-3, width, rows=torch.tensor(rows, dtype=torch.int32, device=DEV),
+                         gate=gate.to(DEV), gate_act=act)
+        xin = _d(x[rows])
+        want = (P.unit_rms(xin, 1e-3) * P.sigmoid(_d(gate)) if act == "sigmoid" else P.unit_rms(xin * P.silu(_d(gate)), 1e-3)) * _d(gain)
+        helpers.assert_close(out[:n], want, out_dtype, f"{act} {width}")
+        assert (out[n] == 3.0).all()
+
+
 @pytest.mark.parametrize("h_dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("branches,n,width", [(1, 3, 40), (2, 70, 64), (3, 5, 300), (4, 2, 1030), (1, 9, 2048), (1, 5, 3000),
                                               (1, 2, 5000), (1, 4, 1024), (2, 3, 2048), (2, 2, 2100)])

@@ -771,53 +771,104 @@ extern "C" int mgpt_grouped_linear_mfma(const void* a, long lda, const int* a_ro
 }
 
 // The same product for tiles of 16 slots (a decode step), laid out for the matrices' way from memory: a workgroup owns a
-// tile x 16 columns, its four waves take the inner size 32 at a time in turn, EXD loads each on their way at once, and
+// tile x 16 columns, its four waves take the inner size 64 at a time in turn, and
 // their sums meet in LDS in wave order.  With a unit (kind >= 0) the expert's matrix is its gate's rows over its up
 // rows, a workgroup owns 16 columns of both, and what it stores is the gated unit of the two sums: n_out is then the
 // hidden size.  tile_expert null: one matrix for all rows, of which the first n_rows are used (slot_token null).
-#define EXD 4
+//
+// A wave brings its slices of the matrix straight into LDS, eight rows of 128 bytes a load, STAGES steps of its own: no barrier, no
+// registers for what is on its way.  A lane's operand, 16 bytes of one of 16 rows, loaded as it is used makes every
+// load touch 16 lines in 16-byte pieces, and the unit that looks the lines up is what bounds it then (the rows are few: theirs are loaded
+// so; through LDS as well they took room that workgroups need).  The 16-byte pieces
+// of a row are XORed with its number, at the source, so that an operand's read from LDS meets no bank twice.  The matrix's first loads
+// leave before the tile's rows are looked up, two trips to memory one behind the other.  us in a graph, matrices from memory, 32 k a
+// step through registers / here: 8 rows, gated, 2048 -> 5440 (44.6 MB) 15.5 / 11.6, -> 1344 7.8 / 6.5, 1024 -> 2688 6.0 / 5.0; 16 pairs for
+// 8 experts 2048 -> 2048 gated (117 MB) 29.8 / 25.6 and down (59 MB) 15.4 / 12.7; 64 pairs for 64 experts 1024 -> 512 21.5 / 17.0,
+// 512 -> 1024 10.4 / 9.9.
+#define EX_STEP 64
 
-template <typename OT, bool GATED>
+template <typename OT, bool GATED, int STAGES>
 __global__ __launch_bounds__(256) void grouped_few_rows_kernel(
     const bf16_t* __restrict__ A, long lda, const int* __restrict__ a_rows, const bf16_t* __restrict__ W, long w_stride,
     const int* __restrict__ tile_expert, const int* __restrict__ slot_token, OT* __restrict__ out, long ldo,
     const int* __restrict__ out_rows, int n_rows, int n_out, int k_dim, int epilogue, int kind, float limit, float sharpness) {
-  constexpr int NJ = GATED ? 2 : 1;
+  constexpr int NJ = GATED ? 2 : 1, SLICE = 16 * EX_STEP;       // elements of 16 rows of a step
+  typedef __attribute__((address_space(1))) const void* global_ptr_t;
+  typedef __attribute__((address_space(3))) void* lds_ptr_t;
+  __shared__ __attribute__((aligned(16))) bf16_t staged[4][STAGES][NJ][SLICE];
   __shared__ ex_f32x4_t part[4][NJ][64];
   const int tile = blockIdx.y;
   const int e = tile_expert ? tile_expert[tile] : 0;
   if (e < 0) return;      // (the whole workgroup)
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, lg = lane >> 4;
+  const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col0 = blockIdx.x * 16;
+  const long up = (long)n_out * k_dim;
+  const bf16_t* const wm = W + (long)e * w_stride;
+  // this lane's part of a load: row 8 i + lane / 8, piece (lane % 8) ^ (row % 8)
+  const int lr = lane >> 3, lp = ((lane & 7) ^ lr) * 8;
+  const bf16_t* wl[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) wl[i] = wm + (long)(col0 + 8 * i + lr < n_out ? col0 + 8 * i + lr : n_out - 1) * k_dim + lp;
+  const int steps = k_dim / EX_STEP;
+  auto load_w = [&](int step, int st) {
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        __builtin_amdgcn_global_load_lds((global_ptr_t)(wl[i] + j * up + (long)step * EX_STEP),
+                                         (lds_ptr_t)(&staged[wave][st][j][i * (SLICE / 2)]), 16, 0, 0);
+  };
+#pragma unroll
+  for (int s = 0; s < STAGES; ++s)
+    if (wave + 4 * s < steps) load_w(wave + 4 * s, s);
+  // rows of the tile; those that are not used are the first one's, and count as zeros
   const int slot = tile * 16 + li;
   const bool a_ok = slot_token ? slot_token[slot] >= 0 : slot < n_rows;
-  const bf16_t* ap = A + (a_ok ? (long)(a_rows ? a_rows[slot] : slot) : 0L) * lda + lg * 8;
-  const bf16_t* wp = W + (long)e * w_stride + (long)(col0 + li < n_out ? col0 + li : n_out - 1) * k_dim + lg * 8;
-  const long up = (long)n_out * k_dim;
+  const int row = a_ok ? (a_rows ? a_rows[slot] : slot) : 0;
+  const bf16_t* ap = A + (long)row * lda + lg * 8;
+  ex_bf16x8_t af[STAGES][2];
+  auto load_a = [&](int step, int st) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) af[st][h] = *reinterpret_cast<const ex_bf16x8_t*>(ap + (long)step * EX_STEP + h * 32);
+  };
+#pragma unroll
+  for (int s = 0; s < STAGES; ++s) load_a(wave + 4 * s < steps ? wave + 4 * s : 0, s);
   const ex_bf16x8_t zero = {0, 0, 0, 0, 0, 0, 0, 0};
   ex_f32x4_t acc[NJ];
 #pragma unroll
   for (int j = 0; j < NJ; ++j) acc[j] = ex_f32x4_t{0.f, 0.f, 0.f, 0.f};
-  const int steps = k_dim / 32;      // whole ones
-  int st = wave;
-  for (; st + 4 * (EXD - 1) < steps; st += 4 * EXD) {
-    ex_bf16x8_t wf[NJ][EXD], af[EXD];
+  const int at0 = li * EX_STEP + ((lg ^ (li & 7)) * 8), at1 = li * EX_STEP + (((lg + 4) ^ (li & 7)) * 8);
+  for (int step0 = wave; step0 < steps; step0 += 4 * STAGES) {
 #pragma unroll
-    for (int d = 0; d < EXD; ++d) {
-      const long k = (long)(st + 4 * d) * 32;
+    for (int st = 0; st < STAGES; ++st) {
+      const int step = step0 + 4 * st;
+      if (step >= steps) break;
+      // A step's loads come together, but for the first steps, whose rows came behind all of their matrices.  The steps behind this one
+      // that are on their way: STAGES - 1, fewer towards the end.
+      if (step0 == wave || step + 4 * (STAGES - 1) >= steps) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      else asm volatile("s_waitcnt vmcnt(%0)" ::"n"((STAGES - 1) * (2 * NJ + 2)) : "memory");
+      ex_bf16x8_t wf[NJ][2];
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) wf[j][d] = *reinterpret_cast<const ex_bf16x8_t*>(wp + j * up + k);
-      af[d] = *reinterpret_cast<const ex_bf16x8_t*>(ap + k);
-    }
+      for (int j = 0; j < NJ; ++j) {
+        wf[j][0] = *reinterpret_cast<const ex_bf16x8_t*>(&staged[wave][st][j][at0]);
+        wf[j][1] = *reinterpret_cast<const ex_bf16x8_t*>(&staged[wave][st][j][at1]);
+      }
+      const ex_bf16x8_t a0 = a_ok ? af[st][0] : zero, a1 = a_ok ? af[st][1] : zero;
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // read before the stage is loaded again
+      if (step + 4 * STAGES < steps) {
+        load_w(step + 4 * STAGES, st);
+        load_a(step + 4 * STAGES, st);
+      }
 #pragma unroll
-    for (int d = 0; d < EXD; ++d) {
-      const ex_bf16x8_t a = a_ok ? af[d] : zero;
+      for (int j = 0; j < NJ; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j][0], a0, acc[j], 0, 0, 0);
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j][d], a, acc[j], 0, 0, 0);
+      for (int j = 0; j < NJ; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j][1], a1, acc[j], 0, 0, 0);
     }
   }
-  for (; st * 32 < k_dim; st += 4) {      // what is left, the last step perhaps not whole
-    const long k = (long)st * 32;
+  // what is left of the inner size, 32 at a time, the last step perhaps not whole
+  const bf16_t* wp = wm + (long)(col0 + li < n_out ? col0 + li : n_out - 1) * k_dim + lg * 8;
+  for (int k = steps * EX_STEP + wave * 32; k < k_dim; k += 128) {
     const bool k_ok = k + lg * 8 < k_dim;
     const ex_bf16x8_t a = a_ok && k_ok ? *reinterpret_cast<const ex_bf16x8_t*>(ap + k) : zero;
 #pragma unroll
@@ -857,8 +908,18 @@ extern "C" int mgpt_grouped_few_rows(const void* a, long lda, const int* a_rows,
   if ((k_dim & 7) || (lda & 7) || (w_stride & 7) || (((size_t)a | (size_t)w) & 15)) return MGPT_ERR_BAD_SHAPE;
   if (n_tiles > 65535) return MGPT_ERR_TOO_LARGE;
   dim3 grid((n_out + 15) / 16, n_tiles), block(256);
+  // One stage a wave while the inner size is short, since more workgroups on a compute unit bring more than more stages do; two under long
+  // ones and for gated experts from 2,048 on (us, one / two / three: gated 2048 -> 5440 11.6 / 12.0 / 12.0, 3072 -> 1024 8.1 / 7.7 / 7.7,
+  // 5440 -> 2048 17.1 / 14.5 / 14.5; experts gated 2048 -> 2048 of 16 pairs 26.8 / 25.6 / 27.8, of 2 9.8 / 10.0 / 9.9, down 12.7 / 13.2 / 13.7,
+  // 4096 -> 1024 13.2 / 12.5 / 12.8).
+  const bool two = k_dim > 2048 || (kind >= 0 && tile_expert && k_dim >= 2048);
 #define GF_LAUNCH(OT, G)                                                                                              \
-  hipLaunchKernelGGL((grouped_few_rows_kernel<OT, G>), grid, block, 0, stream, (const bf16_t*)a, lda, a_rows,         \
+  do {                                                                                                                \
+    if (two) GF_LAUNCH_AS(OT, G, 2);                                                                                  \
+    else GF_LAUNCH_AS(OT, G, 1);                                                                                      \
+  } while (0)
+#define GF_LAUNCH_AS(OT, G, STAGES)                                                                                   \
+  hipLaunchKernelGGL((grouped_few_rows_kernel<OT, G, STAGES>), grid, block, 0, stream, (const bf16_t*)a, lda, a_rows,         \
                      (const bf16_t*)w, w_stride, tile_expert, slot_token, (OT*)out, ldo, out_rows, n_rows, n_out,     \
                      k_dim, epilogue, kind, limit, sharpness)
   if (out_dtype == MGPT_F32) {
@@ -869,6 +930,7 @@ extern "C" int mgpt_grouped_few_rows(const void* a, long lda, const int* a_rows,
     return MGPT_ERR_BAD_DTYPE;
   }
 #undef GF_LAUNCH
+#undef GF_LAUNCH_AS
   return mgpt_last_error();
 }
 

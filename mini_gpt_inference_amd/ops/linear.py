@@ -154,6 +154,17 @@ FOLD_ANY_OUT_MAX_OUT = 8192
 # row (9.4, 16.4, 28.5 us; at an inner size of 1600 it is behind from 4 rows on).
 WIDE_OUT = 8192
 WIDE_OUT_DECODE_WORK = 8192
+
+
+def wide_rows_once(n_rows: int, k_dim: int) -> bool:
+    """Whether a very wide output beyond that work goes to the kernel that reads the matrix once, whole lines a load, for a tile of 16 rows
+    (linear_rows_once).  Its time grows with the rows, from a lower level than the tiled kernel's; and rows of 4,096 bytes and multiples
+    come to the tiled kernel from few of the memory's channels at a time.  Tiled / here, us: 32768 x 768 12.8 / 12.0 at 8 rows, 12.9 / 12.6 at
+    12, 50257 x 768 17.6 / 16.9 at 8; 32768 x 1024 15.1 / 13.6 at 8, 50257 x 1024 20.9 / 20.5 at 8, 21.6 / 21.7 at 12; 32768 x 2048 33.8 / 28.7
+    at 8, 33.9 / 29.8 at 12, 50257 x 2048 44.5 / 43.1 at 8, 45.4 / 45.1 at 12; between, 50257 x 1600 31.7 / 32.6 at 6, 32768 x 2560 34.4 / 34.5 at 8."""
+    return n_rows <= (12 if k_dim % 2048 == 0 else 8 if k_dim <= 1024 else 0)
+
+
 # The decode kernel's time grows with the rows (every workgroup loads all of them for its 16 output
 # columns), the tiled kernel's hardly: under a large matrix with a wide output the tiled kernel (32 x
 # 32 tiles, several steps on their way from memory) is ahead from 17 rows on.  Matrices from memory,
@@ -389,6 +400,9 @@ def linear(ctx, a: Union[torch.Tensor, LazyNorm], w: torch.Tensor, bias: Optiona
                                             scatter)):
         return scatter is not None
     a = as_tensor(ctx, a)
+    if (fast and wide_out and bias is None and scatter is None and epilogue == kernels.EPI_NONE and wide_rows_once(n_rows, w.shape[1])
+            and kernels.linear_rows_once(a, w, out, n_rows)):
+        return False
     if fast and scatter is not None and kernels.linear_mfma(a, w, bias, out, n_rows, epilogue, scatter=scatter):
         return True
     if fast:

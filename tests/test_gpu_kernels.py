@@ -444,6 +444,21 @@ def test_which_float32_products_norm_their_rows(n, o, k, norms):
         assert not kernels.linear_exact_normed(x, gain, None, 1e-5, w, None, torch.zeros(n, o, device=DEV), n)
 
 
+@pytest.mark.parametrize("n,k,o", [(1, 64, 16), (8, 768, 8192), (9, 1030 // 8 * 8, 8200), (12, 2048, 8193), (16, 40, 33), (3, 4096, 100), (16, 320, 48)])
+@pytest.mark.parametrize("o_dt", ["float32", "bfloat16"])
+def test_linear_rows_once(n, k, o, o_dt):
+    """A pass over the matrix for up to 16 rows: one stage and two, inner sizes that are no whole steps, ragged columns; and that
+    very wide outputs of few rows go there."""
+    g = torch.Generator().manual_seed(n * k + o)
+    a, w = rnd(g, n, k, dtype="bfloat16"), rnd(g, o, k, dtype="bfloat16", scale=k ** -0.5)
+    out = torch.full((n + 1, o), 7.0, dtype=torch.float32 if o_dt == "float32" else torch.bfloat16, device=DEV)
+    assert kernels.linear_rows_once(a.to(DEV), w.to(DEV), out, n)
+    helpers.assert_close(out[:n], a.double() @ w.double().T, o_dt, f"{n} {k} {o}")
+    assert (out[n] == 7.0).all()
+    from mini_gpt_inference_amd.ops import linear as L
+    assert L.wide_rows_once(8, 1024) and L.wide_rows_once(12, 2048) and not L.wide_rows_once(9, 1024) and not L.wide_rows_once(1, 1600)
+
+
 @pytest.mark.parametrize("n,k,o", [(1, 1, 4), (1, 1537, 512), (3, 256, 60), (4, 3072, 768), (16, 257, 64), (17, 1026, 68),
                                    (17, 3072, 768), (33, 5000, 260), (70, 2048, 2048), (128, 768, 1028), (130, 4097, 1600)])
 def test_float32_product_left_as_sums_over_its_blocks(n, k, o):

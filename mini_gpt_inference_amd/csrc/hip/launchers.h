@@ -103,6 +103,8 @@ int mgpt_linear_generic(const void* A, int a_dtype, long lda, const void* W, int
 // linear_mfma.hip
 int mgpt_linear_mfma_parts(const void* act, long lda, const void* w, const float* bias, float* partials,
                            long partials_floats, int n_rows, int n_out, int k_dim, hipStream_t stream);
+int mgpt_linear_mfma_shape_parts(int shape, int k_parts, const void* act, long lda, const void* w, const float* bias,
+                                 float* partials, long partials_floats, int n_rows, int n_out, int k_dim, hipStream_t stream);
 int mgpt_linear_mfma(const void* act, long lda, const void* w, const float* bias, void* out, int out_dtype,
     long ldo, int n_rows, int n_out, int k_dim, int epilogue, float* partials, long partials_floats,
     hipStream_t stream);
@@ -296,6 +298,7 @@ int mgpt_linear_mfma_grouped(const void* act, long lda, const void* w, long w_st
   X(mgpt_linear_mfma) \
   X(mgpt_linear_mfma_parts) \
   X(mgpt_linear_mfma_shape) \
+  X(mgpt_linear_mfma_shape_parts) \
   X(mgpt_linear_mfma_xielu) \
   X(mgpt_linear_mfma_qkv) \
   X(mgpt_linear_skinny) \

@@ -834,6 +834,132 @@ int launch_halves(const void* act, long lda, const void* w, const float* bias, v
 #undef MM_LAUNCH
   return MGPT_ERR_BAD_DTYPE;
 }
+// Few rows (NT slices of 16) under a large matrix: a workgroup owns all rows x NC slices of 16 columns, its four waves take the inner
+// size 64 at a time in turn, and their sums meet in LDS in wave order.  Each wave brings its slices of W and of the rows straight
+// into LDS, eight rows of 128 bytes a load, STAGES steps of its own on their way, and waits for nobody: no barrier before the last
+// step.  What bounds it is the matrix's way from memory (16 rows 1600 -> 6400, 20.5 MB: 6.4 us, 3.2 TB/s with the launch; the 32 x 32
+// tiles 7.8, whose barriers hold a step's four waves to the slowest load, on 200 of the 256 compute units); at 32 rows the rows' own, which
+// every workgroup reads again.  More stages than these give nothing.  Rows loaded as operands, without LDS, made the compiler wait for
+// all loads in flight in every round of the loop (1600 -> 6400 9.2 us at 32 rows, 7.4).
+// An element's sum is a chain a step of 64, those of a wave added in order, then the waves': error of 16 rows 6400 -> 1600 against 64
+// bits, relative to the sums' norm, 1.1e-7 (decode kernel 2.4e-7, one chain 5.1e-7), 1600 -> 4800 0.77e-7 (1.2e-7, 2.4e-7).
+template <int NT, int NC, int EPI, typename OT, int STAGES>
+__global__ __launch_bounds__(256) void linear_mfma_rows_kernel(const bf16_t* __restrict__ act, long lda, const bf16_t* __restrict__ w,
+                                                               const float* __restrict__ bias, OT* __restrict__ out, long ldo,
+                                                               int n_rows, int n_out, int k_dim, int k_parts, long part_stride,
+                                                               MfmaScatter sc) {
+  constexpr int SLICE = 16 * MM_BK, SLICES = NC + NT;   // elements of 16 rows of a step; W's slices, then the rows'
+  constexpr int LOADS = 2 * SLICES;                     // of a wave and step
+  static_assert((STAGES - 1) * LOADS < 64, "the counter of loads in flight");
+  static_assert(NT * NC <= 4, "a wave a tile of 16 x 16 behind the last step");
+  typedef __attribute__((address_space(1))) const void* global_ptr_t;
+  typedef __attribute__((address_space(3))) void* lds_ptr_t;
+  extern __shared__ __align__(16) bf16_t lds[];         // [4 waves][STAGES][SLICES][SLICE]
+  __shared__ f32x4_t sums[4][NT * NC][64];
+  const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col0 = blockIdx.x * (16 * NC), part = blockIdx.y;
+  const int all_steps = k_dim / MM_BK, per = (all_steps + k_parts - 1) / k_parts;
+  const int k_begin = part * per * MM_BK, steps = all_steps - part * per < per ? all_steps - part * per : per;
+  const int own = steps > wave ? (steps - wave + 3) / 4 : 0;   // of this wave
+  out += part * part_stride;
+  if (part != 0) bias = nullptr;   // (the first stretch's sums carry it)
+  // this lane's part of a load: row 8 i + lane / 8, chunk (lane % 8) ^ (row % 8)
+  const int lr = lane >> 3, lc = ((lane & 7) ^ lr) * 8;
+  const bf16_t* src[LOADS];
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) {
+    // (columns and rows past the end: the last one's sums, never stored)
+    const int c = col0 + 8 * i + lr, r = 8 * (i - 2 * NC) + lr;
+    src[i] = (i < 2 * NC ? w + (long)(c < n_out ? c : n_out - 1) * k_dim : act + (long)(r < n_rows ? r : n_rows - 1) * lda) +
+             k_begin + wave * MM_BK + lc;
+  }
+  bf16_t* const staged = lds + wave * (STAGES * SLICES * SLICE);
+  auto load = [&](int s, int st) {
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i)
+      __builtin_amdgcn_global_load_lds((global_ptr_t)(src[i] + s * (4 * MM_BK)),
+                                       (lds_ptr_t)(staged + st * (SLICES * SLICE) + i * (SLICE / 2)), 16, 0, 0);
+  };
+  auto arrive = [&](int behind) {   // waits until the loads of at most `behind` steps are on their way
+#define MM_WAIT_CASE(N) \
+  case N: asm volatile("s_waitcnt vmcnt(%0)" ::"n"((N < STAGES ? N : 0) * LOADS) : "memory"); break;
+    switch (behind) {
+      MM_WAIT_CASE(1) MM_WAIT_CASE(2) MM_WAIT_CASE(3)
+      default: asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); break;
+    }
+#undef MM_WAIT_CASE
+  };
+  static_assert(STAGES <= 4, "arrive() knows up to three steps behind the one waited for");
+  // what this wave's tile needs behind the last step: its bias, and where its rows' keys and values go
+  const int n = (wave % NT) * 16 + li, oc = col0 + (wave / NT % NC) * 16 + lg * 4;
+  const bool vec = (n_out & 3) == 0 && (ldo & 3) == 0 && (((size_t)out | (size_t)bias) & 15) == 0;
+  float b4[4];
+  mfma_bias4(bias, oc < n_out ? oc : 0, n_out, vec, b4);
+  int slot = -1;
+  if (EPI == MM_EPI_QKV) slot = sc.slot_mapping[n < n_rows ? n : 0];
+  float a_p = 0.f, a_n = 0.f;
+  if (EPI == MM_EPI_XIELU) a_p = sc.epi_coef[0], a_n = sc.epi_coef[1];
+#pragma unroll
+  for (int s = 0; s < STAGES; ++s)
+    if (s < own) load(s, s);
+  f32x4_t acc[NC][NT];
+#pragma unroll
+  for (int i = 0; i < NC; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  const int at0 = li * MM_BK + ((lg ^ (li & 7)) * 8), at1 = at0 ^ 32;
+  for (int s = 0, st = 0; s < own; ++s) {
+    arrive(own - 1 - s < STAGES - 1 ? own - 1 - s : STAGES - 1);
+    const bf16_t* slice = staged + st * (SLICES * SLICE);
+    bf16x8_t op[SLICES][2];
+#pragma unroll
+    for (int j = 0; j < SLICES; ++j) {
+      op[j][0] = *reinterpret_cast<const bf16x8_t*>(slice + j * SLICE + at0);
+      op[j][1] = *reinterpret_cast<const bf16x8_t*>(slice + j * SLICE + at1);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // read before the stage is loaded again
+    if (s + STAGES < own) load(s + STAGES, st);
+    // a chain a step, added to those before it: chains are short whatever the inner size
+    f32x4_t sum[NC][NT];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < NC; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+          sum[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(op[i][h], op[NC + j][h],
+                                                              h == 0 ? (f32x4_t){0.f, 0.f, 0.f, 0.f} : sum[i][j], 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[i][j][e] += sum[i][j][e];
+    st = st + 1 < STAGES ? st + 1 : 0;
+  }
+#pragma unroll
+  for (int i = 0; i < NC; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) sums[wave][i * NT + j][lane] = acc[i][j];
+  __syncthreads();
+  if (wave >= NT * NC || n >= n_rows || oc >= n_out) return;
+  f32x4_t v;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    v[e] = (sums[0][wave][lane][e] + sums[1][wave][lane][e]) + (sums[2][wave][lane][e] + sums[3][wave][lane][e]);
+  bf16_t* cache_dst = nullptr;
+  if (EPI == MM_EPI_QKV && oc >= sc.q_width && slot >= 0) {
+    const int page = slot / sc.page_size, off = slot - page * sc.page_size;
+    const int c = oc - sc.q_width;   // column among keys then values
+    const bool is_v = c >= sc.kv_width;
+    const int cc = is_v ? c - sc.kv_width : c;
+    const int hh = cc / sc.head_dim, d = cc - hh * sc.head_dim;
+    cache_dst = (is_v ? sc.vpool : sc.kpool) + (((long)page * sc.n_kv_head + hh) * sc.page_size + off) * sc.head_dim + d;
+  }
+  mfma_store4<EPI, OT>(v, b4, out, ldo, n, oc, n_out, vec, cache_dst, a_p, a_n);
+}
+
 template <int WTM, int WTN, int WVM, int WVN, int EPI, typename OT, int AHEAD, int KG = 1, int DIRECT = 0, int CHAINS = 1, int FOLD = 0>
 int launch_one(const void* act, long lda, const void* w, const float* bias, void* out, long ldo, int n_rows,
                int n_out, int k_dim, int k_parts, long part_stride, const MfmaScatter& sc, hipStream_t stream) {
@@ -877,6 +1003,40 @@ int launch_shape(const void* act, long lda, const void* w, const float* bias, vo
   return MGPT_ERR_BAD_DTYPE;
 }
 
+template <int NT, int NC, int EPI, typename OT, int STAGES>
+int launch_rows_one(const void* act, long lda, const void* w, const float* bias, void* out, long ldo, int n_rows, int n_out, int k_dim,
+                    int k_parts, long part_stride, const MfmaScatter& sc, hipStream_t stream) {
+  constexpr size_t lds_bytes = 4ul * STAGES * (NC + NT) * 16 * MM_BK * sizeof(bf16_t), sums_bytes = 4ul * NT * NC * 64 * 16;
+  static_assert(lds_bytes + sums_bytes <= 160 * 1024, "a workgroup's LDS");
+  auto kernel = linear_mfma_rows_kernel<NT, NC, EPI, OT, STAGES>;
+  static bool allowed = false;  // more LDS than a kernel gets without asking
+  if (!allowed) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             (int)lds_bytes);
+    if (e != hipSuccess) return (int)e;
+    allowed = true;
+  }
+  hipLaunchKernelGGL(kernel, dim3((n_out + 16 * NC - 1) / (16 * NC), k_parts), dim3(256), lds_bytes, stream, (const bf16_t*)act, lda,
+                     (const bf16_t*)w, bias, (OT*)out, ldo, n_rows, n_out, k_dim, k_parts, part_stride, sc);
+  return mgpt_last_error();
+}
+
+template <int NT, int NC, int STAGES>
+int launch_rows(const void* act, long lda, const void* w, const float* bias, void* out, int out_dtype, long ldo, int n_rows,
+                int n_out, int k_dim, int epilogue, int k_parts, long part_stride, const MfmaScatter& sc, hipStream_t stream) {
+#define MM_LAUNCH(E, OT)                                                                                                  \
+  return launch_rows_one<NT, NC, E, OT, STAGES>(act, lda, w, bias, out, ldo, n_rows, n_out, k_dim, k_parts, part_stride, sc, stream)
+  if (epilogue == MM_EPI_NONE && out_dtype == MGPT_F32) MM_LAUNCH(MM_EPI_NONE, float);
+  if (epilogue == MM_EPI_RESIDUAL && out_dtype == MGPT_F32) MM_LAUNCH(MM_EPI_RESIDUAL, float);
+  if (epilogue == MM_EPI_NONE && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_NONE, bf16_t);
+  if (epilogue == MM_EPI_GELU && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_GELU, bf16_t);
+  if (epilogue == MM_EPI_RELU2 && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_RELU2, bf16_t);
+  if (epilogue == MM_EPI_XIELU && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_XIELU, bf16_t);
+  if (epilogue == MM_EPI_QKV && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_QKV, bf16_t);
+#undef MM_LAUNCH
+  return MGPT_ERR_BAD_DTYPE;
+}
+
 // The 64 x 64 tile with two wave groups (float32 outputs: plain, or added into the residual stream).
 int launch_two_groups(const void* act, long lda, const void* w, const float* bias, void* out, int out_dtype, long ldo,
                       int n_rows, int n_out, int k_dim, int epilogue, int k_parts, long part_stride,
@@ -911,7 +1071,9 @@ constexpr int MM_DIRECT_HALVES = 5;     // the first of the four variants with t
 // then the same variants with two chains of sums (float32 outputs; those of 128 x 64 and of 128 rows out of step have them)
 constexpr int MM_CHAINS_FIRST = MM_DIRECT_FIRST + MM_DIRECT_VARIANTS;
 constexpr bool MM_HAS_CHAINS[MM_DIRECT_VARIANTS] = {false, false, true, false, false, false, true, false, true};
-constexpr int MM_SHAPE_IDS = MM_CHAINS_FIRST + MM_DIRECT_VARIANTS;
+constexpr int MM_ROWS = MM_CHAINS_FIRST + MM_DIRECT_VARIANTS;   // the kernel for few rows, 16 columns a workgroup, then 32
+constexpr int MM_SHAPE_IDS = MM_ROWS + 2;
+constexpr int MM_ROWS_MAX = 32;
 
 long tiles_of(int shape, int n_rows, int n_out) {
   return (long)((n_rows + MM_TILE_ROWS[shape] - 1) / MM_TILE_ROWS[shape]) *
@@ -943,6 +1105,38 @@ int choose_shape(int n_rows, int n_out) {
   }
   if (tiles_of(3, n_rows, n_out) >= 192) return 3;
   return 4;
+}
+
+// Whether a product of few rows goes to the kernel that has nothing but them and 16 or 32 columns a workgroup, rather than to the decode
+// kernel (from the matrix packed for it) or the 32 x 32 tiles.  us in a graph, matrices from memory, those two / here, where the
+// better one is: 1600 -> 4800 6.5 / 5.3 at 1 row, 7.6 / 5.6 at 8, 7.6 / 5.9 at 16, 7.7 / 7.1 at 32; 1600 -> 6400 9.2 / 6.4 at 16, 8.0 / 7.4
+// at 32; 1600 -> 1600 4.0 / 3.8, 4.8 / 4.1, 5.1 / 4.4, 5.8 / 5.2; 2048 -> 2048 4.8 / 4.5 at 4, 7.7 / 6.0 at 32; 2688 -> 1024 5.9 / 4.6, 9.6 /
+// 6.9; 5440 -> 2048 9.2 / 7.3, 16.5 / 11.8; 768 -> 2304 2.85 / 2.86, 4.5 / 3.3.  Lines: small matrices are a launch and one trip to
+// memory either way (1024 -> 1024 2.6 / 2.8, 768 -> 768 2.6 / 2.7, 512 -> 3072 2.6 / 2.8 at 1 row), and rows of 2,048 bytes and multiples
+// come from few of the memory's channels at a time, which a packed matrix does not (2048 -> 1024 3.6 / 3.7, 4.3 / 4.9; 1024 -> 2048
+// 3.8 / 3.9 at 32).
+bool rows_take(int n_rows, int n_out, int k_dim) {
+  if (n_rows < 1 || n_rows > MM_ROWS_MAX || k_dim % MM_BK != 0 || n_out < 768 || n_out > 8192) return false;
+  if ((long)n_out * k_dim < (k_dim % 1024 == 0 ? 4000000 : 1500000) || (k_dim < 768 && n_rows < 8)) return false;
+  return n_out <= 7168 || n_rows >= 4;   // (2048 -> 8192 at 1 row 8.7 / 8.9)
+}
+
+// Into how many stretches such a product's inner size is cut (choose_split's reasons): every 16 columns read all rows again, and a
+// wave's steps are a chain.  us with the sums added up and into float32 rows, whole / cut: 6400 -> 1600 8.2 / 8.0 at 1 row, 9.3 / 8.6 at 8,
+// 14.2 / 10.6 at 32 (in four, 32 columns a workgroup); 5440 -> 2048 8.6 / 9.0 at 8, 9.7 / 9.2 at 16, 12.3 / 10.5 at 32; 2688 -> 1024 5.9 / 6.3
+// at 16, 7.2 / 6.7 at 32; 8192 -> 2048 12.8 / 13.4 at 16, 15.9 / 12.5 at 32.
+int rows_parts(int n_rows, int n_out, int k_dim) {
+  const int tiles = (n_out + 15) / 16;
+  if (tiles > 160 || k_dim / MM_BK < 32) return 1;
+  const bool many = (long)n_rows * k_dim >= 50000, lengthy = k_dim >= 5120 && tiles <= 100;
+  if (tiles <= 64 || n_rows > 16) return many ? 4 : (tiles > 64 && lengthy ? 2 : 1);
+  return (many || lengthy) && (k_dim % 1024 != 0 || tiles < 128) ? 2 : 1;
+}
+
+// 32 columns a workgroup: where 16 are more workgroups than compute units, and half as many read the rows half as often.
+bool rows_wide(int n_rows, int n_out, int parts) {
+  const int tiles = (n_out + 15) / 16;
+  return parts > 1 ? parts == 4 && n_rows > 16 && tiles >= 80 : tiles > 256;
 }
 
 // Whether the inner size is split into stretches, and then with which tile shape and into how many
@@ -1193,7 +1387,14 @@ int launch_any(int shape, int k_parts, const void* act, long lda, const void* w,
                                               : -1;
     if (chosen >= 0) shape = chosen, k_parts = 1;
   }
-  if (shape >= MM_DIRECT_FIRST) {
+  bool rows = false, rows_32 = false;  // the kernel for few rows, with 32 columns a workgroup
+  if (shape >= MM_ROWS) {
+    if (shape >= MM_SHAPE_IDS || n_rows > MM_ROWS_MAX || sc.row_expert || !direct_ok(act, w, k_dim)) return MGPT_ERR_BAD_SHAPE;
+    rows = true;
+    rows_32 = shape == MM_ROWS + 1;
+    shape = 3;   // (the rules below for the other variants do not apply)
+    ahead = 1;
+  } else if (shape >= MM_DIRECT_FIRST) {
     if (shape >= MM_SHAPE_IDS || !direct_ok(act, w, k_dim)) return MGPT_ERR_BAD_SHAPE;
     chains = shape >= MM_CHAINS_FIRST;
     direct = shape - (chains ? MM_CHAINS_FIRST : MM_DIRECT_FIRST);
@@ -1265,7 +1466,7 @@ int launch_any(int shape, int k_parts, const void* act, long lda, const void* w,
     // a split product are)
     const int dt_here = split ? MGPT_F32 : out_dtype, epi_here = split ? MM_EPI_NONE : epilogue;
     if (dt_here != MGPT_F32 || (epi_here != MM_EPI_NONE && epi_here != MM_EPI_RESIDUAL)) return MGPT_ERR_BAD_SHAPE;
-  } else if (shape == 3 && ahead == 1 && direct < 0) {
+  } else if (shape == 3 && ahead == 1 && direct < 0 && !rows) {
     const int steps_here = ((k_dim + MM_BK - 1) / MM_BK + k_parts - 1) / k_parts;
     const int dt_here = split ? MGPT_F32 : out_dtype, epi_here = split ? MM_EPI_NONE : epilogue;
     two_groups = two_groups_pay(steps_here, tiles_of(3, n_rows, n_out) * k_parts) && dt_here == MGPT_F32 &&
@@ -1288,6 +1489,9 @@ int launch_any(int shape, int k_parts, const void* act, long lda, const void* w,
          : direct == 0 ? launch_one<1, 1, 2, 2, MM_EPI_NONE, float, 1, 1, 4, 1, MM_FOLD>(MM_FOLD_ARGS)
          : ahead > 1   ? launch_one<1, 1, 2, 2, MM_EPI_NONE, float, MM_AHEAD, 1, 0, 1, MM_FOLD>(MM_FOLD_ARGS)
                        : launch_one<1, 1, 2, 2, MM_EPI_NONE, float, 1, 1, 0, 1, MM_FOLD>(MM_FOLD_ARGS);
+  } else if (rows) {
+    if (n_rows <= 16) rc = rows_32 ? launch_rows<1, 2, 3>(MM_ARGS) : launch_rows<1, 1, 4>(MM_ARGS);
+    else rc = rows_32 ? launch_rows<2, 2, 2>(MM_ARGS) : launch_rows<2, 1, 3>(MM_ARGS);
   } else if (direct >= 0 && chains) {
     switch (direct) {
       case 2: rc = launch_shape<2, 2, 4, 2, 1, 3, 2>(MM_ARGS); break;
@@ -1330,6 +1534,14 @@ int launch_any(int shape, int k_parts, const void* act, long lda, const void* w,
 
 }  // namespace
 
+// A product of up to 32 rows in whole steps of 64: 0 where the kernel that has nothing but them and a few columns a workgroup is not the
+// fastest, else its shape for mgpt_linear_mfma_shape + 256 x the stretches of the inner size.
+extern "C" int mgpt_linear_mfma_rows_plan(int n_rows, int n_out, int k_dim, int epilogue) {
+  if (!rows_take(n_rows, n_out, k_dim)) return 0;
+  const int parts = epilogue == MM_EPI_QKV || (n_out & 3) != 0 ? 1 : used_parts(k_dim, rows_parts(n_rows, n_out, k_dim));
+  return MM_ROWS + (rows_wide(n_rows, n_out, parts) ? 1 : 0) + 256 * parts;
+}
+
 // How many floats of scratch the product would use if it were split along its inner size (0: it
 // would not be split).  The caller brings that buffer to mgpt_linear_mfma.
 extern "C" long mgpt_linear_mfma_partials(int n_rows, int n_out, int k_dim, int epilogue) {
@@ -1349,6 +1561,20 @@ extern "C" int mgpt_linear_mfma_parts(const void* act, long lda, const void* w, 
   MfmaScatter sc = {};
   int parts = 0;
   const int rc = launch_any(-1, 0, act, lda, w, bias, partials, MGPT_F32, n_out, n_rows, n_out, k_dim, MM_EPI_RESIDUAL,
+                            partials, partials_floats, sc, stream, &parts);
+  if (rc != MGPT_OK) return rc;
+  return parts > 1 ? MGPT_OK : MGPT_ERR_BAD_SHAPE;
+}
+
+// The same with the shape and the number of stretches given (mgpt_linear_mfma_shape).
+extern "C" int mgpt_linear_mfma_shape_parts(int shape, int k_parts, const void* act, long lda, const void* w, const float* bias,
+                                            float* partials, long partials_floats, int n_rows, int n_out, int k_dim,
+                                            hipStream_t stream) {
+  if (!partials) return MGPT_ERR_NULL;
+  if (shape < 0 || shape >= MM_SHAPE_IDS || k_parts <= 1 || k_parts != used_parts(k_dim, k_parts)) return MGPT_ERR_BAD_SHAPE;
+  MfmaScatter sc = {};
+  int parts = 0;
+  const int rc = launch_any(shape, k_parts, act, lda, w, bias, partials, MGPT_F32, n_out, n_rows, n_out, k_dim, MM_EPI_RESIDUAL,
                             partials, partials_floats, sc, stream, &parts);
   if (rc != MGPT_OK) return rc;
   return parts > 1 ? MGPT_OK : MGPT_ERR_BAD_SHAPE;
@@ -1391,8 +1617,8 @@ extern "C" int mgpt_linear_mfma_xielu(const void* act, long lda, const void* w, 
 // 7 = 64 x 64 with two wave groups a tile (float32 outputs), 8 to 12 = the slices straight into LDS: 32 x 32 and
 // 64 x 64 with four stages, 128 x 64 with three, 128 x 192 with two, 32 x 32 with six (an inner size of whole steps of 64 and operands
 // aligned to 16 bytes, else refused), 13 to 16 = the halves out of step, 256 x 256, 128 x 256, 256 x 192, 128 x 192 (the same
-// conditions, and never split), 19, 23 and 25 = 10, 14 and 16 with two chains of sums (float32 outputs); negative:
-// chosen) and the number of stretches of the inner size given
+// conditions, and never split), 19, 23 and 25 = 10, 14 and 16 with two chains of sums (float32 outputs), 26 and 27 = up to 32 rows
+// with 16 and 32 columns a workgroup (the conditions of 8); negative: chosen) and the number of stretches of the inner size given
 // (k_parts as for launch_any above), instead of chosen by the size: for tests and measurements.
 extern "C" int mgpt_linear_mfma_shape(int shape, int k_parts, const void* act, long lda, const void* w,
                                       const float* bias, void* out, int out_dtype, long ldo, int n_rows,

@@ -740,14 +740,30 @@ def linear_mfma_partials(n_rows: int, n_out: int, k_dim: int, epilogue: int) -> 
     return hit
 
 
+_ROWS_PLANS: dict = {}
+
+
+def linear_rows_plan(n_rows: int, n_out: int, k_dim: int, scatter: bool = False):
+    """(shape, stretches of the inner size) for linear_mfma where a product of few rows is fastest in the kernel made for up to 32 of them
+    (one stretch where it also stores keys and values), or None."""
+    key = (n_rows, n_out, k_dim, scatter)
+    if key not in _ROWS_PLANS:
+        if len(_ROWS_PLANS) > 4096:
+            _ROWS_PLANS.clear()
+        got = library.kernels().mgpt_linear_mfma_rows_plan(n_rows, n_out, k_dim, SK_EPI_QKV if scatter else EPI_NONE)
+        _ROWS_PLANS[key] = (got % 256, got // 256) if got else None
+    return _ROWS_PLANS[key]
+
+
 def linear_mfma_parts(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], partials: torch.Tensor,
-                      n_rows: int) -> bool:
+                      n_rows: int, plan=None) -> bool:
     """The tiled product's first half alone where it splits the inner size: partials[p, :n_rows]
     (float32 [parts, n_rows, out], dense, parts = linear_mfma_partials(n_rows, out, inner, EPI_RESIDUAL)
     // (n_rows * out)) = a[:n_rows] @ w[:, stretch p].T, the first with the bias added; nobody adds
-    them up.  False, having launched nothing, where the product would not be split."""
+    them up.  With a plan (linear_rows_plan's) its shape and stretches instead.  False, having launched nothing, where the product would
+    not be split."""
     n_out, k_dim = w.shape
-    need = linear_mfma_partials(n_rows, n_out, k_dim, EPI_RESIDUAL)
+    need = linear_mfma_partials(n_rows, n_out, k_dim, EPI_RESIDUAL) if plan is None else (plan[1] > 1) * plan[1] * n_rows * n_out
     if (not need or w.dtype != torch.bfloat16 or a.dtype != torch.bfloat16 or a.stride(0) % 8 or a.data_ptr() % 16
             or w.data_ptr() % 16 or k_dim % 16):
         return False
@@ -759,8 +775,11 @@ def linear_mfma_parts(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Ten
     _need(bias is None or (bias.dtype == torch.float32 and bias.numel() == n_out), "bias must be float32 [out]")
     _need(partials.dtype == torch.float32 and partials.is_contiguous() and partials.data_ptr() % 16 == 0
           and tuple(partials.shape) == (parts, n_rows, n_out), f"partials must be dense float32 [{parts}, n_rows, out]")
-    rc = library.kernels().mgpt_linear_mfma_parts(_ptr(a), a.stride(0), _ptr(w), _ptr(bias), _ptr(partials),
-                                                  partials.numel(), n_rows, n_out, k_dim, _stream())
+    args = (_ptr(a), a.stride(0), _ptr(w), _ptr(bias), _ptr(partials), partials.numel(), n_rows, n_out, k_dim, _stream())
+    if plan is None:
+        rc = library.kernels().mgpt_linear_mfma_parts(*args)
+    else:
+        rc = library.kernels().mgpt_linear_mfma_shape_parts(*plan, *args)
     if rc == -2:
         return False
     _check(rc, "linear_mfma_parts")
@@ -786,7 +805,8 @@ def linear_mfma(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], 
     steps on their way from memory, 7 = 64 x 64 with two wave groups that share a tile, float32 outputs, 8 to 12 = operand slices straight
     into LDS with tiles of 32 x 32, 64 x 64, 128 x 64, 128 x 192, 32 x 32 with six stages, 13 to 16 = the same with the
     workgroup's halves out of step and tiles of 256 x 256, 128 x 256, 256 x 192, 128 x 192: an inner size that is a
-    multiple of 64, 19, 23 and 25 = 10, 14 and 16 with float32 sums in two chains, as 7 makes them) and
+    multiple of 64, 19, 23 and 25 = 10, 14 and 16 with float32 sums in two chains, as 7 makes them, 26 and 27 = up to 32 rows with 16 and
+    32 columns a workgroup) and
     `k_parts` fix what the library otherwise chooses by the size.  False when it does not take the shape."""
     if a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
         return False

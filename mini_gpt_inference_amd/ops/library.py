@@ -137,6 +137,8 @@ def _declare_optional(lib: ctypes.CDLL) -> None:
         "mgpt_linear_mfma_shape": [I, I, P, L, P, P, P, I, L, I, I, I, I, P, L, P],
         "mgpt_linear_mfma_partials": [I, I, I, I],
         "mgpt_linear_mfma_choice": [I, I, I, I, I, I],
+        "mgpt_linear_mfma_rows_plan": [I, I, I, I],
+        "mgpt_linear_mfma_shape_parts": [I, I, P, L, P, P, P, L, I, I, I, P],
         "mgpt_linear_exact_kernel": [I, I, I, I],
         "mgpt_linear_exact_norms": [I, I, I],
         "mgpt_linear_exact_normed": [P, P, P, P, F, P, P, P, L, I, I, I, I, P, P, P, I, I, I, I, P],

@@ -215,6 +215,29 @@ def tiled_at_few_rows(n_rows: int, w: torch.Tensor, left: bool = False) -> bool:
     return n_rows >= TILED_ANY_SHAPE_FROM_ROWS or (n_rows >= TILED_FROM_ROWS and n_out >= TILED_MIN_OUT)
 
 
+def folds_before_rows_apart(n_rows: int, n_out: int, k_dim: int) -> bool:
+    """Whether the LayerNorm of a product that has a kernels.linear_rows_plan is folded into the decode kernel instead.  The fold's work
+    grows with the rows in every workgroup; a LayerNorm of its own is a launch of 2 us.  Folded / LayerNorm and product, us: 768 -> 2304
+    3.3 / 4.8 at 1 row, 5.0 / 5.2 at 16, 6.4 / 5.5 at 24; 1024 -> 4096 6.0 / 6.5 at 16, 8.4 / 7.0 at 24; 1280 -> 3840 6.6 / 7.0 at 8, 7.9 / 7.1
+    at 12; with more than a workgroup a compute unit 1280 -> 5120 7.4 / 7.6 at 4, 8.5 / 7.9 at 8, 12.6 / 8.3 at 16; 1600 -> 4800 8.0 / 8.2 at 4,
+    9.5 / 8.5 at 8, 13.1 / 8.9 at 16; 1600 -> 6400 8.3 / 8.8, 9.8 / 9.0, 13.2 / 9.3; short inner sizes never (512 -> 1536 3.9 / 5.5 at 32)."""
+    if n_out > 4096:
+        return n_rows * k_dim <= 8192
+    if k_dim > 1024:
+        return n_rows * k_dim <= 13000
+    return n_rows <= 16 or k_dim < 768
+
+
+def _rows_apart(ctx, plan, a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor, n_rows: int, epilogue: int,
+                scatter) -> bool:
+    """The product as kernels.linear_rows_plan says; False, with nothing launched, where the operands are not aligned for it."""
+    shape, stretches = plan
+    partials = None
+    if stretches > 1:
+        partials = ctx.workspace.get("linear_partials", stretches * n_rows * w.shape[0], 1, torch.float32)
+    return kernels.linear_mfma(a, w, bias, out, n_rows, epilogue, scatter=scatter, shape=shape, partials=partials, k_parts=stretches)
+
+
 def as_tensor(ctx, a: Union[torch.Tensor, LazyNorm]) -> torch.Tensor:
     return a.tensor(ctx) if isinstance(a, LazyNorm) else a
 
@@ -301,7 +324,16 @@ def linear_add(ctx, a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tenso
              and ctx.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and a.dtype == torch.bfloat16
              and 0 < n_rows <= LEAVE_PARTS_MAX_ROWS and n_rows == ctx.n_rows and x.is_contiguous()
              and x.shape[1] == w.shape[0] and w.shape[1] % 16 == 0)
-    if leave and tiled_at_few_rows(n_rows, w, left=True):
+    plan = kernels.linear_rows_plan(n_rows, *w.shape) if leave and n_rows <= 32 else None
+    if plan is not None:
+        # the sums of the kernel for few rows, where it cuts the inner size
+        if 1 < plan[1] <= kernels.residual_parts_limit(w.shape[0]):
+            buf = ctx.workspace.get("residual_parts", plan[1] * n_rows, w.shape[0], torch.float32)
+            parts = buf[:plan[1] * n_rows].view(plan[1], n_rows, w.shape[0])
+            if kernels.linear_mfma_parts(a, w, bias, parts, n_rows, plan):
+                ctx.pending = residual.PendingSums(x, parts, plan[1])
+                return
+    elif leave and tiled_at_few_rows(n_rows, w, left=True):
         # the tiled kernel's split: its stretches' sums are the parts (2 to 8 of them)
         need = kernels.linear_mfma_partials(n_rows, w.shape[0], w.shape[1], kernels.EPI_RESIDUAL)
         n_parts = need // (n_rows * w.shape[0])
@@ -350,7 +382,8 @@ def linear(ctx, a: Union[torch.Tensor, LazyNorm], w: torch.Tensor, bias: Optiona
            tile_best: Optional[TileBest] = None) -> bool:
     """out[:n_rows] = a[:n_rows] @ w.T (+ bias) with the epilogue.
 
-    On the bfloat16 path up to 64 rows (fewer for a very wide output) go to the decode step's MFMA kernels (reading the residual
+    On the bfloat16 path up to 32 rows under all but small matrices and very wide outputs go to the kernel that has nothing but them and a
+    few columns a workgroup; else up to 64 rows (fewer for a very wide output) to the decode step's MFMA kernels (reading the residual
     stream through the folded LayerNorm when `a` is a LazyNorm of a fusable norm and the rows are
     few; splitting a long inner size over workgroups when the rows are many) and more rows to the
     tiled MFMA kernel (which also splits a long inner size when its tiles are few); the 32-bit path, and every shape those refuse, go to the general product
@@ -374,9 +407,11 @@ def linear(ctx, a: Union[torch.Tensor, LazyNorm], w: torch.Tensor, bias: Optiona
                                     tile_best.limit, w_packed=packed_weight(w, ctx)):
             tile_best.filled = True
             return False
+    plan = kernels.linear_rows_plan(n_rows, *w.shape, scatter is not None) if fast and n_rows <= 32 and not wide_out else None
     if fast and n_rows <= 64 and not wide_out and not tiled_at_few_rows(n_rows, w):
         epi = kernels.SK_EPI_QKV if scatter is not None else epilogue
         if (isinstance(a, LazyNorm) and getattr(a.norm, "fusable_layer_norm", False) and a._tensor is None
+                and (plan is None or folds_before_rows_apart(n_rows, *w.shape))
                 and (w.shape[0] <= FOLD_MAX_OUT
                      or (n_rows <= FOLD_ANY_OUT_MAX_ROWS and w.shape[0] <= FOLD_ANY_OUT_MAX_OUT))
                 and (n_rows <= FOLD_MAX_ROWS or kernels.linear_skinny_row_groups(n_rows, w.shape[0], w.shape[1]))):
@@ -387,6 +422,8 @@ def linear(ctx, a: Union[torch.Tensor, LazyNorm], w: torch.Tensor, bias: Optiona
                                          ln_eps=a.norm.eps, ln_rows=a.rows, scatter=scatter,
                                          w_packed=packed_weight(wf, ctx)):
                     return scatter is not None
+        if plan is not None and _rows_apart(ctx, plan, as_tensor(ctx, a), w, bias, out, n_rows, epilogue, scatter):
+            return scatter is not None
         partials = None
         need = kernels.linear_skinny_partials(n_rows, w.shape[0], w.shape[1], False, epi)
         if need:
@@ -403,6 +440,8 @@ def linear(ctx, a: Union[torch.Tensor, LazyNorm], w: torch.Tensor, bias: Optiona
     if (fast and wide_out and bias is None and scatter is None and epilogue == kernels.EPI_NONE and wide_rows_once(n_rows, w.shape[1])
             and kernels.linear_rows_once(a, w, out, n_rows)):
         return False
+    if plan is not None and _rows_apart(ctx, plan, a, w, bias, out, n_rows, epilogue, scatter):
+        return scatter is not None
     if fast and scatter is not None and kernels.linear_mfma(a, w, bias, out, n_rows, epilogue, scatter=scatter):
         return True
     if fast:

@@ -1060,6 +1060,96 @@ def test_linear_mfma_stores_keys_and_values(n, shape, k):
     assert torch.isnan(kflat[untouched]).all() and torch.isnan(vflat[untouched]).all()
 
 
+@pytest.mark.parametrize("n,k,o,parts", [(1, 64, 16, 1), (15, 192, 257, 1), (16, 320, 40, 1), (17, 256, 48, 1), (31, 576, 33, 1),
+                                         (32, 1600, 130, 1), (32, 1344, 66, 1), (3, 2048, 100, 2), (16, 2112, 100, 4), (32, 5440, 36, 4),
+                                         (20, 832, 64, 3)])
+@pytest.mark.parametrize("epi,o_dt", [(kernels.EPI_NONE, "bfloat16"), (kernels.EPI_NONE, "float32"), (kernels.EPI_GELU, "bfloat16"),
+                                      (kernels.EPI_RELU2, "bfloat16"), (kernels.EPI_RESIDUAL, "float32")])
+@pytest.mark.parametrize("shape", [26, 27])
+def test_linear_mfma_of_a_few_rows(n, k, o, parts, epi, o_dt, shape):
+    """The kernel whose waves take steps of their own, with 16 and 32 columns a workgroup: steps for one wave alone and for some of
+    them only, more and fewer than the stages; ragged rows and columns; stretches of the inner size, the last one shorter."""
+    g = torch.Generator().manual_seed(n + k)
+    a, w, bias = rnd(g, n, k, dtype="bfloat16"), rnd(g, o, k, dtype="bfloat16", scale=k ** -0.5), rnd(g, o)
+    prev = rnd(g, n + 2, o, dtype=o_dt)
+    out = prev.clone().to(DEV)
+    scratch = torch.full((parts * n * o,), float("nan"), device=DEV)
+    assert kernels.linear_mfma(a.to(DEV), w.to(DEV), bias.to(DEV), out, n, epi, shape=shape, k_parts=parts, partials=scratch)
+    helpers.assert_close(out[:n], _linear_want(a, w, bias, epi, prev[:n]), "bfloat16", f"shape {shape} {n}x{k}x{o}")
+    assert torch.equal(out[n:], prev[n:].to(DEV)), "rows beyond n_rows were written"
+    many = torch.zeros(33, k, dtype=torch.bfloat16, device=DEV)
+    assert not kernels.linear_mfma(many, w.to(DEV), None, torch.zeros(33, o, dtype=TDT[o_dt], device=DEV), 33, epi, shape=shape)
+    short = torch.zeros(o, 48, dtype=torch.bfloat16, device=DEV)
+    assert not kernels.linear_mfma(many[:, :48].contiguous(), short, None, out, n, epi, shape=shape)
+
+
+@pytest.mark.parametrize("n,shape", [(2, 26), (16, 27), (17, 26), (32, 27)])
+def test_linear_mfma_of_a_few_rows_stores_keys_and_values(n, shape):
+    test_linear_mfma_stores_keys_and_values(n, shape, 320)
+
+
+@pytest.mark.parametrize("n,k,o,rows,split", [
+    (1, 1600, 4800, True, 1), (32, 1600, 4800, True, 1), (33, 1600, 4800, False, None), (4, 768, 2304, True, 1), (8, 704, 2304, True, 1),
+    (7, 704, 2304, False, None), (8, 768, 1920, False, None), (8, 1024, 3072, False, None), (8, 1024, 4096, True, 1),
+    (3, 1600, 7184, False, None), (4, 1600, 7184, True, 1), (8, 1600, 8208, False, None), (8, 4096, 752, False, None),
+    (1, 6400, 1600, True, 2), (32, 6400, 1600, True, 4), (8, 5440, 2048, True, 1), (16, 5440, 2048, True, 2), (32, 5440, 2048, True, 4),
+    (16, 8192, 2048, True, 1), (32, 8192, 2048, True, 4), (18, 2688, 1024, True, 1), (19, 2688, 1024, True, 4), (16, 1616, 1616, False, None)])
+def test_which_products_of_a_few_rows_have_a_kernel_of_their_own(n, k, o, rows, split):
+    """On both sides of the lines; where it is taken, its float32 sums are no further from 64 bits than the decode kernel's and the 32 x 32
+    tiles', also where operands that are not aligned leave it to others."""
+    from types import SimpleNamespace
+
+    from mini_gpt_inference_amd.ops import linear as L
+    from mini_gpt_inference_amd.parts.base import Workspace
+
+    g = torch.Generator().manual_seed(k + n)
+    a, w = rnd(g, n, k, dtype="bfloat16").to(DEV), rnd(g, o, k, dtype="bfloat16", scale=k ** -0.5).to(DEV)
+    plan = kernels.linear_rows_plan(n, o, k)
+    assert (plan is not None) == rows
+    if not rows:
+        return
+    assert plan[1] == split and kernels.linear_rows_plan(n, o, k, True)[1] == 1
+    want = a.double() @ w.double().T
+    error = lambda t: ((t.double() - want).norm() / want.norm()).item()
+    ctx = SimpleNamespace(exact=False, dtype=torch.bfloat16, n_rows=n, pending=None, copy_budget=None, workspace=Workspace(torch.device(DEV)))
+    got, decode, tiles, odd = (torch.zeros(n, o, device=DEV) for _ in range(4))
+    L.linear_add(ctx, a, w, None, got, n, may_leave_parts=True)
+    assert (ctx.pending is not None) == (split > 1)
+    if split > 1:
+        assert kernels.residual_settle(ctx.pending, got, n)
+        ctx.pending, added = None, torch.zeros_like(got)
+        L.linear_add(ctx, a, w, None, added, n)
+        helpers.assert_close(added, got.double().cpu(), "float32", "added up at once")
+    assert kernels.linear_skinny(a, w, None, decode, n, kernels.EPI_RESIDUAL)
+    assert kernels.linear_mfma(a, w, None, tiles, n, kernels.EPI_RESIDUAL, shape=4)
+    assert error(got) <= 1.01 * min(error(decode), error(tiles)), (error(got), error(decode), error(tiles))
+    unaligned = torch.zeros(n * k + 1, dtype=torch.bfloat16, device=DEV)[1:].view(n, k)
+    unaligned.copy_(a)
+    L.linear_add(ctx, unaligned, w, None, odd, n)
+    helpers.assert_close(odd, want, "bfloat16", "operands that are not aligned")
+
+
+@pytest.mark.parametrize("n,k,o", [(16, 768, 2304), (17, 768, 2304), (5, 1600, 4800), (6, 1600, 4800), (10, 1280, 3840), (11, 1280, 3840)])
+def test_layer_norm_in_front_of_a_product_of_a_few_rows(n, k, o):
+    """On both sides of the lines between the LayerNorm folded into the decode kernel and one of its own."""
+    from types import SimpleNamespace
+
+    from mini_gpt_inference_amd.ops import linear as L
+    from mini_gpt_inference_amd.parts.base import Workspace
+
+    g = torch.Generator().manual_seed(n + k)
+    x, w, bias = rnd(g, n, k, scale=2.0).to(DEV), rnd(g, o, k, dtype="bfloat16", scale=k ** -0.5).to(DEV), rnd(g, o).to(DEV)
+    gain, shift = 1.0 + rnd(g, k, scale=0.1).to(DEV), rnd(g, k, scale=0.1).to(DEV)
+    assert kernels.linear_rows_plan(n, o, k) and L.folds_before_rows_apart(n, o, k) == (n in (16, 5, 10))
+    want = _linear_want(P.plain_layer_norm(x.double().cpu(), gain.double().cpu(), shift.double().cpu(), 1e-5), w.cpu(), bias.cpu(), kernels.EPI_GELU, None)
+    ctx = SimpleNamespace(exact=False, dtype=torch.bfloat16, n_rows=n, pending=None, copy_budget=None, workspace=Workspace(torch.device(DEV)))
+    out = torch.empty(n, o, dtype=torch.bfloat16, device=DEV)
+    norm = SimpleNamespace(weight=gain, bias=shift, eps=1e-5, fusable_layer_norm=True,
+                           forward=lambda ctx, x, h, n, rows=None: kernels.layer_norm(x, gain, shift, h, n, 1e-5, rows))
+    L.linear(ctx, L.LazyNorm(norm, x, n), w, bias, out, n, kernels.EPI_GELU)
+    helpers.assert_close(out, want, "bfloat16", "LayerNorm and product")
+
+
 def test_linear_skinny_refuses_what_it_cannot_do():
     w = torch.zeros(32, 64, dtype=torch.bfloat16, device=DEV)
     a = torch.zeros(65, 64, dtype=torch.bfloat16, device=DEV)

@@ -839,8 +839,8 @@ int launch_halves(const void* act, long lda, const void* w, const float* bias, v
 // into LDS, eight rows of 128 bytes a load, STAGES steps of its own on their way, and waits for nobody: no barrier before the last
 // step.  What bounds it is the matrix's way from memory (16 rows 1600 -> 6400, 20.5 MB: 6.4 us, 3.2 TB/s with the launch; the 32 x 32
 // tiles 7.8, whose barriers hold a step's four waves to the slowest load, on 200 of the 256 compute units); at 32 rows the rows' own, which
-// every workgroup reads again.  More stages than these give nothing.  Rows loaded as operands, without LDS, made the compiler wait for
-// all loads in flight in every round of the loop (1600 -> 6400 9.2 us at 32 rows, 7.4).
+// every workgroup reads again.  More stages than these give nothing.  The rows go through LDS because with operands loaded into
+// registers the compiler waits for all loads in flight where the loop closes.
 // An element's sum is a chain a step of 64, those of a wave added in order, then the waves': error of 16 rows 6400 -> 1600 against 64
 // bits, relative to the sums' norm, 1.1e-7 (decode kernel 2.4e-7, one chain 5.1e-7), 1600 -> 4800 0.77e-7 (1.2e-7, 2.4e-7).
 template <int NT, int NC, int EPI, typename OT, int STAGES>

@@ -126,15 +126,14 @@ __device__ __forceinline__ float gelu_tanh(float u) {
   return 0.5f * u * (1.0f + tanhf(inner));
 }
 
-// The same as u / (1 + exp(-2 z)), z the tanh's argument, on the hardware's exp2 and reciprocal (a few ulp of float32): for the
-// kernels whose results are rounded to bfloat16 anyway.  Seven instructions, where 0.5 u (1 + tanh(z)) with the tanh made of the same
-// two takes eleven and loses, by 1 + t, what is left of a negative u.  Error against 64 bits as a share of the results' norm, that
-// form / here: u in [-12, -4) 7.7e-3 / 5.8e-7, [-4, -1) 1.6e-6 / 1.0e-7, [-1, 0) 1.3e-7 / 0.6e-7, [0, 1) 4.0e-8 / 4.6e-8, [1, 4) 3.2e-8 /
-// 4.4e-8; evenly over [-4, 4) 7e-8 / 4e-8.  26 million outputs of a product of 4,096 rows are 3 us less.
+// The same with tanh(z) = 1 - 2 / (exp(2z) + 1) on the hardware's exp2 and reciprocal (a few ulp
+// of float32): for the kernels whose results are rounded to bfloat16 anyway.
 __device__ __forceinline__ float gelu_tanh_fast(float u) {
-  const float k = 2.0f * 0.7978845608028654f * 1.4426950408889634f;  // 2 sqrt(2/pi) log2(e)
-  const float z = u * fmaf(k * 0.044715f, u * u, k);
-  return u * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-z));  // exp2: inf and 0 at the ends are right
+  const float k = 0.7978845608028654f;  // sqrt(2/pi)
+  const float inner = k * (u + 0.044715f * u * u * u);
+  const float e = __builtin_amdgcn_exp2f(inner * 2.8853900817779268f);  // exp(2 inner); inf and 0 at the ends are right
+  const float t = 1.0f - 2.0f * __builtin_amdgcn_rcpf(e + 1.0f);
+  return 0.5f * u * (1.0f + t);
 }
 
 // tanh(z) = 1 - 2 / (exp(2z) + 1) on the hardware's exp2 and reciprocal (a few ulp of float32; the ends are right)

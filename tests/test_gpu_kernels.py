@@ -95,6 +95,29 @@ def _linear_want(a, w, bias, epi, prev):
     return y
 
 
+@pytest.mark.parametrize("low,high,error", [(2.0 ** -7, 1.0, 2.0e-7), (1.0, 4.0, 1.0e-7)])
+def test_gelu_of_the_bfloat16_products_beside_the_midpoints_of_bfloat16(low, high, error):
+    """Inputs whose exact GELU lies within a few 1e-7 of the middle between two bfloat16 values: every one that lies further from it
+    than the activation's error in 32 bits is rounded to its own side.  The farthest that is not lies 1.80e-7 and 0.92e-7 of its value
+    away (4 and 2 % of them are on the wrong side); as u / (1 + exp(-2 z)) it was 1.12e-7 in [1, 4)."""
+    values = (torch.arange(0x3000, 0x4100, dtype=torch.int32) << 16).view(torch.float32).double()
+    middle = (values[:-1] + values[1:]) / 2
+    below, above = torch.zeros_like(middle), torch.full_like(middle, 16.0)
+    for _ in range(80):
+        at = (below + above) / 2
+        under = P.plain_gelu_tanh(at) < middle
+        below, above = torch.where(under, at, below), torch.where(under, above, at)
+    there = (below >= low) & (below < high)
+    u = (below[there].float().view(torch.int32)[:, None] + torch.arange(-8, 9, dtype=torch.int32)).view(torch.float32).flatten()
+    middle = middle[there].repeat_interleave(17)
+    exact = P.plain_gelu_tanh(u.double())
+    out = torch.empty(1, u.numel(), dtype=torch.bfloat16, device=DEV)
+    a, w = torch.zeros(1, 64, dtype=torch.bfloat16, device=DEV), torch.zeros(u.numel(), 64, dtype=torch.bfloat16, device=DEV)
+    assert kernels.linear_mfma(a, w, u.to(DEV), out, 1, kernels.EPI_GELU)
+    wrong = (out[0].double().cpu() > middle) != (exact > middle)
+    assert ((exact - middle).abs() / middle)[wrong].max() <= error
+
+
 @pytest.mark.parametrize("epi", [kernels.EPI_NONE, kernels.EPI_GELU, kernels.EPI_RESIDUAL])
 @pytest.mark.parametrize("a_dt,w_dt,o_dt", [("float32", "float32", "float32"), ("bfloat16", "bfloat16", "bfloat16"),
                                             ("bfloat16", "bfloat16", "float32"), ("bfloat16", "float32", "bfloat16")])

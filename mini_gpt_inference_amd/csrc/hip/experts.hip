@@ -833,7 +833,8 @@ __global__ __launch_bounds__(256) void grouped_few_rows_kernel(
     for (int h = 0; h < 2; ++h) af[st][h] = *reinterpret_cast<const ex_bf16x8_t*>(ap + (long)step * EX_STEP + h * 32);
   };
 #pragma unroll
-  for (int s = 0; s < STAGES; ++s) load_a(wave + 4 * s < steps ? wave + 4 * s : 0, s);
+  for (int s = 0; s < STAGES; ++s)
+    if (wave + 4 * s < steps) load_a(wave + 4 * s, s);     // (no step that is not there: rows may be shorter than one)
   const ex_bf16x8_t zero = {0, 0, 0, 0, 0, 0, 0, 0};
   ex_f32x4_t acc[NJ];
 #pragma unroll

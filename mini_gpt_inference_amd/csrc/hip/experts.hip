@@ -777,7 +777,8 @@ extern "C" int mgpt_grouped_linear_mfma(const void* a, long lda, const int* a_ro
 // hidden size.  tile_expert null: one matrix for all rows, of which the first n_rows are used (slot_token null).
 //
 // A wave brings its slices of the matrix straight into LDS, eight rows of 128 bytes a load, STAGES steps of its own: no barrier, no
-// registers for what is on its way.  A lane's operand, 16 bytes of one of 16 rows, loaded as it is used makes every
+// registers for what is on its way.  (With two, loads stay on their way in one step of two: the rows' operands are loaded into
+// registers, and where the loop closes the compiler waits for all that is in flight.)  A lane's operand, 16 bytes of one of 16 rows, loaded as it is used makes every
 // load touch 16 lines in 16-byte pieces, and the unit that looks the lines up is what bounds it then (the rows are few: theirs are loaded
 // so; through LDS as well they took room that workgroups need).  The 16-byte pieces
 // of a row are XORed with its number, at the source, so that an operand's read from LDS meets no bank twice.  The matrix's first loads
@@ -789,7 +790,7 @@ extern "C" int mgpt_grouped_linear_mfma(const void* a, long lda, const int* a_ro
 
 template <typename OT, bool GATED, int STAGES>
 __global__ __launch_bounds__(256) void grouped_few_rows_kernel(
-    const bf16_t* __restrict__ A, long lda, const int* __restrict__ a_rows, const bf16_t* __restrict__ W, long w_stride,
+    const bf16_t* A, long lda, const int* __restrict__ a_rows, const bf16_t* __restrict__ W, long w_stride,
     const int* __restrict__ tile_expert, const int* __restrict__ slot_token, OT* __restrict__ out, long ldo,
     const int* __restrict__ out_rows, int n_rows, int n_out, int k_dim, int epilogue, int kind, float limit, float sharpness) {
   constexpr int NJ = GATED ? 2 : 1, SLICE = 16 * EX_STEP;       // elements of 16 rows of a step
@@ -846,7 +847,9 @@ __global__ __launch_bounds__(256) void grouped_few_rows_kernel(
       const int step = step0 + 4 * st;
       if (step >= steps) break;
       // A step's loads come together, but for the first steps, whose rows came behind all of their matrices.  The steps behind this one
-      // that are on their way: STAGES - 1, fewer towards the end.
+      // that are on their way: STAGES - 1, fewer towards the end.  The count holds because each of these steps has all its loads,
+      // the rows' too, between the asm statement that ends the reading of its stage and the next wait: they may change places there but not
+      // leave, which is why A is not __restrict__ (what nobody else may write could be loaded behind a statement that says it writes).
       if (step0 == wave || step + 4 * (STAGES - 1) >= steps) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       else asm volatile("s_waitcnt vmcnt(%0)" ::"n"((STAGES - 1) * (2 * NJ + 2)) : "memory");
       ex_bf16x8_t wf[NJ][2];

@@ -467,7 +467,8 @@ def test_which_float32_products_norm_their_rows(n, o, k, norms):
         assert not kernels.linear_exact_normed(x, gain, None, 1e-5, w, None, torch.zeros(n, o, device=DEV), n)
 
 
-@pytest.mark.parametrize("n,k,o", [(1, 64, 16), (8, 768, 8192), (9, 1030 // 8 * 8, 8200), (12, 2048, 8193), (16, 40, 33), (3, 4096, 100), (16, 320, 48)])
+@pytest.mark.parametrize("n,k,o", [(1, 64, 16), (8, 768, 8192), (9, 1030 // 8 * 8, 8200), (12, 2048, 8193), (16, 40, 33), (3, 4096, 100), (16, 320, 48),
+                                   (16, 8, 40), (16, 56, 20), (5, 2120, 50), (16, 2744, 33)])
 @pytest.mark.parametrize("o_dt", ["float32", "bfloat16"])
 def test_linear_rows_once(n, k, o, o_dt):
     """A pass over the matrix for up to 16 rows: one stage and two, inner sizes that are no whole steps, ragged columns; and that

@@ -1675,7 +1675,7 @@ def gated_few_rows(a: torch.Tensor, w: torch.Tensor, act: torch.Tensor, n_rows: 
 
 def linear_rows_once(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, n_rows: int) -> bool:
     """out[:n_rows] = a[:n_rows] @ w.T in one pass over a bfloat16 matrix that is read as it was loaded (up to GATED_FEW_ROWS rows; out
-    float32 or bfloat16).  False, with nothing launched, for other types and unaligned rows."""
+    float32 or bfloat16, perhaps wider).  False, with nothing launched, for other types and unaligned rows."""
     if a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or n_rows > GATED_FEW_ROWS:
         return False
     _need_cuda(a, w, out)
@@ -1683,8 +1683,8 @@ def linear_rows_once(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, n_rows
     _need(w.is_contiguous(), "weight must be dense [out, in]")
     _need(a.dim() == 2 and a.stride(1) == 1 and a.shape[1] == k_dim and a.shape[0] >= n_rows,
           f"activation must be [>=n_rows, {k_dim}] with unit inner stride")
-    _need(out.dim() == 2 and out.stride(1) == 1 and out.shape[1] == n_out and out.shape[0] >= n_rows,
-          f"output must be [>=n_rows, {n_out}] with unit inner stride")
+    _need(out.dim() == 2 and out.stride(1) == 1 and out.shape[1] >= n_out and out.shape[0] >= n_rows,
+          f"output must be [>=n_rows, >={n_out}] with unit inner stride")
     rc = library.kernels().mgpt_grouped_few_rows(_ptr(a), a.stride(0), None, _ptr(w), 0, None, None, _ptr(out), _dtype_code(out),
                                                  out.stride(0), None, 1, n_rows, n_out, k_dim, EPI_NONE, -1, 0.0, 0.0, _stream())
     if rc == -2:

@@ -483,6 +483,24 @@ def test_linear_rows_once(n, k, o, o_dt):
     assert L.wide_rows_once(8, 1024) and L.wide_rows_once(12, 2048) and not L.wide_rows_once(9, 1024) and not L.wide_rows_once(1, 1600)
 
 
+@pytest.mark.parametrize("n,k,o", [(6, 2048, 16384), (3, 4096, 8192), (13, 2048, 16384), (4, 512, 8192)])
+@pytest.mark.parametrize("o_dt", ["float32", "bfloat16"])
+def test_very_wide_output_into_a_wider_buffer(n, k, o, o_dt):
+    """Few rows in one pass over the matrix, and the kernels around that: what lies beside the output's columns is left alone."""
+    from types import SimpleNamespace
+
+    from mini_gpt_inference_amd.ops import linear as L
+    from mini_gpt_inference_amd.parts.base import Workspace
+
+    g = torch.Generator().manual_seed(n)
+    a, w = rnd(g, n, k, dtype="bfloat16").to(DEV), rnd(g, o, k, dtype="bfloat16", scale=k ** -0.5).to(DEV)
+    ctx = SimpleNamespace(exact=False, dtype=torch.bfloat16, n_rows=n, pending=None, copy_budget=None, workspace=Workspace(torch.device(DEV)))
+    out = torch.full((n + 1, o + 24), 7.0, dtype=TDT[o_dt], device=DEV)
+    L.linear(ctx, a, w, None, out, n)
+    helpers.assert_close(out[:n, :o], (a.double() @ w.double().T).cpu(), o_dt if o_dt == "bfloat16" else "float32", f"{n} {k} {o}")
+    assert (out[n] == 7.0).all() and (out[:, o:] == 7.0).all()
+
+
 @pytest.mark.parametrize("n,k,o", [(1, 1, 4), (1, 1537, 512), (3, 256, 60), (4, 3072, 768), (16, 257, 64), (17, 1026, 68),
                                    (17, 3072, 768), (33, 5000, 260), (70, 2048, 2048), (128, 768, 1028), (130, 4097, 1600)])
 def test_float32_product_left_as_sums_over_its_blocks(n, k, o):

@@ -545,6 +545,10 @@ __global__ __launch_bounds__(256, V == 1 ? 1 : MODE == DC_ADDED ? 4 : 3) void de
 #pragma unroll
         for (int i = 0; i < TILES; ++i)
           S[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(Ks[k0 + 4 * g + e][(part + PARTS * i) * 16 + r16], b[k0 / 16][e], S[i], 0, 0, 0);
+    // (a zero key times an infinite value is a NaN, also where there is no channel; Q S adds these up as well)
+#pragma unroll
+    for (int i = 0; i < TILES; ++i)
+      if (part + PARTS * i >= d_tiles) S[i] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
   }
   if (MODE == DC_OUTPUTS && seg != n_seg - 1) return;
 #pragma unroll

@@ -354,6 +354,29 @@ def test_single_tokens_have_the_bits_of_the_walk_over_several(dtype, H, D, E):
         assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
 
 
+@pytest.mark.parametrize("D", [16, 48, 64, 80, 96, 112, 128])
+@pytest.mark.parametrize("cut", [False, True])
+def test_infinite_value_in_a_decaying_state(D, cut):
+    """An infinite value with queries and keys above zero: behind the chunk that holds it the value's channel is infinite, as token
+    by token, and all other channels are what they are without it; head sizes with and without room for more channels."""
+    g = torch.Generator().manual_seed(D)
+    H, E, n = 2, 40, 600
+    z, k_off, v_off, _ = _state_case(g, "float32", [n], H, D, E)
+    z[:, :v_off] = z[:, :v_off].abs() + 0.1
+    z[5, v_off + 3] = float("inf")
+    decay, slots, cu = torch.tensor([0.999, 0.9]).to(DEV), torch.tensor([0], dtype=torch.int32, device=DEV), torch.tensor([0, n], dtype=torch.int32, device=DEV)
+    pos = torch.arange(n, dtype=torch.int32, device=DEV)
+    walked, chunked, state = torch.zeros(n, H * E, device=DEV), torch.zeros(n, H * E, device=DEV), torch.zeros(1, H * D * E, device=DEV)
+    kernels.decay_state(z.to(DEV), 0, k_off, v_off, -1, H, D, E, decay, torch.zeros(1, H * D * E, device=DEV), slots, cu, 1, pos, walked)
+    added = torch.zeros(kernels.decay_state_scratch(n, 1, H, D, E), device=DEV) if cut else None
+    assert kernels.decay_state_chunked(z.to(DEV), 0, k_off, v_off, H, D, E, decay, state, slots, cu, 1, n, pos,
+                                       torch.zeros(n, 2 * H * D, device=DEV), chunked, added=added)
+    assert (walked[32:, 3] == float("inf")).all() and (chunked[32:, 3] == float("inf")).all()
+    assert (state.view(H, D, E)[0, :, 3] == float("inf")).all()
+    others = [c for c in range(H * E) if c != 3]
+    helpers.assert_close(chunked[:, others] / walked[:, others].abs().max(), walked[:, others] / walked[:, others].abs().max(), "float32", "other channels")
+
+
 @pytest.mark.parametrize("H,D,E", [(2, 128, 128), (3, 40, 24), (1, 16, 130)])
 @pytest.mark.parametrize("lens", [[1, 255, 256, 257], [511, 512, 513, 0, 700], [1300], [300] * 70, [4] * 66 + [600]])
 def test_decaying_state_in_segments(lens, H, D, E):

@@ -898,8 +898,6 @@ __global__ __launch_bounds__(256) void linear_mfma_rows_kernel(const bf16_t* __r
   mfma_bias4(bias, oc < n_out ? oc : 0, n_out, vec, b4);
   int slot = -1;
   if (EPI == MM_EPI_QKV) slot = sc.slot_mapping[n < n_rows ? n : 0];
-  float a_p = 0.f, a_n = 0.f;
-  if (EPI == MM_EPI_XIELU) a_p = sc.epi_coef[0], a_n = sc.epi_coef[1];
 #pragma unroll
   for (int s = 0; s < STAGES; ++s)
     if (s < own) load(s, s);
@@ -957,7 +955,7 @@ __global__ __launch_bounds__(256) void linear_mfma_rows_kernel(const bf16_t* __r
     const int hh = cc / sc.head_dim, d = cc - hh * sc.head_dim;
     cache_dst = (is_v ? sc.vpool : sc.kpool) + (((long)page * sc.n_kv_head + hh) * sc.page_size + off) * sc.head_dim + d;
   }
-  mfma_store4<EPI, OT>(v, b4, out, ldo, n, oc, n_out, vec, cache_dst, a_p, a_n);
+  mfma_store4<EPI, OT>(v, b4, out, ldo, n, oc, n_out, vec, cache_dst);
 }
 
 template <int WTM, int WTN, int WVM, int WVN, int EPI, typename OT, int AHEAD, int KG = 1, int DIRECT = 0, int CHAINS = 1, int FOLD = 0>
@@ -1031,7 +1029,6 @@ int launch_rows(const void* act, long lda, const void* w, const float* bias, voi
   if (epilogue == MM_EPI_NONE && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_NONE, bf16_t);
   if (epilogue == MM_EPI_GELU && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_GELU, bf16_t);
   if (epilogue == MM_EPI_RELU2 && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_RELU2, bf16_t);
-  if (epilogue == MM_EPI_XIELU && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_XIELU, bf16_t);
   if (epilogue == MM_EPI_QKV && out_dtype == MGPT_BF16) MM_LAUNCH(MM_EPI_QKV, bf16_t);
 #undef MM_LAUNCH
   return MGPT_ERR_BAD_DTYPE;
@@ -1374,7 +1371,7 @@ int launch_any(int shape, int k_parts, const void* act, long lda, const void* w,
                int out_dtype, long ldo, int n_rows, int n_out, int k_dim, int epilogue, float* partials,
                long partials_floats, const MfmaScatter& sc, hipStream_t stream, int* leave_parts = nullptr) {
   if (n_rows == 0 || n_out == 0) return MGPT_OK;
-  if (!act || !w || !out) return MGPT_ERR_NULL;
+  if (!act || !w || !out || (epilogue == MM_EPI_XIELU && !sc.epi_coef)) return MGPT_ERR_NULL;
   if (!shapes_ok(act, lda, w, out, ldo, n_rows, n_out, k_dim)) return MGPT_ERR_BAD_SHAPE;
   // shapes MM_SHAPES and MM_SHAPES + 1: the two smallest tiles with more steps on their way from memory
   int ahead = 0;  // 0: chosen below
@@ -1618,7 +1615,7 @@ extern "C" int mgpt_linear_mfma_xielu(const void* act, long lda, const void* w, 
 // 64 x 64 with four stages, 128 x 64 with three, 128 x 192 with two, 32 x 32 with six (an inner size of whole steps of 64 and operands
 // aligned to 16 bytes, else refused), 13 to 16 = the halves out of step, 256 x 256, 128 x 256, 256 x 192, 128 x 192 (the same
 // conditions, and never split), 19, 23 and 25 = 10, 14 and 16 with two chains of sums (float32 outputs), 26 and 27 = up to 32 rows
-// with 16 and 32 columns a workgroup (the conditions of 8); negative: chosen) and the number of stretches of the inner size given
+// with 16 and 32 columns a workgroup (the conditions of 8, not with xIELU); negative: chosen) and the number of stretches of the inner size given
 // (k_parts as for launch_any above), instead of chosen by the size: for tests and measurements.
 extern "C" int mgpt_linear_mfma_shape(int shape, int k_parts, const void* act, long lda, const void* w,
                                       const float* bias, void* out, int out_dtype, long ldo, int n_rows,

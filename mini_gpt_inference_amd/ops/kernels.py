@@ -747,12 +747,13 @@ def linear_rows_plan(n_rows: int, n_out: int, k_dim: int, scatter: bool = False)
     """(shape, stretches of the inner size) for linear_mfma where a product of few rows is fastest in the kernel made for up to 32 of them
     (one stretch where it also stores keys and values), or None."""
     key = (n_rows, n_out, k_dim, scatter)
-    if key not in _ROWS_PLANS:
+    hit = _ROWS_PLANS.get(key)          # False: no plan
+    if hit is None:
         if len(_ROWS_PLANS) > 4096:
-            _ROWS_PLANS.clear()
+            _ROWS_PLANS.clear()         # (another thread may be between its own two lines here)
         got = library.kernels().mgpt_linear_mfma_rows_plan(n_rows, n_out, k_dim, SK_EPI_QKV if scatter else EPI_NONE)
-        _ROWS_PLANS[key] = (got % 256, got // 256) if got else None
-    return _ROWS_PLANS[key]
+        hit = _ROWS_PLANS[key] = (got % 256, got // 256) if got else False
+    return hit or None
 
 
 def linear_mfma_parts(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], partials: torch.Tensor,

@@ -4,7 +4,7 @@ import ctypes
 
 import pytest
 
-from mini_gpt_inference_amd.ops import library
+from mini_gpt_inference_amd.ops import kernels, library
 
 NULL_POINTER = -4
 XIELU = 4
@@ -19,3 +19,17 @@ def test_xielu_without_its_coefficients_is_refused(shape, n):
     entry = library.kernels().mgpt_linear_mfma_shape
     assert entry(shape, 0, at, k, at, None, at, 1, o, n, o, k, XIELU, None, 0, None) == NULL_POINTER
     assert library.kernels().mgpt_linear_mfma(at, k, at, None, at, 1, o, n, o, k, XIELU, None, 0, None) == NULL_POINTER
+
+
+def test_plans_that_another_thread_clears(monkeypatch):
+    """The table of plans is bounded: a thread that fills it empties it first, perhaps while another is about to answer from it."""
+    class Emptied(dict):
+        def __setitem__(self, key, value):
+            super().__setitem__(key, value)
+            self.clear()
+
+    sizes = [(16, 4800, 1600), (40, 4800, 1600), (8, 1600, 6400)]
+    want = [kernels.linear_rows_plan(*s) for s in sizes]
+    assert want[0] is not None and want[1] is None
+    monkeypatch.setattr(kernels, "_ROWS_PLANS", Emptied())
+    assert [kernels.linear_rows_plan(*s) for s in sizes] == want

@@ -891,13 +891,16 @@ __global__ __launch_bounds__(256) void linear_mfma_rows_kernel(const bf16_t* __r
 #undef MM_WAIT_CASE
   };
   static_assert(STAGES <= 4, "arrive() knows up to three steps behind the one waited for");
-  // what this wave's tile needs behind the last step: its bias, and where its rows' keys and values go
+  // what this wave's tile needs behind the last step: its bias, where its rows' keys and values go, and what the sums are added to
   const int n = (wave % NT) * 16 + li, oc = col0 + (wave / NT % NC) * 16 + lg * 4;
   const bool vec = (n_out & 3) == 0 && (ldo & 3) == 0 && (((size_t)out | (size_t)bias) & 15) == 0;
   float b4[4];
   mfma_bias4(bias, oc < n_out ? oc : 0, n_out, vec, b4);
   int slot = -1;
   if (EPI == MM_EPI_QKV) slot = sc.slot_mapping[n < n_rows ? n : 0];
+  float4 added = {0.f, 0.f, 0.f, 0.f};
+  if (EPI == MM_EPI_RESIDUAL && vec && wave < NT * NC && n < n_rows && oc < n_out)
+    added = *reinterpret_cast<const float4*>(out + (long)n * ldo + oc);
 #pragma unroll
   for (int s = 0; s < STAGES; ++s)
     if (s < own) load(s, s);
@@ -946,6 +949,13 @@ __global__ __launch_bounds__(256) void linear_mfma_rows_kernel(const bf16_t* __r
 #pragma unroll
   for (int e = 0; e < 4; ++e)
     v[e] = (sums[0][wave][lane][e] + sums[1][wave][lane][e]) + (sums[2][wave][lane][e] + sums[3][wave][lane][e]);
+  if constexpr (EPI == MM_EPI_RESIDUAL) {
+    if (vec) {
+      *reinterpret_cast<float4*>(out + (long)n * ldo + oc) =
+          make_float4(added.x + (v[0] + b4[0]), added.y + (v[1] + b4[1]), added.z + (v[2] + b4[2]), added.w + (v[3] + b4[3]));
+      return;
+    }
+  }
   bf16_t* cache_dst = nullptr;
   if (EPI == MM_EPI_QKV && oc >= sc.q_width && slot >= 0) {
     const int page = slot / sc.page_size, off = slot - page * sc.page_size;
@@ -1106,34 +1116,60 @@ int choose_shape(int n_rows, int n_out) {
 
 // Whether a product of few rows goes to the kernel that has nothing but them and 16 or 32 columns a workgroup, rather than to the decode
 // kernel (from the matrix packed for it) or the 32 x 32 tiles.  us in a graph, matrices from memory, those two / here, where the
-// better one is: 1600 -> 4800 6.5 / 5.3 at 1 row, 7.6 / 5.6 at 8, 7.6 / 5.9 at 16, 7.7 / 7.1 at 32; 1600 -> 6400 9.2 / 6.4 at 16, 8.0 / 7.4
-// at 32; 1600 -> 1600 4.0 / 3.8, 4.8 / 4.1, 5.1 / 4.4, 5.8 / 5.2; 2048 -> 2048 4.8 / 4.5 at 4, 7.7 / 6.0 at 32; 2688 -> 1024 5.9 / 4.6, 9.6 /
-// 6.9; 5440 -> 2048 9.2 / 7.3, 16.5 / 11.8; 768 -> 2304 2.85 / 2.86, 4.5 / 3.3.  Lines: small matrices are a launch and one trip to
-// memory either way (1024 -> 1024 2.6 / 2.8, 768 -> 768 2.6 / 2.7, 512 -> 3072 2.6 / 2.8 at 1 row), and rows of 2,048 bytes and multiples
-// come from few of the memory's channels at a time, which a packed matrix does not (2048 -> 1024 3.6 / 3.7, 4.3 / 4.9; 1024 -> 2048
-// 3.8 / 3.9 at 32).
+// better one is: 1600 -> 4800 6.5 / 5.3 at 1 row, 7.6 / 5.7 at 8, 9.0 / 6.0 at 16, 7.7 / 7.1 at 32; 1600 -> 6400 9.2 / 6.4 at 16, 7.9 / 7.4
+// at 32; 1600 -> 1600 4.0 / 3.8, 4.8 / 4.1, 5.1 / 4.4, 5.8 / 5.2; 2048 -> 2048 4.7 / 4.5 at 4, 7.6 / 7.1 at 32; 2688 -> 1024 4.8 / 4.1, 7.1 /
+// 6.3; 5440 -> 2048 9.9 / 7.8, 14.4 / 10.2; 768 -> 2304 3.2 / 3.0 at 8, 4.6 / 3.4 at 32.
 bool rows_take(int n_rows, int n_out, int k_dim) {
+  const long elements = (long)n_out * k_dim;
   if (n_rows < 1 || n_rows > MM_ROWS_MAX || k_dim % MM_BK != 0 || n_out < 768 || n_out > 8192) return false;
-  if ((long)n_out * k_dim < (k_dim % 1024 == 0 ? 4000000 : 1500000) || (k_dim < 768 && n_rows < 8)) return false;
-  return n_out <= 7168 || n_rows >= 4;   // (2048 -> 8192 at 1 row 8.7 / 8.9)
+  // Small matrices are a launch and one trip to memory either way (1024 -> 1024 2.6 / 2.8, 768 -> 768 2.6 / 2.7, 512 -> 3072 2.6 / 2.8 at 1
+  // row), and rows of 2,048 bytes and multiples come from few of the memory's channels at a time, which a packed matrix does not
+  // (2048 -> 1024 3.6 / 3.7, 4.3 / 4.9; 1024 -> 2048 3.8 / 3.9 at 32).  The decode kernel's time grows with the rows, this one's hardly: with
+  // few of them the lines are further up.  896 -> 1792 3.05 / 3.24 at 4 rows, into float32 rows, 3.28 / 3.26 at 12; 768 -> 2304 3.12 / 3.17 at
+  // 3, 3.21 / 3.18 at 6, 896 -> 2304 3.26 / 3.33 at 6, 3.35 / 3.31 at 8; 896 -> 3072 3.10 / 3.22 at 1, 3.32 / 3.28 at 4; 1600 -> 1024 3.54 /
+  // 3.66 at 4, 3.85 / 3.68 at 12; 1792 -> 1280 3.50 / 3.60 at 1; 2048 -> 4096 5.37 / 5.58 at 1, 5.76 / 5.69 at 4; 2048 -> 7168 7.8 / 8.0 and
+  // 2048 -> 8192 8.7 / 8.9 at 1.
+  if (elements < (k_dim % 1024 == 0 ? 4000000 : 1500000)) return false;
+  if (k_dim < 768 && n_rows < 8) return false;
+  if (k_dim < 1024 && n_rows < (n_out <= 2048 ? 12 : n_out <= 2560 ? (k_dim < 832 ? 4 : 8) : n_out <= 4096 ? 3 : 1)) return false;
+  if (elements < 2400000 && n_out < 1536 && n_rows < 6) return false;
+  if (k_dim == 2048 && (n_out <= 4096 || n_out == 7168) && n_rows < 3) return false;
+  if (n_out > 7168 && n_rows < 4) return false;
+  // A long inner size under few columns before it is cut (rows_parts): 64 workgroups at most, each with a long chain of steps (6144 -> 768
+  // 6.5 / 7.0 at 1 row, 8192 -> 1024 8.1 / 8.6 at 4).
+  if (n_out <= 1024 && k_dim >= 6144 && (long)n_rows * k_dim < (k_dim % 8192 == 0 ? 65536 : 30000)) return false;
+  // Large matrices with rows of 4,096 bytes and multiples: 6144 -> 7168 (44 million) 18.5 / 20.2 at 1 row, 20.4 / 20.2 at 6; 8192 -> 6400 (52)
+  // 24.9 / 26.1 at 4, 26.7 / 26.0 at 8; 8192 -> 8128 (67) 30.6 / 32.5 at 8, equal at 12; 16384 -> 4096 32.9 / 35.4 at 16, 39.2 / 35.8 at 17,
+  // 16384 -> 1536 15.6 / 15.9 at 8.  Not under 257 to 320 tiles of columns, which the decode kernel takes in two rounds (8192 -> 5120 21.9 / 21.5).
+  if (k_dim % 2048 == 0 && (n_out <= 4096 || n_out > 5120) && n_rows * 2500000L <= elements - 36000000) return false;
+  if (k_dim >= 16384 && n_out > 1024 && n_rows <= (n_out > 3072 ? 16 : 12)) return false;
+  // Two tiles of rows read again by every workgroup, where the 32 x 32 tiles fill the chip: 8192 -> 4800 21.9 / 22.2 at 17, 22.6 / 24.2 at 32,
+  // 7680 -> 4800 22.0 / 22.1 at 24, 22.7 / 23.9 at 32; 10240 -> 4096 23.8 / 24.6 at 32.
+  if (n_rows > 16 && n_out > 4096 && n_out <= 5120 && (k_dim % 2048 == 0 ? k_dim >= 8192 : (long)n_rows * k_dim >= 215000)) return false;
+  if (n_rows > 28 && n_out > 2560 && n_out <= 4096 && k_dim >= 10240) return false;
+  return true;
 }
 
 // Into how many stretches such a product's inner size is cut (choose_split's reasons): every 16 columns read all rows again, and a
 // wave's steps are a chain.  us with the sums added up and into float32 rows, whole / cut: 6400 -> 1600 8.2 / 8.0 at 1 row, 9.3 / 8.6 at 8,
 // 14.2 / 10.6 at 32 (in four, 32 columns a workgroup); 5440 -> 2048 8.6 / 9.0 at 8, 9.7 / 9.2 at 16, 12.3 / 10.5 at 32; 2688 -> 1024 5.9 / 6.3
-// at 16, 7.2 / 6.7 at 32; 8192 -> 2048 12.8 / 13.4 at 16, 15.9 / 12.5 at 32.
+// at 16, 7.2 / 6.7 at 32; 8192 -> 2048 12.8 / 13.4 at 16, 15.9 / 12.5 at 32; 5120 -> 1024 7.9 / 7.2 at 8 (in four).  With more than 128 tiles of
+// columns the stretches are more workgroups than the chip takes at once: 2048 -> 2304 6.2 / 8.4 at 32, 4096 -> 2560 9.6 / 11.3; and rows of
+// 16,384 bytes in stretches come from fewer of the memory's channels still: 8192 -> 1536 9.4 / 10.7 at 4, 11.0 / 10.9 at 12.
 int rows_parts(int n_rows, int n_out, int k_dim) {
   const int tiles = (n_out + 15) / 16;
-  if (tiles > 160 || k_dim / MM_BK < 32) return 1;
-  const bool many = (long)n_rows * k_dim >= 50000, lengthy = k_dim >= 5120 && tiles <= 100;
+  if (tiles > 160 || (tiles > 128 && k_dim < 5120) || k_dim / MM_BK < 32) return 1;
+  if (k_dim % 8192 == 0 && tiles > 64 && n_rows <= 12) return 1;
+  const bool many = (long)n_rows * k_dim >= (tiles <= 64 && k_dim >= 5120 ? 30000 : 50000), lengthy = k_dim >= 5120 && tiles <= 100;
   if (tiles <= 64 || n_rows > 16) return many ? 4 : (tiles > 64 && lengthy ? 2 : 1);
   return (many || lengthy) && (k_dim % 1024 != 0 || tiles < 128) ? 2 : 1;
 }
 
-// 32 columns a workgroup: where 16 are more workgroups than compute units, and half as many read the rows half as often.
+// 32 columns a workgroup: where 16 are more workgroups than compute units, and half as many read the rows half as often (in four
+// stretches, 16 / 32 columns: 6400 -> 1088 11.2 / 10.0 at 32 rows, 4096 -> 1152 8.0 / 7.7 at 17; 6400 -> 768 8.4 with 16).
 bool rows_wide(int n_rows, int n_out, int parts) {
   const int tiles = (n_out + 15) / 16;
-  return parts > 1 ? parts == 4 && n_rows > 16 && tiles >= 80 : tiles > 256;
+  return parts > 1 ? parts == 4 && n_rows > 16 && tiles > 64 : tiles > 256;
 }
 
 // Whether the inner size is split into stretches, and then with which tile shape and into how many

@@ -33,3 +33,16 @@ def test_plans_that_another_thread_clears(monkeypatch):
     assert want[0] is not None and want[1] is None
     monkeypatch.setattr(kernels, "_ROWS_PLANS", Emptied())
     assert [kernels.linear_rows_plan(*s) for s in sizes] == want
+
+
+@pytest.mark.parametrize("n,k,o,stretches", [
+    (4, 896, 1792, None), (12, 896, 1792, 1), (3, 768, 2304, None), (4, 768, 2304, 1), (7, 896, 2304, None), (8, 896, 2304, 1), (2, 896, 3072, None),
+    (3, 896, 3072, 1), (5, 1600, 1024, None), (6, 1600, 1024, 1), (2, 2048, 2304, None), (3, 2048, 2304, 1), (4, 6144, 768, None), (5, 6144, 768, 4),
+    (7, 8192, 1024, None), (8, 8192, 1024, 4), (6, 8192, 6400, None), (7, 8192, 6400, 1), (12, 8192, 8128, None), (13, 8192, 8128, 1),
+    (12, 16384, 1536, None), (13, 16384, 1536, 2), (16, 8192, 4800, 1), (17, 8192, 4800, None), (27, 7680, 4800, 1), (28, 7680, 4800, None),
+    (28, 10240, 4096, 1), (29, 10240, 4096, None), (32, 2048, 2304, 1), (32, 4096, 2560, 1), (32, 5440, 2304, 4), (32, 4096, 2048, 4),
+    (5, 5120, 1024, 1), (6, 5120, 1024, 4), (12, 8192, 1536, 1), (13, 8192, 1536, 2), (6, 6400, 1600, 2)])
+def test_lines_of_the_products_of_few_rows(n, k, o, stretches):
+    """Where the kernel for up to 32 rows is left to others, and how often it cuts the inner size, on both sides of each line."""
+    plan = kernels.linear_rows_plan(n, o, k)
+    assert (None if plan is None else plan[1]) == stretches

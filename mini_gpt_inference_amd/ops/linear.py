@@ -217,15 +217,23 @@ def tiled_at_few_rows(n_rows: int, w: torch.Tensor, left: bool = False) -> bool:
 
 def folds_before_rows_apart(n_rows: int, n_out: int, k_dim: int) -> bool:
     """Whether the LayerNorm of a product that has a kernels.linear_rows_plan is folded into the decode kernel instead.  The fold's work
-    grows with the rows in every workgroup; a LayerNorm of its own is a launch of 2 us.  Folded / LayerNorm and product, us: 768 -> 2304
-    3.3 / 4.8 at 1 row, 5.0 / 5.2 at 16, 6.4 / 5.5 at 24; 1024 -> 4096 6.0 / 6.5 at 16, 8.4 / 7.0 at 24; 1280 -> 3840 6.6 / 7.0 at 8, 7.9 / 7.1
-    at 12; with more than a workgroup a compute unit 1280 -> 5120 7.4 / 7.6 at 4, 8.5 / 7.9 at 8, 12.6 / 8.3 at 16; 1600 -> 4800 8.0 / 8.2 at 4,
-    9.5 / 8.5 at 8, 13.1 / 8.9 at 16; 1600 -> 6400 8.3 / 8.8, 9.8 / 9.0, 13.2 / 9.3; short inner sizes never (512 -> 1536 3.9 / 5.5 at 32)."""
+    grows with the rows in every workgroup (in steps of 8 rows, of 4 beyond an inner size of 2,048); a LayerNorm of its own is a launch of
+    2 us, and one of more than 4,096 columns takes ten times that.  Folded / LayerNorm and product, us: 768 -> 2304 3.3 / 4.8 at 1 row, 5.0 /
+    5.2 at 16, 6.4 / 5.5 at 24; 1024 -> 4096 6.0 / 6.3 at 16, 8.3 / 6.7 at 24; 960 -> 1792 5.3 / 5.9 at 32; short inner sizes always (512 ->
+    1536 3.9 / 5.5 at 32).  1280 -> 3840 6.6 / 7.0 at 8, 7.9 / 7.1 at 12; 2048 -> 3072 7.3 / 8.0 at 8, 8.4 / 8.2 at 12; 3072 -> 2048 8.1 / 8.4
+    at 4, 9.3 / 8.7 at 6.  While workgroups of 8 rows and 16 columns all have a compute unit, under small matrices: 1600 -> 1024 5.5 / 6.9 at
+    32, 1408 -> 1280 5.4 / 6.5 at 24 and 7.2 / 6.5 at 28, 1600 -> 1792 5.8 / 6.4 at 16 (1792 -> 1792 8.0 / 6.4).  With more than a workgroup
+    of 16 columns a compute unit: 1280 -> 5120 7.4 / 7.6 at 4, 8.5 / 7.9 at 8, 12.6 / 8.3 at 16; 1600 -> 4800 8.0 / 8.2, 9.5 / 8.5, 13.1 / 8.9;
+    1600 -> 6400 8.3 / 8.8, 9.8 / 9.0, 13.2 / 9.3; 4096 -> 5120 13.7 / 15.2 at 4, 16.0 / 15.4 at 6.  And 5120 -> 2048 16.4 / 44.6 at 12."""
+    if k_dim > 4096:
+        return True
     if n_out > 4096:
-        return n_rows * k_dim <= 8192
+        return n_rows * k_dim <= (16384 if k_dim == 4096 else 8192)
     if k_dim > 1024:
-        return n_rows * k_dim <= 13000
-    return n_rows <= 16 or k_dim < 768
+        if n_out * k_dim < (3_000_000 if k_dim <= 2048 else 2_700_000) and -(-n_out // 16) * -(-n_rows // 8) <= 256:
+            return True
+        return n_rows <= 4 if k_dim > 2048 else n_rows <= 8 or n_rows * k_dim <= 13000
+    return n_rows <= 16 or n_out <= 2048 or k_dim < 768
 
 
 def _rows_apart(ctx, plan, a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor, n_rows: int, epilogue: int,

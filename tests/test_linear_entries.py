@@ -5,6 +5,7 @@ import ctypes
 import pytest
 
 from mini_gpt_inference_amd.ops import kernels, library
+from mini_gpt_inference_amd.ops.linear import folds_before_rows_apart
 
 NULL_POINTER = -4
 XIELU = 4
@@ -46,3 +47,14 @@ def test_lines_of_the_products_of_few_rows(n, k, o, stretches):
     """Where the kernel for up to 32 rows is left to others, and how often it cuts the inner size, on both sides of each line."""
     plan = kernels.linear_rows_plan(n, o, k)
     assert (None if plan is None else plan[1]) == stretches
+
+
+@pytest.mark.parametrize("n,k,o,folds", [
+    (32, 960, 2048, True), (17, 960, 2304, False), (8, 2048, 3072, True), (9, 2048, 3072, False), (10, 1280, 3840, True), (11, 1280, 3840, False),
+    (4, 3072, 2048, True), (5, 3072, 2048, False), (32, 1600, 1024, True), (24, 1408, 1280, True), (25, 1408, 1280, False), (16, 1600, 1792, True),
+    (16, 1792, 1792, False), (16, 2560, 1024, True), (12, 2560, 1280, False), (5, 1600, 4800, True), (6, 1600, 4800, False), (4, 4096, 5120, True),
+    (5, 4096, 5120, False), (32, 5120, 2048, True)])
+def test_lines_of_the_layer_norm_in_front(n, k, o, folds):
+    """Which products of a plan have their LayerNorm folded into the decode kernel instead."""
+    assert kernels.linear_rows_plan(n, o, k) is not None
+    assert folds_before_rows_apart(n, o, k) == folds

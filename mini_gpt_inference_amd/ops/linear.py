@@ -156,13 +156,20 @@ WIDE_OUT = 8192
 WIDE_OUT_DECODE_WORK = 8192
 
 
-def wide_rows_once(n_rows: int, k_dim: int) -> bool:
+def wide_rows_once(n_rows: int, n_out: int, k_dim: int) -> bool:
     """Whether a very wide output beyond that work goes to the kernel that reads the matrix once, whole lines a load, for a tile of 16 rows
-    (linear_rows_once).  Its time grows with the rows, from a lower level than the tiled kernel's; and rows of 4,096 bytes and multiples
-    come to the tiled kernel from few of the memory's channels at a time.  Tiled / here, us: 32768 x 768 12.8 / 12.0 at 8 rows, 12.9 / 12.6 at
-    12, 50257 x 768 17.6 / 16.9 at 8; 32768 x 1024 15.1 / 13.6 at 8, 50257 x 1024 20.9 / 20.5 at 8, 21.6 / 21.7 at 12; 32768 x 2048 33.8 / 28.7
-    at 8, 33.9 / 29.8 at 12, 50257 x 2048 44.5 / 43.1 at 8, 45.4 / 45.1 at 12; between, 50257 x 1600 31.7 / 32.6 at 6, 32768 x 2560 34.4 / 34.5 at 8."""
-    return n_rows <= (12 if k_dim % 2048 == 0 else 8 if k_dim <= 1024 else 0)
+    (linear_rows_once).  Its time grows with the rows, from a lower level than the tiled kernel's where rows of 4,096 bytes and multiples
+    come to that one from few of the memory's channels at a time, and does not jump with the rounds of its tiles (at 8,193 and 10,753
+    columns, less under an inner size of 2,048).  Tiled / here, us: 32768 x 2048 33.8 / 28.7 at 8 rows, 33.9 / 29.8 at 12, 50257 x 2048 44.5 /
+    43.1 and 45.4 / 45.1, 14336 x 2048 14.4 / 13.9 at 5, 14.6 / 14.5 at 12 (8192 x 2048 9.1 / 9.9, 13000 x 2048 12.9 / 13.3 at 5); 8192 x 4096
+    18.6 / 16.2 at 3, 18.7 / 16.4 at 12, 32768 x 4096 63.5 / 51.5, 63.9 / 56.1; 12288 x 6144 38.7 / 32.8 at 2, 38.9 / 32.7 at 8, 13000 x 6144
+    39.5 / 40.0 at 10; 16384 x 8192 57 / 57 at 3 and 12; 14336 x 10240 63.8 / 63.6 at 6, 64.5 / 65.8 at 8; in between, 9216 x 4096 19.6 / 18.6 at
+    3, 20.1 / 21.2 at 12, 9216 x 6144 27.4 / 26.9 at 3, 27.6 / 28.6 at 6."""
+    if k_dim % 2048 or (k_dim == 2048 and n_out < 14336):
+        return False
+    if k_dim > 2048 and 8192 < n_out < 11264:
+        return n_rows * k_dim <= 20000
+    return n_rows <= (12 if k_dim <= 4096 or k_dim == 8192 else 8 if k_dim < 8192 else 6)
 
 
 # The decode kernel's time grows with the rows (every workgroup loads all of them for its 16 output
@@ -445,7 +452,7 @@ def linear(ctx, a: Union[torch.Tensor, LazyNorm], w: torch.Tensor, bias: Optiona
                                             scatter)):
         return scatter is not None
     a = as_tensor(ctx, a)
-    if (fast and wide_out and bias is None and scatter is None and epilogue == kernels.EPI_NONE and wide_rows_once(n_rows, w.shape[1])
+    if (fast and wide_out and bias is None and scatter is None and epilogue == kernels.EPI_NONE and wide_rows_once(n_rows, *w.shape)
             and kernels.linear_rows_once(a, w, out, n_rows)):
         return False
     if plan is not None and _rows_apart(ctx, plan, a, w, bias, out, n_rows, epilogue, scatter):

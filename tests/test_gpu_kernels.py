@@ -471,16 +471,38 @@ def test_which_float32_products_norm_their_rows(n, o, k, norms):
                                    (16, 8, 40), (16, 56, 20), (5, 2120, 50), (16, 2744, 33)])
 @pytest.mark.parametrize("o_dt", ["float32", "bfloat16"])
 def test_linear_rows_once(n, k, o, o_dt):
-    """A pass over the matrix for up to 16 rows: one stage and two, inner sizes that are no whole steps, ragged columns; and that
-    very wide outputs of few rows go there."""
+    """A pass over the matrix for up to 16 rows: one stage and two, inner sizes that are no whole steps, ragged columns."""
     g = torch.Generator().manual_seed(n * k + o)
     a, w = rnd(g, n, k, dtype="bfloat16"), rnd(g, o, k, dtype="bfloat16", scale=k ** -0.5)
     out = torch.full((n + 1, o), 7.0, dtype=torch.float32 if o_dt == "float32" else torch.bfloat16, device=DEV)
     assert kernels.linear_rows_once(a.to(DEV), w.to(DEV), out, n)
     helpers.assert_close(out[:n], a.double() @ w.double().T, o_dt, f"{n} {k} {o}")
     assert (out[n] == 7.0).all()
+
+
+@pytest.mark.parametrize("n,k,o,once", [
+    (4, 2048, 14336, False), (5, 2048, 14336, True), (12, 2048, 14336, True), (13, 2048, 14336, False), (8, 2048, 14320, False), (8, 1024, 50257, False),
+    (9, 1024, 16384, False), (8, 1600, 16384, False), (12, 4096, 8192, True), (13, 4096, 8192, False), (4, 4096, 8208, True), (5, 4096, 8208, False),
+    (12, 4096, 11264, True), (8, 6144, 8192, True), (9, 6144, 8192, False), (3, 6144, 9216, True), (4, 6144, 9216, False), (6, 10240, 8192, True),
+    (7, 10240, 8192, False)])
+def test_which_very_wide_outputs_go_once_over_the_matrix(monkeypatch, n, k, o, once):
+    """Through the entry that chooses, on both sides of the lines: few rows go to the kernel that reads the matrix once, and nothing
+    else does."""
+    from types import SimpleNamespace
+
     from mini_gpt_inference_amd.ops import linear as L
-    assert L.wide_rows_once(8, 1024) and L.wide_rows_once(12, 2048) and not L.wide_rows_once(9, 1024) and not L.wide_rows_once(1, 1600)
+    from mini_gpt_inference_amd.parts.base import Workspace
+
+    calls, plain = [], kernels.linear_rows_once
+    monkeypatch.setattr(kernels, "linear_rows_once", lambda *args: calls.append(plain(*args)) or calls[-1])
+    g = torch.Generator().manual_seed(n + k)
+    a = rnd(g, n, k, dtype="bfloat16").to(DEV)
+    w = (torch.randn(o, k, device=DEV, generator=torch.Generator(DEV).manual_seed(n)) * k ** -0.5).to(torch.bfloat16)
+    ctx = SimpleNamespace(exact=False, dtype=torch.bfloat16, n_rows=n, pending=None, copy_budget=None, workspace=Workspace(torch.device(DEV)))
+    out = torch.empty(n, o, device=DEV)
+    L.linear(ctx, a, w, None, out, n)
+    assert calls == ([True] if once else [])
+    helpers.assert_close(out, a.double() @ w.double().T, "float32", f"{n} {k} {o}")
 
 
 @pytest.mark.parametrize("n,k,o", [(6, 2048, 16384), (3, 4096, 8192), (13, 2048, 16384), (4, 512, 8192)])

@@ -56,11 +56,18 @@ __global__ __launch_bounds__(NT) void decay_state_kernel(
   float* st = state + ((long)slot * n_head + h) * (long)D * E;
   const int first_pos = positions[t_begin];
   const bool fresh = first_pos == 0;            // the request's first token: its state starts at zero
-#pragma unroll
-  for (int j = 0; j < R; ++j) S[j] = j < count ? st[(long)(dg + j * NG) * E + e] : 0.f;
   const int half = rot_dims / 2;
   const int wave = tid >> 6, lane = tid & 63;
 
+  // All of a few values are on their way at once, and chosen from later; many one behind the other (4 heads of 256 x 256, 64 values a
+  // thread: 29 us a token, chosen from later 64).
+  if constexpr (R <= 16) {
+#pragma unroll
+    for (int j = 0; j < R; ++j) S[j] = j < count ? st[(long)(dg + j * NG) * E + e] : 0.f;
+  } else {
+#pragma unroll
+    for (int j = 0; j < R; ++j) S[j] = (j < count && !fresh) ? st[(long)(dg + j * NG) * E + e] : 0.f;
+  }
   if (R <= 16 && t_end - t_begin == 1) {       // (more values a thread leave no registers for it)
     const T* row = z + (long)t_begin * ldz;
     constexpr int GATES = DS_MAX / 64;
@@ -140,8 +147,10 @@ __global__ __launch_bounds__(NT) void decay_state_kernel(
       if (j < count) st[(long)(dg + j * NG) * E + e] = S[j];
     return;
   }
+  if constexpr (R <= 16) {
 #pragma unroll
-  for (int j = 0; j < R; ++j) S[j] = fresh ? 0.f : S[j];
+    for (int j = 0; j < R; ++j) S[j] = fresh ? 0.f : S[j];
+  }
 
   for (int t0 = t_begin; t0 < t_end; t0 += DS_TC) {
     const int nt = t_end - t0 < DS_TC ? t_end - t0 : DS_TC;

@@ -253,7 +253,7 @@ def _state_case(g, dtype, lens, H, D, E):
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("H,D,E", [(2, 16, 24), (1, 64, 64), (2, 128, 128), (3, 20, 12), (1, 256, 64), (2, 8, 256),
-                                   (1, 1, 1)])
+                                   (1, 1, 1), (1, 128, 256), (2, 256, 256)])
 def test_decaying_state_whole_in_portions_and_slots_used_again(dtype, H, D, E):
     """Three requests of unequal lengths in one step against the plain recurrence; then the same
     requests cut into portions (down to one token) over several steps, their states carried in

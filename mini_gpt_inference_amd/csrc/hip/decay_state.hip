@@ -351,7 +351,7 @@ __global__ __launch_bounds__(256) void state_inputs_kernel(const T* __restrict__
 // piece's place costs no division).  V: queries and keys in pieces of V channels (4: head sizes that are multiples of four).  T: the
 // storage type of z.  added: [segments][n_head][E][Dp].
 template <int EB, int MODE, int DL, int V, typename T>
-__global__ __launch_bounds__(256, V == 1 ? 1 : MODE == DC_ADDED ? 4 : 3) void decay_state_chunk_kernel(
+__global__ __launch_bounds__(256, V == 1 && DL == 128 ? 1 : MODE == DC_ADDED ? 4 : 3) void decay_state_chunk_kernel(
     const float* __restrict__ qk, const T* __restrict__ z, long ldz, int v_off, int n_head, int D, int E,
     int act, const int* __restrict__ positions, const float* __restrict__ decay, float* __restrict__ state,
     const int* __restrict__ state_slots, const int* __restrict__ cu_q, float* __restrict__ out, long ldo, int n_req,
@@ -614,10 +614,12 @@ extern "C" int mgpt_decay_state_chunked(const void* z, int dtype, long ldz, int 
     if (dtype == MGPT_F32) {                                                                                               \
       if (vec && D <= 64) DC_LAUNCH_AS(EB, MODE, X, 64, 4, float);                                                              \
       else if (vec) DC_LAUNCH_AS(EB, MODE, X, 128, 4, float);                                                                        \
+      else if (D <= 64) DC_LAUNCH_AS(EB, MODE, X, 64, 1, float);                                                                \
       else DC_LAUNCH_AS(EB, MODE, X, 128, 1, float);                                                                            \
     } else {                                                                                                               \
       if (vec && D <= 64) DC_LAUNCH_AS(EB, MODE, X, 64, 4, bf16_t);                                                             \
       else if (vec) DC_LAUNCH_AS(EB, MODE, X, 128, 4, bf16_t);                                                                       \
+      else if (D <= 64) DC_LAUNCH_AS(EB, MODE, X, 64, 1, bf16_t);                                                               \
       else DC_LAUNCH_AS(EB, MODE, X, 128, 1, bf16_t);                                                                           \
     }                                                                                                                      \
   } while (0)

@@ -377,7 +377,7 @@ def test_infinite_value_in_a_decaying_state(D, cut):
     helpers.assert_close(chunked[:, others] / walked[:, others].abs().max(), walked[:, others] / walked[:, others].abs().max(), "float32", "other channels")
 
 
-@pytest.mark.parametrize("H,D,E", [(2, 128, 128), (3, 40, 24), (1, 16, 130)])
+@pytest.mark.parametrize("H,D,E", [(2, 128, 128), (3, 40, 24), (1, 16, 130), (2, 37, 50), (1, 101, 40)])
 @pytest.mark.parametrize("lens", [[1, 255, 256, 257], [511, 512, 513, 0, 700], [1300], [300] * 70, [4] * 66 + [600]])
 def test_decaying_state_in_segments(lens, H, D, E):
     """Requests cut into segments of 256 tokens that run side by side against their chunks one behind the other (which is

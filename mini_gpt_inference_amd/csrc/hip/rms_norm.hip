@@ -49,7 +49,8 @@ __device__ __forceinline__ float block_sum(float v, float* scratch) {
 // PT * threads values), and everything that it reads is on its way before the first sum; PT = 0: the second pass reads them again.
 // XT, GT, OT: the types of the input, the gate and the output.  What bounds few rows is the trips to memory: with types chosen at run
 // time every value was waited for by itself, and gain and gate came behind the sum.  us in a graph, so / here: 8 rows of 1,024 3.4 / 2.7,
-// with a gate 4.2 / 3.1, of 2,048 4.3 / 3.3, of 8,192 16.5 / 11.1; 4,075 rows of 1,024 8.8 / 7.1, of 8 gated heads of 128 14.0 / 11.7.
+// with a gate 4.2 / 3.1, of 2,048 4.3 / 3.3, of 8,192 16.5 / 11.1; 4,075 rows of 1,024 8.8 / 7.1, of 8 gated heads of 128 14.0 / 11.7.  PT is close to
+// the values there are: those beyond the segment's end are loads as well (4,096 rows of 1,280 14.0 / 17.5 with 16, 11.5 with 6).
 template <int PT, typename XT, typename GT, typename OT>
 __global__ __launch_bounds__(256) void rms_norm_kernel(
     const XT* x, long ldx, const int* __restrict__ rows,      // (out may be x: the norm in place)
@@ -169,6 +170,8 @@ extern "C" int mgpt_rms_norm(const void* x, int x_dtype, long ldx, const int* ro
   const int per_thread = (width + threads - 1) / threads;
   if (per_thread <= 2) RN_TYPES(2);
   else if (per_thread <= 4) RN_TYPES(4);
+  else if (per_thread <= 6) RN_TYPES(6);
+  else if (per_thread <= 8) RN_TYPES(8);
   else if (per_thread <= 16) RN_TYPES(16);
   else RN_TYPES(0);
 #undef RN_TYPES

@@ -777,15 +777,14 @@ extern "C" int mgpt_grouped_linear_mfma(const void* a, long lda, const int* a_ro
 // hidden size.  tile_expert null: one matrix for all rows, of which the first n_rows are used (slot_token null).
 //
 // A wave brings its slices of the matrix straight into LDS, eight rows of 128 bytes a load, STAGES steps of its own: no barrier, no
-// registers for what is on its way.  (With two, loads stay on their way in one step of two: the rows' operands are loaded into
-// registers, and where the loop closes the compiler waits for all that is in flight.)  A lane's operand, 16 bytes of one of 16 rows, loaded as it is used makes every
+// registers for what is on its way.  A lane's operand, 16 bytes of one of 16 rows, loaded as it is used makes every
 // load touch 16 lines in 16-byte pieces, and the unit that looks the lines up is what bounds it then (the rows are few: theirs are loaded
 // so; through LDS as well they took room that workgroups need).  The 16-byte pieces
 // of a row are XORed with its number, at the source, so that an operand's read from LDS meets no bank twice.  The matrix's first loads
 // leave before the tile's rows are looked up, two trips to memory one behind the other.  us in a graph, matrices from memory, 32 k a
-// step through registers / here: 8 rows, gated, 2048 -> 5440 (44.6 MB) 15.5 / 11.6, -> 1344 7.8 / 6.5, 1024 -> 2688 6.0 / 5.0; 16 pairs for
-// 8 experts 2048 -> 2048 gated (117 MB) 29.8 / 25.6 and down (59 MB) 15.4 / 12.7; 64 pairs for 64 experts 1024 -> 512 21.5 / 17.0,
-// 512 -> 1024 10.4 / 9.9.
+// step through registers / here: 8 rows, gated, 2048 -> 5440 (44.6 MB) 16.2 / 12.1, -> 1344 9.0 / 8.5, 1024 -> 2688 6.5 / 5.9; 8 tiles of
+// 8 experts 2048 -> 2048 gated (134 MB) 32.4 / 29.2 and without a unit (67 MB) 17.1 / 16.6; 32 of 32 experts 1024 -> 512 gated 16.1 / 14.4,
+// 512 -> 1024 without 9.4 / 8.7; 2 of 8 experts 2048 -> 2048 without 7.7 / 7.7.
 #define EX_STEP 64
 
 template <typename OT, bool GATED, int STAGES>
@@ -841,35 +840,53 @@ __global__ __launch_bounds__(256) void grouped_few_rows_kernel(
 #pragma unroll
   for (int j = 0; j < NJ; ++j) acc[j] = ex_f32x4_t{0.f, 0.f, 0.f, 0.f};
   const int at0 = li * EX_STEP + ((lg ^ (li & 7)) * 8), at1 = li * EX_STEP + (((lg + 4) ^ (li & 7)) * 8);
-  for (int step0 = wave; step0 < steps; step0 += 4 * STAGES) {
+  ex_bf16x8_t wf[NJ][2], a0, a1;
+  auto read_step = [&](int st) {
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      wf[j][0] = *reinterpret_cast<const ex_bf16x8_t*>(&staged[wave][st][j][at0]);
+      wf[j][1] = *reinterpret_cast<const ex_bf16x8_t*>(&staged[wave][st][j][at1]);
+    }
+    a0 = a_ok ? af[st][0] : zero, a1 = a_ok ? af[st][1] : zero;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // read before the stage is loaded again
+  };
+  auto multiply = [&]() {
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j][0], a0, acc[j], 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j][1], a1, acc[j], 0, 0, 0);
+  };
+  int step0 = wave;
+  if constexpr (STAGES > 1) {
+    // Rounds behind which a whole one follows: every step loads the one STAGES further on, so that STAGES - 1 steps' loads are behind the
+    // one waited for (all of them in the first round, whose rows came behind all of their matrices).  The count holds because each of these
+    // steps has all its loads, the rows' too, between the asm statement that ends the reading of its stage and the next wait: they may change
+    // places there but not leave, which is why A is not __restrict__ (what nobody else may write could be loaded behind a statement that
+    // says it writes).  Loads under a condition made the compiler wait for all of them wherever the rows' operands are used.
+    for (; step0 + 4 * (2 * STAGES - 1) < steps; step0 += 4 * STAGES)
+#pragma unroll
+      for (int st = 0; st < STAGES; ++st) {
+        if (step0 == wave) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(%0)" ::"n"((STAGES - 1) * (2 * NJ + 2)) : "memory");
+        read_step(st);
+        load_w(step0 + 4 * (st + STAGES), st);
+        load_a(step0 + 4 * (st + STAGES), st);
+        multiply();
+      }
+  }
+  for (; step0 < steps; step0 += 4 * STAGES)
 #pragma unroll
     for (int st = 0; st < STAGES; ++st) {
       const int step = step0 + 4 * st;
       if (step >= steps) break;
-      // A step's loads come together, but for the first steps, whose rows came behind all of their matrices.  The steps behind this one
-      // that are on their way: STAGES - 1, fewer towards the end.  The count holds because each of these steps has all its loads,
-      // the rows' too, between the asm statement that ends the reading of its stage and the next wait: they may change places there but not
-      // leave, which is why A is not __restrict__ (what nobody else may write could be loaded behind a statement that says it writes).
-      if (step0 == wave || step + 4 * (STAGES - 1) >= steps) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      else asm volatile("s_waitcnt vmcnt(%0)" ::"n"((STAGES - 1) * (2 * NJ + 2)) : "memory");
-      ex_bf16x8_t wf[NJ][2];
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) {
-        wf[j][0] = *reinterpret_cast<const ex_bf16x8_t*>(&staged[wave][st][j][at0]);
-        wf[j][1] = *reinterpret_cast<const ex_bf16x8_t*>(&staged[wave][st][j][at1]);
-      }
-      const ex_bf16x8_t a0 = a_ok ? af[st][0] : zero, a1 = a_ok ? af[st][1] : zero;
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // read before the stage is loaded again
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      read_step(st);
       if (step + 4 * STAGES < steps) {
         load_w(step + 4 * STAGES, st);
         load_a(step + 4 * STAGES, st);
       }
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j][0], a0, acc[j], 0, 0, 0);
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j][1], a1, acc[j], 0, 0, 0);
+      multiply();
     }
-  }
   // what is left of the inner size, 32 at a time, the last step perhaps not whole
   const bf16_t* wp = wm + (long)(col0 + li < n_out ? col0 + li : n_out - 1) * k_dim + lg * 8;
   for (int k = steps * EX_STEP + wave * 32; k < k_dim; k += 128) {
@@ -913,10 +930,11 @@ extern "C" int mgpt_grouped_few_rows(const void* a, long lda, const int* a_rows,
   if (n_tiles > 65535) return MGPT_ERR_TOO_LARGE;
   dim3 grid((n_out + 15) / 16, n_tiles), block(256);
   // One stage a wave while the inner size is short, since more workgroups on a compute unit bring more than more stages do; two under long
-  // ones and for gated experts from 2,048 on (us, one / two / three: gated 2048 -> 5440 11.6 / 12.0 / 12.0, 3072 -> 1024 8.1 / 7.7 / 7.7,
-  // 5440 -> 2048 17.1 / 14.5 / 14.5; experts gated 2048 -> 2048 of 16 pairs 26.8 / 25.6 / 27.8, of 2 9.8 / 10.0 / 9.9, down 12.7 / 13.2 / 13.7,
-  // 4096 -> 1024 13.2 / 12.5 / 12.8).
-  const bool two = k_dim > 2048 || (kind >= 0 && tile_expert && k_dim >= 2048);
+  // ones, for gated experts from 2,048 on, and for few workgroups without a unit (us, one / two: gated 2048 -> 5440 11.6 / 11.9, 3072 -> 1024
+  // 10.8 / 8.9, 5440 -> 1024 17.1 / 13.0; experts gated 2048 -> 2048 of 8 tiles 30.5 / 29.2, of 4 17.3 / 17.3, of 1 9.2 / 8.4; without a unit of
+  // 2 tiles 8.6 / 7.7, of 4 10.6 / 10.5, of 8 16.6 / 17.2; 1024 -> 512 of 8 4.75 / 4.50, of 16 6.5 / 6.6; 4096 -> 1024 of 2 12.6 / 9.6).
+  const long groups = (long)((n_out + 15) / 16) * n_tiles;
+  const bool two = k_dim > 2048 || (kind >= 0 ? tile_expert && k_dim >= 2048 : k_dim >= 512 && groups <= (k_dim > 1024 ? 512 : 256));
 #define GF_LAUNCH(OT, G)                                                                                              \
   do {                                                                                                                \
     if (two) GF_LAUNCH_AS(OT, G, 2);                                                                                  \

@@ -459,7 +459,9 @@ def test_float32_product_that_norms_its_rows_has_the_bits_of_both_kernels(n, k, 
 
 
 @pytest.mark.parametrize("n,o,k,norms", [(16, 4096, 512, True), (16, 4097, 512, False), (32, 2048, 512, True), (33, 2048, 512, False),
-                                         (3, 300, 768, True), (3, 300, 772, False), (3, 300, 66, False)])
+                                         (3, 300, 768, True), (3, 300, 772, False), (3, 300, 66, False),
+                                         (16, 4096, 516, True), (17, 1536, 640, True), (17, 1537, 640, False), (32, 2048, 516, False),
+                                         (64, 768, 768, True), (64, 784, 768, False)])
 def test_which_float32_products_norm_their_rows(n, o, k, norms):
     assert kernels.linear_exact_norms(n, o, k) == norms
     if not norms:

@@ -35,7 +35,7 @@ __device__ __forceinline__ void ds_meet() { asm volatile("s_waitcnt lgkmcnt(0)\n
 // A request's single token (every request of a decode step) takes three phases between two barriers, with everything that it reads on its
 // way at once: the state, the gate, and for each work item of the inputs (a rotated pair of channels of q and k, a channel that is not
 // rotated, a value) what that needs.  What bounds it is that chain of latencies: the walk below reads queries, keys, values,
-// angles and the gate one behind the other.  8 requests x 8 heads of 128 x 128 in a decode step: 11.9 us by that walk, so 8.9.
+// angles and the gate one behind the other.  8 requests x 8 heads of 128 x 128 with norm and gate: 11.1 us by that walk, so 7.7.
 template <int R, int NT, typename T>
 __global__ __launch_bounds__(NT) void decay_state_kernel(
     const T* __restrict__ z, long ldz, int q_off, int k_off, int v_off, int g_off, int n_head, int D, int E,
@@ -61,9 +61,18 @@ __global__ __launch_bounds__(NT) void decay_state_kernel(
 
   // All of a few values are on their way at once, and chosen from later; many one behind the other (4 heads of 256 x 256, 64 values a
   // thread: 29 us a token, chosen from later 64).
+  // With more than a workgroup a compute unit bytes count for more than the wait for the position, and a new request's state is left
+  // alone.  us, always loaded / so: 128 new requests x 8 heads of 128 x 128 35.6 / 22.1, x 16 60.2 / 37.6, 32 x 16 17.3 / 14.0; 128 that are not
+  // new x 8 35.3 / 32.3, 8 requests x 8 8.2 / 7.2 (the same loads, with fewer conditions at each); 32 requests of 3 tokens x 16 22.2 / 23.0.
   if constexpr (R <= 16) {
+    const bool leave = gridDim.x * gridDim.y > 256 && fresh;
+    if (leave) {
 #pragma unroll
-    for (int j = 0; j < R; ++j) S[j] = j < count ? st[(long)(dg + j * NG) * E + e] : 0.f;
+      for (int j = 0; j < R; ++j) S[j] = 0.f;
+    } else {
+#pragma unroll
+      for (int j = 0; j < R; ++j) S[j] = j < count ? st[(long)(dg + j * NG) * E + e] : 0.f;
+    }
   } else {
 #pragma unroll
     for (int j = 0; j < R; ++j) S[j] = (j < count && !fresh) ? st[(long)(dg + j * NG) * E + e] : 0.f;

@@ -324,6 +324,36 @@ def test_decaying_state_whole_in_portions_and_slots_used_again(dtype, H, D, E):
         helpers.assert_close(state[1:4], whole_state[1:4], "float32", f"{variant} state")
 
 
+@pytest.mark.parametrize("H,D,E,n_req", [(2, 16, 24, 128), (2, 16, 24, 129), (3, 64, 64, 86), (2, 128, 128, 129), (1, 256, 128, 257)])
+def test_many_requests_have_the_bits_of_a_few_at_a_time(H, D, E, n_req):
+    """Beyond 256 workgroups a new request's state is not read at all: slots that hold NaN, every third request new, one and three
+    tokens, against the same requests 16 at a time."""
+    g = torch.Generator().manual_seed(n_req)
+    lens = [3 if r % 5 == 4 else 1 for r in range(n_req)]
+    z, k_off, v_off, g_off = _state_case(g, "bfloat16", lens, H, D, E)
+    first = [0 if r % 3 == 0 else 7 for r in range(n_req)]
+    start = _rnd(g, n_req, H * D * E)
+    start[[r for r in range(n_req) if r % 3 == 0]] = float("nan")
+    decay = torch.tensor([0.999, 0.6, 0.9][:H], device=DEV)
+
+    def run(at_once):
+        state, outs = start.to(DEV), []
+        for r0 in range(0, n_req, at_once):
+            rs = range(r0, min(r0 + at_once, n_req))
+            cu = torch.tensor([0] + [lens[r] for r in rs]).cumsum(0)
+            pos = torch.tensor([first[r] + t for r in rs for t in range(lens[r])], dtype=torch.int32, device=DEV)
+            o = torch.zeros(int(cu[-1]), H * E, dtype=torch.bfloat16, device=DEV)
+            base = sum(lens[:r0])
+            kernels.decay_state(z[base:base + int(cu[-1])].to(DEV), 0, k_off, v_off, g_off, H, D, E, decay, state,
+                                torch.tensor(list(rs), dtype=torch.int32, device=DEV), cu.to(torch.int32).to(DEV), len(rs), pos, o,
+                                silu_inputs=True, norm_eps=1e-5)
+            outs.append(o)
+        return torch.cat(outs), state
+
+    (out, state), (want_out, want_state) = run(n_req), run(16)
+    assert torch.isfinite(state).all() and torch.equal(state, want_state) and torch.equal(out, want_out)
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("H,D,E", [(2, 128, 128), (3, 20, 12), (1, 256, 64), (2, 8, 256), (1, 37, 50), (1, 64, 65)])
 def test_single_tokens_have_the_bits_of_the_walk_over_several(dtype, H, D, E):

@@ -1117,7 +1117,8 @@ int choose_shape(int n_rows, int n_out) {
 // Whether a product of few rows goes to the kernel that has nothing but them and 16 or 32 columns a workgroup, rather than to the decode
 // kernel (from the matrix packed for it) or the 32 x 32 tiles.  us in a graph, matrices from memory, those two / here, where the
 // better one is: 1600 -> 4800 6.5 / 5.3 at 1 row, 7.6 / 5.7 at 8, 9.0 / 6.0 at 16, 7.7 / 7.1 at 32; 1600 -> 6400 9.2 / 6.4 at 16, 7.9 / 7.4
-// at 32; 1600 -> 1600 4.0 / 3.8, 4.8 / 4.1, 5.1 / 4.4, 5.8 / 5.2; 2048 -> 2048 4.7 / 4.5 at 4, 7.6 / 7.1 at 32; 2688 -> 1024 4.8 / 4.1, 7.1 /
+// at 32; 1600 -> 1600 4.0 / 3.8, 4.8 / 4.1, 5.1 / 4.4, 5.8 / 5.2
+// (into the residual rows of a decode step at 32 rows 6.1 / 5.9); 2048 -> 2048 4.7 / 4.5 at 4, 7.6 / 7.1 at 32; 2688 -> 1024 4.8 / 4.1, 7.1 /
 // 6.3; 5440 -> 2048 9.9 / 7.8, 14.4 / 10.2; 768 -> 2304 3.2 / 3.0 at 8, 4.6 / 3.4 at 32.
 bool rows_take(int n_rows, int n_out, int k_dim) {
   const long elements = (long)n_out * k_dim;

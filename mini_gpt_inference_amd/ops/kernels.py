@@ -2111,8 +2111,9 @@ def decay_state_segments(n_tokens: int, n_req: int, max_q_len: int, n_head: int,
     chunks, heads and 32 value channels.  Whole / cut: 2 requests of 1,024 tokens x 8 heads 175 / 129, x 16 heads 184 / 193;
     one of 2,048 x 16 337 / 160; 8 of 100 to 1,024 x 8 236 / 205; 4 of 600 x 16 153 / 204; 16 of 1,024 x 8 332 / 482.  A chunk
     of smaller heads is less work, of 64 x 64 0.72 of that: one request of 300 x 4 40 / 50, of 1,024 x 4 111 / 54, two of 600 x 16
-    75 / 65.  (By now all of these take 0.55 to 0.6 of that, on both sides: 102 / 81, 106 / 102, 195 / 91, 129 / 103, 86 / 108,
-    222 / 289; 25 / 31, 69 / 34, 49 / 44.  The line is where it was.)"""
+    75 / 65.  These are times of the kernels before the state moved into registers, from which the line was drawn; now they are 0.50 to
+    0.68 of that: 102 / 81, 106 / 102, 195 / 91, 129 / 103, 86 / 108, 222 / 289; 25 / 31, 69 / 34, 49 / 44.  The line still takes the faster side
+    of all but one of them (2 requests of 1,024 x 16 stay whole, 4 % slower than cut)."""
     blocks = -(-value_dim // 32) * n_head
     chunk = 0.44 + 0.56 * head_dim / 128
     whole = max_q_len / 32 * chunk * (6.75 if n_req * blocks >= 256 else 5.1)

@@ -61,11 +61,16 @@ __global__ __launch_bounds__(NT) void decay_state_kernel(
 
   // All of a few values are on their way at once, and chosen from later; many one behind the other (4 heads of 256 x 256, 64 values a
   // thread: 29 us a token, chosen from later 64).
-  // With more than a workgroup a compute unit bytes count for more than the wait for the position, and a new request's state is left
-  // alone.  us, always loaded / so: 128 new requests x 8 heads of 128 x 128 35.6 / 22.1, x 16 60.2 / 37.6, 32 x 16 17.3 / 14.0; 128 that are not
-  // new x 8 35.3 / 32.3, 8 requests x 8 8.2 / 7.2 (the same loads, with fewer conditions at each); 32 requests of 3 tokens x 16 22.2 / 23.0.
-  if constexpr (R <= 16) {
-    const bool leave = gridDim.x * gridDim.y > 256 && fresh;
+  // Of large states with more than a workgroup a compute unit bytes count for more than the wait for the position, and a new request's are
+  // left alone.  us, always loaded / so: 128 new requests x 8 heads of 128 x 128 36.2 / 21.9, x 16 59.6 / 37.1, 32 x 16 17.2 / 13.8; 128 that
+  // are not new x 8 36.2 / 32.6, 8 requests x 8 8.1 / 7.1 (the same loads, in a branch); 32 requests of 3 tokens x 16 22.4 / 22.8.
+  if constexpr (R == 16) {
+    bool leave = false;
+    if (gridDim.x * gridDim.y > 256) {
+      int first = first_pos;
+      asm volatile("" : "+s"(first));             // (waited for here only)
+      leave = first == 0;
+    }
     if (leave) {
 #pragma unroll
       for (int j = 0; j < R; ++j) S[j] = 0.f;
@@ -73,6 +78,9 @@ __global__ __launch_bounds__(NT) void decay_state_kernel(
 #pragma unroll
       for (int j = 0; j < R; ++j) S[j] = j < count ? st[(long)(dg + j * NG) * E + e] : 0.f;
     }
+  } else if constexpr (R < 16) {
+#pragma unroll
+    for (int j = 0; j < R; ++j) S[j] = j < count ? st[(long)(dg + j * NG) * E + e] : 0.f;
   } else {
 #pragma unroll
     for (int j = 0; j < R; ++j) S[j] = (j < count && !fresh) ? st[(long)(dg + j * NG) * E + e] : 0.f;

@@ -326,7 +326,7 @@ def test_decaying_state_whole_in_portions_and_slots_used_again(dtype, H, D, E):
 
 @pytest.mark.parametrize("H,D,E,n_req", [(2, 16, 24, 128), (2, 16, 24, 129), (3, 64, 64, 86), (2, 128, 128, 129), (1, 256, 128, 257)])
 def test_many_requests_have_the_bits_of_a_few_at_a_time(H, D, E, n_req):
-    """Beyond 256 workgroups a new request's state is not read at all: slots that hold NaN, every third request new, one and three
+    """Beyond 256 workgroups a new request's large state is not read at all: slots that hold NaN, every third request new, one and three
     tokens, against the same requests 16 at a time."""
     g = torch.Generator().manual_seed(n_req)
     lens = [3 if r % 5 == 4 else 1 for r in range(n_req)]

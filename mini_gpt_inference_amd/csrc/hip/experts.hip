@@ -934,7 +934,11 @@ extern "C" int mgpt_grouped_few_rows(const void* a, long lda, const int* a_rows,
   // 10.8 / 8.9, 5440 -> 1024 17.1 / 13.0; experts gated 2048 -> 2048 of 8 tiles 30.5 / 29.2, of 4 17.3 / 17.3, of 1 9.2 / 8.4; without a unit of
   // 2 tiles 8.6 / 7.7, of 4 10.6 / 10.5, of 8 16.6 / 17.2; 1024 -> 512 of 8 4.75 / 4.50, of 16 6.5 / 6.6; 4096 -> 1024 of 2 12.6 / 9.6).
   const long groups = (long)((n_out + 15) / 16) * n_tiles;
-  const bool two = k_dim > 2048 || (kind >= 0 ? tile_expert && k_dim >= 2048 : k_dim >= 512 && groups <= (k_dim > 1024 ? 512 : 256));
+  // Five and six whole steps are one for some waves and two for others, and room for two costs no workgroup without a unit (32 tiles 328 ->
+  // 1248 11.0 / 9.7, 8 of 384 -> 2624 6.86 / 6.45, 1 of 320 -> 11248 4.61 / 4.38; with seven 4 tiles 448 -> 3136 5.9 / 6.4).
+  const bool two = k_dim > 2048 || (kind >= 0 ? tile_expert && k_dim >= 2048
+                                              : (k_dim >= 5 * EX_STEP && k_dim < 7 * EX_STEP) ||
+                                                    (k_dim >= 512 && groups <= (k_dim > 1024 ? 512 : 256)));
 #define GF_LAUNCH(OT, G)                                                                                              \
   do {                                                                                                                \
     if (two) GF_LAUNCH_AS(OT, G, 2);                                                                                  \

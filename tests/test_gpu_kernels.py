@@ -470,7 +470,7 @@ def test_which_float32_products_norm_their_rows(n, o, k, norms):
 
 
 @pytest.mark.parametrize("n,k,o", [(1, 64, 16), (8, 768, 8192), (9, 1030 // 8 * 8, 8200), (12, 2048, 8193), (16, 40, 33), (3, 4096, 100), (16, 320, 48),
-                                   (16, 8, 40), (16, 56, 20), (5, 2120, 50), (16, 2744, 33)])
+                                   (16, 8, 40), (16, 56, 20), (5, 2120, 50), (16, 2744, 33), (7, 312, 40), (16, 328, 20), (3, 440, 33), (2, 504, 17)])
 @pytest.mark.parametrize("o_dt", ["float32", "bfloat16"])
 def test_linear_rows_once(n, k, o, o_dt):
     """A pass over the matrix for up to 16 rows: one stage and two, inner sizes that are no whole steps, ragged columns."""

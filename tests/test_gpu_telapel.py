@@ -588,7 +588,7 @@ UNITS = {"silu": lambda g, u: g * P.sigmoid(g) * u, "relu": lambda g, u: torch.c
 
 @pytest.mark.parametrize("activation", sorted(UNITS))
 @pytest.mark.parametrize("n,width,hidden", [(1, 64, 48), (5, 40, 37), (16, 2048, 1360), (7, 520, 16), (3, 1000, 100), (4, 8, 20),
-                                            (3, 2120, 70), (16, 2744, 48), (2, 4096, 33)])
+                                            (3, 2120, 70), (16, 2744, 48), (2, 4096, 33), (5, 384, 40), (6, 392, 24), (16, 504, 33)])
 def test_gated_products_of_few_rows_with_their_unit(activation, n, width, hidden):
     """One matrix pair for all rows, and pairs of four experts in tiles of 16 slots, gathered and in order; inner sizes with
     and without a rest of less than 32, shorter than a step, and long ones with two steps on their way, not the same number for every

@@ -40,18 +40,19 @@ static bf16_t* ends_at_a_page(size_t values) {
   if (at == MAP_FAILED || mprotect(at + pages, page, PROT_NONE)) exit(3);
   return (bf16_t*)(at + pages - bytes);
 }
-template <bool GATED, int STAGES> void walk(int k, int rows, int o) {
+template <bool GATED, int STAGES, bool REST> void walk(int k, int rows, int o) {
   const bf16_t *a = ends_at_a_page((size_t)rows * k), *w = ends_at_a_page((size_t)(GATED ? 2 : 1) * o * k);
   float out[1];
   for (blockIdx.x = 0; blockIdx.x < (o + 15) / 16; ++blockIdx.x)
     for (threadIdx.x = 0; threadIdx.x < 256; ++threadIdx.x)
       try {
-        grouped_few_rows_kernel<float, GATED, STAGES>(a, k, nullptr, w, 0, nullptr, nullptr, out, o, nullptr, rows, o, k, 0, GATED ? 0 : -1, 0.f, 0.f);
+        grouped_few_rows_kernel<float, GATED, STAGES, REST>(a, k, nullptr, w, 0, nullptr, nullptr, out, o, nullptr, rows, o, k, 0, GATED ? 0 : -1, 0.f, 0.f);
       } catch (Met) {}
 }
 int main(int, char** argv) {
   const int k = atoi(argv[1]), rows = atoi(argv[2]), o = atoi(argv[3]);
-  walk<true, 1>(k, rows, o), walk<true, 2>(k, rows, o), walk<false, 1>(k, rows, o), walk<false, 2>(k, rows, o);
+  walk<true, 1, false>(k, rows, o), walk<true, 2, false>(k, rows, o), walk<false, 1, false>(k, rows, o), walk<false, 2, false>(k, rows, o);
+  walk<true, 1, true>(k, rows, o), walk<false, 1, true>(k, rows, o), walk<false, 2, true>(k, rows, o);
 }
 """
 
@@ -60,7 +61,7 @@ int main(int, char** argv) {
 def walk(tmp_path_factory):
     with open(os.path.join(build.HIP_DIR, "experts.hip"), encoding="utf-8") as fh:
         source = fh.read()
-    kernel = re.search(r"template <typename OT, bool GATED, int STAGES>\n__global__.*?\n}\n", source, re.S).group()
+    kernel = re.search(r"template <typename OT, bool GATED, int STAGES, bool REST>\n__global__.*?\n}\n", source, re.S).group()
     step = re.search(r"#define EX_STEP (\d+)", source).group(1)
     text = PROGRAM.replace("STEP_OF_THE_SOURCE", step).replace("KERNEL_OF_THE_SOURCE", re.sub(r"asm volatile\([^;]*\);", ";", kernel))
     folder = tmp_path_factory.mktemp("walk")
